@@ -10,6 +10,7 @@
 // order (two-stage, partials then an ordered sum), so results are bitwise
 // reproducible run to run.
 #include "mpc_internal.hpp"
+#include <algorithm>
 
 namespace {
 
@@ -18,7 +19,7 @@ constexpr int RB = 256;          // rows per workgroup
 // ---------------------------------------------------------------- SYMV
 // y = A x for symmetric A reading only the upper triangle (i <= j) of the
 // column-major FP32 (or FP64) matrix: half the HBM traffic of a full GEMV.
-// One workgroup per SY_E x SY_E super-tile (I <= J) of SY_S x SY_S tiles of
+// One workgroup per E x E super-tile (I <= J, E = 64 S) of S x S tiles of
 // 64, walked tile by tile through LDS (the next tile's loads are in flight
 // while the current one is summed).  Waves 0-1 form row sums (A_IJ x_J: lane
 // = row, wave = half of the tile's columns), waves 2-3 column sums
@@ -29,22 +30,25 @@ constexpr int RB = 256;          // rows per workgroup
 //                   column-sum partial of super-tile (L, K)
 // (a diagonal super-tile writes its row and column sums as one partial), and
 // symv_reduce adds P[K][0..nst) in order (deterministic).  The partials take
-// nst^2 SY_E SJ doubles, SJ <= 8 right-hand sides per pass: n^2 SJ / 32
-// bytes, 1/128 of the FP32 matrix per right-hand side; more right-hand sides
-// than 8 run in passes of 8 over the same buffer.
+// nst^2 E NJ doubles, NJ <= 4 right-hand sides per pass (at n = 16384, S = 4,
+// one right-hand side: 1/64 of the bytes read from A).  More than four
+// right-hand sides go through the matrix cores in passes of 16 over the whole
+// matrix (k_mrhs.hip): twice the bytes, but the FMAs here read x from LDS per
+// element and right-hand side and so cost more than the bytes (n = 8192: 48 us
+// for 4, where 16 take 62 there; n = 6000: 34 and 53).
 constexpr int SY_T = 64;
-constexpr int SY_S = 4;
-constexpr int SY_E = SY_T * SY_S;
-constexpr int SY_JMAX = 8;
-template <typename T> struct vec16 { using type = float4; };
-template <> struct vec16<double> { using type = double2; };
+constexpr int SY_JMAX = 4;
+// 16-byte loads of columns that are aligned to their elements only (an odd
+// leading dimension): global loads need no more than 4-byte alignment
+template <typename T> struct vec16 { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct vec16<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
 
-template <typename T, int NJ>
+template <typename T, int NJ, int S>
 __global__ __launch_bounds__(256) void symv_super_kernel(const T* __restrict__ A, int64_t lda,
                                                         int64_t n, int nst, int j0, int nj,
                                                         const double* __restrict__ X, int64_t ldx,
                                                         double* __restrict__ P) {
-    constexpr int ST = SY_T, S = SY_S, E = SY_E;
+    constexpr int ST = SY_T, E = SY_T * S;
     using V16 = typename vec16<T>::type;
     constexpr int VE = 16 / (int)sizeof(T);        // elements per 16-byte load
     constexpr int RV = ST / VE;                     // loads per tile column
@@ -77,12 +81,11 @@ __global__ __launch_bounds__(256) void symv_super_kernel(const T* __restrict__ A
         xc[j][k] = (!diag && j < nj && C0 + k < n) ? vc : 0.0;
     }
     const double* xcol = diag ? &xr[0][0] : &xc[0][0];
-    const bool fast_ok = lda % VE == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
     const int q = tid % RV, cq = tid / RV;
     V16 v[NP];
     auto load_tile = [&](int a, int b) {
         const int64_t r0 = R0 + a * ST, c0 = C0 + b * ST;
-        if (fast_ok && r0 + ST <= n && c0 + ST <= n) {
+        if (r0 + ST <= n && c0 + ST <= n) {
 #pragma unroll
             for (int p = 0; p < NP; ++p)
                 v[p] = *reinterpret_cast<const V16*>(A + r0 + VE * q + (c0 + p * CPP + cq) * lda);
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(256) void symv_super_kernel(const T* __restrict__ A
 // super-tiles [w q, (w+1) q), q = ceil(nst / 4), in batches of 16
 // independent loads (clamped index, zero weight past the end) in order; the
 // four quarter sums are then added in order.
-__global__ __launch_bounds__(256) void symv_reduce_kernel(int64_t n, int nst, int NJ, int j0,
+__global__ __launch_bounds__(256) void symv_reduce_kernel(int64_t n, int E, int nst, int NJ, int j0,
                                                          const double* __restrict__ P,
                                                          double* __restrict__ Y, int64_t ldy) {
     __shared__ double red[4][64];
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(256) void symv_reduce_kernel(int64_t n, int nst, in
     const int64_t row0 = (int64_t)blockIdx.x * 64 + lane;
     const int64_t row = row0 < n ? row0 : n - 1;
     const int j = blockIdx.y;
-    const int64_t K = row / SY_E, r = row % SY_E;
+    const int64_t K = row / E, r = row % E;
     const int q = (nst + 3) / 4, l0 = w * q, l1 = l0 + q < nst ? l0 + q : nst;
     double s = 0.0;
     for (int L0 = l0; L0 < l1; L0 += 16) {
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(256) void symv_reduce_kernel(int64_t n, int nst, in
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             const int64_t L = L0 + u < l1 ? L0 + u : l1 - 1;
-            v[u] = P[((K * nst + L) * NJ + j) * SY_E + r];
+            v[u] = P[((K * nst + L) * NJ + j) * E + r];
         }
 #pragma unroll
         for (int u = 0; u < 16; ++u) s += L0 + u < l1 ? v[u] : 0.0;
@@ -523,34 +526,58 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + RB - 1) / RB); }
 
 }  // namespace
 
-// per pass of at most SY_JMAX right-hand sides
+// right-hand sides of the next pass: at most SY_JMAX (padded to 1, 2 or 4) with
+// the symmetric kernel, at most MPC_MM_NJ as a product with the whole matrix
 static int symv_pass_rhs(int nrhs) {
-    return nrhs <= 1 ? 1 : nrhs <= 2 ? 2 : nrhs <= 4 ? 4 : SY_JMAX;
+    return nrhs > SY_JMAX ? std::min(nrhs, MPC_MM_NJ) : nrhs <= 1 ? 1 : nrhs <= 2 ? 2 : SY_JMAX;
 }
+// Tiles per super-tile side: small matrices need the workgroups (n = 777, one
+// right-hand side: 8.7 / 10.5 / 20 us with 1 / 2 / 4; n = 3001: 11.8 / 13.9 /
+// 25), large ones the fewer partial sums (n = 6000: 25.6 / 25.1 / 27.7, 12000:
+// 72 / 55 / 62, 16384: 145 / 132 / 121, 36864: 671 / 580 / 540).
+static int symv_tiles(int64_t n) { return n >= 14336 ? 4 : n >= 4608 ? 2 : 1; }
+static int64_t symv_splits(int64_t n) { return mpc_mm_splits(n, n); }
 
 int64_t mpc_symv_partial_doubles(int64_t n, int nrhs) {
-    const int64_t nst = (n + SY_E - 1) / SY_E;
-    return nst * nst * SY_E * symv_pass_rhs(nrhs);
+    const int64_t E = SY_T * symv_tiles(n), nst = (n + E - 1) / E;
+    const int64_t sym = nst * nst * E * (nrhs > 2 ? SY_JMAX : nrhs);
+    return nrhs > SY_JMAX ? std::max(sym, symv_splits(n) * n * std::min(nrhs, MPC_MM_NJ)) : sym;
+}
+
+template <typename T, int S>
+static void launch_symv_pass(hipStream_t st, const T* A, int64_t lda, int64_t n, int NJ, int j0,
+                             int nj, const double* X, int64_t ldx, double* Y, int64_t ldy,
+                             double* part) {
+    const int64_t E = SY_T * S, nst = (n + E - 1) / E;
+    const dim3 g((unsigned)(nst * (nst + 1) / 2)), b(256);
+    switch (NJ) {
+    case 1: hipLaunchKernelGGL((symv_super_kernel<T, 1, S>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
+    case 2: hipLaunchKernelGGL((symv_super_kernel<T, 2, S>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
+    default: hipLaunchKernelGGL((symv_super_kernel<T, SY_JMAX, S>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
+    }
+    hipLaunchKernelGGL(symv_reduce_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)nj), dim3(256), 0,
+                       st, n, (int)E, (int)nst, NJ, j0, part, Y, ldy);
 }
 
 template <typename T>
 static int launch_symv_t(hipStream_t st, const T* A, int64_t lda, int64_t n, int nrhs,
                          const double* X, int64_t ldx, double* Y, int64_t ldy, double* part) {
-    const int64_t nst = (n + SY_E - 1) / SY_E;
-    const int64_t ntile = nst * (nst + 1) / 2;
-    const int NJ = symv_pass_rhs(nrhs);
-    for (int j0 = 0; j0 < nrhs; j0 += NJ) {
-        const int nj = nrhs - j0 < NJ ? nrhs - j0 : NJ;
-        const dim3 g((unsigned)ntile), b(256);
-        switch (NJ) {
-        case 1: hipLaunchKernelGGL((symv_super_kernel<T, 1>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
-        case 2: hipLaunchKernelGGL((symv_super_kernel<T, 2>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
-        case 4: hipLaunchKernelGGL((symv_super_kernel<T, 4>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
-        default: hipLaunchKernelGGL((symv_super_kernel<T, SY_JMAX>), g, b, 0, st, A, lda, n, (int)nst, j0, nj, X, ldx, part); break;
+    for (int j0 = 0; j0 < nrhs;) {
+        const int NJ = symv_pass_rhs(nrhs - j0), nj = std::min(nrhs - j0, NJ);
+        if (NJ > SY_JMAX) {
+            const int64_t S = symv_splits(n);
+            int rc = mpc_launch_mm_n(st, A, lda, n, n, X + j0 * ldx, ldx, nj, part, S);
+            if (!rc) rc = mpc_launch_mm_sum(st, n, nj, n, S, part, nullptr, 0, 1.0, Y + j0 * ldy, ldy);
+            if (rc) return rc;
+        } else {
+            switch (symv_tiles(n)) {
+            case 1: launch_symv_pass<T, 1>(st, A, lda, n, NJ, j0, nj, X, ldx, Y, ldy, part); break;
+            case 2: launch_symv_pass<T, 2>(st, A, lda, n, NJ, j0, nj, X, ldx, Y, ldy, part); break;
+            default: launch_symv_pass<T, 4>(st, A, lda, n, NJ, j0, nj, X, ldx, Y, ldy, part); break;
+            }
+            MPC_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(symv_reduce_kernel, dim3((unsigned)((n + 63) / 64), (unsigned)nj), dim3(256),
-                           0, st, n, (int)nst, NJ, j0, part, Y, ldy);
-        MPC_LAUNCH_CHECK();
+        j0 += nj;
     }
     return 0;
 }

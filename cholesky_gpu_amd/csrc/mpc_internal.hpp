@@ -255,6 +255,19 @@ int mpc_launch_syrk_classes(hipStream_t st, float* C, int64_t m, int64_t ldc, in
 // compute classes / FP8 element formats that a factor configuration can produce
 void mpc_syrk_masks(int update_prec, const int* ladder, int n_ladder, unsigned* class_mask,
                     unsigned* fp8_mask);
+// k_mrhs.hip: products with up to MPC_MM_NJ right-hand sides X (nj columns,
+// ld ldx), as partial sums over S column chunks, and their sum
+constexpr int MPC_MM_NJ = 16;
+constexpr int MPC_MM_GROUP_N = 16;                           // chunk granularity
+int64_t mpc_mm_splits(int64_t rows, int64_t kc);             // chunks that fill the chip
+// part[(s nj + j) m + r] = sum over chunk s of A[r][c] X[j][c]
+int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc,
+                    const double* X, int64_t ldx, int nj, double* part, int64_t S);
+int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc,
+                    const double* X, int64_t ldx, int nj, double* part, int64_t S);
+// Y[j][r] = (B ? B[j][r] : 0) + a sum_s part[(s nj + j) m + r]
+int mpc_launch_mm_sum(hipStream_t st, int64_t m, int nj, int64_t kc, int64_t S,
+                      const double* part, const double* B, int64_t ldb, double a, double* Y, int64_t ldy);
 // k_pcg.hip
 int mpc_launch_symv(hipStream_t st, const float* A, int64_t lda, int64_t n, int nrhs,
                     const double* X, int64_t ldx, double* Y, int64_t ldy, double* part);

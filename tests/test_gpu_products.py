@@ -1,0 +1,39 @@
+"""GPU tests of the products with blocks of right-hand sides (libmpchol through
+the C ABI) at the edges of their tiles, chunks and passes."""
+import numpy as np
+import pytest
+import torch
+
+from cholesky_gpu_amd import _lib as L
+from cholesky_gpu_amd import solver as S
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[case]", *a, flush=True)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 1000, 4609, 14337])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 5, 16, 21])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_symmetric_product(handle, n, nrhs, dtype):
+    """The operator's product A X, read off the true residual of a PCG that
+    starts at X and takes no step (B the exact product to FP64, L = I): an
+    FP64 sum of n exact products is within n u |A| |X| of it, and B too."""
+    say("product", n, nrhs, dtype)
+    if n > 10000 and (nrhs in (2, 3, 21) or dtype is torch.float64):
+        pytest.skip("one large size per kernel is enough")
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn(n, n, generator=g, device="cuda", dtype=torch.float32).to(dtype)
+    A = torch.tril(A) + torch.tril(A, -1).T.contiguous()
+    X = torch.randn(nrhs, n, generator=g, device="cuda", dtype=torch.float64)
+    Xt = X.T.contiguous()
+    rows = [A[r:r + 2048].to(torch.float64) for r in range(0, n, 2048)]
+    B = torch.cat([R @ Xt for R in rows]).T.contiguous()
+    mag = torch.cat([R.abs() @ Xt.abs() for R in rows]).T
+    bound = float((2 * n * 2.0 ** -53 * mag.norm(dim=1) / B.norm(dim=1)).max())
+    eye = torch.eye(n, device="cuda", dtype=torch.float32)
+    f = S.pcg if dtype is torch.float32 else S.pcg64
+    _, pi, _ = f(handle, A, eye, B, nb=64, X=X.clone(), opts=S.pcg_opts(x0_mode=2, maxit=0))
+    assert pi.relres <= bound, (pi.relres, bound)
