@@ -5,10 +5,12 @@
 // D = a b with a[m][k] = the right-hand sides (m) and b[k][n] = the matrix.
 // Lane (q, k) = (lane % 16, lane / 16) of a wave supplies a[q][k], b[k][q] and
 // receives in register e the element D[4e + k][q].
-// Rows of the matrix are the outputs: a lane loads rows 4q .. 4q+3 of
-// one column, 16 bytes, so 16 lanes read a 256-byte column segment, and
-// its element i is the operand of the product whose n stands for row
-// 4n + i: no transpose and no LDS.
+//   mm_n (rows of the matrix are the outputs): a lane loads rows 4q .. 4q+3 of
+//     one column, 16 bytes, so 16 lanes read a 256-byte column segment, and
+//     its element i is the operand of the product whose n stands for row
+//     4n + i: no transpose and no LDS.
+//   mm_t (columns are the outputs): lane (q, k) loads rows 4k .. 4k+3 of
+//     column q; element i is the operand with k <-> row 4k + i.
 // The right-hand sides are read as operands straight from L2.  Per 8 KB of an
 // FP32 matrix a wave issues 32 products of 64 cycles, 9.8 TB/s over 1024 SIMDs:
 // above what HBM delivers.  With 16 right-hand sides (A X, FP32 A) n = 8192
@@ -21,17 +23,29 @@ namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
-constexpr int MR = 64;          // output rows of a workgroup
+constexpr int MR = 64;          // output rows of a workgroup (mm_n)
 constexpr int MU = 4;           // columns of a group per lane (8: two waves per SIMD
                                 // instead of three, 5-15 % slower)
 constexpr int MG = MPC_MM_GROUP_N;      // columns of a group
 static_assert(MG == 4 * MU, "group");
+constexpr int MFL = 8;          // groups per partial sum of a wave
+constexpr int MTC = 32;         // output columns of a workgroup (mm_t)
+constexpr int MTG = MPC_MM_GROUP_T;     // rows of a group (mm_t)
+
+// which column chunks [s cw, (s+1) cw) have work for row block r0 (mode 1:
+// lower triangle, columns up to the row; 2: upper, columns from the row on)
+__device__ __forceinline__ void split_range(int mode, int64_t r0, int64_t rows, int64_t cw, int S,
+                                            int& s0, int& s1) {
+    s0 = mode == 2 ? (int)(r0 / cw) : 0;
+    const int64_t last = mode == 1 ? (r0 + rows - 1) / cw + 1 : S;
+    s1 = last < S ? (int)last : S;
+}
 
 // part[(s nj + j) m + r] = sum_{c in chunk s} A[r][c] X[j][c] for the 64 rows of
 // blockIdx.x, chunk s = blockIdx.y of cw columns (a multiple of MG).  Wave w
 // takes the chunk's column groups w, w + 4, ..; the four waves' sums are added
 // in wave order through LDS.
-template <typename T>
+template <typename T, int MODE>
 __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int64_t lda, int64_t m,
                                                   int64_t kc, int64_t cw, const double* __restrict__ X,
                                                   int64_t ldx, int nj, double* __restrict__ part) {
@@ -40,7 +54,11 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane & 15, k = lane >> 4;
     const int64_t r0 = (int64_t)blockIdx.x * MR, cs = (int64_t)blockIdx.y * cw;
-    const int64_t ce = cs + cw < kc ? cs + cw : kc;
+    int64_t ce = cs + cw < kc ? cs + cw : kc;
+    if (MODE == 1 && ce > r0 + MR) ce = r0 + MR < kc ? r0 + MR : kc;
+    int64_t cb = cs;
+    if (MODE == 2 && cb < r0) cb = r0 & ~(int64_t)(MG - 1);
+    if (cb >= ce) return;                        // (the sum skips this chunk)
     const double* __restrict__ Xj = X + (int64_t)(q < nj ? q : nj - 1) * ldx;
     const int64_t r = r0 + 4 * q;
     const bool rfull = r0 + MR <= m;
@@ -70,13 +88,28 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
                 x[s] = c + s < kc ? y : 0.0;
             }
         }
-    };
-    v4d acc[4];
+        if (MODE == 1 && c0 + MG > r0) {         // zeros above the diagonal
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = v4d{};
-    int64_t c0 = cs + MG * wave;
+            for (int s = 0; s < MU; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[s][i] = c + s <= r + i ? v[s][i] : T(0);
+        }
+        if (MODE == 2 && c0 < r0 + MR) {         // zeros below the diagonal
+#pragma unroll
+            for (int s = 0; s < MU; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[s][i] = c + s >= r + i ? v[s][i] : T(0);
+        }
+    };
+    // Sums of MFL groups (128 terms) are added up apart: one running sum over
+    // the chunk loses accuracy with its length, which a residual at cond 1e8
+    // shows (n = 65536: 8192 terms a wave).
+    v4d acc[4], tot[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = tot[i] = v4d{};
+    int64_t c0 = cb + MG * wave;
     if (c0 < ce) load(c0);
-    for (; c0 < ce; c0 += 4 * MG) {
+    for (int g = 1; c0 < ce; c0 += 4 * MG, ++g) {
         vec4 w[MU];
         double y[MU];
 #pragma unroll
@@ -90,7 +123,16 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[s], (double)w[s][i], acc[i], 0, 0, 0);
+        if (g % MFL == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                tot[i] += acc[i];
+                acc[i] = v4d{};
+            }
+        }
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += tot[i];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -107,40 +149,136 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
     }
 }
 
+// part[(s nj + j) nc + c] = sum_{r in chunk s} A[r][c] X[j][r] for the 32
+// columns of blockIdx.x, chunk s = blockIdx.y of rw rows (a multiple of MTG).
+// Wave w takes the chunk's row groups w, w + 4, ..
+__global__ __launch_bounds__(256) void mm_t_kernel(const float* __restrict__ A, int64_t lda,
+                                                  int64_t m, int64_t nc, int64_t rw,
+                                                  const double* __restrict__ X, int64_t ldx, int nj,
+                                                  double* __restrict__ part) {
+    typedef float vec4 __attribute__((ext_vector_type(4), aligned(4)));
+    __shared__ double red[4][MPC_MM_NJ][MTC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int q = lane & 15, k = lane >> 4;
+    const int64_t c0 = (int64_t)blockIdx.x * MTC, rs = (int64_t)blockIdx.y * rw;
+    const int64_t re = rs + rw < m ? rs + rw : m;
+    const double* __restrict__ Xj = X + (int64_t)(q < nj ? q : nj - 1) * ldx;
+    const float* __restrict__ col[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        const int64_t c = c0 + 16 * g + q;
+        col[g] = A + (c < nc ? c : nc - 1) * lda;    // (sums of a column past the end are dropped)
+    }
+    vec4 v[2][4];
+    double x[16];
+    auto load = [&](int64_t r0) {
+        const int64_t r = r0 + 4 * k;
+        if (r0 + MTG <= m) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) v[g][u] = *reinterpret_cast<const vec4*>(col[g] + r + 16 * u);
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const d2 y = *reinterpret_cast<const d2*>(Xj + r + 16 * u + i);
+                    x[4 * u + i] = y[0];
+                    x[4 * u + i + 1] = y[1];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int64_t rr = r + 16 * u + i, rc = rr < m ? rr : m - 1;
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) {
+                        const float y = col[g][rc];
+                        v[g][u][i] = rr < m ? y : 0.f;
+                    }
+                    const double y = Xj[rc];
+                    x[4 * u + i] = rr < m ? y : 0.0;
+                }
+        }
+    };
+    v4d acc[2][2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) acc[g][0] = acc[g][1] = v4d{};
+    int64_t r0 = rs + MTG * wave;
+    if (r0 < re) load(r0);
+    for (; r0 < re; r0 += 4 * MTG) {
+        vec4 w[2][4];
+        double y[16];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g) w[g][u] = v[g][u];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[4 * u + i] = x[4 * u + i];
+        }
+        if (r0 + 4 * MTG < re) load(r0 + 4 * MTG);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+                    acc[g][i & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[4 * u + i], (double)w[g][u][i],
+                                                                         acc[g][i & 1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave][4 * e + k][16 * g + q] = acc[g][0][e] + acc[g][1][e];
+    __syncthreads();
+    const int c = tid & 31;
+    if (c0 + c < nc) {
+#pragma unroll
+        for (int j = tid >> 5; j < MPC_MM_NJ; j += 8)
+            if (j < nj)
+                part[((int64_t)blockIdx.y * nj + j) * nc + c0 + c] =
+                    ((red[0][j][c] + red[1][j][c]) + red[2][j][c]) + red[3][j][c];
+    }
+}
+
 // Y[j][r] = (B ? B[j][r] : 0) + a sum_s part[(s nj + j) m + r], chunks in order;
 // thread = row, 8 loads in flight (clamped chunk, zero weight past the end)
-__global__ __launch_bounds__(256) void mm_sum_kernel(int64_t m, int S,
+__global__ __launch_bounds__(256) void mm_sum_kernel(int64_t m, int S, int mode, int64_t cw,
                                                     const double* __restrict__ part,
                                                     const double* __restrict__ B, int64_t ldb,
                                                     double a, double* __restrict__ Y, int64_t ldy) {
     const int64_t r0 = (int64_t)blockIdx.x * 256 + threadIdx.x, r = r0 < m ? r0 : m - 1;
     const int j = blockIdx.y, nj = gridDim.y;
+    int s0 = 0, s1 = S;
+    if (mode) split_range(mode, r & ~(int64_t)(MR - 1), MR, cw, S, s0, s1);
     double sum = 0.0;
-    for (int s = 0; s < S; s += 8) {
+    for (int s = s0; s < s1; s += 8) {
         double v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            v[u] = part[((int64_t)(s + u < S ? s + u : S - 1) * nj + j) * m + r];
+            v[u] = part[((int64_t)(s + u < s1 ? s + u : s1 - 1) * nj + j) * m + r];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) sum += s + u < S ? v[u] : 0.0;
+        for (int u = 0; u < 8; ++u) sum += s + u < s1 ? v[u] : 0.0;
     }
     if (r0 < m) Y[j * ldy + r] = B ? fma(a, sum, B[j * ldb + r]) : a * sum;
 }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // columns of a chunk when kc columns are split S ways (whole groups)
-inline int64_t chunk(int64_t kc, int64_t S) { return cdiv(cdiv(kc, S), MG) * MG; }
+inline int64_t chunk(int64_t kc, int64_t S, int64_t unit) { return cdiv(cdiv(kc, S), unit) * unit; }
 
 template <typename T>
-int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc,
+int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc, int mode,
                 const double* X, int64_t ldx, int nj, double* part, int64_t S) {
     if (nj < 1 || nj > MPC_MM_NJ || S < 1) {
         mpc_set_error("mm_n: %d right-hand sides, %lld chunks", nj, (long long)S);
         return MPC_ERR_ARG;
     }
-    const int64_t cw = chunk(kc, S);
+    const int64_t cw = chunk(kc, S, MG);
     const dim3 g((unsigned)cdiv(m, MR), (unsigned)cdiv(kc, cw)), b(256);
-    hipLaunchKernelGGL(mm_n_kernel<T>, g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
+    if (mode == 1) hipLaunchKernelGGL((mm_n_kernel<T, 1>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
+    else if (mode == 2) hipLaunchKernelGGL((mm_n_kernel<T, 2>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
+    else hipLaunchKernelGGL((mm_n_kernel<T, 0>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     MPC_LAUNCH_CHECK();
     return 0;
 }
@@ -150,25 +288,40 @@ int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc,
 // Enough chunks for about 2048 workgroups, each wave of which has a column
 // group.  768 run at once, so fewer leave a last wave nearly empty (16
 // columns: n = 6000 67 us with 1024 workgroups, 53 with 2048, 54 with 4096;
-// n = 8192 60, 62, 68), and every chunk costs a partial sum per output.
+// n = 8192 60, 62, 68), and every chunk costs a partial sum per output.  At
+// most 8192 columns a chunk (see MFL).
 int64_t mpc_mm_splits(int64_t rows, int64_t kc) {
-    const int64_t want = cdiv(2048, cdiv(rows, MR)), most = cdiv(kc, 4 * MG);
+    const int64_t want = std::max(cdiv(2048, cdiv(rows, MR)), cdiv(kc, 8192)), most = cdiv(kc, 4 * MG);
     return std::max<int64_t>(1, std::min(want, most));
 }
 
-int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc,
+int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc, int mode,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S) {
-    return launch_mm_n<float>(st, A, lda, m, kc, X, ldx, nj, part, S);
+    return launch_mm_n<float>(st, A, lda, m, kc, mode, X, ldx, nj, part, S);
 }
-int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc,
+int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc, int mode,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S) {
-    return launch_mm_n<double>(st, A, lda, m, kc, X, ldx, nj, part, S);
+    return launch_mm_n<double>(st, A, lda, m, kc, mode, X, ldx, nj, part, S);
 }
 
-int mpc_launch_mm_sum(hipStream_t st, int64_t m, int nj, int64_t kc, int64_t S,
+int mpc_launch_mm_t(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t nc,
+                    const double* X, int64_t ldx, int nj, double* part, int64_t S) {
+    if (nj < 1 || nj > MPC_MM_NJ || S < 1) {
+        mpc_set_error("mm_t: %d right-hand sides, %lld chunks", nj, (long long)S);
+        return MPC_ERR_ARG;
+    }
+    const int64_t rw = chunk(m, S, MTG);
+    hipLaunchKernelGGL(mm_t_kernel, dim3((unsigned)cdiv(nc, MTC), (unsigned)cdiv(m, rw)), dim3(256), 0,
+                       st, A, lda, m, nc, rw, X, ldx, nj, part);
+    MPC_LAUNCH_CHECK();
+    return 0;
+}
+
+int mpc_launch_mm_sum(hipStream_t st, int64_t m, int nj, int64_t kc, int64_t S, int mode, int unit,
                       const double* part, const double* B, int64_t ldb, double a, double* Y, int64_t ldy) {
+    const int64_t cw = chunk(kc, S, unit);
     hipLaunchKernelGGL(mm_sum_kernel, dim3((unsigned)cdiv(m, 256), (unsigned)nj), dim3(256), 0, st, m,
-                       (int)cdiv(kc, chunk(kc, S)), part, B, ldb, a, Y, ldy);
+                       (int)cdiv(kc, cw), mode, cw, part, B, ldb, a, Y, ldy);
     MPC_LAUNCH_CHECK();
     return 0;
 }

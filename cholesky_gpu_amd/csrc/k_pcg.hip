@@ -566,8 +566,8 @@ static int launch_symv_t(hipStream_t st, const T* A, int64_t lda, int64_t n, int
         const int NJ = symv_pass_rhs(nrhs - j0), nj = std::min(nrhs - j0, NJ);
         if (NJ > SY_JMAX) {
             const int64_t S = symv_splits(n);
-            int rc = mpc_launch_mm_n(st, A, lda, n, n, X + j0 * ldx, ldx, nj, part, S);
-            if (!rc) rc = mpc_launch_mm_sum(st, n, nj, n, S, part, nullptr, 0, 1.0, Y + j0 * ldy, ldy);
+            int rc = mpc_launch_mm_n(st, A, lda, n, n, 0, X + j0 * ldx, ldx, nj, part, S);
+            if (!rc) rc = mpc_launch_mm_sum(st, n, nj, n, S, 0, MPC_MM_GROUP_N, part, nullptr, 0, 1.0, Y + j0 * ldy, ldy);
             if (rc) return rc;
         } else {
             switch (symv_tiles(n)) {

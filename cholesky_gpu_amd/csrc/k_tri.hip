@@ -14,25 +14,122 @@
 // inside.  Winv_I is built by recursive doubling from the 32x32 inverses the
 // POTRF kernel leaves behind:
 //   [A 0; B C]^{-1} = [A^-1 0; -C^-1 B A^-1  C^-1]
-// with a batched FP32 MFMA GEMM (v_mfma_f32_32x32x2f32) that skips the zero
-// triangles of A^-1 and C^-1.  The temporary B A^-1 lives in the unused upper
-// triangle of the Winv block.
+// with a batched GEMM on the matrix cores that skips the zero triangles of
+// A^-1 and C^-1.  The temporary B A^-1 lives in the unused upper triangle of
+// the Winv block.
 #include "mpc_internal.hpp"
 #include <algorithm>
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
+// ---------------------------------------------------------------- block inverses
+// The products of the build are FP32 operands with FP64 sums
+// (v_mfma_f64_16x16x4), rounded to FP32 once when stored: the rounding errors
+// of FP32 sums grow with the block (z of a 2048-point RBF factor is then off
+// by 1.5e-7 with Bo = 256 and 7e-7 with Bo = 2048; with FP64 sums 7e-8 for
+// every Bo).  D = a b: lane (q, k) = (lane % 16, lane / 16) supplies a[q][k] and
+// b[k][q]; its register e is D[4e + k][q].
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
-// ---------------------------------------------------------------- batched GEMM
-// For batch (q, I) and an output tile (T x T at m0, n0):
-//   C[m][n] = alpha * sum_k A[m][k] B[k][n]    (column-major, ld per operand)
-// a_lower: A[m][k] = 0 for k > m; b_lower: B[k][n] = 0 for k < n.  Both are
-// applied per element while staging (the strict upper parts of inverse
-// blocks hold temporaries of the previous doubling level) and per tile when
-// choosing the K range.  Batch b = blockIdx.z = I * nq + q.
+// The 128 x 128 diagonal blocks of the inverse (both W and W^T): the 32 x 32
+// inverses and the two doubling levels above them, in LDS.  One workgroup per
+// block, wave w = one 16 x 16 quadrant of every 32 x 32 product.  Rows and
+// columns beyond n are the identity's.  The products run from short loops
+// (20 us; 24 as straight-line code, each line of which is fetched once).
+constexpr int LF = 128;
+constexpr int LFD = LF + 1;
+__global__ __launch_bounds__(256) void winv_leaf_kernel(const float* __restrict__ L, int64_t ldl,
+                                                       const float* __restrict__ dinv, int64_t n,
+                                                       int Bo, float* __restrict__ W,
+                                                       float* __restrict__ WT, int64_t b0) {
+    // column-major: the 32 x 32 inverses on the diagonal, L below them until
+    // the inverse takes its place, temporaries above
+    __shared__ float Ws[LF * LFD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t r0 = (b0 + blockIdx.x) * LF;
+    {
+        const int r = tid & (LF - 1), h = tid >> 7;
+        const int64_t gr = r0 + r < n ? r0 + r : n - 1;
+        const float* Lr = L + gr;
+        const float* dr = dinv + (gr >> 5) * 1024 + (gr & 31);
+#pragma unroll 1
+        for (int c0 = h; c0 < LF; c0 += 64) {
+            float v[32];
+#pragma unroll
+            for (int u = 0; u < 32; ++u) {
+                const int c = c0 + 2 * u;
+                const int64_t gc = r0 + c < n ? r0 + c : n - 1;
+                v[u] = (r >> 5) == (c >> 5) ? dr[(gc & 31) * 32] : Lr[gc * ldl];
+            }
+#pragma unroll
+            for (int u = 0; u < 32; ++u) {
+                const int c = c0 + 2 * u;
+                Ws[r + c * LFD] = (r0 + r < n && r0 + c < n) ? v[u] : (r == c ? 1.f : 0.f);
+            }
+        }
+    }
+    __syncthreads();
+    const int q = lane & 15, k = lane >> 4, qr = 16 * (wave & 1), qc = 16 * (wave >> 1);
+    // block (r, c) = sgn sum_s A(ar, ac + 32 s) B(br + 32 s, bc), s < ns; lane
+    // (q, k)'s register e: row qr + q, column qc + 4e + k (a = B^T, b = A^T)
+    auto product = [&](int ns, int ar, int ac, int br, int bc, int r, int c, double sgn) {
+        v4d acc = v4d{};
+#pragma unroll 1
+        for (int s = 0; s < ns; ++s) {
+            float x[8], y[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                x[t] = Ws[ar + qr + q + (ac + 32 * s + 8 * k + t) * LFD];
+                y[t] = Ws[br + 32 * s + 8 * k + t + (bc + qc + q) * LFD];
+            }
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)y[t], (double)x[t], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Ws[r + qr + q + (c + qc + 4 * e + k) * LFD] = (float)(sgn * acc[e]);
+    };
+    // level 32, pairs at p = 0 and 64: T = L21 A^-1 above the diagonal, then
+    // -C^-1 T below it; level 64 the same in 32 x 32 blocks (i, j) of the
+    // 64 x 64 products, whose zero blocks are left out
+#pragma unroll 1
+    for (int p = 0; p < LF; p += 64) product(1, p + 32, p, p, p, p, p + 32, 1.0);
+    __syncthreads();
+#pragma unroll 1
+    for (int p = 0; p < LF; p += 64) product(1, p + 32, p + 32, p, p + 32, p + 32, p, -1.0);
+    __syncthreads();
+#pragma unroll 1
+    for (int o = 0; o < 4; ++o) {
+        const int i = 32 * (o & 1), j = 32 * (o >> 1);
+        product(2 - (o >> 1), 64 + i, j, j, j, i, 64 + j, 1.0);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int o = 0; o < 4; ++o) {
+        const int i = 32 * (o & 1), j = 32 * (o >> 1);
+        product(1 + (o & 1), 64 + i, 64, 0, 64 + j, 64 + i, j, -1.0);
+    }
+    __syncthreads();
+    const int64_t I = r0 / Bo, p = r0 - I * Bo;       // (Bo is a multiple of LF: inside W_I)
+    float* Wi = W + I * (int64_t)Bo * Bo + p + p * Bo;
+    float* Ti = WT + I * (int64_t)Bo * Bo + p + p * Bo;
+    const int r = tid & (LF - 1);
+#pragma unroll 4
+    for (int c = tid >> 7; c < LF; c += 2) {
+        const float v = r >= c ? Ws[r + c * LFD] : Ws[c + r * LFD];
+        (r >= c ? Wi : Ti)[r + (uint32_t)c * (uint32_t)Bo] = v;
+        if (r == c) Ti[r + (uint32_t)c * (uint32_t)Bo] = v;
+    }
+}
+
+// One doubling product for pair q of big block I (batch blockIdx.z = I nq + q):
+//   C[m][n] = alpha sum_k A[m][k] B[k][n]    (column-major, ld per operand)
+// a_lower: A[m][k] = 0 for k > m; b_lower: B[k][n] = 0 for k < n (applied per
+// element while staging, the other triangles hold temporaries, and per tile to
+// the K range).  CT (optional): C^T as well.
 struct gemm_batch {
-    const float* A; const float* B; float* C;
+    const float* A; const float* B; float* C; float* CT;
     int64_t lda, ldb, ldc;
     int64_t sA, sB, sC;          // stride between pairs q (elements)
     int64_t tA, tB, tC;          // stride between big blocks I
@@ -42,121 +139,118 @@ struct gemm_batch {
     int a_lower, b_lower;
 };
 
-template <int T>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(gemm_batch g) {
-    constexpr int WT = T / 2;          // per-wave tile (2 x 2 waves)
-    constexpr int NB = WT / 32;        // 32x32 MFMA blocks per wave side
-    __shared__ float As[32][T + 4];    // As[k][m]
-    __shared__ float Bs[32][T + 4];    // Bs[k][n]
-    const int64_t q = blockIdx.z % g.nq, I = blockIdx.z / g.nq;
-    const float* A = g.A + q * g.sA + I * g.tA;
-    const float* B = g.B + q * g.sB + I * g.tB;
-    float* C = g.C + q * g.sC + I * g.tC;
-    const int m0 = blockIdx.x * T, n0 = blockIdx.y * T;
-    if (m0 >= g.m || n0 >= g.n) return;
+// 32 x 64 tiles, wave w = a 16 x 32 quadrant; 64 K per stage, the next stage's
+// loads in flight during the products (16 steps of two products of 76 cycles).
+// Stages inside the operands' triangles and edges move 16 bytes per load and
+// LDS store: with a masked 4-byte element each, the staging cost more than the
+// products (K = 1024: 50-60 us).  The LDS strides put the 64 lanes of an
+// operand read on 64 banks.  Tiles with the longest K range come first.
+constexpr int GM = 32, GN = 64, GK = 64;
+constexpr int GAS = GM + 16, GBS = GK + 4;
+// T = float (v_mfma_f32_16x16x4: FP32 sums, half the time per product; register
+// e is D[4k + e][q]) for matrices of more than 8192 rows, whose blocks are
+// built beside the factor and compete with it.
+template <typename T>
+__global__ __launch_bounds__(256) void gemm_kernel(gemm_batch g) {
+    typedef T v4 __attribute__((ext_vector_type(4)));
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float As[GK * GAS];   // As[k][m]
+    __shared__ __align__(16) float Bs[GN * GBS];   // Bs[n][k]
+    const int64_t q_ = blockIdx.z % g.nq, I = blockIdx.z / g.nq;
+    const float* A = g.A + q_ * g.sA + I * g.tA;
+    const float* B = g.B + q_ * g.sB + I * g.tB;
+    const int bm = g.a_lower ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    const int m0 = bm * GM, n0 = blockIdx.y * GN;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * WT, wn = (wave & 1) * WT;
+    const int q = lane & 15, k = lane >> 4, wm = 16 * (wave & 1), wn = 32 * (wave >> 1);
     int klo = 0, khi = g.k;
-    if (g.a_lower && m0 + T < khi) khi = m0 + T;
+    if (g.a_lower && m0 + GM < khi) khi = m0 + GM;
     if (g.b_lower) klo = n0;
-    klo &= ~31;
-    v16f acc[NB][NB];
-#pragma unroll
-    for (int a = 0; a < NB; ++a)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[a][b] = v16f{};
-    // Staging: every load of a K step issued together from clamped
-    // (in-bounds) addresses and masked by a select when stored to LDS
-    // (conditional loads would serialise); the next step's loads are issued
-    // before this step's products, so their latency overlaps the MFMA work.
-    constexpr int NL = T * 32 / 256;
-    float xa[NL], xb[NL];
+    v4 acc[2] = {v4{}, v4{}};
+    // a thread's vectors of a stage: A rows 4 am .. +3 of columns ak + 32 u, B
+    // rows 4 bk .. +3 of columns bn + 16 u
+    const int am = 4 * (tid & 7), ak = tid >> 3, bk = 4 * (tid & 15), bn = tid >> 4;
+    const float* Ap = A + m0 + am + (int64_t)ak * g.lda;
+    const float* Bp = B + bk + (int64_t)(n0 + bn) * g.ldb;
+    const bool aedge = m0 + GM > g.m, bedge = n0 + GN > g.n;
+    f4 xa[2], xb[4];
     auto gload = [&](int k0) {
+        if (!aedge && k0 + GK <= khi && (!g.a_lower || k0 + GK <= m0 + 1)) {
 #pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int idx = tid + 256 * u;
-            const int gm = m0 + idx % T, gk = k0 + idx / T;
-            xa[u] = A[(gm < g.m ? gm : g.m - 1) + (int64_t)(gk < g.k ? gk : g.k - 1) * g.lda];
-            const int gk2 = k0 + (idx & 31), gn = n0 + (idx >> 5);
-            xb[u] = B[(gk2 < g.k ? gk2 : g.k - 1) + (int64_t)(gn < g.n ? gn : g.n - 1) * g.ldb];
+            for (int u = 0; u < 2; ++u) xa[u] = *reinterpret_cast<const f4u*>(Ap + (int64_t)(k0 + 32 * u) * g.lda);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int gm = m0 + am + i, gk = k0 + ak + 32 * u;
+                    const float x = A[(gm < g.m ? gm : g.m - 1) + (int64_t)(gk < khi ? gk : khi - 1) * g.lda];
+                    xa[u][i] = (gm < g.m && gk < khi && (!g.a_lower || gk <= gm)) ? x : 0.f;
+                }
+        }
+        if (!bedge && k0 + GK <= khi && (!g.b_lower || k0 + 1 >= n0 + GN)) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) xb[u] = *reinterpret_cast<const f4u*>(Bp + k0 + (int64_t)(16 * u) * g.ldb);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int gk = k0 + bk + i, gn = n0 + bn + 16 * u;
+                    const float x = B[(gk < khi ? gk : khi - 1) + (int64_t)(gn < g.n ? gn : g.n - 1) * g.ldb];
+                    xb[u][i] = (gk < khi && gn < g.n && (!g.b_lower || gk >= gn)) ? x : 0.f;
+                }
         }
     };
     if (klo < khi) gload(klo);
-    for (int k0 = klo; k0 < khi; k0 += 32) {
+    for (int k0 = klo; k0 < khi; k0 += GK) {
 #pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int idx = tid + 256 * u;
-            const int mm = idx % T, kk = idx / T, gm = m0 + mm, gk = k0 + kk;
-            const bool aok = gm < g.m && gk < g.k && (!g.a_lower || gk <= gm);
-            As[kk][mm] = aok ? xa[u] : 0.f;
-            const int k2 = idx & 31, nn = idx >> 5, gk2 = k0 + k2, gn = n0 + nn;
-            const bool bok = gk2 < g.k && gn < g.n && (!g.b_lower || gk2 >= gn);
-            Bs[k2][nn] = bok ? xb[u] : 0.f;
-        }
+        for (int u = 0; u < 2; ++u) *reinterpret_cast<f4*>(As + (ak + 32 * u) * GAS + am) = xa[u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<f4*>(Bs + (bn + 16 * u) * GBS + bk) = xb[u];
         __syncthreads();
-        if (k0 + 32 < khi) gload(k0 + 32);
-        const int r = lane & 31, h = lane >> 5;
+        if (k0 + GK < khi) gload(k0 + GK);
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            float av[NB], bv[NB];
+        for (int u = 0; u < 16; u += 8) {
+            float x[8], y[2][8];
 #pragma unroll
-            for (int a = 0; a < NB; ++a) av[a] = As[2 * s + h][wm + 32 * a + r];
-#pragma unroll
-            for (int b = 0; b < NB; ++b) bv[b] = Bs[2 * s + h][wn + 32 * b + r];
-#pragma unroll
-            for (int a = 0; a < NB; ++a)
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a], bv[b], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    const int n = lane & 31, h = lane >> 5;
-#pragma unroll
-    for (int a = 0; a < NB; ++a)
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                int mm = m0 + wm + 32 * a + 8 * (i >> 2) + 4 * h + (i & 3);
-                int nn = n0 + wn + 32 * b + n;
-                if (mm < g.m && nn < g.n) C[mm + (int64_t)nn * g.ldc] = g.alpha * acc[a][b][i];
+            for (int t = 0; t < 8; ++t) {
+                x[t] = As[(4 * (u + t) + k) * GAS + wm + q];
+                y[0][t] = Bs[(wn + q) * GBS + 4 * (u + t) + k];
+                y[1][t] = Bs[(wn + 16 + q) * GBS + 4 * (u + t) + k];
             }
-}
-
-// copy the 32x32 inverses onto the diagonal of the Winv blocks
-__global__ __launch_bounds__(256) void winv_init_kernel(const float* __restrict__ dinv, int64_t n,
-                                                       int Bo, float* __restrict__ W, int64_t b0) {
-    const int64_t b = b0 + blockIdx.x;
-    const int64_t r0 = b * 32;
-    const int64_t I = r0 / Bo;
-    const int64_t p = r0 - I * Bo;
-    float* Wi = W + I * (int64_t)Bo * Bo;
-    for (int idx = threadIdx.x; idx < 1024; idx += 256) {
-        int r = idx & 31, c = idx >> 5;
-        float v = (r0 + r < n && r0 + c < n) ? dinv[b * 1024 + r + c * 32] : (r == c ? 1.f : 0.f);
-        Wi[(p + r) + (p + c) * (int64_t)Bo] = v;
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    if constexpr (sizeof(T) == 8)
+                        acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)y[b][t], (double)x[t], acc[b], 0, 0, 0);
+                    else
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[b][t], x[t], acc[b], 0, 0, 0);
+                }
+        }
+        __syncthreads();
     }
-}
-
-// WT = Winv^T for each big block (lower part only is meaningful in Winv)
-__global__ __launch_bounds__(256) void transpose_blocks_kernel(const float* __restrict__ W,
-                                                              float* __restrict__ WT, int Bo,
-                                                              int64_t I0) {
-    __shared__ float t[32][33];
-    const int64_t I = I0 + blockIdx.z;
-    const float* Wi = W + I * (int64_t)Bo * Bo;
-    float* Ti = WT + I * (int64_t)Bo * Bo;
-    const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
-    if (r0 < c0) return;                              // upper tiles of Winv are unused
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int j = ty; j < 32; j += 8) {
-        float v = Wi[(r0 + tx) + (int64_t)(c0 + j) * Bo];
-        if (r0 == c0 && r0 + tx < c0 + j) v = 0.f;     // strict upper part of a diagonal tile
-        t[j][tx] = v;
-    }
+    // lane (q, k)'s register e of acc[b]: row wm + q, column wn + 16 b + 4e + k
+    // (FP32: 4k + e)
+    float* C = g.C + q_ * g.sC + I * g.tC;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + wm + q, n = n0 + (sizeof(T) == 8 ? 4 * e + k : 4 * k + e) + wn + 16 * b, nn = n - n0;
+            const float v = (float)((T)g.alpha * acc[b][e]);
+            if (m < g.m && n < g.n) C[m + (int64_t)n * g.ldc] = v;
+            if (g.CT) Bs[nn * GBS + wm + q] = v;
+        }
+    if (!g.CT) return;
     __syncthreads();
-    for (int j = ty; j < 32; j += 8) Ti[(c0 + tx) + (int64_t)(r0 + j) * Bo] = t[tx][j];
+    float* CT = g.CT + q_ * g.sC + I * g.tC;
+    for (int idx = tid; idx < GM * GN; idx += 256) {
+        const int nn = idx & (GN - 1), mm = idx / GN;
+        if (m0 + mm < g.m && n0 + nn < g.n) CT[n0 + nn + (int64_t)(m0 + mm) * g.ldc] = Bs[nn * GBS + mm];
+    }
 }
 
 // ---------------------------------------------------------------- TRSV kernels
@@ -192,8 +286,6 @@ __global__ __launch_bounds__(256) void fwd_gemv_partial_kernel(
     const int i = blockIdx.x * 64 + lane;
     const int ic = i < bI ? i : bI - 1;
     const int sp = blockIdx.y;
-    const int j0 = blockIdx.z * NR;
-    const int nj = nrhs - j0 < NR ? nrhs - j0 : NR;
     const int64_t cs = (int64_t)sp * FW_CW;
     const float* Lr = L + (p0 + ic);
     float l[FW_CPW];
@@ -207,16 +299,16 @@ __global__ __launch_bounds__(256) void fwd_gemv_partial_kernel(
     for (int q = 0; q < NR * FW_CW / 256; ++q) {
         const int idx = tid + 256 * q, j = idx / FW_CW, cc = idx % FW_CW;
         const int64_t c = cs + cc;
-        const int jj = j < nj ? j : nj - 1;
-        const double v = Y[(int64_t)(j0 + jj) * ldy + (c < p0 ? c : p0 - 1)];
-        ys[j][cc] = (j < nj && c < p0) ? v : 0.0;
+        const int jj = j < nrhs ? j : nrhs - 1;
+        const double v = Y[(int64_t)jj * ldy + (c < p0 ? c : p0 - 1)];
+        ys[j][cc] = (j < nrhs && c < p0) ? v : 0.0;
     }
     __syncthreads();
     double acc[NR];
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
         double a0 = 0.0, a1 = 0.0;
-        if (j < nj) {
+        if (j < nrhs) {
 #pragma unroll
             for (int u = 0; u < FW_CPW; u += 2) {
                 a0 = fma((double)l[u], ys[j][wave * FW_CPW + u], a0);
@@ -231,8 +323,8 @@ __global__ __launch_bounds__(256) void fwd_gemv_partial_kernel(
     if (wave == 0 && i < bI) {
 #pragma unroll
         for (int j = 0; j < NR; ++j)
-            if (j < nj)
-                part[((int64_t)sp * nrhs + j0 + j) * bI + i] =
+            if (j < nrhs)
+                part[((int64_t)sp * nrhs + j) * bI + i] =
                     ((red[0][j][lane] + red[1][j][lane]) + red[2][j][lane]) + red[3][j][lane];
     }
 }
@@ -252,8 +344,6 @@ __global__ __launch_bounds__(256) void bwd_gemv_partial_kernel(
     const int sp = blockIdx.y;
     const int64_t rs = p1 + (int64_t)sp * BW_RW;
     const int c0 = blockIdx.x * (4 * BW_CPW) + wave * BW_CPW;
-    const int j0 = blockIdx.z * NR;
-    const int nj = nrhs - j0 < NR ? nrhs - j0 : NR;
     float l[BW_CPW][BW_RPL];
 #pragma unroll
     for (int cc = 0; cc < BW_CPW; ++cc) {
@@ -267,8 +357,8 @@ __global__ __launch_bounds__(256) void bwd_gemv_partial_kernel(
     }
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
-        if (j < nj) {
-            const double* x = X + (int64_t)(j0 + j) * ldx;
+        if (j < nrhs) {
+            const double* x = X + (int64_t)j * ldx;
             double xv[BW_RPL];
 #pragma unroll
             for (int k = 0; k < BW_RPL; ++k) {
@@ -294,7 +384,7 @@ __global__ __launch_bounds__(256) void bwd_gemv_partial_kernel(
             v += __shfl_xor(v, 2);
             v += __shfl_xor(v, 4);
             if (q == 0 && c0 + col < bI)
-                part[((int64_t)sp * nrhs + j0 + j) * bI + c0 + col] = v;
+                part[((int64_t)sp * nrhs + j) * bI + c0 + col] = v;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();                 // buf is rewritten next
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -341,8 +431,6 @@ __global__ __launch_bounds__(64 * TT_NW) void tri_gemv_tile_kernel(const float* 
     const int i = ib * TG + lane;
     const int j0 = jb * TG;
     const int c0 = j0 + TT_CW * wave;      // this wave's first column
-    const int r0 = blockIdx.y * NR;
-    const int nj = nrhs - r0 < NR ? nrhs - r0 : NR;
     // This wave's 16 columns of the tile, all loads issued before any use.  A
     // load guarded by a condition (or whose use is) would be sunk into a
     // branch with its own wait, serialising the loads; hence three shapes:
@@ -379,8 +467,8 @@ __global__ __launch_bounds__(64 * TT_NW) void tri_gemv_tile_kernel(const float* 
     // lane u of every wave builds a part of v[j0 + u]
     const int jl = j0 + lane < bI ? j0 + lane : bI - 1;
     const int64_t sstride = (int64_t)nrhs * bI;
-    for (int r = 0; r < nj; ++r) {
-        const double* pr = pin + (int64_t)(r0 + r) * bI + jl;
+    for (int r = 0; r < nrhs; ++r) {
+        const double* pr = pin + (int64_t)r * bI + jl;
         double sum = 0.0;
         int sp = wave;
         for (; sp + 7 * TT_NW < S; sp += 8 * TT_NW) {      // batches of 8 independent loads
@@ -397,7 +485,7 @@ __global__ __launch_bounds__(64 * TT_NW) void tri_gemv_tile_kernel(const float* 
             double tot = vsum[0][lane];
 #pragma unroll
             for (int w = 1; w < TT_NW; ++w) tot += vsum[w][lane];
-            vs[lane] = V[(int64_t)(r0 + r) * ldv + jl] - tot;
+            vs[lane] = V[(int64_t)r * ldv + jl] - tot;
         }
         __syncthreads();
         double a0 = 0.0, a1 = 0.0;
@@ -412,7 +500,7 @@ __global__ __launch_bounds__(64 * TT_NW) void tri_gemv_tile_kernel(const float* 
             double tot = acc_w[0][lane];
 #pragma unroll
             for (int w = 1; w < TT_NW; ++w) tot += acc_w[w][lane];
-            part[((int64_t)jb * nrhs + r0 + r) * bI + i] = tot;
+            part[((int64_t)jb * nrhs + r) * bI + i] = tot;
         }
         __syncthreads();                    // vsum, vs and acc_w are reused
     }
@@ -452,18 +540,10 @@ __global__ __launch_bounds__(256) void tri_gemv_reduce_kernel(const double* __re
 
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
-// 128x128 tiles when they give at least two workgroups per CU of a 256-CU
-// device, else 64x64 tiles (the deep levels of the doubling are a few large
-// products: four times the workgroups for the same work)
-int launch_gemm(hipStream_t st, const gemm_batch& g, int nbatch) {
-    const int64_t t128 = (int64_t)cdiv(g.m, 128) * cdiv(g.n, 128) * nbatch;
-    if (g.m >= 128 && g.n >= 128 && t128 >= 512) {
-        dim3 grid(cdiv(g.m, 128), cdiv(g.n, 128), (unsigned)nbatch);
-        hipLaunchKernelGGL(gemm_f32_kernel<128>, grid, dim3(256), 0, st, g);
-    } else {
-        dim3 grid(cdiv(g.m, 64), cdiv(g.n, 64), (unsigned)nbatch);
-        hipLaunchKernelGGL(gemm_f32_kernel<64>, grid, dim3(256), 0, st, g);
-    }
+int launch_gemm(hipStream_t st, const gemm_batch& g, int nbatch, bool f64) {
+    const dim3 grid(cdiv(g.m, GM), cdiv(g.n, GN), (unsigned)nbatch);
+    if (f64) hipLaunchKernelGGL(gemm_kernel<double>, grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL(gemm_kernel<float>, grid, dim3(256), 0, st, g);
     MPC_LAUNCH_CHECK();
     return 0;
 }
@@ -471,11 +551,11 @@ int launch_gemm(hipStream_t st, const gemm_batch& g, int nbatch) {
 }  // namespace
 
 // Build Winv_I = L_II^{-1} for every big block (Bo x Bo, column-major, ld Bo,
-// block I at W + I*Bo*Bo) from L and its 32x32 diagonal inverses, then
-// WT_I = Winv_I^T.  Full big blocks are batched per level; a ragged last big
-// block is handled by its own launches with clipped sizes.
-static int double_level(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo, float* W,
-                        int h, int64_t I0, int nblk, int64_t rows, int q0, int nq, int hc) {
+// block I at W + I*Bo*Bo) and WT_I = Winv_I^T from L and its 32x32 diagonal
+// inverses.  Full big blocks are batched per level; a ragged last big block is
+// handled by its own launches with clipped sizes.
+static int double_level(hipStream_t st, const float* L, int64_t ldl, int Bo, float* W, float* WT,
+                        int h, int64_t I0, int nblk, int q0, int nq, int hc, bool f64) {
     const int64_t base = I0 * Bo;
     const int64_t p = 2 * (int64_t)h * q0;
     float* Wi = W + I0 * (int64_t)Bo * Bo;
@@ -484,24 +564,25 @@ static int double_level(hipStream_t st, const float* L, int64_t ldl, int64_t n, 
     g1.A = L + (base + p + h) + (base + p) * ldl;  g1.lda = ldl;
     g1.B = Wi + p + p * (int64_t)Bo;              g1.ldb = Bo;
     g1.C = Wi + p + (p + h) * (int64_t)Bo;        g1.ldc = Bo;
+    g1.CT = nullptr;
     g1.sA = 2 * (int64_t)h * (1 + ldl);
     g1.sB = g1.sC = 2 * (int64_t)h * (1 + Bo);
     g1.tA = (int64_t)Bo * (1 + ldl);
     g1.tB = g1.tC = bs;
     g1.nq = nq;
     g1.m = hc; g1.n = h; g1.k = h; g1.alpha = 1.f; g1.a_lower = 0; g1.b_lower = 1;
-    int rc = launch_gemm(st, g1, nq * nblk);
+    int rc = launch_gemm(st, g1, nq * nblk, f64);
     if (rc) return rc;
     gemm_batch g2;                                       // X21 = -Cinv * T -> (p+h, p)
     g2.A = Wi + (p + h) + (p + h) * (int64_t)Bo;  g2.lda = Bo;
     g2.B = Wi + p + (p + h) * (int64_t)Bo;        g2.ldb = Bo;
     g2.C = Wi + (p + h) + p * (int64_t)Bo;        g2.ldc = Bo;
+    g2.CT = WT + I0 * bs + p + (p + h) * (int64_t)Bo;
     g2.sA = g2.sB = g2.sC = 2 * (int64_t)h * (1 + Bo);
     g2.tA = g2.tB = g2.tC = bs;
     g2.nq = nq;
     g2.m = hc; g2.n = h; g2.k = hc; g2.alpha = -1.f; g2.a_lower = 1; g2.b_lower = 0;
-    (void)rows;
-    return launch_gemm(st, g2, nq * nblk);
+    return launch_gemm(st, g2, nq * nblk, f64);
 }
 
 // Big blocks [I0, I1) only (each depends on L_II and the 32x32 inverses of
@@ -509,24 +590,24 @@ static int double_level(hipStream_t st, const float* L, int64_t ldl, int64_t n, 
 int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
                                    const float* dinv, float* W, float* WT, int64_t I0,
                                    int64_t I1) {
-    if (Bo % 64 || Bo < 64) {
-        mpc_set_error("block inverse: Bo must be a multiple of 64");
+    if (Bo % LF || Bo < LF) {
+        mpc_set_error("block inverse: Bo must be a multiple of %d", LF);
         return MPC_ERR_ARG;
     }
     const int64_t nI = (n + Bo - 1) / Bo;
     const int64_t nfull = n / Bo;                 // big blocks with Bo rows
     if (I1 > nI) I1 = nI;
     if (I0 >= I1) return 0;
-    const int64_t b0 = I0 * (Bo / 32), b1 = std::min<int64_t>((n + 31) / 32, I1 * (Bo / 32));
-    hipLaunchKernelGGL(winv_init_kernel, dim3((unsigned)(b1 - b0)), dim3(256), 0, st, dinv, n, Bo, W,
-                       b0);
+    const int64_t b0 = I0 * (Bo / LF), b1 = std::min<int64_t>(cdiv(n, LF), I1 * (Bo / LF));
+    hipLaunchKernelGGL(winv_leaf_kernel, dim3((unsigned)(b1 - b0)), dim3(256), 0, st, L, ldl, dinv, n,
+                       Bo, W, WT, b0);
     MPC_LAUNCH_CHECK();
     const int64_t f1 = std::min(I1, nfull);      // full blocks in the range: [I0, f1)
+    const bool f64 = n <= 8192;
     int rc;
-    for (int h = 32; h < Bo; h *= 2) {
+    for (int h = LF; h < Bo; h *= 2) {
         const int pairs = Bo / (2 * h);
-        if (f1 > I0 &&
-            (rc = double_level(st, L, ldl, n, Bo, W, h, I0, (int)(f1 - I0), Bo, 0, pairs, h)))
+        if (f1 > I0 && (rc = double_level(st, L, ldl, Bo, W, WT, h, I0, (int)(f1 - I0), 0, pairs, h, f64)))
             return rc;
         if (nI > nfull && nfull >= I0 && nfull < I1) {   // ragged last big block
             const int64_t I = nfull, rows = n - I * Bo;
@@ -535,17 +616,14 @@ int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, 
                 if (2 * h * q + h < rows) npair = q + 1;
             if (npair == 0) continue;
             const int full = (2 * h * (npair - 1) + 2 * h <= rows) ? npair : npair - 1;
-            if (full > 0 && (rc = double_level(st, L, ldl, n, Bo, W, h, I, 1, rows, 0, full, h)))
+            if (full > 0 && (rc = double_level(st, L, ldl, Bo, W, WT, h, I, 1, 0, full, h, f64)))
                 return rc;
             if (npair > full) {
                 const int hc = (int)(rows - 2 * (int64_t)h * full - h);
-                if ((rc = double_level(st, L, ldl, n, Bo, W, h, I, 1, rows, full, 1, hc))) return rc;
+                if ((rc = double_level(st, L, ldl, Bo, W, WT, h, I, 1, full, 1, hc, f64))) return rc;
             }
         }
     }
-    dim3 tg((unsigned)(Bo / 32), (unsigned)(Bo / 32), (unsigned)(I1 - I0));
-    hipLaunchKernelGGL(transpose_blocks_kernel, tg, dim3(256), 0, st, W, WT, Bo, I0);
-    MPC_LAUNCH_CHECK();
     return 0;
 }
 
@@ -558,7 +636,7 @@ static int tri_gemv(hipStream_t st, const float* M, int Bo, int bI, int upper, c
                     int64_t ldv, int nrhs, const double* pin, int S, double* part, double* out,
                     int64_t ldo) {
     const int nb = (bI + TG - 1) / TG;
-    const dim3 grid((unsigned)(nb * (nb + 1) / 2), cdiv(nrhs, NR));
+    const dim3 grid((unsigned)(nb * (nb + 1) / 2));
     if (upper)
         hipLaunchKernelGGL(tri_gemv_tile_kernel<true>, grid, dim3(64 * TT_NW), 0, st, M, Bo, bI, V,
                            ldv, nrhs, pin, S, part);
@@ -578,8 +656,38 @@ static int64_t gemv_splits_max(int64_t n, int Bo) {
     return std::max<int64_t>((n + FW_CW - 1) / FW_CW, (n + BW_RW - 1) / BW_RW);
 }
 
+// right-hand sides of the next pass over the factor: at most NR in the GEMV
+// kernels above, else at most MPC_MM_NJ on the matrix cores
+static int sweep_pass(int nrhs) { return nrhs > NR ? std::min(nrhs, MPC_MM_NJ) : nrhs; }
+
+// chunks of a product with at most Bo output rows, in units of Bo partial sums:
+// the chunks of bI < Bo rows take at most bI rounded up to a row block times
+// ceil(2048 / blocks), which is less than Bo beyond those of Bo rows
+static int64_t mm_chunks(int Bo, int64_t kc) { return mpc_mm_splits(Bo, kc) + 1; }
+
+// scratch of a pass: GEMV kernels: the triangular product's partial sums, then
+// the off-diagonal one's; matrix cores: the same with v between them
 int64_t mpc_block_prec_partial_doubles(int64_t n, int Bo, int nrhs) {
-    return ((int64_t)(Bo + TG - 1) / TG + gemv_splits_max(n, Bo)) * Bo * nrhs;
+    const int64_t gemv = ((int64_t)(Bo + TG - 1) / TG + gemv_splits_max(n, Bo)) * Bo *
+                         std::min(nrhs, NR);
+    if (nrhs <= NR) return gemv;
+    return std::max(gemv, (mm_chunks(Bo, n) + mm_chunks(Bo, Bo) + 1) * Bo * std::min(nrhs, MPC_MM_NJ));
+}
+
+// One stage on the matrix cores: v = R_I - (sum of the S chunks of the off-
+// diagonal product in gpart), out_I = M v with the triangular M (mode 1 lower,
+// 2 upper).
+static int mm_stage(hipStream_t st, const float* M, int Bo, int bI, int mode, const double* V,
+                    int64_t ld, int nj, const double* gpart, int64_t kc, int64_t S, int unit,
+                    double* v, double* tpart, double* out) {
+    int rc;
+    if (kc > 0) {
+        if ((rc = mpc_launch_mm_sum(st, bI, nj, kc, S, 0, unit, gpart, V, ld, -1.0, v, bI))) return rc;
+        V = v;
+    }
+    const int64_t St = mpc_mm_splits(bI, bI);
+    if ((rc = mpc_launch_mm_n(st, M, Bo, bI, bI, mode, V, kc > 0 ? bI : ld, nj, tpart, St))) return rc;
+    return mpc_launch_mm_sum(st, bI, nj, bI, St, mode, MPC_MM_GROUP_N, tpart, nullptr, 0, 1.0, out, ld);
 }
 
 // z = L^{-T} L^{-1} r for nrhs columns: R (in), Y (forward result), Z (out).
@@ -590,39 +698,48 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
                          double* Z, int64_t ld, int nrhs, double* part, hipEvent_t late_ev,
                          int64_t I_late) {
     const int64_t nI = (n + Bo - 1) / Bo;
-    const unsigned gz = cdiv(nrhs, NR);
-    double* gpart = part + (int64_t)((Bo + TG - 1) / TG) * Bo * nrhs;   // GEMV partial sums
     int rc;
-    for (int64_t I = 0; I < nI; ++I) {
-        const int64_t p0 = I * Bo;
-        const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
-        int S = 0;
-        if (p0 > 0) {
-            S = (int)cdiv(p0, FW_CW);
-            hipLaunchKernelGGL(fwd_gemv_partial_kernel, dim3(cdiv(bI, 64), (unsigned)S, gz),
-                               dim3(256), 0, st, L, ldl, p0, bI, Y, ld, nrhs, gpart);
+    for (int j0 = 0, nj; j0 < nrhs; j0 += nj, R += nj * ld, Y += nj * ld, Z += nj * ld) {
+        nj = sweep_pass(nrhs - j0);
+        const bool mm = nj > NR;
+        double* v = part + (mm ? mm_chunks(Bo, Bo) : (Bo + TG - 1) / TG) * Bo * nj;
+        double* gpart = mm ? v + (int64_t)Bo * nj : v;
+        for (int64_t I = 0; I < nI; ++I) {
+            const int64_t p0 = I * Bo;
+            const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
+            const float* Wi = Winv + I * (int64_t)Bo * Bo;
+            const int64_t S = mm ? mpc_mm_splits(bI, p0) : cdiv(p0, FW_CW);
+            if (p0 > 0 && mm) {
+                if ((rc = mpc_launch_mm_n(st, L + p0, ldl, bI, p0, 0, Y, ld, nj, gpart, S))) return rc;
+            } else if (p0 > 0) {
+                hipLaunchKernelGGL(fwd_gemv_partial_kernel, dim3(cdiv(bI, 64), (unsigned)S), dim3(256), 0,
+                                   st, L, ldl, p0, bI, Y, ld, nj, gpart);
+            }
+            if (late_ev && j0 == 0 && I == I_late && hipStreamWaitEvent(st, late_ev, 0) != hipSuccess) {
+                mpc_set_error("apply_block_prec: stream wait failed");
+                return MPC_ERR_HIP;
+            }
+            rc = mm ? mm_stage(st, Wi, Bo, bI, 1, R + p0, ld, nj, gpart, p0, S, MPC_MM_GROUP_N, v, part, Y + p0)
+                    : tri_gemv(st, Wi, Bo, bI, 0, R + p0, ld, nj, gpart, (int)S, part, Y + p0, ld);
+            if (rc) return rc;
         }
-        const float* Wi = Winv + I * (int64_t)Bo * Bo;
-        if (late_ev && I == I_late && hipStreamWaitEvent(st, late_ev, 0) != hipSuccess) {
-            mpc_set_error("apply_block_prec: stream wait failed");
-            return MPC_ERR_HIP;
+        for (int64_t I = nI - 1; I >= 0; --I) {
+            const int64_t p0 = I * Bo;
+            const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
+            const int64_t p1 = p0 + bI;
+            const float* WTi = WinvT + I * (int64_t)Bo * Bo;
+            const int64_t S = mm ? mpc_mm_splits(bI, n - p1) : cdiv(n - p1, BW_RW);
+            if (p1 < n && mm) {
+                if ((rc = mpc_launch_mm_t(st, L + p1 + p0 * ldl, ldl, n - p1, bI, Z + p1, ld, nj, gpart, S)))
+                    return rc;
+            } else if (p1 < n) {
+                hipLaunchKernelGGL(bwd_gemv_partial_kernel, dim3(cdiv(bI, 4 * BW_CPW), (unsigned)S),
+                                   dim3(256), 0, st, L, ldl, p0, bI, n, Z, ld, nj, gpart);
+            }
+            rc = mm ? mm_stage(st, WTi, Bo, bI, 2, Y + p0, ld, nj, gpart, n - p1, S, MPC_MM_GROUP_T, v, part, Z + p0)
+                    : tri_gemv(st, WTi, Bo, bI, 1, Y + p0, ld, nj, gpart, (int)S, part, Z + p0, ld);
+            if (rc) return rc;
         }
-        if ((rc = tri_gemv(st, Wi, Bo, bI, 0, R + p0, ld, nrhs, gpart, S, part, Y + p0, ld)))
-            return rc;
-    }
-    for (int64_t I = nI - 1; I >= 0; --I) {
-        const int64_t p0 = I * Bo;
-        const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
-        const int64_t p1 = p0 + bI;
-        int S = 0;
-        if (p1 < n) {
-            S = (int)cdiv(n - p1, BW_RW);
-            hipLaunchKernelGGL(bwd_gemv_partial_kernel, dim3(cdiv(bI, 4 * BW_CPW), (unsigned)S, gz),
-                               dim3(256), 0, st, L, ldl, p0, bI, n, Z, ld, nrhs, gpart);
-        }
-        const float* WTi = WinvT + I * (int64_t)Bo * Bo;
-        if ((rc = tri_gemv(st, WTi, Bo, bI, 1, Y + p0, ld, nrhs, gpart, S, part, Z + p0, ld)))
-            return rc;
     }
     MPC_LAUNCH_CHECK();
     return 0;

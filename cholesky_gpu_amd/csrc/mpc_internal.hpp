@@ -256,17 +256,22 @@ int mpc_launch_syrk_classes(hipStream_t st, float* C, int64_t m, int64_t ldc, in
 void mpc_syrk_masks(int update_prec, const int* ladder, int n_ladder, unsigned* class_mask,
                     unsigned* fp8_mask);
 // k_mrhs.hip: products with up to MPC_MM_NJ right-hand sides X (nj columns,
-// ld ldx), as partial sums over S column chunks, and their sum
+// ld ldx), as partial sums over S column (row) chunks, and their sum
 constexpr int MPC_MM_NJ = 16;
-constexpr int MPC_MM_GROUP_N = 16;                           // chunk granularity
+constexpr int MPC_MM_GROUP_N = 16, MPC_MM_GROUP_T = 64;      // chunk granularity of mm_n, mm_t
 int64_t mpc_mm_splits(int64_t rows, int64_t kc);             // chunks that fill the chip
-// part[(s nj + j) m + r] = sum over chunk s of A[r][c] X[j][c]
-int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc,
+// part[(s nj + j) m + r] = sum over chunk s of A[r][c] X[j][c]; mode 1: c <= r,
+// 2: c >= r (square A; the rest is not read as data)
+int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc, int mode,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S);
-int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc,
+int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc, int mode,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S);
-// Y[j][r] = (B ? B[j][r] : 0) + a sum_s part[(s nj + j) m + r]
-int mpc_launch_mm_sum(hipStream_t st, int64_t m, int nj, int64_t kc, int64_t S,
+// part[(s nj + j) nc + c] = sum over row chunk s of A[r][c] X[j][r]
+int mpc_launch_mm_t(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t nc,
+                    const double* X, int64_t ldx, int nj, double* part, int64_t S);
+// Y[j][r] = (B ? B[j][r] : 0) + a sum_s part[(s nj + j) m + r], the S chunks of
+// kc columns (in units of `unit`) that mode leaves to row r
+int mpc_launch_mm_sum(hipStream_t st, int64_t m, int nj, int64_t kc, int64_t S, int mode, int unit,
                       const double* part, const double* B, int64_t ldb, double a, double* Y, int64_t ldy);
 // k_pcg.hip
 int mpc_launch_symv(hipStream_t st, const float* A, int64_t lda, int64_t n, int nrhs,
@@ -343,7 +348,17 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
                          double* Z, int64_t ld, int nrhs, double* part,
                          hipEvent_t late_ev = nullptr, int64_t I_late = -1);
 int64_t mpc_block_prec_partial_doubles(int64_t n, int Bo, int nrhs);
-inline int mpc_block_bo(int64_t n) { return n > 8192 ? 2048 : (n > 2048 ? 1024 : 256); }
+// Big-block edge of the sweeps: the whole matrix up to 2048 rows (rounded up to
+// a power of two), else 2048.  A stage costs six dependent launches per
+// application; a larger block costs its inverse, which for the last one is not
+// hidden by the factor.  Solves (us, Bo = 1024 / 2048 / 4096): n = 2048 2244 /
+// 2149 / -, 4096 3335 / 3172 / 3555, 8192 6397 / 6111 / 6802, 12000 11041 / 10060
+// / 10644; n = 777: 1354 / 1155 / 1143 with 256 / 512 / 1024.
+inline int mpc_block_bo(int64_t n) {
+    int bo = 128;
+    while (bo < 2048 && bo < n) bo *= 2;
+    return bo;
+}
 
 // host-side generators shared with mpc_matgen (RNG identical to the device one)
 void mpc_philox4x32(const uint32_t ctr[4], const uint32_t key[2], uint32_t out[4]);

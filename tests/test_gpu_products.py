@@ -37,3 +37,22 @@ def test_symmetric_product(handle, n, nrhs, dtype):
     f = S.pcg if dtype is torch.float32 else S.pcg64
     _, pi, _ = f(handle, A, eye, B, nb=64, X=X.clone(), opts=S.pcg_opts(x0_mode=2, maxit=0))
     assert pi.relres <= bound, (pi.relres, bound)
+
+
+@pytest.mark.parametrize("n", [65, 256, 1000, 2049, 4200, 8300])
+@pytest.mark.parametrize("nrhs", [1, 4, 5, 16, 21])
+def test_apply_precond_blocks(handle, n, nrhs):
+    """z = (L L^T)^-1 r for the sizes and passes of the blocked sweeps against
+    FP64 triangular solves with the same L (diagonally dominant, cond <= 3, so
+    that the FP32 block inverses are within a few hundred u32 of exact)."""
+    say("apply_precond", n, nrhs)
+    g = torch.Generator(device="cuda").manual_seed(n + nrhs)
+    T = torch.randn(n, n, generator=g, device="cuda") * (0.25 / n ** 0.5)
+    T = torch.triu(T, 1) + torch.eye(n, device="cuda")            # tensor = L^T
+    T = T + torch.tril(torch.full_like(T, float("nan")), -1)      # A's upper part is not read
+    R = torch.randn(nrhs, n, generator=g, device="cuda", dtype=torch.float64)
+    Z = S.apply_precond(handle, T.contiguous(), R)
+    L64 = torch.triu(T).nan_to_num(0.0).to(torch.float64).T.contiguous()
+    Y = torch.linalg.solve_triangular(L64, R.T.contiguous(), upper=False)
+    X = torch.linalg.solve_triangular(L64.T.contiguous(), Y, upper=True).T
+    assert float((Z - X).norm() / X.norm()) < 256 * 2.0 ** -24
