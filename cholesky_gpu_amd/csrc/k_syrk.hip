@@ -413,9 +413,8 @@ __device__ __forceinline__ void mm_16(const operand_src& oc, const operand_src& 
         k_loop<0, 16>(k, [&](int kc) { body(kc, std::false_type{}); });
 }
 
-// NATIVE (runtime-K form only): both operands stored in FP32
-// SPLIT: 0 never, 1 always (the launch holds only such pairs), 2 per pair
-template <int QA, int KC, bool NATIVE, int SPLIT>
+// SPLIT: FP32 against FP8/BF16 as bf16 products (else no such pair occurs)
+template <int QA, int KC, bool SPLIT>
 __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src& orow,
                                        const tile_ctx& t, int k, v16f acc[QA][QA]) {
     const int h = (threadIdx.x & 63) >> 5;
@@ -425,8 +424,8 @@ __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src&
     // FP32 operand as hi + mid + lo (exact), three bf16 products per 16-wide
     // chunk; the products are exact and the sums FP32, as in the FP32
     // matrix-core op, at a sixth of its cost per k
-    if (SPLIT == 1 || (SPLIT == 2 && (oc.prec == MPC_PREC_FP32) != (orow.prec == MPC_PREC_FP32) &&
-                       oc.prec != MPC_PREC_FP16 && orow.prec != MPC_PREC_FP16)) {
+    if (SPLIT && (oc.prec == MPC_PREC_FP32) != (orow.prec == MPC_PREC_FP32) &&
+        oc.prec != MPC_PREC_FP16 && orow.prec != MPC_PREC_FP16) {
         const bool col32 = oc.prec == MPC_PREC_FP32;
         k_loop<0, 16>(k, [&](int kc) {
             const int k0 = kc + 8 * h;
@@ -484,51 +483,6 @@ __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src&
             k_loop<KC, 16>(k, [&](int kc) { body(kc, std::true_type{}); });
         else
             k_loop<KC, 16>(k, [&](int kc) { body(kc, std::false_type{}); });
-    } else if constexpr (NATIVE) {
-        // both operands FP32: one branch-free loop, the next chunk's operands
-        // loaded before this chunk's products (the FP32 class is MFMA-bound
-        // only if its loads overlap the products)
-        const float* pa[QA];
-        const float* pb[QA];
-#pragma unroll
-        for (int q = 0; q < QA; ++q) {
-            pa[q] = reinterpret_cast<const float*>(oc.payload + ra[q] * oc.row_stride) + 8 * h;
-            pb[q] = reinterpret_cast<const float*>(orow.payload + rb[q] * orow.row_stride) + 8 * h;
-        }
-        float4 A[QA][2], B[QA][2];
-#pragma unroll
-        for (int q = 0; q < QA; ++q) {
-            A[q][0] = *reinterpret_cast<const float4*>(pa[q]);
-            A[q][1] = *reinterpret_cast<const float4*>(pa[q] + 4);
-            B[q][0] = *reinterpret_cast<const float4*>(pb[q]);
-            B[q][1] = *reinterpret_cast<const float4*>(pb[q] + 4);
-        }
-        for (int kc = 0; kc < k; kc += 16) {
-            const int kn = kc + 16 < k ? kc + 16 : kc;       // the last chunk reloads itself
-            float4 An[QA][2], Bn[QA][2];
-#pragma unroll
-            for (int q = 0; q < QA; ++q) {
-                An[q][0] = *reinterpret_cast<const float4*>(pa[q] + kn);
-                An[q][1] = *reinterpret_cast<const float4*>(pa[q] + kn + 4);
-                Bn[q][0] = *reinterpret_cast<const float4*>(pb[q] + kn);
-                Bn[q][1] = *reinterpret_cast<const float4*>(pb[q] + kn + 4);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-#pragma unroll
-                for (int a = 0; a < QA; ++a)
-#pragma unroll
-                    for (int b = 0; b < QA; ++b) {
-                        const float av = e < 4 ? A[b][0][e] : A[b][1][e - 4];
-                        const float bv = e < 4 ? B[a][0][e] : B[a][1][e - 4];
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[a][b], 0, 0, 0);
-                    }
-#pragma unroll
-            for (int q = 0; q < QA; ++q) {
-                A[q][0] = An[q][0]; A[q][1] = An[q][1];
-                B[q][0] = Bn[q][0]; B[q][1] = Bn[q][1];
-            }
-        }
     } else {
         // an FP32 operand against a lower format (rare): expanded per chunk
         for (int kc = 0; kc < k; kc += 16) {
@@ -574,44 +528,28 @@ struct syrk_shape {
     int64_t mt, tcol0, tcol1, rect_tr0, rect_ncol;
 };
 
-template <int QA, int CLS, int FA, int FB, int KC>
-__device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
-                                          const mpc_syrk_panels& P, int64_t row_stride,
-                                          int tile_rows, const syrk_shape& G, int64_t pid,
-                                          const syrk_lists& L);
-
-// LISTED: a later launch of a sequence, over its work list (L.mode 2);
-// otherwise one workgroup per tile pair (L.mode 0, or 1 to build the lists)
-template <int QA, int CLS, int FA, int FB, int KC, bool LISTED>
-__global__ __launch_bounds__(256, 2) void syrk_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
-                                                   int k, const mpc_syrk_panels P,
-                                                   int64_t row_stride, int tile_rows,
-                                                   const mpc_small* __restrict__ sm, int64_t npair,
-                                                   int64_t per_xcd, const syrk_shape G,
-                                                   const syrk_lists L) {
-    if (sm && sm->info != 0) return;
-    if constexpr (LISTED) {
-        const int rank = launch_rank_of(CLS, FA, FB);
-        const int count = L.base[rank];
-        const int* list = L.base + kListHead + (int64_t)rank * L.cap;
-        for (int it = blockIdx.x; it < count; it += gridDim.x)
-            syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L);
-        return;
+// Launch sequence, first launch: the pair goes to the lists of the later
+// launches (ranks above `rank`) that have work on it.
+__device__ __forceinline__ void note_pair(const syrk_lists& L, const mpc_syrk_panels& P, int tile_rows,
+                                          int64_t trow, int64_t tcol, int64_t pid, int rank) {
+    if (threadIdx.x != 0) return;
+    unsigned need = 0;
+    for (int q = 0; q < P.np; ++q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+        need |= 1u << launch_rank(prec[trow], prec[tcol]);
     }
-    // XCD-aware remap: hardware places block b on XCD b % 8
-    const int64_t b = blockIdx.x;
-    const int64_t pid = (b & 7) * per_xcd + (b >> 3);
-    if (pid >= npair) return;
-    syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L);
+    need &= ~((2u << rank) - 1u);
+    for (int r = 0; r < kListHead; ++r)
+        if ((need >> r) & 1u) {
+            const int slot = atomicAdd(&L.base[r], 1);
+            L.base[kListHead + (int64_t)r * L.cap + slot] = (int)pid;
+        }
 }
 
-template <int QA, int CLS, int FA, int FB, int KC>
-__device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
-                                          const mpc_syrk_panels& P, int64_t row_stride,
-                                          int tile_rows, const syrk_shape& G, int64_t pid,
-                                          const syrk_lists& L) {
-    constexpr int TILE = 64 * QA;
-    int64_t ti, tj;
+// tile pair pid of the launch -> tile row ti, tile column tj
+template <int TILE>
+__device__ __forceinline__ void tile_of(const syrk_shape& G, int64_t pid, int64_t& ti, int64_t& tj) {
     if (G.rect_ncol > 0) {
         ti = G.rect_tr0 + pid / G.rect_ncol;
         tj = G.tcol0 + pid % G.rect_ncol;
@@ -664,23 +602,49 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
             ti = rbase + inner % rows;
         }
     }
-    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+}
 
-    if (L.mode == 1 && threadIdx.x == 0) {
-        // the later launches of the sequence with work on this tile pair
-        unsigned need = 0;
-        for (int q = 0; q < P.np; ++q) {
-            const int slot = (P.p0 + q) % P.slots;
-            const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
-            need |= 1u << launch_rank(prec[trow], prec[tcol]);
-        }
-        need &= ~((2u << launch_rank_of(CLS, FA, FB)) - 1u);
-        for (int r = 0; r < kListHead; ++r)
-            if ((need >> r) & 1u) {
-                const int slot = atomicAdd(&L.base[r], 1);
-                L.base[kListHead + (int64_t)r * L.cap + slot] = (int)pid;
-            }
+template <int QA, int CLS, int FA, int FB, int KC>
+__device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                          const mpc_syrk_panels& P, int64_t row_stride,
+                                          int tile_rows, const syrk_shape& G, int64_t pid,
+                                          const syrk_lists& L);
+
+// LISTED: a later launch of a sequence, over its work list (L.mode 2);
+// otherwise one workgroup per tile pair (L.mode 0, or 1 to build the lists)
+template <int QA, int CLS, int FA, int FB, int KC, bool LISTED>
+__global__ __launch_bounds__(256, 2) void syrk_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
+                                                   int k, const mpc_syrk_panels P,
+                                                   int64_t row_stride, int tile_rows,
+                                                   const mpc_small* __restrict__ sm, int64_t npair,
+                                                   int64_t per_xcd, const syrk_shape G,
+                                                   const syrk_lists L) {
+    if (sm && sm->info != 0) return;
+    if constexpr (LISTED) {
+        const int rank = launch_rank_of(CLS, FA, FB);
+        const int count = L.base[rank];
+        const int* list = L.base + kListHead + (int64_t)rank * L.cap;
+        for (int it = blockIdx.x; it < count; it += gridDim.x)
+            syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L);
+        return;
     }
+    // XCD-aware remap: hardware places block b on XCD b % 8
+    const int64_t b = blockIdx.x;
+    const int64_t pid = (b & 7) * per_xcd + (b >> 3);
+    if (pid >= npair) return;
+    syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L);
+}
+
+template <int QA, int CLS, int FA, int FB, int KC>
+__device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                          const mpc_syrk_panels& P, int64_t row_stride,
+                                          int tile_rows, const syrk_shape& G, int64_t pid,
+                                          const syrk_lists& L) {
+    constexpr int TILE = 64 * QA;
+    int64_t ti, tj;
+    tile_of<TILE>(G, pid, ti, tj);
+    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, launch_rank_of(CLS, FA, FB));
 
     const int wave = threadIdx.x >> 6, wr = wave >> 1, wc = wave & 1;
     const bool diag = ti == tj;
@@ -774,15 +738,356 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
         } else if (c == MPC_PREC_FP16) {
             mm_16<QA, false, KC>(ocol, orow, t, k, acc);
         } else if (CLS == MPC_PREC_FP32) {
-            if constexpr (FA == 1) mm_f32<QA, KC, true, 0>(ocol, orow, t, k, acc);
-            else if constexpr (FA == 2) mm_f32<QA, KC, false, 1>(ocol, orow, t, k, acc);
-            else mm_f32<QA, KC, false, 0>(ocol, orow, t, k, acc);
+            mm_f32<QA, KC, false>(ocol, orow, t, k, acc);   // FP32 x FP16
         } else {                   // mixed-class launch: FP32 against an 8-bit or BF16 tile
-            mm_f32<QA, KC, false, 2>(ocol, orow, t, k, acc);
+            mm_f32<QA, KC, true>(ocol, orow, t, k, acc);
         }
     }
     if constexpr (!kPrefetchC) load_c<QA>(t, cv);
     store_c<QA>(t, cv, acc);
+}
+
+
+// ---------------------------------------------------------------- FP32 x FP32
+// The pairs of two FP32 tiles, with v_mfma_f32_32x32x2f32 in the K order of
+// mm_f32 (bit for bit the same sums).  The operands of 128 columns and 128
+// rows of C are staged through LDS, 16 K at a time in two buffers: four lanes
+// load a row's 64 bytes, where the matrix op's own layout (a lane per row)
+// reads 64 rows' separate lines per load, which bound the kernel (m = 16128,
+// K = 256: 832 us = 80 TFLOP/s of the 157 peak).  In LDS a block of 32 rows is in operand
+// order, two groups of 16-byte elements (k 8h .. +3 and 8h + 4 .. +7 of lane
+// half h), so a wave's operand is one 1 KB read.
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int FSK = 16;                       // K of a chunk
+constexpr int FSB = 8 * 2 * 1024;             // bytes of a buffer: 8 blocks of 2 groups
+
+__device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                              const mpc_syrk_panels& P, int64_t row_stride,
+                                              int tile_rows, const syrk_shape& G, int64_t pid,
+                                              const syrk_lists& L, char* lds) {
+    constexpr int TILE = MPC_SYRK_TILE;
+    int64_t ti, tj;
+    tile_of<TILE>(G, pid, ti, tj);
+    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+    const int rank = launch_rank_of(MPC_PREC_FP32, 1, 0);
+    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
+
+    unsigned use = 0;                        // the panels of this launch
+    int lo = 99;                             // first launch with work on the tile
+    for (int q = 0; q < P.np; ++q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+        const int r = launch_rank(prec[trow], prec[tcol]);
+        lo = r < lo ? r : lo;
+        if (r == rank) use |= 1u << q;
+    }
+    if (!use) return;
+
+    tile_ctx t;
+    t.C = C;
+    t.Cs = P.csrc && lo == rank ? P.csrc : C;
+    t.ldc = ldc;
+    t.m = m;
+    t.rowbase = ti * TILE + 64 * wr;
+    t.colbase = tj * TILE + 64 * wc;
+    t.diag = ti == tj && wr == wc;
+    // (waves without a quadrant stage and meet the barriers all the same)
+    const bool live = !(ti == tj && wr == 0 && wc == 1) && t.rowbase < m && t.colbase < m;
+
+    // staging: thread (r4, l4) moves k 4 l4 .. +3 of operand rows r4 + 64 u (u < 2:
+    // the columns of C, else its rows; past m the last row again)
+    const int l4 = tid & 3, r4 = tid >> 2;
+    char* const sd = lds + ((r4 >> 5) * 2 + (l4 & 1)) * 1024 + (l4 >> 1) * 512 + (r4 & 31) * 16;
+    v4f st[4];
+    const float* src[4];
+    auto panel = [&](int q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const int64_t roff = P.rows0 - (int64_t)q * P.nb;    // C row 0 within this panel
+        const uint8_t* pay = P.payload + slot * P.pstride + roff * row_stride + 16 * l4;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            int64_t row = (u < 2 ? tj : ti) * TILE + 64 * (u & 1) + r4;
+            if (row >= m) row = m - 1;
+            src[u] = reinterpret_cast<const float*>(pay + row * row_stride);
+        }
+    };
+    int q = __builtin_ctz(use), kc = 0;
+    bool more = true;
+    auto load = [&]() {                      // the next chunk into st
+#pragma unroll
+        for (int u = 0; u < 4; ++u) st[u] = *reinterpret_cast<const v4f*>(src[u] + kc);
+        kc += FSK;
+        if (kc >= k) {
+            use &= ~(1u << q);
+            kc = 0;
+            more = use != 0;
+            if (more) {
+                q = __builtin_ctz(use);
+                panel(q);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<v4f*>(sd + buf * FSB + u * 4096) = st[u];
+    };
+    v16f acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
+    const char* const opa = lds + (2 * wc) * 2048 + lane * 16;
+    const char* const opb = lds + (4 + 2 * wr) * 2048 + lane * 16;
+    panel(q);
+    load();
+    store(0);
+    bool staged = true;                      // a chunk is in the current buffer
+    bool held = more;                        // a chunk is in st
+    if (more) load();
+    for (int buf = 0; staged; buf ^= 1) {
+        mpc_lds_barrier();
+        if (live) {
+            v4f A[2][2], B[2][2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    A[b][g] = *reinterpret_cast<const v4f*>(opa + buf * FSB + b * 2048 + g * 1024);
+                    B[b][g] = *reinterpret_cast<const v4f*>(opb + buf * FSB + b * 2048 + g * 1024);
+                }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const float av = A[b][e >> 2][e & 3];
+                        const float bv = B[a][e >> 2][e & 3];
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[a][b], 0, 0, 0);
+                    }
+        }
+        staged = held;
+        if (held) {
+            store(buf ^ 1);                  // (last read before this chunk's barrier)
+            held = more;
+            if (more) load();
+        }
+    }
+    if (!live) return;
+    c_frag<2> cv;
+    load_c<2>(t, cv);
+    store_c<2>(t, cv, acc);
+}
+
+// ---------------------------------------------------------------- FP32 x FP8 / BF16
+// The pairs of an FP32 tile and an FP8 or BF16 one, as the three exact bf16
+// products of mm_f32 (bit for bit the same sums).  Staged as above, but as bf16
+// planes made once per workgroup: three of the FP32 side's 128 rows (hi, mid,
+// lo by truncation), one of the other side's (its values are exact in bf16).
+// In LDS a plane's 32-row block is 1 KB in operand order (16 bytes = k 8h .. +7
+// of a lane).  Split by every wave for itself from row-per-lane loads, these
+// pairs took longer than FP32 x FP32 ones.
+constexpr int SPB = 16 * 1024;                // bytes of a buffer: (3 + 1) planes of 4 blocks
+
+__device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                                const mpc_syrk_panels& P, int64_t row_stride,
+                                                int tile_rows, const syrk_shape& G, int64_t pid,
+                                                const syrk_lists& L, char* lds) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    constexpr int TILE = MPC_SYRK_TILE;
+    int64_t ti, tj;
+    tile_of<TILE>(G, pid, ti, tj);
+    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+    const int rank = launch_rank_of(MPC_PREC_FP32, 2, 0);
+    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
+
+    unsigned use = 0;                        // the panels of this launch
+    int lo = 99;                             // first launch with work on the tile
+    for (int q = 0; q < P.np; ++q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+        const int r = launch_rank(prec[trow], prec[tcol]);
+        lo = r < lo ? r : lo;
+        if (r == rank) use |= 1u << q;
+    }
+    if (!use) return;
+
+    tile_ctx t;
+    t.C = C;
+    t.Cs = P.csrc && lo == rank ? P.csrc : C;
+    t.ldc = ldc;
+    t.m = m;
+    t.rowbase = ti * TILE + 64 * wr;
+    t.colbase = tj * TILE + 64 * wc;
+    t.diag = ti == tj && wr == wc;
+    const bool live = !(ti == tj && wr == 0 && wc == 1) && t.rowbase < m && t.colbase < m;
+
+    // staging: thread (r4, l4) moves k 4 l4 .. +3 of rows r4 and r4 + 64 of each
+    // side (past m the last row again)
+    const int l4 = tid & 3, r4 = tid >> 2;
+    char* const sd = lds + (r4 >> 5) * 1024 + (l4 >> 1) * 512 + (r4 & 31) * 16 + (l4 & 1) * 8;
+    v4f sf[2];                               // the FP32 side
+    uint32_t sl[2][2];                       // the other: FP8 bytes and scale, or four BF16
+    const uint8_t *pay = nullptr, *sc = nullptr;
+    bool col32 = false;                      // of the panel being loaded
+    int plow = 0, slow = 0;                  // the other side's format: loaded panel, staged chunk
+    bool scol32 = false;
+    int64_t rf[2], rl[2];                    // rows of the two sides within the panel
+    auto panel = [&](int q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const int64_t roff = P.rows0 - (int64_t)q * P.nb;    // C row 0 within this panel
+        const uint8_t* prec = P.prec + slot * 1024 + roff / tile_rows;
+        pay = P.payload + slot * P.pstride;
+        sc = P.scales + slot * P.sstride;
+        col32 = prec[tcol] == MPC_PREC_FP32;
+        plow = col32 ? prec[trow] : prec[tcol];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int64_t c = tj * TILE + 64 * u + r4, r = ti * TILE + 64 * u + r4;
+            const int64_t cc = roff + (c < m ? c : m - 1), rc = roff + (r < m ? r : m - 1);
+            rf[u] = col32 ? cc : rc;
+            rl[u] = col32 ? rc : cc;
+        }
+    };
+    int q = __builtin_ctz(use), kc = 0;
+    bool more = true;
+    auto load = [&]() {                      // the next chunk into sf, sl
+        const int kk = kc + 4 * l4;
+        scol32 = col32;
+        slow = plow;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sf[u] = *reinterpret_cast<const v4f*>(pay + rf[u] * row_stride + 4 * kk);
+        if (plow == MPC_PREC_BF16) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const u32x2 v = *reinterpret_cast<const u32x2*>(pay + rl[u] * row_stride + 2 * kk);
+                sl[u][0] = v[0];
+                sl[u][1] = v[1];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                sl[u][0] = *reinterpret_cast<const uint32_t*>(pay + mpc_f8_offset(rl[u], kk, row_stride));
+                sl[u][1] = sc[rl[u] * (k >> 5) + (kk >> 5)];
+            }
+        }
+        kc += FSK;
+        if (kc >= k) {
+            use &= ~(1u << q);
+            kc = 0;
+            more = use != 0;
+            if (more) {
+                q = __builtin_ctz(use);
+                panel(q);
+            }
+        }
+    };
+    auto pack = [](float a, float b) {       // the leading 16 bits of each
+        return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            char* d = sd + buf * SPB + u * 2048;
+            v4f f = sf[u];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                *reinterpret_cast<u32x2*>(d + p * 4096) = u32x2{pack(f[0], f[1]), pack(f[2], f[3])};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[e] -= __uint_as_float(__float_as_uint(f[e]) & 0xffff0000u);
+            }
+            u32x2 w = {sl[u][0], sl[u][1]};
+            if (slow != MPC_PREC_BF16) {
+                const float s = mpc_dev_exp2i((int)sl[u][1] - 127);
+                v2f a, b;
+                if (mpc_dev_is_e4m3(slow)) {
+                    a = __builtin_amdgcn_cvt_pk_f32_fp8((int)sl[u][0], false);
+                    b = __builtin_amdgcn_cvt_pk_f32_fp8((int)sl[u][0], true);
+                } else {
+                    a = __builtin_amdgcn_cvt_pk_f32_bf8((int)sl[u][0], false);
+                    b = __builtin_amdgcn_cvt_pk_f32_bf8((int)sl[u][0], true);
+                }
+                w = u32x2{pack(a.x * s, a.y * s), pack(b.x * s, b.y * s)};
+            }
+            *reinterpret_cast<u32x2*>(d + 3 * 4096) = w;
+        }
+    };
+    v16f acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
+    panel(q);
+    load();
+    store(0);
+    bool col = scol32;                       // of the chunk in the current buffer
+    bool staged = true;                      // a chunk is in the current buffer
+    bool held = more;                        // a chunk is in sf, sl
+    if (more) load();
+    for (int buf = 0; staged; buf ^= 1) {
+        mpc_lds_barrier();
+        if (live) {
+            const char* o = lds + buf * SPB + lane * 16;
+            v8bf F[2][3], W[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    F[b][p] = *reinterpret_cast<const v8bf*>(o + p * 4096 + (2 * (col ? wc : wr) + b) * 1024);
+                W[b] = *reinterpret_cast<const v8bf*>(o + 3 * 4096 + (2 * (col ? wr : wc) + b) * 1024);
+            }
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        acc[a][b] = col ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(F[b][p], W[a], acc[a][b], 0, 0, 0)
+                                        : __builtin_amdgcn_mfma_f32_32x32x16_bf16(W[b], F[a][p], acc[a][b], 0, 0, 0);
+        }
+        staged = held;
+        if (held) {
+            col = scol32;
+            store(buf ^ 1);                  // (last read before this chunk's barrier)
+            held = more;
+            if (more) load();
+        }
+    }
+    if (!live) return;
+    c_frag<2> cv;
+    load_c<2>(t, cv);
+    store_c<2>(t, cv, acc);
+}
+
+// KIND 1: FP32 x FP32; 2: FP32 x FP8 / BF16 (the FA of launch_rank_of)
+template <int KIND, bool LISTED>
+__global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
+                                                          int k, const mpc_syrk_panels P,
+                                                          int64_t row_stride, int tile_rows,
+                                                          const mpc_small* __restrict__ sm, int64_t npair,
+                                                          int64_t per_xcd, const syrk_shape G,
+                                                          const syrk_lists L) {
+    __shared__ __align__(16) char lds[2 * (KIND == 1 ? FSB : SPB)];
+    if (sm && sm->info != 0) return;
+    auto tile = [&](int64_t pid) {
+        if constexpr (KIND == 1) syrk_f32_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        else syrk_split_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+    };
+    if constexpr (LISTED) {
+        const int rank = launch_rank_of(MPC_PREC_FP32, KIND, 0);
+        const int count = L.base[rank];
+        const int* list = L.base + kListHead + (int64_t)rank * L.cap;
+        for (int it = blockIdx.x; it < count; it += gridDim.x) {
+            tile(list[it]);
+            mpc_lds_barrier();               // the buffers are rewritten
+        }
+        return;
+    }
+    const int64_t b = blockIdx.x;
+    const int64_t pid = (b & 7) * per_xcd + (b >> 3);
+    if (pid < npair) tile(pid);
 }
 
 }  // namespace
@@ -839,6 +1144,19 @@ static bool syrk_geometry(int64_t m, int tile, int64_t tcol0, int64_t tcol1, syr
             hipLaunchKernelGGL((syrk_kernel<QA, CLS, FA, FB, KC, false>), g.grid, dim3(256), 0, \
                                st, C, m, ldc, k, P, row_stride, tile_rows, sm, g.npair,        \
                                g.per_xcd, g.shape, L_);                                        \
+    } while (0)
+
+#define MPC_SYRK_STAGED(KIND)                                                                  \
+    do {                                                                                       \
+        const syrk_lists L_ = next_lists();                                                    \
+        if (L_.mode == 2)                                                                      \
+            hipLaunchKernelGGL((syrk_staged_kernel<KIND, true>), list_grid, dim3(256), 0, st,  \
+                               C, m, ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd, \
+                               g.shape, L_);                                                   \
+        else                                                                                   \
+            hipLaunchKernelGGL((syrk_staged_kernel<KIND, false>), g.grid, dim3(256), 0, st, C, \
+                               m, ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd,    \
+                               g.shape, L_);                                                   \
     } while (0)
 
 // C(lower) -= Q Q^T restricted to the tile columns [tcol0, tcol1) of C, one
@@ -936,13 +1254,14 @@ int mpc_launch_syrk_panels(hipStream_t st, float* C, int64_t m, int64_t ldc, int
     if (e5) MPC_SYRK_LAUNCH(2, MPC_PREC_E4M3, 1, 1, 0);
     if (class_mask & (1u << MPC_PREC_BF16)) MPC_SYRK_LAUNCH(2, MPC_PREC_BF16, 0, 0, 0);
     if (class_mask & (1u << MPC_PREC_FP16)) MPC_SYRK_LAUNCH(2, MPC_PREC_FP16, 0, 0, 0);
-    if (f32) MPC_SYRK_LAUNCH(2, MPC_PREC_FP32, 1, 0, 0);         // FP32 x FP32
-    if (f32s) MPC_SYRK_LAUNCH(2, MPC_PREC_FP32, 2, 0, 0);        // FP32 x FP8 / BF16 (split)
+    if (f32) MPC_SYRK_STAGED(1);                                 // FP32 x FP32
+    if (f32s) MPC_SYRK_STAGED(2);                                // FP32 x FP8 / BF16 (split)
     if (f32h) MPC_SYRK_LAUNCH(2, MPC_PREC_FP32, 0, 0, 0);        // FP32 x FP16
     MPC_LAUNCH_CHECK();
     return 0;
 }
 #undef MPC_SYRK_LAUNCH
+#undef MPC_SYRK_STAGED
 
 int mpc_launch_syrk(hipStream_t st, float* C, int64_t m, int64_t ldc, int k,
                     const uint8_t* payload, int64_t row_stride, const uint8_t* scales,
