@@ -19,11 +19,16 @@
 //              (the FP32 operand split as hi + mid + lo)
 //
 // Launch: one workgroup (4 waves) per 128x128 lower tile of C, wave (wr, wc)
-// owns a 64x64 quadrant as 2x2 MFMA blocks (64x64 tiles of 1x1 blocks for the
-// look-ahead's block column).  The MFMA "row" index runs along
-// C's columns and the "column" index along C's rows, so each accumulator
-// register maps to 32 consecutive rows of the column-major C (128 B per
-// half-wave).  Block ids are remapped so consecutive tiles share an XCD.
+// owns a 64x64 quadrant as 2x2 MFMA blocks, with the operands staged through
+// LDS (one kernel per class and pair of formats); 64x64 tiles of 1x1 blocks,
+// every class in one kernel, for the look-ahead's block column.  The MFMA
+// "row" index runs along C's columns and the "column" index along C's rows, so
+// each accumulator register maps to 32 consecutive rows of the column-major C
+// (128 B per half-wave).  Block ids are remapped so consecutive tiles share an
+// XCD.  At m = 16128 an E4M3 update takes 213 us with K = 64 (C's traffic at 4.9
+// TB/s), 231 with 256, 253 with 512, 321 with 1024 (830 TFLOP/s); with operands
+// loaded by every wave for itself 222, 234, 297 and 488.  BF16 K = 512: 464 (667
+// before); FP16 437 (674).
 #include "mpc_internal.hpp"
 #include "mpc_formats.hpp"
 #include <type_traits>
@@ -271,32 +276,8 @@ __device__ __forceinline__ void operand_rows(const tile_ctx& t, int64_t ra[QA], 
     }
 }
 
-// body(kc) for kc = 0, STEP, 2 STEP, ... < k: fully unrolled when the extent
-// KC is a compile-time constant (every chunk's loads can then be issued
-// before the first product), a plain loop otherwise
-template <int KC, int STEP, typename F>
-__device__ __forceinline__ void k_loop(int k, F&& body) {
-    if constexpr (KC > 0) {
-#pragma unroll
-        for (int kc = 0; kc < KC; kc += STEP) body(kc);
-    } else {
-        for (int kc = 0; kc < k; kc += STEP) body(kc);
-    }
-}
-
-// K chunks of the 8-bit products kept in flight ahead of the chunk being
-// multiplied (register buffers; the runtime-K loop is otherwise bound by one
-// operand-load latency per 64-wide chunk)
-constexpr int kFp8Ahead = 0;
-
-template <int QA>
-struct f8_frag {
-    v8i A[QA], B[QA];
-    int sa[QA], sb[QA];
-};
-
 // FP8 class: A operand = column-side rows, B operand = row-side rows.
-template <int QA, int FA, int FB, int KC>
+template <int QA, int FA, int FB>
 __device__ __forceinline__ void mm_fp8(const operand_src& oc, const operand_src& orow,
                                        const tile_ctx& t, int k, v16f acc[QA][QA]) {
     const int h = (threadIdx.x & 63) >> 5;
@@ -318,78 +299,43 @@ __device__ __forceinline__ void mm_fp8(const operand_src& oc, const operand_src&
         ba[q] = oc.payload + (t.colbase + 32 * q) * oc.row_stride + lane32;
         bb[q] = orow.payload + (t.rowbase + 32 * q) * orow.row_stride + lane32;
     }
-    auto load = [&](int kc, f8_frag<QA>& f) {
+    for (int kc = 0; kc < k; kc += 64) {
         const int koff = kc + 32 * h;          // scale block of this lane half
         const int64_t co = (int64_t)(kc >> 6) * 2048;
+        v8i A[QA], B[QA];
+        int sa[QA], sb[QA];
 #pragma unroll
         for (int q = 0; q < QA; ++q) {
             const uint8_t* pa = ba[q] + co;
             const uint8_t* pb = bb[q] + co;
             uint4 a0 = *reinterpret_cast<const uint4*>(pa), a1 = *reinterpret_cast<const uint4*>(pa + 16);
             uint4 b0 = *reinterpret_cast<const uint4*>(pb), b1 = *reinterpret_cast<const uint4*>(pb + 16);
-            f.A[q] = v8i{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
-            f.B[q] = v8i{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-            f.sa[q] = oc.scales[ra[q] * oc.kb + (koff >> 5)];
-            f.sb[q] = orow.scales[rb[q] * orow.kb + (koff >> 5)];
+            A[q] = v8i{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
+            B[q] = v8i{(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
+            sa[q] = oc.scales[ra[q] * oc.kb + (koff >> 5)];
+            sb[q] = orow.scales[rb[q] * orow.kb + (koff >> 5)];
         }
-    };
-    auto mma = [&](const f8_frag<QA>& f) {
 #pragma unroll
         for (int a = 0; a < QA; ++a)
 #pragma unroll
             for (int b = 0; b < QA; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                    f.A[b], f.B[a], acc[a][b], FA, FB, 0, f.sa[b], 0, f.sb[a]);
-    };
-    if constexpr (KC > 0) {
-        k_loop<KC, 64>(k, [&](int kc) {
-            f8_frag<QA> f;
-            load(kc, f);
-            mma(f);
-        });
-    } else {
-        // rolling buffer of kFp8Ahead + 1 chunks; past the end, the last
-        // chunk is loaded again (branch-free) and never multiplied
-        constexpr int NB = kFp8Ahead + 1;
-        f8_frag<QA> buf[NB];
-        const int klast = k - 64;
-#pragma unroll
-        for (int i = 0; i < kFp8Ahead; ++i) load(64 * i < klast ? 64 * i : klast, buf[i]);
-        for (int kc = 0; kc < k; kc += 64 * NB) {
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const int c = kc + 64 * i;                       // chunk multiplied now
-                const int cn = c + 64 * kFp8Ahead;               // chunk loaded now
-                load(cn < klast ? cn : klast, buf[(i + kFp8Ahead) % NB]);
-                if (c < k) mma(buf[i]);
-            }
-        }
+                acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A[b], B[a], acc[a][b], FA, FB, 0,
+                                                                           sa[b], 0, sb[a]);
     }
 }
 
-template <int QA, bool BF, int KC>
+template <int QA, bool BF>
 __device__ __forceinline__ void mm_16(const operand_src& oc, const operand_src& orow,
                                       const tile_ctx& t, int k, v16f acc[QA][QA]) {
     const int h = (threadIdx.x & 63) >> 5;
     int64_t ra[QA], rb[QA];
     operand_rows<QA>(t, ra, rb);
-    const int native = BF ? MPC_PREC_BF16 : MPC_PREC_FP16;
-    auto body = [&](int kc, auto both_native) {
+    for (int kc = 0; kc < k; kc += 16) {
         const int k0 = kc + 8 * h;
         if constexpr (BF) {
             v8bf A[QA], B[QA];
 #pragma unroll
-            for (int q = 0; q < QA; ++q) {
-                if constexpr (decltype(both_native)::value) {
-                    A[q] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(
-                                                        oc.payload + ra[q] * oc.row_stride + 2 * k0));
-                    B[q] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(
-                                                        orow.payload + rb[q] * orow.row_stride + 2 * k0));
-                } else {
-                    A[q] = load8_bf16(oc, ra[q], k0);
-                    B[q] = load8_bf16(orow, rb[q], k0);
-                }
-            }
+            for (int q = 0; q < QA; ++q) { A[q] = load8_bf16(oc, ra[q], k0); B[q] = load8_bf16(orow, rb[q], k0); }
 #pragma unroll
             for (int a = 0; a < QA; ++a)
 #pragma unroll
@@ -405,16 +351,11 @@ __device__ __forceinline__ void mm_16(const operand_src& oc, const operand_src& 
                 for (int b = 0; b < QA; ++b)
                     acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[b], B[a], acc[a][b], 0, 0, 0);
         }
-    };
-    // both operands stored in the class's own format: no per-load format branch
-    if (KC > 0 && oc.prec == native && orow.prec == native)
-        k_loop<KC, 16>(k, [&](int kc) { body(kc, std::true_type{}); });
-    else
-        k_loop<0, 16>(k, [&](int kc) { body(kc, std::false_type{}); });
+    }
 }
 
 // SPLIT: FP32 against FP8/BF16 as bf16 products (else no such pair occurs)
-template <int QA, int KC, bool SPLIT>
+template <int QA, bool SPLIT>
 __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src& orow,
                                        const tile_ctx& t, int k, v16f acc[QA][QA]) {
     const int h = (threadIdx.x & 63) >> 5;
@@ -427,7 +368,7 @@ __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src&
     if (SPLIT && (oc.prec == MPC_PREC_FP32) != (orow.prec == MPC_PREC_FP32) &&
         oc.prec != MPC_PREC_FP16 && orow.prec != MPC_PREC_FP16) {
         const bool col32 = oc.prec == MPC_PREC_FP32;
-        k_loop<0, 16>(k, [&](int kc) {
+        for (int kc = 0; kc < k; kc += 16) {
             const int k0 = kc + 8 * h;
             v8bf F[QA][3], Lw[QA];
 #pragma unroll
@@ -446,67 +387,25 @@ __device__ __forceinline__ void mm_f32(const operand_src& oc, const operand_src&
                         acc[a][b] = col32
                             ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(F[b][s3], Lw[a], acc[a][b], 0, 0, 0)
                             : __builtin_amdgcn_mfma_f32_32x32x16_bf16(Lw[b], F[a][s3], acc[a][b], 0, 0, 0);
-        });
+        }
         return;
     }
     // k permutation: half h takes the 8-element groups k = 16c + 8h .. +8
-    if constexpr (KC > 0) {
-        // unrolled (small launches): branch-free loads for the all-FP32 pair
-        auto body = [&](int kc, auto both_native) {
-            const int k0 = kc + 8 * h;
-            float A[QA][8], B[QA][8];
+    for (int kc = 0; kc < k; kc += 16) {
+        const int k0 = kc + 8 * h;
+        float A[QA][8], B[QA][8];
 #pragma unroll
-            for (int q = 0; q < QA; ++q) {
-                if constexpr (decltype(both_native)::value) {
-                    const float* pa = reinterpret_cast<const float*>(oc.payload + ra[q] * oc.row_stride) + k0;
-                    const float* pb = reinterpret_cast<const float*>(orow.payload + rb[q] * orow.row_stride) + k0;
-                    const float4 a0 = *reinterpret_cast<const float4*>(pa), a1 = *reinterpret_cast<const float4*>(pa + 4);
-                    const float4 b0 = *reinterpret_cast<const float4*>(pb), b1 = *reinterpret_cast<const float4*>(pb + 4);
-                    A[q][0] = a0.x; A[q][1] = a0.y; A[q][2] = a0.z; A[q][3] = a0.w;
-                    A[q][4] = a1.x; A[q][5] = a1.y; A[q][6] = a1.z; A[q][7] = a1.w;
-                    B[q][0] = b0.x; B[q][1] = b0.y; B[q][2] = b0.z; B[q][3] = b0.w;
-                    B[q][4] = b1.x; B[q][5] = b1.y; B[q][6] = b1.z; B[q][7] = b1.w;
-                } else {
-                    load8_f32(oc, ra[q], k0, A[q]);
-                    load8_f32(orow, rb[q], k0, B[q]);
-                }
-            }
+        for (int q = 0; q < QA; ++q) { load8_f32(oc, ra[q], k0, A[q]); load8_f32(orow, rb[q], k0, B[q]); }
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < 8; ++e)
 #pragma unroll
-                for (int a = 0; a < QA; ++a)
+            for (int a = 0; a < QA; ++a)
 #pragma unroll
-                    for (int b = 0; b < QA; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[b][e], B[a][e], acc[a][b], 0, 0, 0);
-        };
-        if (oc.prec == MPC_PREC_FP32 && orow.prec == MPC_PREC_FP32)
-            k_loop<KC, 16>(k, [&](int kc) { body(kc, std::true_type{}); });
-        else
-            k_loop<KC, 16>(k, [&](int kc) { body(kc, std::false_type{}); });
-    } else {
-        // an FP32 operand against a lower format (rare): expanded per chunk
-        for (int kc = 0; kc < k; kc += 16) {
-            const int k0 = kc + 8 * h;
-            float A[QA][8], B[QA][8];
-#pragma unroll
-            for (int q = 0; q < QA; ++q) { load8_f32(oc, ra[q], k0, A[q]); load8_f32(orow, rb[q], k0, B[q]); }
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-#pragma unroll
-                for (int a = 0; a < QA; ++a)
-#pragma unroll
-                    for (int b = 0; b < QA; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[b][e], B[a][e], acc[a][b], 0, 0, 0);
-        }
+                for (int b = 0; b < QA; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[b][e], B[a][e], acc[a][b], 0, 0, 0);
     }
 }
 
-// The products of the P.np panels are summed in the accumulators (K = np*k)
-// and subtracted from C once.  CLS >= 0: only the panels whose pair on this
-// tile has that compute class (and, for the FP8 class, that element-format
-// pair FA/FB) are used, and a tile with none exits without touching C; a
-// tile mixing classes across panels is updated once per class launch.
-// CLS < 0: every panel, the class chosen per workgroup and panel.
 // Work lists of a launch sequence (int32): 16 counters indexed by launch
 // rank (launch_rank_of), then one list of tile pair ids per rank at
 // 16 + rank * cap.  The first launch of a sequence runs over every tile pair
@@ -604,15 +503,21 @@ __device__ __forceinline__ void tile_of(const syrk_shape& G, int64_t pid, int64_
     }
 }
 
-template <int QA, int CLS, int FA, int FB, int KC>
+template <int QA, bool F32H>
 __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                           const mpc_syrk_panels& P, int64_t row_stride,
                                           int tile_rows, const syrk_shape& G, int64_t pid,
                                           const syrk_lists& L);
 
+// The products of the P.np panels are summed in the accumulators (K = np*k)
+// and subtracted from C once.  F32H: only the pairs of FP32 and FP16 tiles (a
+// later launch of a sequence whose others are the staged kernels below), and
+// a tile without one exits without touching C; a tile mixing classes across
+// panels is updated once per class launch.  Otherwise every panel, the class
+// chosen per workgroup and panel.
 // LISTED: a later launch of a sequence, over its work list (L.mode 2);
 // otherwise one workgroup per tile pair (L.mode 0, or 1 to build the lists)
-template <int QA, int CLS, int FA, int FB, int KC, bool LISTED>
+template <int QA, bool F32H, bool LISTED>
 __global__ __launch_bounds__(256, 2) void syrk_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
                                                    int k, const mpc_syrk_panels P,
                                                    int64_t row_stride, int tile_rows,
@@ -621,21 +526,21 @@ __global__ __launch_bounds__(256, 2) void syrk_kernel(float* __restrict__ C, int
                                                    const syrk_lists L) {
     if (sm && sm->info != 0) return;
     if constexpr (LISTED) {
-        const int rank = launch_rank_of(CLS, FA, FB);
+        const int rank = launch_rank_of(MPC_PREC_FP32, 0, 0);
         const int count = L.base[rank];
         const int* list = L.base + kListHead + (int64_t)rank * L.cap;
         for (int it = blockIdx.x; it < count; it += gridDim.x)
-            syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L);
+            syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L);
         return;
     }
     // XCD-aware remap: hardware places block b on XCD b % 8
     const int64_t b = blockIdx.x;
     const int64_t pid = (b & 7) * per_xcd + (b >> 3);
     if (pid >= npair) return;
-    syrk_tile<QA, CLS, FA, FB, KC>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L);
+    syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L);
 }
 
-template <int QA, int CLS, int FA, int FB, int KC>
+template <int QA, bool F32H>
 __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                           const mpc_syrk_panels& P, int64_t row_stride,
                                           int tile_rows, const syrk_shape& G, int64_t pid,
@@ -644,7 +549,8 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
     int64_t ti, tj;
     tile_of<TILE>(G, pid, ti, tj);
     const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
-    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, launch_rank_of(CLS, FA, FB));
+    const int rank = launch_rank_of(MPC_PREC_FP32, 0, 0);
+    if (F32H && L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
 
     const int wave = threadIdx.x >> 6, wr = wave >> 1, wc = wave & 1;
     const bool diag = ti == tj;
@@ -665,24 +571,17 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
     for (int a = 0; a < QA; ++a)
 #pragma unroll
         for (int b2 = 0; b2 < QA; ++b2) acc[a][b2] = v16f{};
-    bool any = false;
     if (P.csrc) {
         // C's old values come from csrc in the first launch, in the host's
         // launch order, whose class covers one of this tile's panels
-        int first = 0;
-        if (CLS >= 0) {
-            int lo = 99;
-            for (int q = 0; q < P.np; ++q) {
-                const int slot = (P.p0 + q) % P.slots;
-                const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
-                const int r = launch_rank(prec[trow], prec[tcol]);
-                lo = r < lo ? r : lo;
-            }
-            first = lo == launch_rank_of(CLS, FA, FB);
-        } else {
-            first = 1;                 // one launch for every class
+        int lo = 99;
+        for (int q = 0; q < P.np; ++q) {
+            const int slot = (P.p0 + q) % P.slots;
+            const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+            const int r = launch_rank(prec[trow], prec[tcol]);
+            lo = r < lo ? r : lo;
         }
-        if (first) t.Cs = P.csrc;
+        if (!F32H || lo == rank) t.Cs = P.csrc;
     }
     // the panels this launch applies to the tile (bit q: panel q)
     auto operands = [&](int q, operand_src& orow, operand_src& ocol) {
@@ -700,19 +599,7 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
     for (int q = 0; q < P.np; ++q) {
         operand_src orow, ocol;
         operands(q, orow, ocol);
-        if (CLS >= 0) {            // this launch computes one class (and format pair) only
-            // FP32 class: FA 1 both FP32, 2 FP32 against a bf16-exact
-            // format (split products), 0 FP32 against FP16
-            const int cls = pair_class(orow.prec, ocol.prec);
-            const int fa = mpc_dev_is_e4m3(ocol.prec) ? 0 : 1, fb = mpc_dev_is_e4m3(orow.prec) ? 0 : 1;
-            const bool f32pair = orow.prec == MPC_PREC_FP32 && ocol.prec == MPC_PREC_FP32;
-            const bool f16 = orow.prec == MPC_PREC_FP16 || ocol.prec == MPC_PREC_FP16;
-            const int f32kind = f32pair ? 1 : (f16 ? 0 : 2);
-            if (cls != CLS || (CLS == MPC_PREC_E4M3 && (fa != FA || fb != FB)) ||
-                (CLS == MPC_PREC_FP32 && f32kind != FA))
-                continue;
-        }
-        use |= 1u << q;
+        if (!F32H || launch_rank(orow.prec, ocol.prec) == rank) use |= 1u << q;
     }
     if (!use) return;              // no panel of this launch's class on this tile
     // C's old values in flight during the products (64-row tiles only: at
@@ -724,23 +611,23 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
         if (!((use >> q) & 1u)) continue;
         operand_src orow, ocol;
         operands(q, orow, ocol);
-        const int cls = pair_class(orow.prec, ocol.prec);
-        const int fa = mpc_dev_is_e4m3(ocol.prec) ? 0 : 1, fb = mpc_dev_is_e4m3(orow.prec) ? 0 : 1;
-        const int c = CLS >= 0 ? CLS : cls;
-        if (c == MPC_PREC_E4M3) {
-            if (CLS >= 0) mm_fp8<QA, FA, FB, KC>(ocol, orow, t, k, acc);
-            else if (fa == 0 && fb == 0) mm_fp8<QA, 0, 0, KC>(ocol, orow, t, k, acc);
-            else if (fa == 0) mm_fp8<QA, 0, 1, KC>(ocol, orow, t, k, acc);
-            else if (fb == 0) mm_fp8<QA, 1, 0, KC>(ocol, orow, t, k, acc);
-            else mm_fp8<QA, 1, 1, KC>(ocol, orow, t, k, acc);
-        } else if (c == MPC_PREC_BF16) {
-            mm_16<QA, true, KC>(ocol, orow, t, k, acc);
-        } else if (c == MPC_PREC_FP16) {
-            mm_16<QA, false, KC>(ocol, orow, t, k, acc);
-        } else if (CLS == MPC_PREC_FP32) {
-            mm_f32<QA, KC, false>(ocol, orow, t, k, acc);   // FP32 x FP16
-        } else {                   // mixed-class launch: FP32 against an 8-bit or BF16 tile
-            mm_f32<QA, KC, true>(ocol, orow, t, k, acc);
+        if constexpr (F32H) {
+            mm_f32<QA, false>(ocol, orow, t, k, acc);
+        } else {
+            const int c = pair_class(orow.prec, ocol.prec);
+            const int fa = mpc_dev_is_e4m3(ocol.prec) ? 0 : 1, fb = mpc_dev_is_e4m3(orow.prec) ? 0 : 1;
+            if (c == MPC_PREC_E4M3) {
+                if (fa == 0 && fb == 0) mm_fp8<QA, 0, 0>(ocol, orow, t, k, acc);
+                else if (fa == 0) mm_fp8<QA, 0, 1>(ocol, orow, t, k, acc);
+                else if (fb == 0) mm_fp8<QA, 1, 0>(ocol, orow, t, k, acc);
+                else mm_fp8<QA, 1, 1>(ocol, orow, t, k, acc);
+            } else if (c == MPC_PREC_BF16) {
+                mm_16<QA, true>(ocol, orow, t, k, acc);
+            } else if (c == MPC_PREC_FP16) {
+                mm_16<QA, false>(ocol, orow, t, k, acc);
+            } else {
+                mm_f32<QA, true>(ocol, orow, t, k, acc);
+            }
         }
     }
     if constexpr (!kPrefetchC) load_c<QA>(t, cv);
@@ -888,6 +775,9 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
 // In LDS a plane's 32-row block is 1 KB in operand order (16 bytes = k 8h .. +7
 // of a lane).  Split by every wave for itself from row-per-lane loads, these
 // pairs took longer than FP32 x FP32 ones.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {      // the leading 16 bits of each
+    return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
+}
 constexpr int SPB = 16 * 1024;                // bytes of a buffer: (3 + 1) planes of 4 blocks
 
 __device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
@@ -984,9 +874,6 @@ __device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m
             }
         }
     };
-    auto pack = [](float a, float b) {       // the leading 16 bits of each
-        return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
-    };
     auto store = [&](int buf) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -994,7 +881,7 @@ __device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m
             v4f f = sf[u];
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
-                *reinterpret_cast<u32x2*>(d + p * 4096) = u32x2{pack(f[0], f[1]), pack(f[2], f[3])};
+                *reinterpret_cast<u32x2*>(d + p * 4096) = u32x2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) f[e] -= __uint_as_float(__float_as_uint(f[e]) & 0xffff0000u);
             }
@@ -1009,7 +896,7 @@ __device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m
                     a = __builtin_amdgcn_cvt_pk_f32_bf8((int)sl[u][0], false);
                     b = __builtin_amdgcn_cvt_pk_f32_bf8((int)sl[u][0], true);
                 }
-                w = u32x2{pack(a.x * s, a.y * s), pack(b.x * s, b.y * s)};
+                w = u32x2{pack_bf16(a.x * s, a.y * s), pack_bf16(b.x * s, b.y * s)};
             }
             *reinterpret_cast<u32x2*>(d + 3 * 4096) = w;
         }
@@ -1061,24 +948,349 @@ __device__ __forceinline__ void syrk_split_tile(float* __restrict__ C, int64_t m
     store_c<2>(t, cv, acc);
 }
 
-// KIND 1: FP32 x FP32; 2: FP32 x FP8 / BF16 (the FA of launch_rank_of)
-template <int KIND, bool LISTED>
+// ---------------------------------------------------------------- FP8 x FP8
+// The pairs of two 8-bit tiles with element formats FA (columns) and FB (rows),
+// v_mfma_scale_f32_32x32x64_f8f6f4 in the K order of mm_fp8 (bit for bit the
+// same sums).  The payload is in operand order already; staging it means that
+// a workgroup reads each operand once instead of twice, and that three chunks
+// of 64 K are in flight: two in registers, one in the LDS buffer being filled.
+// A block of 32 rows is 2 KB per chunk, the lanes' first 16 bytes and then
+// their second, so that every read is 1 KB in lane order.  The chunk's two
+// scale bytes of a row go through LDS as well.
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+constexpr int F8B = 8 * 2048 + 512;           // bytes of a buffer: 8 blocks, 256 rows' scales
+
+template <int FA, int FB>
+__device__ __forceinline__ void syrk_f8_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                             const mpc_syrk_panels& P, int64_t row_stride,
+                                             int tile_rows, const syrk_shape& G, int64_t pid,
+                                             const syrk_lists& L, char* lds) {
+    constexpr int TILE = MPC_SYRK_TILE;
+    int64_t ti, tj;
+    tile_of<TILE>(G, pid, ti, tj);
+    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+    const int rank = launch_rank_of(MPC_PREC_E4M3, FA, FB);
+    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
+
+    unsigned use = 0;                        // the panels of this launch
+    int lo = 99;                             // first launch with work on the tile
+    for (int q = 0; q < P.np; ++q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+        const int r = launch_rank(prec[trow], prec[tcol]);
+        lo = r < lo ? r : lo;
+        if (r == rank) use |= 1u << q;
+    }
+    if (!use) return;
+
+    tile_ctx t;
+    t.C = C;
+    t.Cs = P.csrc && lo == rank ? P.csrc : C;
+    t.ldc = ldc;
+    t.m = m;
+    t.rowbase = ti * TILE + 64 * wr;
+    t.colbase = tj * TILE + 64 * wc;
+    t.diag = ti == tj && wr == wc;
+    const bool live = !(ti == tj && wr == 0 && wc == 1) && t.rowbase < m && t.colbase < m;
+
+    // staging: wave w moves blocks 2w and 2w + 1 (blocks 0..3 the columns of C,
+    // 4..7 its rows; past m the last one again), lane l 32 bytes of each; thread
+    // t the scales of operand row t
+    const int64_t bmax = (m - 1) & ~(int64_t)31;
+    int64_t blk[2], srow;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int b = 2 * wave + u;
+        const int64_t r = (b < 4 ? tj : ti) * TILE + 32 * (b & 3);
+        blk[u] = r < bmax ? r : bmax;
+    }
+    srow = (tid < 128 ? tj : ti) * TILE + (tid & 127);
+    if (srow >= m) srow = m - 1;
+    v4u st[2][2][2];                       // [set][block][half]
+    uint32_t ss[2];
+    const uint8_t *pb[2] = {}, *ps = nullptr;
+    auto panel = [&](int q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const int64_t roff = P.rows0 - (int64_t)q * P.nb;    // C row 0 within this panel
+        const uint8_t* pay = P.payload + slot * P.pstride;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) pb[u] = pay + (roff + blk[u]) * row_stride + lane * 32;
+        ps = P.scales + slot * P.sstride + (roff + srow) * (k >> 5);
+    };
+    int q = __builtin_ctz(use), kc = 0;
+    int left = 0;                            // chunks not loaded yet
+    for (unsigned v = use; v; v &= v - 1) left += k >> 6;
+    auto load = [&](v4u (&v)[2][2], uint32_t& s) {         // the next chunk
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+                v[u][g] = *reinterpret_cast<const v4u*>(pb[u] + (int64_t)(kc >> 6) * 2048 + 16 * g);
+        s = *reinterpret_cast<const uint16_t*>(ps + (kc >> 5));
+        --left;
+        kc += 64;
+        if (kc >= k) {
+            use &= ~(1u << q);
+            kc = 0;
+            if (use) {
+                q = __builtin_ctz(use);
+                panel(q);
+            }
+        }
+    };
+    auto store = [&](const v4u (&v)[2][2], uint32_t s, int buf) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+                *reinterpret_cast<v4u*>(lds + buf * F8B + (2 * wave + u) * 2048 + g * 1024 + lane * 16) = v[u][g];
+        *reinterpret_cast<uint16_t*>(lds + buf * F8B + 8 * 2048 + 2 * tid) = (uint16_t)s;
+    };
+    v16f acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
+    auto operand = [&](const char* o) {
+        const v4u x = *reinterpret_cast<const v4u*>(o), y = *reinterpret_cast<const v4u*>(o + 1024);
+        return v8i{(int)x[0], (int)x[1], (int)x[2], (int)x[3], (int)y[0], (int)y[1], (int)y[2], (int)y[3]};
+    };
+    auto multiply = [&](int buf) {
+        const char* o = lds + buf * F8B;
+        const char* s = o + 8 * 2048 + 2 * (lane & 31) + (lane >> 5);
+        v8i A[2], B[2];
+        int sa[2], sb[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            A[b] = operand(o + (2 * wc + b) * 2048 + lane * 16);
+            B[b] = operand(o + (4 + 2 * wr + b) * 2048 + lane * 16);
+            sa[b] = *reinterpret_cast<const uint8_t*>(s + 64 * (2 * wc + b));
+            sb[b] = *reinterpret_cast<const uint8_t*>(s + 64 * (4 + 2 * wr + b));
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                    A[b], B[a], acc[a][b], FA, FB, 0, sa[b], 0, sb[a]);
+    };
+    panel(q);
+    int todo = left;                         // chunks not multiplied yet
+    load(st[0], ss[0]);
+    if (left) load(st[1], ss[1]);
+    store(st[0], ss[0], 0);
+    if (left) load(st[0], ss[0]);
+    // chunk c is in buffer c & 1, c + 1 in set (c + 1) & 1, c + 2 in set c & 1
+    for (;;) {
+        mpc_lds_barrier();
+        if (todo > 1) {
+            store(st[1], ss[1], 1);
+            if (left) load(st[1], ss[1]);
+        }
+        if (live) multiply(0);
+        if (--todo == 0) break;
+        mpc_lds_barrier();
+        if (todo > 1) {
+            store(st[0], ss[0], 0);
+            if (left) load(st[0], ss[0]);
+        }
+        if (live) multiply(1);
+        if (--todo == 0) break;
+    }
+    if (!live) return;
+    c_frag<2> cv;
+    load_c<2>(t, cv);
+    store_c<2>(t, cv, acc);
+}
+
+// ---------------------------------------------------------------- 16-bit classes
+// The pairs of the BF16 class (BF16 or FP8 tiles, at least one BF16; CLS BF16)
+// and of two FP16 tiles (CLS FP16), in the K order of mm_16 (bit for bit the
+// same sums), staged like the bf16 planes above with one plane a side.
+constexpr int S16B = 8 * 1024;                // bytes of a buffer
+
+template <int CLS>
+__device__ __forceinline__ void syrk_16_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
+                                             const mpc_syrk_panels& P, int64_t row_stride,
+                                             int tile_rows, const syrk_shape& G, int64_t pid,
+                                             const syrk_lists& L, char* lds) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    constexpr int TILE = MPC_SYRK_TILE;
+    int64_t ti, tj;
+    tile_of<TILE>(G, pid, ti, tj);
+    const int64_t trow = (ti * TILE) / tile_rows, tcol = (tj * TILE) / tile_rows;
+    const int rank = launch_rank_of(CLS, 0, 0);
+    if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
+
+    unsigned use = 0;                        // the panels of this launch
+    int lo = 99;                             // first launch with work on the tile
+    for (int q = 0; q < P.np; ++q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
+        const int r = launch_rank(prec[trow], prec[tcol]);
+        lo = r < lo ? r : lo;
+        if (r == rank) use |= 1u << q;
+    }
+    if (!use) return;
+
+    tile_ctx t;
+    t.C = C;
+    t.Cs = P.csrc && lo == rank ? P.csrc : C;
+    t.ldc = ldc;
+    t.m = m;
+    t.rowbase = ti * TILE + 64 * wr;
+    t.colbase = tj * TILE + 64 * wc;
+    t.diag = ti == tj && wr == wc;
+    const bool live = !(ti == tj && wr == 0 && wc == 1) && t.rowbase < m && t.colbase < m;
+
+    // staging: thread (r4, l4) moves k 4 l4 .. +3 of operand rows r4 + 64 u (u < 2:
+    // the columns of C, else its rows; past m the last row again)
+    const int l4 = tid & 3, r4 = tid >> 2;
+    char* const sd = lds + (r4 >> 5) * 1024 + (l4 >> 1) * 512 + (r4 & 31) * 16 + (l4 & 1) * 8;
+    uint32_t st[4][2];                       // four 16-bit values, or FP8 bytes and scale
+    const uint8_t *pay = nullptr, *sc = nullptr;
+    int pf[2] = {0, 0}, sf[2] = {0, 0};      // formats of the sides: loaded panel, staged chunk
+    int64_t row[4];
+    auto panel = [&](int q) {
+        const int slot = (P.p0 + q) % P.slots;
+        const int64_t roff = P.rows0 - (int64_t)q * P.nb;    // C row 0 within this panel
+        const uint8_t* prec = P.prec + slot * 1024 + roff / tile_rows;
+        pay = P.payload + slot * P.pstride;
+        sc = P.scales + slot * P.sstride;
+        pf[0] = prec[tcol];
+        pf[1] = prec[trow];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t r = (u < 2 ? tj : ti) * TILE + 64 * (u & 1) + r4;
+            row[u] = roff + (r < m ? r : m - 1);
+        }
+    };
+    int q = __builtin_ctz(use), kc = 0;
+    bool more = true;
+    auto load = [&]() {                      // the next chunk into st
+        const int kk = kc + 4 * l4;
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            sf[side] = pf[side];
+            if (CLS == MPC_PREC_FP16 || pf[side] == MPC_PREC_BF16) {
+#pragma unroll
+                for (int u = 2 * side; u < 2 * side + 2; ++u) {
+                    const u32x2 v = *reinterpret_cast<const u32x2*>(pay + row[u] * row_stride + 2 * kk);
+                    st[u][0] = v[0];
+                    st[u][1] = v[1];
+                }
+            } else {
+#pragma unroll
+                for (int u = 2 * side; u < 2 * side + 2; ++u) {
+                    st[u][0] = *reinterpret_cast<const uint32_t*>(pay + mpc_f8_offset(row[u], kk, row_stride));
+                    st[u][1] = sc[row[u] * (k >> 5) + (kk >> 5)];
+                }
+            }
+        }
+        kc += FSK;
+        if (kc >= k) {
+            use &= ~(1u << q);
+            kc = 0;
+            more = use != 0;
+            if (more) {
+                q = __builtin_ctz(use);
+                panel(q);
+            }
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            u32x2 w = {st[u][0], st[u][1]};
+            if (CLS != MPC_PREC_FP16 && sf[u >> 1] != MPC_PREC_BF16) {
+                const float s = mpc_dev_exp2i((int)st[u][1] - 127);
+                v2f a, b;
+                if (mpc_dev_is_e4m3(sf[u >> 1])) {
+                    a = __builtin_amdgcn_cvt_pk_f32_fp8((int)st[u][0], false);
+                    b = __builtin_amdgcn_cvt_pk_f32_fp8((int)st[u][0], true);
+                } else {
+                    a = __builtin_amdgcn_cvt_pk_f32_bf8((int)st[u][0], false);
+                    b = __builtin_amdgcn_cvt_pk_f32_bf8((int)st[u][0], true);
+                }
+                w = u32x2{pack_bf16(a.x * s, a.y * s), pack_bf16(b.x * s, b.y * s)};
+            }
+            *reinterpret_cast<u32x2*>(sd + buf * S16B + u * 2048) = w;
+        }
+    };
+    v16f acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
+    panel(q);
+    load();
+    store(0);
+    bool staged = true;                      // a chunk is in the current buffer
+    bool held = more;                        // a chunk is in st
+    if (more) load();
+    for (int buf = 0; staged; buf ^= 1) {
+        mpc_lds_barrier();
+        if (live) {
+            const char* o = lds + buf * S16B + lane * 16;
+            v4u A[2], B[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                A[b] = *reinterpret_cast<const v4u*>(o + (2 * wc + b) * 1024);
+                B[b] = *reinterpret_cast<const v4u*>(o + (4 + 2 * wr + b) * 1024);
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    if constexpr (CLS == MPC_PREC_FP16)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            __builtin_bit_cast(v8h, A[b]), __builtin_bit_cast(v8h, B[a]), acc[a][b], 0, 0, 0);
+                    else
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(v8bf, A[b]), __builtin_bit_cast(v8bf, B[a]), acc[a][b], 0, 0, 0);
+                }
+        }
+        staged = held;
+        if (held) {
+            store(buf ^ 1);                  // (last read before this chunk's barrier)
+            held = more;
+            if (more) load();
+        }
+    }
+    if (!live) return;
+    c_frag<2> cv;
+    load_c<2>(t, cv);
+    store_c<2>(t, cv, acc);
+}
+
+// The staged kernels by launch rank: 0-3 FP8 element pairs, 4 BF16, 5 FP16,
+// 6 FP32 x FP32, 7 FP32 x FP8 / BF16.
+template <int RANK, bool LISTED>
 __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
                                                           int k, const mpc_syrk_panels P,
                                                           int64_t row_stride, int tile_rows,
                                                           const mpc_small* __restrict__ sm, int64_t npair,
                                                           int64_t per_xcd, const syrk_shape G,
                                                           const syrk_lists L) {
-    __shared__ __align__(16) char lds[2 * (KIND == 1 ? FSB : SPB)];
+    constexpr int kBuf = RANK < 4 ? F8B : RANK < 6 ? S16B : RANK == 6 ? FSB : SPB;
+    __shared__ __align__(16) char lds[2 * kBuf];
     if (sm && sm->info != 0) return;
     auto tile = [&](int64_t pid) {
-        if constexpr (KIND == 1) syrk_f32_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
-        else syrk_split_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        if constexpr (RANK < 4)
+            syrk_f8_tile<RANK / 2, RANK % 2>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        else if constexpr (RANK < 6)
+            syrk_16_tile<RANK == 4 ? MPC_PREC_BF16 : MPC_PREC_FP16>(C, m, ldc, k, P, row_stride, tile_rows,
+                                                                    G, pid, L, lds);
+        else if constexpr (RANK == 6)
+            syrk_f32_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        else
+            syrk_split_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
     };
     if constexpr (LISTED) {
-        const int rank = launch_rank_of(MPC_PREC_FP32, KIND, 0);
-        const int count = L.base[rank];
-        const int* list = L.base + kListHead + (int64_t)rank * L.cap;
+        const int count = L.base[RANK];
+        const int* list = L.base + kListHead + (int64_t)RANK * L.cap;
         for (int it = blockIdx.x; it < count; it += gridDim.x) {
             tile(list[it]);
             mpc_lds_barrier();               // the buffers are rewritten
@@ -1133,29 +1345,17 @@ static bool syrk_geometry(int64_t m, int tile, int64_t tcol0, int64_t tcol1, syr
     return true;
 }
 
-#define MPC_SYRK_LAUNCH(QA, CLS, FA, FB, KC)                                                   \
+// MPC_SYRK_LAUNCH(KERNEL, template arguments but LISTED)
+#define MPC_SYRK_LAUNCH(KERNEL, ...)                                                           \
     do {                                                                                       \
         const syrk_lists L_ = next_lists();                                                    \
         if (L_.mode == 2)                                                                      \
-            hipLaunchKernelGGL((syrk_kernel<QA, CLS, FA, FB, KC, true>), list_grid, dim3(256), \
-                               0, st, C, m, ldc, k, P, row_stride, tile_rows, sm, g.npair,     \
-                               g.per_xcd, g.shape, L_);                                        \
-        else                                                                                   \
-            hipLaunchKernelGGL((syrk_kernel<QA, CLS, FA, FB, KC, false>), g.grid, dim3(256), 0, \
-                               st, C, m, ldc, k, P, row_stride, tile_rows, sm, g.npair,        \
-                               g.per_xcd, g.shape, L_);                                        \
-    } while (0)
-
-#define MPC_SYRK_STAGED(KIND)                                                                  \
-    do {                                                                                       \
-        const syrk_lists L_ = next_lists();                                                    \
-        if (L_.mode == 2)                                                                      \
-            hipLaunchKernelGGL((syrk_staged_kernel<KIND, true>), list_grid, dim3(256), 0, st,  \
-                               C, m, ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd, \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, true>), list_grid, dim3(256), 0, st, C, m, \
+                               ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd,       \
                                g.shape, L_);                                                   \
         else                                                                                   \
-            hipLaunchKernelGGL((syrk_staged_kernel<KIND, false>), g.grid, dim3(256), 0, st, C, \
-                               m, ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd,    \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, false>), g.grid, dim3(256), 0, st, C, m,   \
+                               ldc, k, P, row_stride, tile_rows, sm, g.npair, g.per_xcd,       \
                                g.shape, L_);                                                   \
     } while (0)
 
@@ -1221,9 +1421,8 @@ int mpc_launch_syrk_panels(hipStream_t st, float* C, int64_t m, int64_t ldc, int
         // unrolled for k = 256 took 240 VGPRs (two workgroups per CU, two
         // rounds of workgroups at the first steps); the runtime-k loop takes
         // 152 (three per CU) and made the solve 0.3 ms faster.
-        const dim3 list_grid = g.grid;
-        auto next_lists = [&]() { return none; };
-        MPC_SYRK_LAUNCH(1, -1, 0, 0, 0);
+        hipLaunchKernelGGL((syrk_kernel<1, false, false>), g.grid, dim3(256), 0, st, C, m, ldc, k, P,
+                           row_stride, tile_rows, sm, g.npair, g.per_xcd, g.shape, none);
         MPC_LAUNCH_CHECK();
         return 0;
     }
@@ -1249,19 +1448,21 @@ int mpc_launch_syrk_panels(hipStream_t st, float* C, int64_t m, int64_t ldc, int
         ++launched;
         return L;
     };
-    if (e4) MPC_SYRK_LAUNCH(2, MPC_PREC_E4M3, 0, 0, 0);
-    if (e4 && e5) { MPC_SYRK_LAUNCH(2, MPC_PREC_E4M3, 0, 1, 0); MPC_SYRK_LAUNCH(2, MPC_PREC_E4M3, 1, 0, 0); }
-    if (e5) MPC_SYRK_LAUNCH(2, MPC_PREC_E4M3, 1, 1, 0);
-    if (class_mask & (1u << MPC_PREC_BF16)) MPC_SYRK_LAUNCH(2, MPC_PREC_BF16, 0, 0, 0);
-    if (class_mask & (1u << MPC_PREC_FP16)) MPC_SYRK_LAUNCH(2, MPC_PREC_FP16, 0, 0, 0);
-    if (f32) MPC_SYRK_STAGED(1);                                 // FP32 x FP32
-    if (f32s) MPC_SYRK_STAGED(2);                                // FP32 x FP8 / BF16 (split)
-    if (f32h) MPC_SYRK_LAUNCH(2, MPC_PREC_FP32, 0, 0, 0);        // FP32 x FP16
+    if (e4) MPC_SYRK_LAUNCH(syrk_staged_kernel, 0);
+    if (e4 && e5) {
+        MPC_SYRK_LAUNCH(syrk_staged_kernel, 1);
+        MPC_SYRK_LAUNCH(syrk_staged_kernel, 2);
+    }
+    if (e5) MPC_SYRK_LAUNCH(syrk_staged_kernel, 3);
+    if (class_mask & (1u << MPC_PREC_BF16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 4);
+    if (class_mask & (1u << MPC_PREC_FP16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 5);
+    if (f32) MPC_SYRK_LAUNCH(syrk_staged_kernel, 6);             // FP32 x FP32
+    if (f32s) MPC_SYRK_LAUNCH(syrk_staged_kernel, 7);            // FP32 x FP8 / BF16 (split)
+    if (f32h) MPC_SYRK_LAUNCH(syrk_kernel, 2, true);             // FP32 x FP16
     MPC_LAUNCH_CHECK();
     return 0;
 }
 #undef MPC_SYRK_LAUNCH
-#undef MPC_SYRK_STAGED
 
 int mpc_launch_syrk(hipStream_t st, float* C, int64_t m, int64_t ldc, int k,
                     const uint8_t* payload, int64_t row_stride, const uint8_t* scales,
