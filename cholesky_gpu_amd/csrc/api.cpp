@@ -533,16 +533,21 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     hipStream_t st = h->stream;
     int rc;
     if ((rc = wait_winv(h, st))) return rc;       // it reads dinv and the factor
-    // panels live in a ring: 2 buffers, or 2 * agg_panels when the updates
-    // beyond a group of agg_panels block columns are aggregated (the group
-    // being aggregated and the group being factored)
+    // panels live in a ring: 2 buffers, or 2 * PG * agg_panels when the updates
+    // beyond a group of agg_panels block columns are aggregated (the PG groups
+    // being aggregated and the groups being factored meanwhile)
     const bool prof = o->profile != 0;
     const int AG = agg_panels_of(o);
     if (first_src && (AG < 2 || (int64_t)AG * nb >= n)) {
         mpc_set_error("factor: a deferred copy needs the aggregated schedule");
         return MPC_ERR_ARG;
     }
-    const int nslot = 2 * AG;
+    // groups whose far updates go together: two, unless every update is FP32
+    // (bound by the matrix cores, not by C's traffic; n = 16384: 22.1 ms a solve
+    // with one, 22.7 with two, where E4M3/FP32 switching takes 15.08 and 14.66 and
+    // the 60000-point MXFP8 solve 446 and 367) or the panel ring has no room
+    const int PG = AG == 2 && o->update_prec != MPC_PREC_FP32 ? 2 : 1;
+    const int nslot = 2 * PG * AG;
     if ((rc = mpc_ws_reserve(h->panel, (size_t)nslot * (n + 128) * nb * 4))) return rc;
     if ((rc = mpc_ws_reserve(h->scales, (size_t)nslot * (n + 128) * (nb / 32)))) return rc;
     if ((rc = mpc_ws_reserve(h->dinv, (size_t)(nt * nb / 32 + 8) * 1024 * sizeof(float)))) return rc;
@@ -628,6 +633,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         P.p0 = (int)(p0 % nslot);
         P.np = np;
         P.nb = nb;
+        // (panel 0 is in the first update of every column beyond its group)
         P.csrc = (first_src && p0 == 0) ? first_src + e + e * lda : nullptr;
         return mpc_launch_syrk_panels(us, dA + e + e * lda, n - e, lda, nb, P, (int64_t)nb * 4, tr,
                                       sm, t0, t1, qa, cmask, fmask, lists_of(us));
@@ -656,13 +662,20 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // One-deep look-ahead with aggregated far updates.  Block columns
         // come in groups of AG.  Inside a group, as below: panel j updates
         // block column j+1 on pstream and the rest of the group's columns on
-        // st.  The columns beyond the group are updated once per group with
-        // all AG panels (K = AG nb): block column E (the next group's first)
-        // on pstream, the rest of the next group on st, everything beyond
-        // that on fstream, where it overlaps the next group's panels.
+        // st.  The columns beyond the group are updated with all AG panels of
+        // the group (K = AG nb): block column E (the next group's first) on
+        // pstream, the rest of the next group on st, everything beyond that
+        // on fstream, where it overlaps the next groups' panels.
+        // With PG = 2 the columns beyond the next two groups take two groups'
+        // panels at once (K = 2 AG nb), which halves the traffic of C that
+        // bounds those updates: after an even group fstream updates only the
+        // strip of the group after next; after an odd one the next group but
+        // one first (the chain waits for it at the end of the next group),
+        // then the rest, each with both groups.
         // Ordering: a writer of a block column waits for its previous writer
-        // (ev_bulk: st's last update; ev_far: fstream's last); a panel slot
-        // is reused AG panels after the group that read it was aggregated.
+        // (ev_bulk: st's last update; ev_far: fstream's last update of the
+        // group that the chain enters next); a panel slot is reused 2 PG AG
+        // panels later, after the updates that read it.
         hipStream_t ps = h->pstream, fs = h->fstream;
         MPC_HIP(hipEventRecord(h->ev_col, st));
         MPC_HIP(hipStreamWaitEvent(ps, h->ev_col, 0));
@@ -675,6 +688,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // costs several microseconds of the chain even when the event is
         // long complete, so ps waits only for st work it has not seen
         bool bulk_seen = true;
+        const int64_t gt = (int64_t)AG * nb / MPC_SYRK_TILE;      // SYRK tiles of a group
         for (int64_t j = 0; j + 1 < nt; ++j) {
             const int64_t g = j / AG, E = std::min<int64_t>((g + 1) * AG, nt);
             const int64_t bs1 = std::min<int64_t>(nb, n - (j + 1) * nb);
@@ -703,12 +717,20 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 MPC_HIP(hipEventRecord(h->ev_panel, ps));
                 MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
                 MPC_HIP(hipStreamWaitEvent(fs, h->ev_panel, 0));
-                if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, (int64_t)AG * nb / MPC_SYRK_TILE, st, 2)))
-                    return rc;
+                if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, gt, st, 2))) return rc;
                 MPC_HIP(hipEventRecord(h->ev_bulk, st));
                 bulk_seen = false;
-                if ((rc = agg(p0, np, E, (int64_t)AG * nb / MPC_SYRK_TILE, -1, fs, 2))) return rc;
-                MPC_HIP(hipEventRecord(h->ev_far, fs));
+                if (PG == 1) {
+                    if ((rc = agg(p0, np, E, gt, -1, fs, 2))) return rc;
+                    MPC_HIP(hipEventRecord(h->ev_far, fs));
+                } else if (g % 2 == 0) {
+                    if ((rc = agg(p0, np, E, gt, 2 * gt, fs, 2))) return rc;
+                    MPC_HIP(hipEventRecord(h->ev_far, fs));
+                } else {
+                    if ((rc = agg(p0 - AG, 2 * AG, E, gt, 2 * gt, fs, 2))) return rc;
+                    MPC_HIP(hipEventRecord(h->ev_far, fs));
+                    if ((rc = agg(p0 - AG, 2 * AG, E, 2 * gt, -1, fs, 2))) return rc;
+                }
                 far_pending = true;
             }
             if ((rc = panel(j + 1, ps))) return rc;
@@ -716,7 +738,10 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         }
         MPC_HIP(hipEventRecord(h->ev_panel, ps));
         MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
-        if (far_pending) MPC_HIP(hipStreamWaitEvent(st, h->ev_far, 0));
+        if (far_pending) {
+            MPC_HIP(hipEventRecord(h->ev_far, fs));
+            MPC_HIP(hipStreamWaitEvent(st, h->ev_far, 0));
+        }
     } else if (!prof) {
         // One-deep look-ahead.  pstream carries the critical chain: the update
         // of block column j+1 by panel j (one mixed-class launch of small

@@ -39,3 +39,25 @@ def test_staged_updates(handle, oracle, m, k, first, other):
     assert err[low & ~pair8].max(initial=0.0) <= k * 2.0 ** -24
     assert err[low & pair8].max(initial=0.0) < 1e-4
     assert np.array_equal(np.triu(got, 1), np.triu(Cm, 1))
+
+
+@pytest.mark.parametrize("n", [1024, 1280, 1600, 2304, 2816])
+@pytest.mark.parametrize("prec", [L.PREC_BF16, L.PREC_MXE4M3])
+def test_factor_group_pairs(handle, n, prec):
+    """Two-group far updates (4 to 11 block columns of 256: groups without,
+    with one and with several pairs, full and partial last ones): the backward
+    error of the factor is that of the per-panel updates (agg_panels = 1) up
+    to 10 %, and two runs agree bit for bit."""
+    print("[case]", n, L.PREC_NAMES[prec], flush=True)
+    A, _ = S.matgen_householder(handle, n, cond=20.0, lam_max=20.0, seed=n)
+    err, outs = {}, []
+    for agg in (1, 2, 2):
+        T = A.clone()
+        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=256, update_prec=prec, ladder=(prec,),
+                                                        fallback=0, agg_panels=agg))
+        assert rc == 0
+        L64 = torch.triu(T).to(torch.float64).T.contiguous()
+        err[agg] = float((L64 @ L64.T.contiguous() - A.to(torch.float64)).norm() / A.to(torch.float64).norm())
+        outs.append(T)
+    assert torch.equal(outs[1], outs[2])
+    assert err[2] <= 1.1 * err[1], err
