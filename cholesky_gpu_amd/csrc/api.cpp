@@ -653,12 +653,46 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         return mpc_build_block_inverses_range(h->wstream, dA, lda, n, Bo, dinv, W, WT, I, I + 1);
     };
 
+    // The last kOneStream columns go on one stream: panel, then its whole
+    // trailing update, with no event in between.  There the update is no
+    // longer than the waits that overlapping it would take (5..10 us for each
+    // event on the chain, and as much of host time).  Measured as whole
+    // factors, overlapped and on one stream: n = 4096, nb = 128 FP32 2181 and
+    // 1670 us, E4M3/FP32 1750 and 1393, nb = 256 FP32 1784 and 1590; n = 768,
+    // nb = 64 570 and 405.  Beyond it the update is the longer part: the last
+    // 8192 columns of n = 16384 that way cost an FP32 solve 21.3 -> 21.7 ms,
+    // E4M3/FP32 14.01 -> 14.28.
+    constexpr int64_t kOneStream = 4096;
+    // FP32-only updates of at least kWide columns take the 128-row kernel (too
+    // few workgroups for the chip below: n = 4000 factor 1774 us without it,
+    // 1754, 1717, 1696, 1694 and 1713 from 1024, 1536, 2048, 2560 and 3072)
+    constexpr int64_t kWide = 2304;
+    auto one_stream = [&](int64_t j0, hipStream_t ps) -> int {
+        for (int64_t j = j0; j + 1 < nt; ++j) {
+            const int wide = n - (j + 1) * nb >= kWide && cmask == (1u << MPC_PREC_FP32);
+            int r;
+            if ((r = AG > 1 ? agg(j, 1, j + 1, 0, -1, ps, wide ? 2 : 1)
+                            : update(j, 0, -1, ps, !wide)))
+                return r;
+            if ((r = panel(j + 1, ps))) return r;
+            if ((r = build_w(j + 1, ps))) return r;
+        }
+        return 0;
+    };
+
     double tp = 0, tt = 0, tq = 0, ts = 0;
     owned_events<2> tev;
     if ((rc = tev.create())) return rc;
     hipEvent_t e0 = tev.e[0], e1 = tev.e[1];
     MPC_HIP(hipEventRecord(e0, st));
-    if (!prof && AG > 1) {
+    if (!prof && n <= kOneStream) {
+        // (wstream: the inverses of an earlier factor were waited for on st)
+        MPC_HIP(hipEventRecord(h->ev_col, st));
+        MPC_HIP(hipStreamWaitEvent(h->wstream, h->ev_col, 0));
+        if ((rc = panel(0, st))) return rc;
+        if ((rc = build_w(0, st))) return rc;
+        if ((rc = one_stream(0, st))) return rc;
+    } else if (!prof && AG > 1) {
         // One-deep look-ahead with aggregated far updates.  Block columns
         // come in groups of AG.  Inside a group, as below: panel j updates
         // block column j+1 on pstream and the rest of the group's columns on
@@ -672,6 +706,9 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // strip of the group after next; after an odd one the next group but
         // one first (the chain waits for it at the end of the next group),
         // then the rest, each with both groups.
+        // The next panel is enqueued before the updates on st and fstream: the
+        // chain does not wait for the host to issue those, and POTRF's one
+        // workgroup gets a CU before their thousands.
         // Ordering: a writer of a block column waits for its previous writer
         // (ev_bulk: st's last update; ev_far: fstream's last update of the
         // group that the chain enters next); a panel slot is reused 2 PG AG
@@ -689,7 +726,9 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // long complete, so ps waits only for st work it has not seen
         bool bulk_seen = true;
         const int64_t gt = (int64_t)AG * nb / MPC_SYRK_TILE;      // SYRK tiles of a group
-        for (int64_t j = 0; j + 1 < nt; ++j) {
+        int64_t j = 0;
+        for (; j + 1 < nt; ++j) {
+            if (j % (PG * AG) == 0 && n - j * nb <= kOneStream) break;
             const int64_t g = j / AG, E = std::min<int64_t>((g + 1) * AG, nt);
             const int64_t bs1 = std::min<int64_t>(nb, n - (j + 1) * nb);
             const int64_t split = (bs1 + MPC_SYRK_TILE - 1) / MPC_SYRK_TILE;
@@ -701,8 +740,9 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 // inside the group: block column j+1, then the group's other columns
                 if ((rc = update(j, 0, 2 * split, ps, 1))) return rc;
                 const int64_t wend = (E - (j + 1)) * nb / MPC_SYRK_TILE;
+                if (wend > split) MPC_HIP(hipEventRecord(h->ev_panel, ps));
+                if ((rc = panel(j + 1, ps))) return rc;
                 if (wend > split) {
-                    MPC_HIP(hipEventRecord(h->ev_panel, ps));
                     MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
                     if ((rc = update(j, split, wend, st, 0))) return rc;
                     MPC_HIP(hipEventRecord(h->ev_bulk, st));
@@ -715,6 +755,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 if (far_pending) MPC_HIP(hipStreamWaitEvent(ps, h->ev_far, 0));
                 if ((rc = agg(p0, np, E, 0, nb / 64, ps, 1))) return rc;
                 MPC_HIP(hipEventRecord(h->ev_panel, ps));
+                if ((rc = panel(j + 1, ps))) return rc;
                 MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
                 MPC_HIP(hipStreamWaitEvent(fs, h->ev_panel, 0));
                 if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, gt, st, 2))) return rc;
@@ -733,15 +774,18 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 }
                 far_pending = true;
             }
-            if ((rc = panel(j + 1, ps))) return rc;
             if ((rc = build_w(j + 1, ps))) return rc;
+        }
+        if (far_pending) {
+            MPC_HIP(hipEventRecord(h->ev_far, fs));
+            MPC_HIP(hipStreamWaitEvent(j + 1 < nt ? ps : st, h->ev_far, 0));
+        }
+        if (j + 1 < nt) {
+            if (!bulk_seen) MPC_HIP(hipStreamWaitEvent(ps, h->ev_bulk, 0));
+            if ((rc = one_stream(j, ps))) return rc;
         }
         MPC_HIP(hipEventRecord(h->ev_panel, ps));
         MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
-        if (far_pending) {
-            MPC_HIP(hipEventRecord(h->ev_far, fs));
-            MPC_HIP(hipStreamWaitEvent(st, h->ev_far, 0));
-        }
     } else if (!prof) {
         // One-deep look-ahead.  pstream carries the critical chain: the update
         // of block column j+1 by panel j (one mixed-class launch of small
@@ -759,7 +803,9 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         MPC_HIP(hipStreamWaitEvent(h->wstream, h->ev_col, 0));
         if ((rc = panel(0, ps))) return rc;
         if ((rc = build_w(0, ps))) return rc;
-        for (int64_t j = 0; j + 1 < nt; ++j) {
+        int64_t j = 0;
+        for (; j + 1 < nt; ++j) {
+            if (j > 0 && n - j * nb <= kOneStream) break;
             const int64_t bs1 = std::min<int64_t>(nb, n - (j + 1) * nb);
             const int64_t split = (bs1 + MPC_SYRK_TILE - 1) / MPC_SYRK_TILE;
             if (j > 0) MPC_HIP(hipStreamWaitEvent(ps, h->ev_bulk, 0));    // bulk j-1
@@ -768,11 +814,15 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
             // small launch then has the chip to itself (sharing it with the
             // bulk's workgroups made it several times slower)
             MPC_HIP(hipEventRecord(h->ev_panel, ps));
+            if ((rc = panel(j + 1, ps))) return rc;
             MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
             if ((rc = update(j, split, -1, st, 0))) return rc;
             MPC_HIP(hipEventRecord(h->ev_bulk, st));
-            if ((rc = panel(j + 1, ps))) return rc;
             if ((rc = build_w(j + 1, ps))) return rc;
+        }
+        if (j + 1 < nt) {
+            MPC_HIP(hipStreamWaitEvent(ps, h->ev_bulk, 0));
+            if ((rc = one_stream(j, ps))) return rc;
         }
         MPC_HIP(hipEventRecord(h->ev_panel, ps));
         MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));

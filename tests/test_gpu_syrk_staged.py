@@ -61,3 +61,26 @@ def test_factor_group_pairs(handle, n, prec):
         outs.append(T)
     assert torch.equal(outs[1], outs[2])
     assert err[2] <= 1.1 * err[1], err
+
+
+@pytest.mark.parametrize("n,nb", [(65, 64), (2303, 128), (4096, 256), (4097, 256), (4352, 256),
+                                  (5000, 128), (5120, 256), (4480, 64)])
+@pytest.mark.parametrize("prec", [L.PREC_FP32, L.PREC_SWITCH])
+def test_factor_one_stream_tail(handle, n, nb, prec):
+    """The last 4096 columns on one stream (whole factors and the ends of
+    larger ones, from a group's start on): the backward error is that of the
+    phase-by-phase schedule up to 10 %, and two runs agree bit for bit."""
+    print("[case]", n, nb, prec, flush=True)
+    A, _ = S.matgen_householder(handle, n, cond=20.0, lam_max=20.0, seed=n)
+    err, outs = [], []
+    for prof in (1, 0, 0):
+        T = A.clone()
+        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=prec, eps_prime=0.125,
+                                                        ladder=(L.PREC_E4M3, L.PREC_FP32),
+                                                        fallback=0, profile=prof))
+        assert rc == 0
+        L64 = torch.triu(T).to(torch.float64).T.contiguous()
+        err.append(float((L64 @ L64.T.contiguous() - A.to(torch.float64)).norm() / A.to(torch.float64).norm()))
+        outs.append(T)
+    assert torch.equal(outs[1], outs[2])
+    assert err[1] <= 1.1 * err[0], err
