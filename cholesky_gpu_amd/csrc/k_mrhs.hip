@@ -14,7 +14,7 @@
 // The right-hand sides are read as operands straight from L2.  Per 8 KB of an
 // FP32 matrix a wave issues 32 products of 64 cycles, 9.8 TB/s over 1024 SIMDs:
 // above what HBM delivers.  With 16 right-hand sides (A X, FP32 A) n = 8192
-// takes 62 us (4.3 TB/s), where two passes of 8 over half the symmetric matrix
+// takes 55 us (4.9 TB/s), where two passes of 8 over half the symmetric matrix
 // with FP64 FMAs from LDS took 244.
 #include "mpc_internal.hpp"
 #include <algorithm>
@@ -45,6 +45,11 @@ __device__ __forceinline__ void split_range(int mode, int64_t r0, int64_t rows, 
 // blockIdx.x, chunk s = blockIdx.y of cw columns (a multiple of MG).  Wave w
 // takes the chunk's column groups w, w + 4, ..; the four waves' sums are added
 // in wave order through LDS.
+//
+// A last row block that is not full (m >= 64) moves up to end at row m and
+// stores only its own rows: with predicated 4-byte loads its workgroups ran
+// several times as long as the others (16 right-hand sides: n = 12000 185 us,
+// now 112; n = 8684 108, now 72).
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int64_t lda, int64_t m,
                                                   int64_t kc, int64_t cw, const double* __restrict__ X,
@@ -53,7 +58,8 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
     __shared__ double red[4][MPC_MM_NJ][MR];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane & 15, k = lane >> 4;
-    const int64_t r0 = (int64_t)blockIdx.x * MR, cs = (int64_t)blockIdx.y * cw;
+    const int64_t rb = (int64_t)blockIdx.x * MR, cs = (int64_t)blockIdx.y * cw;
+    const int64_t r0 = m >= MR && rb + MR > m ? m - MR : rb;
     int64_t ce = cs + cw < kc ? cs + cw : kc;
     if (MODE == 1 && ce > r0 + MR) ce = r0 + MR < kc ? r0 + MR : kc;
     int64_t cb = cs;
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[wave][4 * e + k][4 * q + i] = acc[i][e];
     __syncthreads();
-    if (r0 + lane < m) {
+    if (r0 + lane < m && r0 + lane >= rb) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int j = wave + 4 * u;
@@ -285,13 +291,19 @@ int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc, 
 
 }  // namespace
 
-// Enough chunks for about 2048 workgroups, each wave of which has a column
-// group.  768 run at once, so fewer leave a last wave nearly empty (16
-// columns: n = 6000 67 us with 1024 workgroups, 53 with 2048, 54 with 4096;
-// n = 8192 60, 62, 68), and every chunk costs a partial sum per output.  At
-// most 8192 columns a chunk (see MFL).
-int64_t mpc_mm_splits(int64_t rows, int64_t kc) {
-    const int64_t want = std::max(cdiv(2048, cdiv(rows, MR)), cdiv(kc, 8192)), most = cdiv(kc, 4 * MG);
+// Enough chunks for about wgs workgroups, each wave of which has a column
+// group, at most 8192 columns a chunk (see MFL).  Every chunk costs a partial
+// sum per output.
+int64_t mpc_mm_splits(int64_t rows, int64_t kc, int64_t wgs) {
+    const int64_t want = std::max(wgs / cdiv(rows, MR), cdiv(kc, 8192)), most = cdiv(kc, 4 * MG);
+    return std::max<int64_t>(1, std::min(want, most));
+}
+
+// One workgroup a CU, each wave of which has a row group (2048 columns, 16
+// right-hand sides, 2048 / 4096 / 6144 rows: 8.3 / 12.6 / 16.8 us; two a CU 8.3 /
+// 16 / 23; 3328 workgroups, half of whose waves had no row group, 24 / 41 / 46)
+int64_t mpc_mm_splits_t(int64_t cols, int64_t kc) {
+    const int64_t want = std::max(256 / cdiv(cols, MTC), cdiv(kc, 8192)), most = cdiv(kc, 4 * MTG);
     return std::max<int64_t>(1, std::min(want, most));
 }
 

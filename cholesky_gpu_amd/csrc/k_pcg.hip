@@ -536,7 +536,11 @@ static int symv_pass_rhs(int nrhs) {
 // 25), large ones the fewer partial sums (n = 6000: 25.6 / 25.1 / 27.7, 12000:
 // 72 / 55 / 62, 16384: 145 / 132 / 121, 36864: 671 / 580 / 540).
 static int symv_tiles(int64_t n) { return n >= 14336 ? 4 : n >= 4608 ? 2 : 1; }
-static int64_t symv_splits(int64_t n) { return mpc_mm_splits(n, n); }
+// Workgroups of the product with the whole matrix: 768 run at once (16 columns:
+// n = 3000 15.0 / 17.4 / 18.0 / 20.2 us with 512 / 1024 / 1536 / 2048, 8192 53 /
+// 56 / 57 / 61, 8684 79 / 73 / 72 / 74, 12000 138 / 116 / 112 / 120, 16384 192 /
+// 191 / 196 / 201)
+static int64_t symv_splits(int64_t n) { return mpc_mm_splits(n, n, n <= 4096 ? 512 : 1024); }
 
 int64_t mpc_symv_partial_doubles(int64_t n, int nrhs) {
     const int64_t E = SY_T * symv_tiles(n), nst = (n + E - 1) / E;

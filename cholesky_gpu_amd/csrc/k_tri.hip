@@ -660,10 +660,17 @@ static int64_t gemv_splits_max(int64_t n, int Bo) {
 // kernels above, else at most MPC_MM_NJ on the matrix cores
 static int sweep_pass(int nrhs) { return nrhs > NR ? std::min(nrhs, MPC_MM_NJ) : nrhs; }
 
+// Chunks of the products with a big block's rows: two workgroups a CU (2048
+// rows, 16 right-hand sides: the triangle 7.2 us, 9.7 with three or four; 2048 /
+// 4096 / 6144 columns beside it 8 / 11.5 / 15 us, with eight 10.6 / 22 / 22)
+static int64_t mm_splits(int64_t bI, int64_t kc) { return mpc_mm_splits(bI, kc, 512); }
+
 // chunks of a product with at most Bo output rows, in units of Bo partial sums:
 // the chunks of bI < Bo rows take at most bI rounded up to a row block times
-// ceil(2048 / blocks), which is less than Bo beyond those of Bo rows
-static int64_t mm_chunks(int Bo, int64_t kc) { return mpc_mm_splits(Bo, kc) + 1; }
+// 512 / blocks or one a column group, no more than those of Bo rows
+static int64_t mm_chunks(int Bo, int64_t kc) {
+    return std::max(mm_splits(Bo, kc), mpc_mm_splits_t(Bo, kc)) + 1;
+}
 
 // scratch of a pass: GEMV kernels: the triangular product's partial sums, then
 // the off-diagonal one's; matrix cores: the same with v between them
@@ -685,7 +692,7 @@ static int mm_stage(hipStream_t st, const float* M, int Bo, int bI, int mode, co
         if ((rc = mpc_launch_mm_sum(st, bI, nj, kc, S, 0, unit, gpart, V, ld, -1.0, v, bI))) return rc;
         V = v;
     }
-    const int64_t St = mpc_mm_splits(bI, bI);
+    const int64_t St = mm_splits(bI, bI);
     if ((rc = mpc_launch_mm_n(st, M, Bo, bI, bI, mode, V, kc > 0 ? bI : ld, nj, tpart, St))) return rc;
     return mpc_launch_mm_sum(st, bI, nj, bI, St, mode, MPC_MM_GROUP_N, tpart, nullptr, 0, 1.0, out, ld);
 }
@@ -708,7 +715,7 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
             const int64_t p0 = I * Bo;
             const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
             const float* Wi = Winv + I * (int64_t)Bo * Bo;
-            const int64_t S = mm ? mpc_mm_splits(bI, p0) : cdiv(p0, FW_CW);
+            const int64_t S = mm ? mm_splits(bI, p0) : cdiv(p0, FW_CW);
             if (p0 > 0 && mm) {
                 if ((rc = mpc_launch_mm_n(st, L + p0, ldl, bI, p0, 0, Y, ld, nj, gpart, S))) return rc;
             } else if (p0 > 0) {
@@ -728,7 +735,7 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
             const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
             const int64_t p1 = p0 + bI;
             const float* WTi = WinvT + I * (int64_t)Bo * Bo;
-            const int64_t S = mm ? mpc_mm_splits(bI, n - p1) : cdiv(n - p1, BW_RW);
+            const int64_t S = mm ? mpc_mm_splits_t(bI, n - p1) : cdiv(n - p1, BW_RW);
             if (p1 < n && mm) {
                 if ((rc = mpc_launch_mm_t(st, L + p1 + p0 * ldl, ldl, n - p1, bI, Z + p1, ld, nj, gpart, S)))
                     return rc;
