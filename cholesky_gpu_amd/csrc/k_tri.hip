@@ -255,21 +255,21 @@ __global__ __launch_bounds__(256) void gemm_kernel(gemm_batch g) {
 
 // ---------------------------------------------------------------- TRSV kernels
 // Both sweeps are left-looking: the update a big block receives from the
-// blocks solved before it is one GEMV over all of them, split into many
-// workgroups (partial sums per split, in a fixed order), and the partial sums
-// are folded into the right-hand side inside the triangular GEMV that
-// applies the block's inverse.  Per block: two or three launches, each wide
-// enough to fill the chip, instead of a narrow per-block update of every
-// later block.
+// blocks solved before it is one GEMV over all of them, then the block's
+// inverse is applied.  Where the columns of a matrix are the outputs (backward,
+// and both inverses: W and its transpose are stored) a wave owns whole columns,
+// so nothing is left to add up afterwards.  The forward GEMV, whose outputs are
+// rows, is split into many workgroups with partial sums in a fixed order.
 constexpr int NR = 4;       // right-hand sides per pass
-constexpr int TG = 64;      // tile edge of the triangular GEMV
 // forward: columns per split (4 waves x FW_CPW).  At n = 16384 (Bo = 2048)
 // 128 beat 64, 256 and 512: more workgroups with fewer loads in flight each.
 constexpr int FW_CW = 128;
 constexpr int FW_CPW = FW_CW / 4;
-constexpr int BW_CPW = 8;   // backward: columns per wave (32 per workgroup)
-constexpr int BW_RW = 512;  // backward: rows per split (BW_RPL per lane)
+constexpr int BW_CPW = 8;   // backward by partial sums: columns per wave (32 per workgroup)
+constexpr int BW_RW = 512;  // and rows per split (BW_RPL per lane)
 constexpr int BW_RPL = BW_RW / 64;
+constexpr int TD = 2048;    // most columns of a big block
+constexpr int BW_CH = 1024; // backward: rows at a time
 
 // Forward, big block I = rows [p0, p0 + bI):
 //   part[(s nrhs + j) bI + i] = sum_{c in split s} L[p0 + i][c] Y[c][j],  c < p0
@@ -329,7 +329,8 @@ __global__ __launch_bounds__(256) void fwd_gemv_partial_kernel(
     }
 }
 
-// Backward, big block I = columns [p0, p0 + bI), rows below it [p1, n):
+// Backward with 3 or 4 right-hand sides, big block I = columns [p0, p0 + bI),
+// rows below it [p1, n):
 //   part[(s nrhs + j) bI + c] = sum_{r in split s} L[r][p0 + c] X[r][j]
 // 32 columns per workgroup (8 per wave), split s = BW_RW rows; lane k of a
 // wave holds rows lane + 64k, k < BW_RPL, of each of its columns (coalesced
@@ -392,150 +393,197 @@ __global__ __launch_bounds__(256) void bwd_gemv_partial_kernel(
     }
 }
 
-// Triangular GEMV on a diagonal big block, out[i] = sum_j M[i + j*ld] v[j]
-// over j <= i (lower: M = Winv, forward) or j >= i (upper: M = Winv^T,
-// backward), i, j < bI, where v[j] = V[j] - sum_{s < S} pin[(s nrhs + r) bI + j]
-// (the off-diagonal GEMV's partial sums).  One workgroup of TT_NW waves per
-// 64 x 64 tile (row block ib, column chunk jb) of the triangle; lane = row.
-// Wave w adds the partial sums s = w, w + TT_NW, .. of the tile's 64 v
-// entries (batches of 8 independent loads); the waves' sums are combined in
-// LDS in wave order.  Wave w then multiplies its TT_CW columns of the tile
-// (their loads in flight at once, v read back from LDS) and the waves'
-// products are added in wave order.  Partial sums go to
-// part[(jb * nrhs + j) * bI + i]; tri_gemv_reduce adds the chunks of a row
-// in order (deterministic).
-#ifndef MPC_TT_NW
-#define MPC_TT_NW 4
-#endif
-constexpr int TT_NW = MPC_TT_NW;          // waves per tile
-constexpr int TT_CW = TG / TT_NW;          // tile columns per wave
-template <bool UPPER>
-__global__ __launch_bounds__(64 * TT_NW) void tri_gemv_tile_kernel(const float* __restrict__ M,
-                                                                  int ld, int bI,
-                                                                  const double* __restrict__ V,
-                                                                  int64_t ldv, int nrhs,
-                                                                  const double* __restrict__ pin,
-                                                                  int S,
-                                                                  double* __restrict__ part) {
-    __shared__ double vsum[TT_NW][64];
-    __shared__ double vs[64];
-    __shared__ double acc_w[TT_NW][64];
-    // tile t -> (ib, jb): lower ib >= jb, t = ib (ib + 1) / 2 + jb; upper mirrors it
-    const int t = blockIdx.x;
-    int a = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-    while (a * (a + 1) / 2 > t) --a;
-    while ((a + 1) * (a + 2) / 2 <= t) ++a;
-    const int b = t - a * (a + 1) / 2;
-    const int ib = UPPER ? b : a, jb = UPPER ? a : b;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i = ib * TG + lane;
-    const int j0 = jb * TG;
-    const int c0 = j0 + TT_CW * wave;      // this wave's first column
-    // This wave's 16 columns of the tile, all loads issued before any use.  A
-    // load guarded by a condition (or whose use is) would be sunk into a
-    // branch with its own wait, serialising the loads; hence three shapes:
-    float m[TT_CW];
-    const bool full = j0 + TG <= bI && ib * TG + TG <= bI;
-    if (full && ib != jb) {                  // interior: no mask
-        const float* Mi = M + i + (int64_t)c0 * ld;
+// Sum over the 64 lanes, in every lane: rotations within 16 lanes, then the
+// four sixteens in order
+template <int CTRL>
+__device__ __forceinline__ double rotate16(double v) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double sum64(double v) {
+    v += rotate16<0x128>(v);
+    v += rotate16<0x124>(v);
+    v += rotate16<0x122>(v);
+    v += rotate16<0x121>(v);
+    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));     // 16-byte load, any column start
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+// Where 256 values that lane l reads as 4l .. 4l+3 lie in LDS: 4l and 4l+1 of
+// all lanes in a row, then 4l+2 and 4l+3 (two 16-byte reads without conflicts)
+__device__ __forceinline__ int dot_slot(int x) { return (x & 2) * 64 + (x >> 2) * 2 + (x & 1); }
+
+// Backward, big block I = columns [p0, p0 + bI), rows below it [p1, n):
+//   v[j bI + c] = V[j ldv + c] - sum_{r >= p1} L[r][p0 + c] X[j][r]
+// A column per wave, BW_CH rows at a time: lane l reads rows 4l .. 4l+3 of
+// every 256 (16 bytes), the next rows' loads in flight during the products; the
+// workgroup shares the rows' X values through LDS.  Bound by memory (n = 16384,
+// one right-hand side: 14.9 us on average for 59 MB); two columns a wave are
+// too few workgroups (20.7), 2048 rows at a time the same for long columns and
+// slower for short ones (n = 8684: 9.3 / 10.8).  Two right-hand sides take 17.0;
+// with four the X values are the larger part (28 us, n = 60000 89, where the
+// partial sums above and their addition take 67).
+template <int NJ>
+__global__ __launch_bounds__(256, 2) void bwd_dot_kernel(const float* __restrict__ L, int64_t ldl,
+                                                        int64_t p0, int bI, int64_t n,
+                                                        const double* __restrict__ X, int64_t ldx,
+                                                        int nj, const double* __restrict__ V,
+                                                        int64_t ldv, double* __restrict__ v) {
+    constexpr int NK = BW_CH / 256;
+    __shared__ __align__(16) double xs[NJ][BW_CH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = blockIdx.x * 4 + wave;
+    const float* col = L + (p0 + (c < bI ? c : bI - 1)) * ldl;
+    v4f l[NK];
+    double x[NJ][NK];
+    auto load = [&](int64_t rs) {
+        if (rs + BW_CH <= n) {
 #pragma unroll
-        for (int u = 0; u < TT_CW; ++u) m[u] = Mi[(int64_t)u * ld];
-    } else if (full) {                       // diagonal tile: per-lane triangle select
-        const float* Mi = M + i + (int64_t)c0 * ld;
+            for (int k = 0; k < NK; ++k)
+                l[k] = *reinterpret_cast<const v4u*>(col + rs + 256 * k + 4 * lane);
+        } else {
+            // the last rows: loads that end at row n at the latest (n > Bo >= 4
+            // where there are rows below a block), moved into place
 #pragma unroll
-        for (int u = 0; u < TT_CW; ++u) m[u] = Mi[(int64_t)u * ld];
-#pragma unroll
-        for (int u = 0; u < TT_CW; ++u) {
-            const int cl = TT_CW * wave + u;              // column within the tile
-            const bool keep = UPPER ? cl >= lane : cl <= lane;
-            m[u] = keep ? m[u] : 0.f;
+            for (int k = 0; k < NK; ++k) {
+                const int64_t r = rs + 256 * k + 4 * lane, rc = r < n - 4 ? r : n - 4, off = r - rc;
+                const v4f y = *reinterpret_cast<const v4u*>(col + rc);
+                l[k][0] = off == 0 ? y[0] : off == 1 ? y[1] : off == 2 ? y[2] : off == 3 ? y[3] : 0.f;
+                l[k][1] = off == 0 ? y[1] : off == 1 ? y[2] : off == 2 ? y[3] : 0.f;
+                l[k][2] = off == 0 ? y[2] : off == 1 ? y[3] : 0.f;
+                l[k][3] = off == 0 ? y[3] : 0.f;
+            }
         }
-    } else {                                 // ragged last block: clamped addresses
-        const int ic = i < bI ? i : bI - 1;
 #pragma unroll
-        for (int u = 0; u < TT_CW; ++u) {
-            const int j = c0 + u;
-            m[u] = M[ic + (int64_t)(j < bI ? j : bI - 1) * ld];
-        }
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int u = 0; u < TT_CW; ++u) {
-            const int j = c0 + u;
-            const bool keep = j < bI && (UPPER ? j >= i : j <= i);
-            m[u] = keep ? m[u] : 0.f;
-        }
+            for (int k = 0; k < NK; ++k) {
+                const int64_t r = rs + 256 * k + tid;
+                const double y = X[(int64_t)(j < nj ? j : nj - 1) * ldx + (r < n ? r : n - 1)];
+                x[j][k] = r < n ? y : 0.0;
+            }
+    };
+    double acc[NJ] = {};
+    int64_t rs = p0 + bI;
+    load(rs);
+    for (; rs < n; rs += BW_CH) {
+        v4f w[NK];
+#pragma unroll
+        for (int k = 0; k < NK; ++k) w[k] = l[k];
+        __syncthreads();                         // the last rows' values are read
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int k = 0; k < NK; ++k) xs[j][256 * k + dot_slot(tid)] = x[j][k];
+        __syncthreads();
+        if (rs + BW_CH < n) load(rs + BW_CH);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int k = 0; k < NK; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const d2 y = *reinterpret_cast<const d2*>(&xs[j][256 * k + 64 * i + 2 * lane]);
+                    acc[j] = fma((double)w[k][i], y[0], acc[j]);
+                    acc[j] = fma((double)w[k][i + 1], y[1], acc[j]);
+                }
     }
-    // lane u of every wave builds a part of v[j0 + u]
-    const int jl = j0 + lane < bI ? j0 + lane : bI - 1;
-    const int64_t sstride = (int64_t)nrhs * bI;
-    for (int r = 0; r < nrhs; ++r) {
-        const double* pr = pin + (int64_t)r * bI + jl;
-        double sum = 0.0;
-        int sp = wave;
-        for (; sp + 7 * TT_NW < S; sp += 8 * TT_NW) {      // batches of 8 independent loads
-            double pv[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) pv[q] = pr[(int64_t)(sp + q * TT_NW) * sstride];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) sum += pv[q];
-        }
-        for (; sp < S; sp += TT_NW) sum += pr[(int64_t)sp * sstride];
-        vsum[wave][lane] = sum;
-        __syncthreads();
-        if (wave == 0) {
-            double tot = vsum[0][lane];
-#pragma unroll
-            for (int w = 1; w < TT_NW; ++w) tot += vsum[w][lane];
-            vs[lane] = V[(int64_t)r * ldv + jl] - tot;
-        }
-        __syncthreads();
-        double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-        for (int u = 0; u < TT_CW; u += 2) {
-            a0 = fma((double)m[u], vs[TT_CW * wave + u], a0);
-            a1 = fma((double)m[u + 1], vs[TT_CW * wave + u + 1], a1);
-        }
-        acc_w[wave][lane] = a0 + a1;
-        __syncthreads();
-        if (wave == 0 && i < bI) {
-            double tot = acc_w[0][lane];
-#pragma unroll
-            for (int w = 1; w < TT_NW; ++w) tot += acc_w[w][lane];
-            part[((int64_t)jb * nrhs + r) * bI + i] = tot;
-        }
-        __syncthreads();                    // vsum, vs and acc_w are reused
+    for (int j = 0; j < NJ; ++j) {
+        const double sum = sum64(acc[j]);
+        if (lane == 0 && j < nj && c < bI) v[(int64_t)j * bI + c] = V[(int64_t)j * ldv + c] - sum;
     }
 }
 
-// 64 rows per workgroup (lane = row, one TG chunk row).  Wave w sums the
-// chunks jlo + w, jlo + w + 4, ... in batches of 8 independent loads
-// (clamped chunk index, zero weight beyond jhi): one batch when the block
-// has at most 32 chunks.  The four wave sums are then added in order.
-__global__ __launch_bounds__(256) void tri_gemv_reduce_kernel(const double* __restrict__ part,
-                                                             int bI, int nrhs, int upper,
-                                                             double* __restrict__ out,
-                                                             int64_t ldo) {
+// v[j bI + i] = V[j ldv + i] - sum_s part[(s nj + j) bI + i] (a GEMV's partial
+// sums); wave w of a workgroup adds s = w, w + 4, .. of 64 rows
+__global__ __launch_bounds__(256) void gemv_sum_kernel(const double* __restrict__ part, int bI, int S,
+                                                     const double* __restrict__ V, int64_t ldv,
+                                                     double* __restrict__ v) {
     __shared__ double red[4][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i0 = blockIdx.x * 64 + lane;
-    const int i = i0 < bI ? i0 : bI - 1;
-    const int r = blockIdx.y;
-    const int nb = (bI + TG - 1) / TG, ib = i / TG;
-    const int jlo = upper ? ib : 0, jhi = upper ? nb - 1 : ib;
-    double s = 0.0;
-    for (int j0 = jlo + w; j0 <= jhi; j0 += 32) {
-        double v[8];
+    const int i0 = blockIdx.x * 64 + lane, i = i0 < bI ? i0 : bI - 1;
+    const int j = blockIdx.y, nj = gridDim.y;
+    double sum = 0.0;
+    for (int s0 = w; s0 < S; s0 += 64) {
+        double x[16];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int jb = j0 + 4 * u <= jhi ? j0 + 4 * u : jhi;
-            v[u] = part[((int64_t)jb * nrhs + r) * bI + i];
+        for (int u = 0; u < 16; ++u) {
+            const int s = s0 + 4 * u < S ? s0 + 4 * u : S - 1;
+            x[u] = part[((int64_t)s * nj + j) * bI + i];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) s += j0 + 4 * u <= jhi ? v[u] : 0.0;
+        for (int u = 0; u < 16; ++u) sum += s0 + 4 * u < S ? x[u] : 0.0;
     }
-    red[w][lane] = s;
+    red[w][lane] = sum;
     __syncthreads();
     if (w == 0 && i0 < bI)
-        out[i0 + (int64_t)r * ldo] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+        v[(int64_t)j * bI + i0] = V[(int64_t)j * ldv + i0] -
+                                  (((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
+}
+
+// A big block's inverse applied: out[r] = sum_c Mt[c + r ld] v[c] over c <= r
+// (forward, Mt = Winv^T) or c >= r (backward, Mt = Winv), r, c < bI.  A wave
+// owns an output: its column of Mt (16-byte loads, all in flight at once, a
+// 256-row piece outside the triangle replaced by its neighbour) times v from
+// LDS.  bI = 2048, one right-hand side 5.3 us, four 7.0 (two outputs a wave 6.0
+// and 7.6; 64 x 64 tiles over rows of M and a launch to add them up 10 and 15).
+template <bool UPPER, int NJ>
+__global__ __launch_bounds__(256, 2) void tri_dot_kernel(const float* __restrict__ Mt, int ld, int bI,
+                                                        const double* __restrict__ V, int64_t ldv,
+                                                        int nj, double* __restrict__ out, int64_t ldo) {
+    constexpr int NK = TD / 256;
+    __shared__ __align__(16) double vs[NJ][TD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = blockIdx.x * 4 + wave;
+    const int kd = r >> 8;                       // the diagonal's 256-row piece
+    const int klo = UPPER ? kd : 0, khi = UPPER ? (bI - 1) >> 8 : kd;
+    v4f m[NK];
+    const float* col = Mt + (int64_t)(r < bI ? r : bI - 1) * ld;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        const int c = 256 * (k < klo ? klo : k > khi ? khi : k) + 4 * lane;
+        m[k] = *reinterpret_cast<const v4f*>(col + (c < ld ? c : ld - 4));
+    }
+    for (int c = 256 * klo + tid; c < 256 * (khi + 1); c += 256)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            vs[j][(c & ~255) + dot_slot(tid)] = V[(int64_t)(j < nj ? j : nj - 1) * ldv + (c < bI ? c : bI - 1)];
+    __syncthreads();
+    double acc[NJ] = {};
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        if (k < klo || k > khi) continue;
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+            double w[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int c = 256 * k + 4 * lane + i + u;
+                w[u] = (UPPER ? c >= r && c < bI : c <= r) ? (double)m[k][i + u] : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const d2 y = *reinterpret_cast<const d2*>(&vs[j][256 * k + 64 * i + 2 * lane]);
+                acc[j] = fma(w[1], y[1], fma(w[0], y[0], acc[j]));
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const double sum = sum64(acc[j]);
+        if (lane == 0 && j < nj && r < bI) out[(int64_t)j * ldo + r] = sum;
+    }
 }
 
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
@@ -632,28 +680,42 @@ int mpc_build_block_inverses(hipStream_t st, const float* L, int64_t ldl, int64_
     return mpc_build_block_inverses_range(st, L, ldl, n, Bo, dinv, W, WT, 0, (n + Bo - 1) / Bo);
 }
 
-static int tri_gemv(hipStream_t st, const float* M, int Bo, int bI, int upper, const double* V,
-                    int64_t ldv, int nrhs, const double* pin, int S, double* part, double* out,
-                    int64_t ldo) {
-    const int nb = (bI + TG - 1) / TG;
-    const dim3 grid((unsigned)(nb * (nb + 1) / 2));
-    if (upper)
-        hipLaunchKernelGGL(tri_gemv_tile_kernel<true>, grid, dim3(64 * TT_NW), 0, st, M, Bo, bI, V,
-                           ldv, nrhs, pin, S, part);
-    else
-        hipLaunchKernelGGL(tri_gemv_tile_kernel<false>, grid, dim3(64 * TT_NW), 0, st, M, Bo, bI, V,
-                           ldv, nrhs, pin, S, part);
-    hipLaunchKernelGGL(tri_gemv_reduce_kernel, dim3(cdiv(bI, 64), (unsigned)nrhs), dim3(256), 0, st,
-                       part, bI, nrhs, upper, out, ldo);
+static int tri_dot(hipStream_t st, const float* Mt, int Bo, int bI, bool upper, const double* V,
+                   int64_t ldv, int nj, double* out, int64_t ldo) {
+    const dim3 g(cdiv(bI, 4)), b(256);
+#define MPC_TRI_DOT(U, J) \
+    hipLaunchKernelGGL((tri_dot_kernel<U, J>), g, b, 0, st, Mt, Bo, bI, V, ldv, nj, out, ldo)
+    if (upper) {
+        if (nj == 1) MPC_TRI_DOT(true, 1);
+        else if (nj == 2) MPC_TRI_DOT(true, 2);
+        else MPC_TRI_DOT(true, 4);
+    } else {
+        if (nj == 1) MPC_TRI_DOT(false, 1);
+        else if (nj == 2) MPC_TRI_DOT(false, 2);
+        else MPC_TRI_DOT(false, 4);
+    }
+#undef MPC_TRI_DOT
     MPC_LAUNCH_CHECK();
     return 0;
 }
 
-// splits of the off-diagonal GEMVs: at most n / FW_CW (forward, over p0 < n
-// columns) and n / BW_RW (backward, over fewer than n rows)
-static int64_t gemv_splits_max(int64_t n, int Bo) {
-    (void)Bo;
-    return std::max<int64_t>((n + FW_CW - 1) / FW_CW, (n + BW_RW - 1) / BW_RW);
+static int bwd_gemv(hipStream_t st, const float* L, int64_t ldl, int64_t p0, int bI, int64_t n,
+                   const double* X, int64_t ldx, int nj, const double* V, int64_t ldv, double* v,
+                    double* part) {
+    const dim3 g(cdiv(bI, 4)), b(256);
+    if (nj > 2) {
+        const unsigned S = cdiv(n - p0 - bI, BW_RW);
+        hipLaunchKernelGGL(bwd_gemv_partial_kernel, dim3(cdiv(bI, 4 * BW_CPW), S), b, 0, st, L, ldl, p0,
+                           bI, n, X, ldx, nj, part);
+        hipLaunchKernelGGL(gemv_sum_kernel, dim3(cdiv(bI, 64), (unsigned)nj), b, 0, st, part, bI, (int)S,
+                           V, ldv, v);
+    } else if (nj == 2) {
+        hipLaunchKernelGGL(bwd_dot_kernel<2>, g, b, 0, st, L, ldl, p0, bI, n, X, ldx, nj, V, ldv, v);
+    } else {
+        hipLaunchKernelGGL(bwd_dot_kernel<1>, g, b, 0, st, L, ldl, p0, bI, n, X, ldx, nj, V, ldv, v);
+    }
+    MPC_LAUNCH_CHECK();
+    return 0;
 }
 
 // right-hand sides of the next pass over the factor: at most NR in the GEMV
@@ -672,11 +734,11 @@ static int64_t mm_chunks(int Bo, int64_t kc) {
     return std::max(mm_splits(Bo, kc), mpc_mm_splits_t(Bo, kc)) + 1;
 }
 
-// scratch of a pass: GEMV kernels: the triangular product's partial sums, then
-// the off-diagonal one's; matrix cores: the same with v between them
+// scratch of a pass: GEMV kernels: v, then the off-diagonal product's partial
+// sums (over fewer than n columns, or n rows); matrix cores: the triangular product's partial sums, v,
+// the off-diagonal one's
 int64_t mpc_block_prec_partial_doubles(int64_t n, int Bo, int nrhs) {
-    const int64_t gemv = ((int64_t)(Bo + TG - 1) / TG + gemv_splits_max(n, Bo)) * Bo *
-                         std::min(nrhs, NR);
+    const int64_t gemv = (1 + (n + FW_CW - 1) / FW_CW) * Bo * std::min(nrhs, NR);
     if (nrhs <= NR) return gemv;
     return std::max(gemv, (mm_chunks(Bo, n) + mm_chunks(Bo, Bo) + 1) * Bo * std::min(nrhs, MPC_MM_NJ));
 }
@@ -709,42 +771,43 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
     for (int j0 = 0, nj; j0 < nrhs; j0 += nj, R += nj * ld, Y += nj * ld, Z += nj * ld) {
         nj = sweep_pass(nrhs - j0);
         const bool mm = nj > NR;
-        double* v = part + (mm ? mm_chunks(Bo, Bo) : (Bo + TG - 1) / TG) * Bo * nj;
-        double* gpart = mm ? v + (int64_t)Bo * nj : v;
+        double* v = part + (mm ? mm_chunks(Bo, Bo) * Bo * nj : 0);
+        double* gpart = v + (int64_t)Bo * nj;
         for (int64_t I = 0; I < nI; ++I) {
             const int64_t p0 = I * Bo;
             const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
-            const float* Wi = Winv + I * (int64_t)Bo * Bo;
             const int64_t S = mm ? mm_splits(bI, p0) : cdiv(p0, FW_CW);
             if (p0 > 0 && mm) {
                 if ((rc = mpc_launch_mm_n(st, L + p0, ldl, bI, p0, 0, Y, ld, nj, gpart, S))) return rc;
             } else if (p0 > 0) {
                 hipLaunchKernelGGL(fwd_gemv_partial_kernel, dim3(cdiv(bI, 64), (unsigned)S), dim3(256), 0,
                                    st, L, ldl, p0, bI, Y, ld, nj, gpart);
+                hipLaunchKernelGGL(gemv_sum_kernel, dim3(cdiv(bI, 64), (unsigned)nj), dim3(256), 0, st,
+                                   gpart, bI, (int)S, R + p0, ld, v);
             }
             if (late_ev && j0 == 0 && I == I_late && hipStreamWaitEvent(st, late_ev, 0) != hipSuccess) {
                 mpc_set_error("apply_block_prec: stream wait failed");
                 return MPC_ERR_HIP;
             }
-            rc = mm ? mm_stage(st, Wi, Bo, bI, 1, R + p0, ld, nj, gpart, p0, S, MPC_MM_GROUP_N, v, part, Y + p0)
-                    : tri_gemv(st, Wi, Bo, bI, 0, R + p0, ld, nj, gpart, (int)S, part, Y + p0, ld);
+            const int64_t wI = I * (int64_t)Bo * Bo;
+            rc = mm ? mm_stage(st, Winv + wI, Bo, bI, 1, R + p0, ld, nj, gpart, p0, S, MPC_MM_GROUP_N, v, part, Y + p0)
+                    : tri_dot(st, WinvT + wI, Bo, bI, false, p0 ? v : R, p0 ? bI : ld, nj, Y + p0, ld);
             if (rc) return rc;
         }
         for (int64_t I = nI - 1; I >= 0; --I) {
             const int64_t p0 = I * Bo;
             const int bI = (int)(n - p0 < Bo ? n - p0 : Bo);
-            const int64_t p1 = p0 + bI;
-            const float* WTi = WinvT + I * (int64_t)Bo * Bo;
-            const int64_t S = mm ? mpc_mm_splits_t(bI, n - p1) : cdiv(n - p1, BW_RW);
-            if (p1 < n && mm) {
-                if ((rc = mpc_launch_mm_t(st, L + p1 + p0 * ldl, ldl, n - p1, bI, Z + p1, ld, nj, gpart, S)))
+            const int64_t p1 = p0 + bI, wI = I * (int64_t)Bo * Bo;
+            const bool off = p1 < n;
+            if (mm) {
+                const int64_t S = mpc_mm_splits_t(bI, n - p1);
+                if (off && (rc = mpc_launch_mm_t(st, L + p1 + p0 * ldl, ldl, n - p1, bI, Z + p1, ld, nj, gpart, S)))
                     return rc;
-            } else if (p1 < n) {
-                hipLaunchKernelGGL(bwd_gemv_partial_kernel, dim3(cdiv(bI, 4 * BW_CPW), (unsigned)S),
-                                   dim3(256), 0, st, L, ldl, p0, bI, n, Z, ld, nj, gpart);
+                rc = mm_stage(st, WinvT + wI, Bo, bI, 2, Y + p0, ld, nj, gpart, n - p1, S, MPC_MM_GROUP_T, v, part, Z + p0);
+            } else {
+                if (off && (rc = bwd_gemv(st, L, ldl, p0, bI, n, Z, ld, nj, Y + p0, ld, v, gpart))) return rc;
+                rc = tri_dot(st, Winv + wI, Bo, bI, true, off ? v : Y + p0, off ? bI : ld, nj, Z + p0, ld);
             }
-            rc = mm ? mm_stage(st, WTi, Bo, bI, 2, Y + p0, ld, nj, gpart, n - p1, S, MPC_MM_GROUP_T, v, part, Z + p0)
-                    : tri_gemv(st, WTi, Bo, bI, 1, Y + p0, ld, nj, gpart, (int)S, part, Z + p0, ld);
             if (rc) return rc;
         }
     }

@@ -56,3 +56,12 @@ def test_apply_precond_blocks(handle, n, nrhs):
     Y = torch.linalg.solve_triangular(L64, R.T.contiguous(), upper=False)
     X = torch.linalg.solve_triangular(L64.T.contiguous(), Y, upper=True).T
     assert float((Z - X).norm() / X.norm()) < 256 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n", [1, 127, 255, 257, 2047, 2050, 2051, 2052, 3073, 4097, 5121])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 4, 6])
+def test_apply_precond_edges(handle, n, nrhs):
+    """The sweeps where a column ends: one to four rows below a big block, one
+    past 1024 (the backward products' step), pieces of 256 that are not full,
+    last row blocks of 1 to 63 rows.  Tolerance as above."""
+    test_apply_precond_blocks(handle, n, nrhs)
