@@ -5,7 +5,7 @@
 //    fp8_chol.cuh:73-85; switching_chol.cuh:98-110 calls a LEFT form that is
 //    out of bounds).  One wave owns a 32-row slab and substitutes over the
 //    32-column blocks of the panel with the inverses of L_jj's 32x32 diagonal
-//    sub-blocks (MFMA 32x32x2 f32) plus one refinement step per block.  The epilogue computes each row's sum of
+//    sub-blocks (MFMA 32x32x2 f32).  The epilogue computes each row's sum of
 //    squares, subtracts it from the Schur-diagonal tracker (update_diag,
 //    kernels_macros.cuh:177-190) and folds the tile amax / max row sum of
 //    squares into per-tile slots with order-independent atomics.
@@ -22,23 +22,27 @@
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int sigma(int s, int h) { return 8 * (s >> 2) + 4 * h + (s & 3); }
 
-// one refinement step after the product with the explicit 32x32 inverse
-constexpr bool kTrsmRefine = false;
-
-// One workgroup of NW waves per 32-row slab.  Wave w owns the column blocks
-// b = w, w + NW, ...  Step b: the owner finishes X_b = acc_b Dinv_b^T (one
-// refinement step against L_bb when REF), publishes it in LDS; after the
-// barrier every wave subtracts X_b L_{b'b}^T from its owned blocks b' > b,
-// the soonest-needed block first.  The L operands for a step are loaded
-// before the barrier so their latency overlaps the owner's solve.
+// One workgroup per 32-row slab, wave w = the panel's 32-column block w.  Step
+// b: wave b finishes X_b = acc_b Dinv_b^T and publishes it in LDS; after the
+// barrier the waves w > b subtract X_b L_wb^T from their blocks.  The chain
+// (update of block b + 1, its product with the inverse, LDS and barrier: 32
+// MFMAs of 64 cycles a step) bounds the launch: nothing else may sit on it.  The
+// inverse is read at the start, the L operands of step b + 1 during step b,
+// statistics and stores follow the barrier, and the chain's wave has priority
+// over the wave that shares its SIMD.  A wave per block (two blocks each on four
+// waves, operands read where they are used: nb = 256 30 us for 2000 to 10000
+// rows, nb = 128 11.3).
 // MFMA roles (32x32x2 f32, k index sig(t, h) on both operands): A = L or
 // Dinv rows (lane m = lane % 32), B = X or acc columns (lane n = row of the
-// slab); accumulator register i of lane (n, h) holds column sig(i, h), row n.
-template <int NBK, int NW, bool REF>
-__global__ __launch_bounds__(NW * 64, 2) void trsm_stats_kernel(float* __restrict__ A21, int64_t lda,
+// slab); accumulator register i of lane (n, h) holds column sig(i, h), row n,
+// negated, so that the products add.  So the lane's X operand of k step t is its
+// own register t of X_b.
+template <int NB>
+__global__ __launch_bounds__(NB * 64, 4) void trsm_stats_kernel(float* __restrict__ A21, int64_t lda,
                                                          int64_t s, const float* __restrict__ dinv_j,
                                                          const float* __restrict__ Ljj,
                                                          float* __restrict__ rowss,
@@ -49,87 +53,73 @@ __global__ __launch_bounds__(NW * 64, 2) void trsm_stats_kernel(float* __restric
                                                          int64_t row0,
                                                          const float* __restrict__ diag0,
                                                          int slot) {
-    constexpr int NO = NBK / NW;          // blocks per wave
-    constexpr int XLD = 33;
-    __shared__ float Xs[NBK][32 * XLD];
-    __shared__ float red_ss[NW][64], red_am[NW][64];
-    if (sm->info != 0) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ v4f Xs[NB][4][64];
+    __shared__ float red_ss[NB][64], red_am[NB][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int64_t r0 = row0 + (int64_t)blockIdx.x * 32;
     const int64_t row = r0 + n;
     const bool valid = row < s;
-    const int64_t rowc = valid ? row : s - 1;     // loads from clamped rows, then select
+    // one lane offset for all columns, which are scalars; rows beyond s read as
+    // 0 and are not written (offset out of range)
+    const __amdgpu_buffer_rsrc_t ra =
+        __builtin_amdgcn_make_buffer_rsrc(A21 + r0, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rl =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Ljj), 0, 0x7fffffff, 0x00020000);
+    const uint32_t ld4 = 4u * (uint32_t)lda;
+    const uint32_t va = valid ? 4u * (uint32_t)n + 4u * (uint32_t)h * ld4 : 0x80000000u;
+    const uint32_t vl = 4u * (uint32_t)(32 * wave + n) + 4u * (uint32_t)h * ld4;
+    auto soff = [&](int b, int t) -> uint32_t { return (uint32_t)(32 * b + sigma(t, 0)) * ld4; };
 
-    v16f acc[NO];
+    v16f acc;
+    float dv[16], lv[2][16];
+    auto load_l = [&](int b) {               // L(32 wave + n, 32 b + sig(t, h))
 #pragma unroll
-    for (int o = 0; o < NO; ++o) {
-        const int b = wave + NW * o;
+        for (int t = 0; t < 16; ++t)
+            lv[b & 1][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rl, vl, soff(b, t), 0));
+    };
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float x = A21[rowc + (int64_t)(32 * b + sigma(i, h)) * lda];
-            acc[o][i] = valid ? x : 0.f;
-        }
-    }
+    for (int i = 0; i < 16; ++i)
+        acc[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ra, va, soff(wave, i), 0));
+#pragma unroll
+    for (int t = 0; t < 16; ++t) dv[t] = dinv_j[wave * 1024 + n + sigma(t, h) * 32];
+    load_l(0);
+    if (sm->info != 0) return;
+    acc = -acc;
     float ss = 0.f, am = 0.f;
+    v16f xb = {};
+    auto solve = [&](int b) {
+        xb = v16f{};
 #pragma unroll
-    for (int b = 0; b < NBK; ++b) {
-        // prefetch this step's L operands: -L(32 b' + m, 32 b + sig(t, h)) for owned b' > b
-        float lv[NO][16];
+        for (int t = 0; t < 16; ++t)
+            xb = __builtin_amdgcn_mfma_f32_32x32x2f32(dv[t], acc[t], xb, 0, 0, 0);
+        xb = -xb;
 #pragma unroll
-        for (int o = 0; o < NO; ++o) {
-            const int bp = wave + NW * o;
+        for (int v = 0; v < 4; ++v)
+            Xs[b][v][lane] = v4f{xb[4 * v], xb[4 * v + 1], xb[4 * v + 2], xb[4 * v + 3]};
+    };
+    if (wave == 0) solve(0);
 #pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const float x = Ljj[(32 * bp + n) + (int64_t)(32 * b + sigma(t, h)) * lda];
-                lv[o][t] = bp > b ? -x : 0.f;
-            }
-        }
-        if (b % NW == wave) {
-            const int o = b / NW;
-            const float* Db = dinv_j + b * 1024;
-            v16f xb = {};
+    for (int b = 0; b < NB; ++b) {
+        mpc_lds_barrier();                   // X_b
+        if (wave > b) {
+            if (wave == b + 1) __builtin_amdgcn_s_setprio(3);
+            if (b + 2 < NB) load_l(b + 1);
+            v4f x[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) x[v] = Xs[b][v][lane];
 #pragma unroll
             for (int t = 0; t < 16; ++t)
-                xb = __builtin_amdgcn_mfma_f32_32x32x2f32(Db[n + sigma(t, h) * 32], acc[o][t], xb, 0,
-                                                          0, 0);
-            if constexpr (REF) {
-                // r = acc - xb L_bb^T (strict upper part of L_jj holds A: masked), xb += r Dinv^T
-                v16f rr = acc[o];
-#pragma unroll
-                for (int t = 0; t < 16; ++t) {
-                    const int q = sigma(t, h);
-                    const float x = Ljj[(32 * b + n) + (int64_t)(32 * b + q) * lda];
-                    const float a = q <= n ? -x : 0.f;
-                    rr = __builtin_amdgcn_mfma_f32_32x32x2f32(a, xb[t], rr, 0, 0, 0);
-                }
-#pragma unroll
-                for (int t = 0; t < 16; ++t)
-                    xb = __builtin_amdgcn_mfma_f32_32x32x2f32(Db[n + sigma(t, h) * 32], rr[t], xb, 0,
-                                                              0, 0);
-            }
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(lv[b & 1][t], x[t >> 2][t & 3], acc, 0, 0, 0);
+            if (wave == b + 1) solve(b + 1);
+        } else if (wave == b) {              // (off the chain)
+            __builtin_amdgcn_s_setprio(0);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                Xs[b][n + sigma(i, h) * XLD] = xb[i];
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(xb[i]), ra, va, soff(wave, i), 0);
                 ss = fmaf(xb[i], xb[i], ss);
                 am = fmaxf(am, fabsf(xb[i]));
-            }
-            if (valid) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) A21[row + (int64_t)(32 * b + sigma(i, h)) * lda] = xb[i];
-            }
-        }
-        if (b + 1 < NBK) {
-            mpc_lds_barrier();
-#pragma unroll
-            for (int o = 0; o < NO; ++o) {
-                const int bp = wave + NW * o;
-                if (bp > b) {
-#pragma unroll
-                    for (int t = 0; t < 16; ++t)
-                        acc[o] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                            lv[o][t], Xs[b][n + sigma(t, h) * XLD], acc[o], 0, 0, 0);
-                }
             }
         }
     }
@@ -141,7 +131,7 @@ __global__ __launch_bounds__(NW * 64, 2) void trsm_stats_kernel(float* __restric
     float tss = 0.f, tam = 0.f;
     if (lane < 32) {
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < NB; ++w) {
             tss += red_ss[w][lane] + red_ss[w][lane + 32];
             tam = fmaxf(tam, fmaxf(red_am[w][lane], red_am[w][lane + 32]));
         }
@@ -353,20 +343,24 @@ int mpc_launch_trsm_stats(hipStream_t st, float* A21, int64_t lda, int64_t s, in
         mpc_set_error("trsm: row range end %lld not a multiple of 32", (long long)row1);
         return MPC_ERR_ARG;
     }
+    if (lda > (1 << 21)) {                   // 32-bit offsets within a slab
+        mpc_set_error("trsm: leading dimension %lld above 2^21", (long long)lda);
+        return MPC_ERR_ARG;
+    }
     dim3 grid((unsigned)((row1 - row0 + 31) / 32));
     switch (nb) {
     case 64:
-        hipLaunchKernelGGL((trsm_stats_kernel<2, 2, kTrsmRefine>), grid, dim3(128), 0, st, A21,
+        hipLaunchKernelGGL(trsm_stats_kernel<2>, grid, dim3(128), 0, st, A21,
                            lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
                            tile_maxrs, row0, diag0, slot & 1);
         break;
     case 128:
-        hipLaunchKernelGGL((trsm_stats_kernel<4, 4, kTrsmRefine>), grid, dim3(256), 0, st, A21,
+        hipLaunchKernelGGL(trsm_stats_kernel<4>, grid, dim3(256), 0, st, A21,
                            lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
                            tile_maxrs, row0, diag0, slot & 1);
         break;
     case 256:
-        hipLaunchKernelGGL((trsm_stats_kernel<8, 4, kTrsmRefine>), grid, dim3(256), 0, st, A21,
+        hipLaunchKernelGGL(trsm_stats_kernel<8>, grid, dim3(512), 0, st, A21,
                            lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
                            tile_maxrs, row0, diag0, slot & 1);
         break;
