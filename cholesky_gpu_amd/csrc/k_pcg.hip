@@ -391,134 +391,182 @@ __global__ __launch_bounds__(RB) void copy_f32_kernel(int64_t rows, int64_t cols
 // s x s products and updates of the block recurrence (s <= MPC_BLOCK_PCG_MAX
 // right-hand sides, n x s blocks column-major).
 constexpr int BS = MPC_BLOCK_PCG_MAX;   // largest block
-constexpr int GCH = 2048;         // rows per gram workgroup
-constexpr int GSUB = 128;         // rows staged in LDS at a time
+constexpr int GROWS = 256;        // rows of a gram workgroup at a time, 64 per wave
+constexpr int GWG = 32;           // most gram workgroups (the last one adds their sums)
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
-// G = X^T Y: workgroup c forms the s^2 partial dots of rows
-// [c GCH, (c+1) GCH) (thread p = a + s b, rows ascending) and the last one
-// to finish adds the partials of every chunk in order.
-__global__ __launch_bounds__(256) void gram_kernel(int64_t n, int s, const double* __restrict__ X,
-                                                  int64_t ldx, const double* __restrict__ Y,
-                                                  int64_t ldy, double* __restrict__ part,
-                                                  double* __restrict__ G, int* __restrict__ tick) {
-    __shared__ double xs[BS][GSUB + 1], ys[BS][GSUB + 1];
-    const int tid = threadIdx.x;
+int64_t gram_rows(int64_t n) {    // rows of a workgroup
+    const int64_t per = (n + GWG * GROWS - 1) / (GWG * GROWS);
+    return per * GROWS;
+}
+
+// G = X^T Y on the FP64 matrix cores (v_mfma_f64_16x16x4): lane (q, k) of a wave
+// holds 16 rows 16k .. 16k+15 of column q of both blocks (whole lines), product
+// t multiplies the rows 16k + t, and register e of the lane is G[4e + k][q].
+// Workgroup c takes rows [c chunk, (c+1) chunk), its waves' sums are added in
+// wave order and the last workgroup to finish adds the workgroups' in order.
+// (One thread per entry of G over 2048 rows took 74 us at n = 6000.)
+__global__ __launch_bounds__(256, 2) void gram_kernel(int64_t n, int s, int64_t chunk,
+                                                     const double* __restrict__ X, int64_t ldx,
+                                                     const double* __restrict__ Y, int64_t ldy,
+                                                     double* __restrict__ part,
+                                                     double* __restrict__ G, int* __restrict__ tick) {
+    __shared__ double red[4][BS * BS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int q = lane & 15, k = lane >> 4, qc = q < s ? q : s - 1;
     const int s2 = s * s;
-    const int a = tid % s, b = tid / s;
-    const int64_t r0 = (int64_t)blockIdx.x * GCH;
-    double acc = 0.0;
-    for (int64_t q0 = r0; q0 < r0 + GCH && q0 < n; q0 += GSUB) {
-        for (int idx = tid; idx < s * GSUB; idx += 256) {
-            const int c = idx / GSUB, r = idx % GSUB;
-            const int64_t gr = q0 + r;
-            const int64_t rc = gr < n ? gr : n - 1;
-            const double vx = X[c * ldx + rc], vy = Y[c * ldy + rc];
-            xs[c][r] = gr < n ? vx : 0.0;
-            ys[c][r] = gr < n ? vy : 0.0;
+    const int64_t r0 = (int64_t)blockIdx.x * chunk, r1 = r0 + chunk < n ? r0 + chunk : n;
+    const double* Xq = X + qc * ldx;
+    const double* Yq = Y + qc * ldy;
+    v4d acc = {};
+    for (int64_t rw = r0 + 64 * wave; rw < r1; rw += GROWS) {
+        const int64_t r = rw + 16 * k;
+        double x[16], y[16];
+        if (rw + 64 <= n) {
+#pragma unroll
+            for (int t = 0; t < 16; t += 2) {
+                const d2u u = *reinterpret_cast<const d2u*>(Xq + r + t);
+                const d2u v = *reinterpret_cast<const d2u*>(Yq + r + t);
+                x[t] = u[0]; x[t + 1] = u[1];
+                y[t] = v[0]; y[t + 1] = v[1];
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                const int64_t rc = r + t < n ? r + t : n - 1;
+                const double u = Xq[rc], v = Yq[rc];
+                x[t] = r + t < n ? u : 0.0;
+                y[t] = r + t < n ? v : 0.0;
+            }
         }
-        __syncthreads();
-        if (tid < s2) {
-#pragma unroll 8
-            for (int r = 0; r < GSUB; ++r) acc = fma(xs[a][r], ys[b][r], acc);
-        }
-        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[t], acc, 0, 0, 0);
     }
-    if (tid < s2) part[(int64_t)blockIdx.x * s2 + tid] = acc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][(4 * e + k) + BS * q] = acc[e];
+    __syncthreads();
+    const int a = tid % s, b = tid / s;
+    if (tid < s2) {
+        const int i = a + BS * b;
+        part[(int64_t)blockIdx.x * s2 + tid] = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
+    }
     if (!mpc_last_arrival(tick, (int)gridDim.x)) return;
     if (tid < s2) {
-        double t = 0.0;
-        for (int c = 0; c < (int)gridDim.x; ++c) t += part[(int64_t)c * s2 + tid];
+        double v[GWG], t = 0.0;
+#pragma unroll
+        for (int c = 0; c < GWG; ++c)
+            v[c] = part[(int64_t)(c < (int)gridDim.x ? c : 0) * s2 + tid];
+#pragma unroll
+        for (int c = 0; c < GWG; ++c) t += c < (int)gridDim.x ? v[c] : 0.0;
         G[tid] = t;
     }
 }
 
 // Xo = G^-1 H for s x s G (its lower triangle, SPD) and H, through the
-// Cholesky factor of G in LDS (one thread factors, thread c solves column
-// c).  A pivot not above kSpdRelPivot times its diagonal entry (G singular
+// Cholesky factor of G.  One wave, a row of G per lane in registers: column j's
+// entries are broadcast to the lanes below by lane reads; then lane c solves
+// column c.  A pivot not above kSpdRelPivot times its diagonal entry (G singular
 // to working precision, e.g. dependent columns), or not finite, sets *flag
 // and gives Xo = 0, so the updates that use Xo leave their blocks unchanged.
+// (One thread for the factor: 45 us at s = 16.)
 constexpr double kSpdRelPivot = 1e-13;
+__device__ __forceinline__ double lane_double(double v, int l) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
 __global__ __launch_bounds__(64) void spd_solve_kernel(int s, const double* __restrict__ Gm,
                                                       const double* __restrict__ H,
                                                       double* __restrict__ Xo,
                                                       int* __restrict__ flag) {
-    __shared__ double C[BS][BS + 1];
-    __shared__ int bad;
-    const int tid = threadIdx.x;
-    for (int idx = tid; idx < s * s; idx += 64) C[idx % s][idx / s] = Gm[idx];
-    __syncthreads();
-    if (tid == 0) {
-        int b = 0;
-        for (int j = 0; j < s && !b; ++j) {
-            const double g = C[j][j];
-            double d = g;
-            for (int k = 0; k < j; ++k) d -= C[j][k] * C[j][k];
-            if (!(d > kSpdRelPivot * g) || !(d < INFINITY)) { b = 1; break; }
-            d = sqrt(d);
-            C[j][j] = d;
-            for (int i = j + 1; i < s; ++i) {
-                double v = C[i][j];
-                for (int k = 0; k < j; ++k) v -= C[i][k] * C[j][k];
-                C[i][j] = v / d;
+    __shared__ double C[BS][BS];                 // C[k][i] = L(i, k)
+    const int tid = threadIdx.x, r = tid < s ? tid : s - 1;
+    double c[BS], x[BS];
+#pragma unroll
+    for (int k = 0; k < BS; ++k) {
+        const int kc = k < s ? k : s - 1;
+        c[k] = Gm[r + kc * s];
+        x[k] = H[kc + r * s];
+    }
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < BS; ++j) {
+        if (j < s && !bad) {                     // (uniform)
+            const double d = lane_double(c[j], j), g = Gm[j + j * s];
+            if (!(d > kSpdRelPivot * g) || !(d < INFINITY)) {
+                bad = true;
+            } else {
+                const double l = sqrt(d);
+                c[j] = tid == j ? l : c[j] / l;  // lanes above j hold nothing of use
+#pragma unroll
+                for (int k = j + 1; k < BS; ++k)
+                    if (k < s) c[k] = fma(-c[j], lane_double(c[j], k), c[k]);
             }
         }
-        bad = b;
-        if (b) flag[0] = 1;
+        if (tid < BS) C[j][tid] = c[j];
     }
+    if (bad && tid == 0) flag[0] = 1;
     __syncthreads();
-    if (tid < s) {
-        double x[BS];
+    if (tid >= s) return;
+    if (!bad) {
 #pragma unroll
-        for (int i = 0; i < BS; ++i) x[i] = 0.0;
-        if (!bad) {
+        for (int i = 0; i < BS; ++i) {                 // L y = h
+            if (i < s) {
 #pragma unroll
-            for (int i = 0; i < BS; ++i) {                 // C y = h
-                if (i < s) {
-                    double v = H[i + tid * s];
-#pragma unroll
-                    for (int k = 0; k < i; ++k) v -= C[i][k] * x[k];
-                    x[i] = v / C[i][i];
-                }
-            }
-#pragma unroll
-            for (int i = BS - 1; i >= 0; --i) {            // C^T x = y
-                if (i < s) {
-                    double v = x[i];
-#pragma unroll
-                    for (int k = i + 1; k < BS; ++k)
-                        if (k < s) v -= C[k][i] * x[k];
-                    x[i] = v / C[i][i];
-                }
+                for (int k = 0; k < i; ++k) x[i] = fma(-C[k][i], x[k], x[i]);
+                x[i] /= C[i][i];
             }
         }
 #pragma unroll
-        for (int i = 0; i < BS; ++i)
-            if (i < s) Xo[i + tid * s] = x[i];
+        for (int i = BS - 1; i >= 0; --i) {            // L^T x = y
+            if (i < s) {
+#pragma unroll
+                for (int k = i + 1; k < BS; ++k)
+                    if (k < s) x[i] = fma(-C[i][k], x[k], x[i]);
+                x[i] /= C[i][i];
+            }
+        }
     }
+#pragma unroll
+    for (int i = 0; i < BS; ++i)
+        if (i < s) Xo[i + tid * s] = bad ? 0.0 : x[i];
 }
 
 // Y[r][j] = (Z ? Z[r][j] : Y[r][j]) + a sum_k M[r][k] Cm[k][j], one thread
-// per row; the row of M is read before any write, so Y may be M.
-__global__ __launch_bounds__(256) void block_axpy_kernel(int64_t n, int s, const double* M,
-                                                        int64_t ldm,
-                                                        const double* __restrict__ Cm, double a,
-                                                        const double* Z, int64_t ldz, double* Y,
-                                                        int64_t ldy) {
+// per row; the row of M is read before any write, so Y may be M.  All loads of
+// a row are in flight at once, and a workgroup is one wave, so that a few
+// thousand rows reach many CUs (n = 6000, s = 16: 17.3 us with 256 rows a
+// workgroup and a base column at a time).
+__global__ __launch_bounds__(64) void block_axpy_kernel(int64_t n, int s, const double* M,
+                                                       int64_t ldm, const double* __restrict__ Cm,
+                                                       double a, const double* Z, int64_t ldz,
+                                                       double* Y, int64_t ldy) {
     __shared__ double cs[BS * BS];
-    for (int idx = threadIdx.x; idx < s * s; idx += 256) cs[idx] = Cm[idx];
+    const int64_t r0 = (int64_t)blockIdx.x * 64 + threadIdx.x, r = r0 < n ? r0 : n - 1;
+    const double* B = Z ? Z : Y;
+    const int64_t ldb = Z ? ldz : ldy;
+    double m[BS], y[BS];
+#pragma unroll
+    for (int k = 0; k < BS; ++k) {
+        const int kc = k < s ? k : s - 1;
+        m[k] = M[kc * ldm + r];
+        y[k] = B[kc * ldb + r];
+    }
+    for (int idx = threadIdx.x; idx < s * s; idx += 64) cs[idx] = Cm[idx];
     __syncthreads();
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= n) return;
-    double m[BS];
+    if (r0 >= n) return;
 #pragma unroll
-    for (int k = 0; k < BS; ++k) m[k] = k < s ? M[k * ldm + r] : 0.0;
-    for (int j = 0; j < s; ++j) {
-        double v = 0.0;
+    for (int j = 0; j < BS; ++j) {
+        if (j < s) {
+            double v = 0.0;
 #pragma unroll
-        for (int k = 0; k < BS; ++k)
-            if (k < s) v = fma(m[k], cs[k + j * s], v);
-        const double base = Z ? Z[j * ldz + r] : Y[j * ldy + r];
-        Y[j * ldy + r] = fma(a, v, base);
+            for (int k = 0; k < BS; ++k)
+                if (k < s) v = fma(m[k], cs[k + j * s], v);
+            Y[j * ldy + r] = fma(a, v, y[j]);
+        }
     }
 }
 
@@ -677,7 +725,8 @@ int mpc_launch_copy_f32(hipStream_t st, int64_t rows, int64_t cols, const float*
 }
 
 int64_t mpc_gram_partial_doubles(int64_t n, int s) {
-    return ((n + GCH - 1) / GCH) * (int64_t)s * s;
+    (void)n;
+    return GWG * (int64_t)s * s;
 }
 
 int mpc_launch_gram(hipStream_t st, int64_t n, int s, const double* X, int64_t ldx,
@@ -686,8 +735,9 @@ int mpc_launch_gram(hipStream_t st, int64_t n, int s, const double* X, int64_t l
         mpc_set_error("gram: block of %d columns (1..%d)", s, BS);
         return MPC_ERR_ARG;
     }
-    hipLaunchKernelGGL(gram_kernel, dim3((unsigned)((n + GCH - 1) / GCH)), dim3(256), 0, st, n, s,
-                       X, ldx, Y, ldy, part, G, tick);
+    const int64_t chunk = gram_rows(n);
+    hipLaunchKernelGGL(gram_kernel, dim3((unsigned)((n + chunk - 1) / chunk)), dim3(256), 0, st, n, s,
+                       chunk, X, ldx, Y, ldy, part, G, tick);
     MPC_LAUNCH_CHECK();
     return 0;
 }
@@ -702,7 +752,7 @@ int mpc_launch_spd_solve(hipStream_t st, int s, const double* G, const double* H
 int mpc_launch_block_axpy(hipStream_t st, int64_t n, int s, const double* M, int64_t ldm,
                           const double* Cm, double a, const double* Z, int64_t ldz, double* Y,
                           int64_t ldy) {
-    hipLaunchKernelGGL(block_axpy_kernel, dim3(blocks_for(n)), dim3(256), 0, st, n, s, M, ldm, Cm,
+    hipLaunchKernelGGL(block_axpy_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, n, s, M, ldm, Cm,
                        a, Z, ldz, Y, ldy);
     MPC_LAUNCH_CHECK();
     return 0;
