@@ -22,14 +22,41 @@
 namespace {
 
 constexpr int GT = 64;        // tile edge
-constexpr int GRC = 32;       // solve columns staged per pass
-constexpr int GLD = GRC + 1;
+typedef double v4d __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void gp_grad_tile_kernel(
+// sum over the 64 lanes, in every lane: rotations within 16 lanes, then the
+// four sixteens in order
+template <int CTRL>
+__device__ __forceinline__ double rotate16(double v) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double sum64(double v) {
+    v += rotate16<0x128>(v);
+    v += rotate16<0x124>(v);
+    v += rotate16<0x122>(v);
+    v += rotate16<0x121>(v);
+    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+// One 64 x 64 tile of the lower triangle per workgroup, a 32 x 32 quarter per
+// wave.  m comes from the FP64 matrix cores (v_mfma_f64_16x16x4, operands
+// straight from L2: lane (q, k) of a product holds row q, solve column k, and
+// receives in register e the element (4e + k, q)); the 16 elements of a lane
+// then share the loops over the dimensions.  Bound by the FP64 vector
+// operations of the kernel entries (exp and two passes over the dimensions).
+__global__ __launch_bounds__(256, 2) void gp_grad_tile_kernel(
     const float* __restrict__ X, int64_t n, int d, int64_t ldx, const double* __restrict__ inv_ls,
     int n_ls, double variance, const double* __restrict__ U, const double* __restrict__ V,
-    int64_t ldu, int R, int nt, double* __restrict__ part) {
-    __shared__ double Ui[GT * GLD], Vi[GT * GLD], Uj[GT * GLD], Vj[GT * GLD];
+    int64_t ldu, int R, double* __restrict__ part) {
     __shared__ double xi[MPC_GP_MAXD][GT], xj[MPC_GP_MAXD][GT];
     __shared__ double red[4][MPC_GP_MAXD + 2];
     // lower tile (I >= J): t = I (I + 1) / 2 + J
@@ -39,8 +66,9 @@ __global__ __launch_bounds__(256) void gp_grad_tile_kernel(
     while ((I + 1) * (I + 2) / 2 <= t) ++I;
     const int64_t J = t - I * (I + 1) / 2;
     const int64_t i0 = I * GT, j0 = J * GT;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    (void)nt;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int q = lane & 15, k = lane >> 4;
+    const int bi = 32 * (wave & 1), bj = 32 * (wave >> 1);       // this wave's quarter
 
     for (int idx = tid; idx < d * GT; idx += 256) {
         const int c = idx / GT, p = idx % GT;
@@ -50,80 +78,115 @@ __global__ __launch_bounds__(256) void gp_grad_tile_kernel(
         xi[c][p] = i0 + p < n ? a : 0.0;
         xj[c][p] = j0 + p < n ? b : 0.0;
     }
-    // m[u][v] for i = i0 + tx + 16u, j = j0 + ty + 16v
-    double m[4][4] = {};
-    for (int r0 = 0; r0 < R; r0 += GRC) {
-        __syncthreads();
-        for (int idx = tid; idx < GT * GRC; idx += 256) {
-            const int p = idx % GT, r = idx / GT;
-            const bool okr = r0 + r < R;
-            const int64_t gi = i0 + p, gj = j0 + p;
-            const int64_t gic = gi < n ? gi : n - 1, gjc = gj < n ? gj : n - 1;
-            const int64_t o = (int64_t)(okr ? r0 + r : R - 1) * ldu;
-            const double ui = U[o + gic], vi = V[o + gic], uj = U[o + gjc], vj = V[o + gjc];
-            Ui[p * GLD + r] = okr && gi < n ? ui : 0.0;
-            Vi[p * GLD + r] = okr && gi < n ? vi : 0.0;
-            Uj[p * GLD + r] = okr && gj < n ? uj : 0.0;
-            Vj[p * GLD + r] = okr && gj < n ? vj : 0.0;
-        }
-        __syncthreads();
-        for (int r = 0; r < GRC; ++r) {
-            double ui[4], vi[4], uj[4], vj[4];
+    // m = (U V^T)_ij + (U V^T)_ji
+    v4d m[2][2] = {};
+    int64_t gi[2], gj[2];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                ui[u] = Ui[(tx + 16 * u) * GLD + r];
-                vi[u] = Vi[(tx + 16 * u) * GLD + r];
-                uj[u] = Uj[(ty + 16 * u) * GLD + r];
-                vj[u] = Vj[(ty + 16 * u) * GLD + r];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) m[u][v] = fma(ui[u], vj[v], fma(uj[v], vi[u], m[u][v]));
-        }
+    for (int u = 0; u < 2; ++u) {
+        const int64_t i = i0 + bi + 16 * u + q, j = j0 + bj + 16 * u + q;
+        gi[u] = i < n ? i : n - 1;           // (rows past the end are dropped below)
+        gj[u] = j < n ? j : n - 1;
     }
-    // m = (U V^T)_ij + (U V^T)_ji, which counts the diagonal twice: halved there
-    double gl[MPC_GP_MAXD], gvar = 0.0, gnoise = 0.0;
+    double ui[2], vi[2], uj[2], vj[2];
+    auto load = [&](int r0) {
+        const int r = r0 + k;
+        const int64_t o = (int64_t)(r < R ? r : R - 1) * ldu;
 #pragma unroll
-    for (int c = 0; c < MPC_GP_MAXD; ++c) gl[c] = 0.0;
+        for (int u = 0; u < 2; ++u) {
+            const double a = U[o + gi[u]], b = V[o + gi[u]], c = U[o + gj[u]], e = V[o + gj[u]];
+            ui[u] = r < R ? a : 0.0;
+            vi[u] = r < R ? b : 0.0;
+            uj[u] = r < R ? c : 0.0;
+            vj[u] = r < R ? e : 0.0;
+        }
+    };
+    load(0);
+    for (int r0 = 0; r0 < R; r0 += 4) {
+        double a[2], b[2], c[2], e[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < 2; ++u) {
+            a[u] = ui[u];
+            b[u] = vi[u];
+            c[u] = uj[u];
+            e[u] = vj[u];
+        }
+        if (r0 + 4 < R) load(r0 + 4);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int pi = tx + 16 * u, pj = ty + 16 * v;
-            const int64_t i = i0 + pi, j = j0 + pj;
-            if (i >= n || j >= n || j > i) continue;
-            double w = m[u][v];
-            if (i == j) {
-                w *= 0.5;
-                gnoise += w;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                m[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], e[v], m[u][v], 0, 0, 0);
+                m[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[u], c[v], m[u][v], 0, 0, 0);
             }
-            double s2 = 0.0;
-            for (int c = 0; c < d; ++c) {
-                const double df = xi[c][pi] - xj[c][pj];
-                s2 = fma(df, df, s2);
-            }
-            const double kij = variance * exp(-0.5 * s2);
-            const double wk = w * kij;
-            gvar += wk;
-            if (n_ls == 1) {
-                gl[0] += wk * s2;          // times 1/ls on the host
-            } else {
-                for (int c = 0; c < d; ++c) {
-                    const double df = xi[c][pi] - xj[c][pj];
-                    gl[c] = fma(wk, df * df, gl[c]);
+    }
+    __syncthreads();
+    // element x = 8u + 4v + e of this lane: (pi(u, e), pj(v))
+    auto pi = [&](int u, int e) { return bi + 16 * u + 4 * e + k; };
+    auto pj = [&](int v) { return bj + 16 * v + q; };
+    double s2[16] = {};
+    for (int c = 0; c < d; ++c) {
+        double y[2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) y[v] = xj[c][pj(v)];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double x = xi[c][pi(u, e)];
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    const double df = x - y[v];
+                    s2[8 * u + 4 * v + e] = fma(df, df, s2[8 * u + 4 * v + e]);
                 }
             }
-        }
-    // workgroup reduction (wave shuffles, then 4 waves in order)
-    const int nout = (n_ls == 1 ? 1 : d) + 2;
-    const int lane = tid & 63, wave = tid >> 6;
-    for (int q = 0; q < nout; ++q) {
-        double v = q < nout - 2 ? gl[q] : (q == nout - 2 ? gvar : gnoise);
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-        if (lane == 0) red[wave][q] = v;
     }
+    // the lower triangle's weights; m counts the diagonal twice
+    double wk[16], gvar = 0.0, gnoise = 0.0, giso = 0.0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int x = 8 * u + 4 * v + e;
+                const int64_t i = i0 + pi(u, e), j = j0 + pj(v);
+                double w = i < n && j <= i ? m[u][v][e] : 0.0;
+                if (i == j) {
+                    w *= 0.5;
+                    gnoise += w;
+                }
+                wk[x] = w * (variance * exp(-0.5 * s2[x]));
+                gvar += wk[x];
+                giso = fma(wk[x], s2[x], giso);
+            }
+    const int nout = (n_ls == 1 ? 1 : d) + 2;
+    auto out = [&](int c, double v) {
+        v = sum64(v);
+        if (lane == 0) red[wave][c] = v;
+    };
+    if (n_ls == 1) {
+        out(0, giso);                        // times 1/ls on the host
+    } else {
+        for (int c = 0; c < d; ++c) {
+            double y[2], g = 0.0;
+#pragma unroll
+            for (int v = 0; v < 2; ++v) y[v] = xj[c][pj(v)];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double x = xi[c][pi(u, e)];
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const double df = x - y[v];
+                        g = fma(wk[8 * u + 4 * v + e], df * df, g);
+                    }
+                }
+            out(c, g);
+        }
+    }
+    out(nout - 2, gvar);
+    out(nout - 1, gnoise);
     __syncthreads();
     if (tid < nout) part[t * nout + tid] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
 }
@@ -185,7 +248,7 @@ int mpc_launch_gp_grad(hipStream_t st, const float* X, int64_t n, int d, int64_t
     const int64_t ntile = nt * (nt + 1) / 2;
     const int nout = (n_ls == 1 ? 1 : d) + 2;
     hipLaunchKernelGGL(gp_grad_tile_kernel, dim3((unsigned)ntile), dim3(256), 0, st, X, n, d, ldx,
-                       inv_ls, n_ls, variance, U, V, ldu, R, (int)nt, part);
+                       inv_ls, n_ls, variance, U, V, ldu, R, part);
     hipLaunchKernelGGL(gp_grad_reduce_kernel, dim3((unsigned)nout), dim3(256), 0, st, part, ntile,
                        nout, out);
     MPC_LAUNCH_CHECK();

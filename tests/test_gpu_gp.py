@@ -127,3 +127,26 @@ def test_gp_autograd_function(handle, oracle):
     assert abs(var.grad.item() - 3.0 * rvar) <= 1e-6 * abs(3.0 * rvar)
     assert abs(noise.grad.item() - 3.0 * rno) <= 1e-6 * abs(3.0 * rno)
     assert rel(bt.grad.cpu().numpy(), 3.0 * rb) < 1e-9
+
+
+@pytest.mark.parametrize("n,d,ard,P", [(1, 2, True, 1), (31, 16, True, 3), (64, 1, True, 2), (65, 5, False, 4),
+                                       (129, 16, False, 7), (193, 3, True, 33)])
+def test_gp_gradient_tile_edges(handle, oracle, n, d, ard, P):
+    """Tiles that are not full (quarters of 32, 64), 1 and 16 dimensions,
+    solve columns (1 + probes) that are not a multiple of 4.  Solves to 1e-11
+    with cond(A) <= n variance / noise + 1 <= 2.4e4, so 1e-6 as above."""
+    say("gp grad edges", n, d, ard, P)
+    X, ls, b = gp_case(n, d, seed=n)
+    if not ard:
+        ls = ls[:1]
+    var, noise, seed = 1.2, 1e-2, 77
+    o = S.gp_opts(n_probes=P, probe_seed=seed, factor=S.factor_opts(nb=64),
+                  pcg=S.pcg_opts(tol=1e-11, maxit=400))
+    _, gb, gls, gvar, gno, _ = S.gp_loss_grad(handle, torch.from_numpy(X).cuda(), ls, var, noise,
+                                              torch.from_numpy(b).cuda(), o)
+    _, rb, rls, rvar, rno = oracle.gp_loss_grad_f64(X, ls, var, noise, b, Z=oracle.probes(n, P, seed))
+    assert rel(gb.cpu().numpy(), rb) < 1e-6
+    # a single point has no distances: both are zero
+    assert np.linalg.norm(np.asarray(gls) - rls) <= 1e-6 * np.linalg.norm(rls), (gls, rls)
+    assert abs(gvar - rvar) <= 1e-6 * abs(rvar)
+    assert abs(gno - rno) <= 1e-6 * abs(rno)
