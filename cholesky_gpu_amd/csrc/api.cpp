@@ -593,11 +593,17 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
             return r;
         if (s == 0) return 0;
         float* A21 = dA + e + c0 * lda;
+        const bool fp32 = o->update_prec == MPC_PREC_FP32;
+        const mpc_fp32_panel out = {payload + q * pstride, (int64_t)nb * 4, scales + q * sstride,
+                                    sm->tile_prec[q], map ? map + (j + 1) + j * nt : nullptr,
+                                    tr / nb, nt - (j + 1)};
         if ((r = mpc_launch_trsm_stats(ps, A21, lda, s, nb, dinv + (c0 / 32) * 1024, Ajj,
                                        rowss + e, tracker + e, tr, sm, sm->tile_amax[b],
                                        sm->tile_maxrs[b], 0, -1,
-                                       rule == MPC_RULE_SCHUR ? diag0 + e : nullptr, b)))
+                                       rule == MPC_RULE_SCHUR ? diag0 + e : nullptr, b,
+                                       fp32 ? &out : nullptr)))
             return r;
+        if (fp32) return 0;
         return mpc_launch_quantize_ex(ps, A21, s, nb, lda, tr, nullptr, sm->tile_amax[b],
                                       sm->tile_maxrs[b], sm, o->update_prec, ladder, o->n_ladder,
                                       eps, sm->tile_prec[q], map ? map + (j + 1) + j * nt : nullptr,
@@ -969,11 +975,12 @@ static int factor_impl(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         if (!map) map = base + (d_tracker ? 0 : (size_t)(n + 64) * sizeof(float));
     }
     // backup for the fallback path when the caller gave no source to restore from
+    // (an FP32 failure is final: nothing to restore)
     const float* src = restore_from;
     int64_t src_ld = restore_ld;
-    if (o->fallback && !src) {
+    if (o->fallback && !src && o->update_prec != MPC_PREC_FP32) {
         if ((rc = mpc_ws_reserve(h->amat, sizeof(float) * (size_t)n * n))) return rc;
-        if ((rc = mpc_launch_copy_f32(h->stream, n, n, dA, lda, (float*)h->amat.ptr, n))) return rc;
+        if ((rc = mpc_launch_copy_lower(h->stream, n, n, dA, lda, (float*)h->amat.ptr, n))) return rc;
         src = (const float*)h->amat.ptr;
         src_ld = n;
     }
@@ -1001,7 +1008,7 @@ static int factor_impl(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         const bool all_fp32 = cur.update_prec == MPC_PREC_FP32;
         if ((rc2_wait = wait_winv(h, h->stream))) return rc2_wait;   // before A is restored
         if (all_fp32) break;
-        int rc2 = mpc_launch_copy_f32(h->stream, n, n, src, src_ld, dA, lda);
+        int rc2 = mpc_launch_copy_lower(h->stream, n, n, src, src_ld, dA, lda);
         if (rc2) return rc2;
         ++attempt;
         if (cur.update_prec == MPC_PREC_SWITCH && attempt <= 2) eps /= 16.0;
@@ -1695,7 +1702,7 @@ extern "C" int mpc_precond_cg(mpc_handle* h, const float* dA, int64_t lda, int64
     if ((rc = validate_factor_opts(fo))) return rc;
     const int AG = agg_panels_of(fo);
     const bool defer = lda == n && AG > 1 && (int64_t)AG * fo->nb < n;
-    if ((rc = mpc_launch_copy_f32(h->stream, n, defer ? (int64_t)AG * fo->nb : n, dA, lda, L, n)))
+    if ((rc = mpc_launch_copy_lower(h->stream, n, defer ? (int64_t)AG * fo->nb : n, dA, lda, L, n)))
         return rc;
     // the caller's A stays intact, so the fallback restores from it
     rc = factor_impl(h, L, n, n, fo, nullptr, nullptr, finfo, dA, lda, true, defer ? dA : nullptr);
@@ -1799,11 +1806,16 @@ extern "C" int mpc_gp_loss_grad(mpc_handle* h, const float* dX, int64_t n, int d
     MPC_HIP(hipMemcpyAsync(dinvls, inv.data(), sizeof(double) * n_ls, hipMemcpyHostToDevice, st));
     if ((rc = mpc_launch_rbf64(st, dX, n, d, ldx, dinvls, n_ls, variance, noise, A64, n, A32, n)))
         return rc;
-    if ((rc = mpc_launch_copy_f32(st, n, n, A32, n, L, n))) return rc;
+    // (the rest of A32 goes over with the first aggregated update, as in mpc_precond_cg)
+    if ((rc = validate_factor_opts(&o->factor))) return rc;
+    const int64_t first = (int64_t)agg_panels_of(&o->factor) * o->factor.nb;
+    const bool defer = agg_panels_of(&o->factor) > 1 && first < n;
+    if ((rc = mpc_launch_copy_lower(st, n, defer ? first : n, A32, n, L, n))) return rc;
     // 2. mixed-precision factor of the FP32 copy (the preconditioner)
     mpc_factor_info fi;
     std::memset(&fi, 0, sizeof fi);
-    rc = factor_impl(h, L, n, n, &o->factor, nullptr, nullptr, &fi, A32, n, true);
+    rc = factor_impl(h, L, n, n, &o->factor, nullptr, nullptr, &fi, A32, n, true,
+                     defer ? A32 : nullptr);
     if (info) info->factor = fi;
     if (rc != 0) return rc;
     // 3. adjoint solve A [alpha, w_1..w_P] = [b, z_1..z_P] with the FP64 operator

@@ -41,7 +41,9 @@ __device__ __forceinline__ int sigma(int s, int h) { return 8 * (s >> 2) + 4 * h
 // slab); accumulator register i of lane (n, h) holds column sig(i, h), row n,
 // negated, so that the products add.  So the lane's X operand of k step t is its
 // own register t of X_b.
-template <int NB>
+// OUT: X also goes to the SYRK operand (an all-FP32 factor takes no decision and
+// rounds nothing, so no launch of the quantiser: 4.7 us a step).
+template <int NB, bool OUT>
 __global__ __launch_bounds__(NB * 64, 4) void trsm_stats_kernel(float* __restrict__ A21, int64_t lda,
                                                          int64_t s, const float* __restrict__ dinv_j,
                                                          const float* __restrict__ Ljj,
@@ -52,7 +54,7 @@ __global__ __launch_bounds__(NB * 64, 4) void trsm_stats_kernel(float* __restric
                                                          uint32_t* __restrict__ t_maxrs,
                                                          int64_t row0,
                                                          const float* __restrict__ diag0,
-                                                         int slot) {
+                                                         int slot, const mpc_fp32_panel P) {
     __shared__ v4f Xs[NB][4][64];
     __shared__ float red_ss[NB][64], red_am[NB][64];
     const int lane = threadIdx.x & 63;
@@ -121,6 +123,24 @@ __global__ __launch_bounds__(NB * 64, 4) void trsm_stats_kernel(float* __restric
                 ss = fmaf(xb[i], xb[i], ss);
                 am = fmaxf(am, fabsf(xb[i]));
             }
+            if constexpr (OUT) {
+                if (valid) {
+                    float* dst = reinterpret_cast<float*>(P.payload + row * P.row_stride) + 32 * wave + 4 * h;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        *reinterpret_cast<v4f*>(dst + 8 * v) =
+                            v4f{xb[4 * v], xb[4 * v + 1], xb[4 * v + 2], xb[4 * v + 3]};
+                    if (h == 0) P.scales[row * NB + wave] = 127;
+                }
+            }
+        }
+    }
+    if constexpr (OUT) {
+        if (r0 % tile_rows == 0 && threadIdx.x == 0) {
+            const int64_t tile = r0 / tile_rows;
+            P.prec[tile] = MPC_PREC_FP32;
+            for (int u = 0; u < P.map_rep && P.map_col; ++u)
+                if (tile * P.map_rep + u < P.map_len) P.map_col[tile * P.map_rep + u] = MPC_PREC_FP32;
         }
     }
     // row statistics: lane (n, h) of every wave holds part of row n
@@ -329,7 +349,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(
 int mpc_launch_trsm_stats(hipStream_t st, float* A21, int64_t lda, int64_t s, int nb,
                           const float* dinv_j, const float* Ljj, float* rowss, float* tracker,
                           int tile_rows, mpc_small* sm, uint32_t* tile_amax, uint32_t* tile_maxrs,
-                          int64_t row0, int64_t row1, const float* diag0, int slot) {
+                          int64_t row0, int64_t row1, const float* diag0, int slot,
+                          const mpc_fp32_panel* out) {
     if (row1 < 0 || row1 > s) row1 = s;
     if (row1 <= row0) return 0;
     if (tile_rows % 32 || row0 % 32) {
@@ -348,22 +369,24 @@ int mpc_launch_trsm_stats(hipStream_t st, float* A21, int64_t lda, int64_t s, in
         return MPC_ERR_ARG;
     }
     dim3 grid((unsigned)((row1 - row0 + 31) / 32));
+#define MPC_TRSM(N, O)                                                                             \
+    hipLaunchKernelGGL((trsm_stats_kernel<N, O>), grid, dim3(64 * N), 0, st, A21, lda, s, dinv_j,   \
+                       Ljj, rowss, tracker, tile_rows, sm, tile_amax, tile_maxrs, row0, diag0,      \
+                       slot & 1, out ? *out : mpc_fp32_panel{})
     switch (nb) {
     case 64:
-        hipLaunchKernelGGL(trsm_stats_kernel<2>, grid, dim3(128), 0, st, A21,
-                           lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
-                           tile_maxrs, row0, diag0, slot & 1);
+        if (out) MPC_TRSM(2, true);
+        else MPC_TRSM(2, false);
         break;
     case 128:
-        hipLaunchKernelGGL(trsm_stats_kernel<4>, grid, dim3(256), 0, st, A21,
-                           lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
-                           tile_maxrs, row0, diag0, slot & 1);
+        if (out) MPC_TRSM(4, true);
+        else MPC_TRSM(4, false);
         break;
     case 256:
-        hipLaunchKernelGGL(trsm_stats_kernel<8>, grid, dim3(512), 0, st, A21,
-                           lda, s, dinv_j, Ljj, rowss, tracker, tile_rows, sm, tile_amax,
-                           tile_maxrs, row0, diag0, slot & 1);
+        if (out) MPC_TRSM(8, true);
+        else MPC_TRSM(8, false);
         break;
+#undef MPC_TRSM
     default:
         mpc_set_error("trsm: unsupported block size %d", nb);
         return MPC_ERR_ARG;

@@ -192,11 +192,23 @@ int mpc_launch_potrf(hipStream_t st, float* A, int64_t lda, int bs, int col0,
 // k_panel.hip
 // rows [row0, row1) of the s-row panel (row1 < 0: s); the panel kernels
 // index tiles and statistics by the row within the whole panel
+// The SYRK operand of an all-FP32 panel, written by the TRSM itself (as the
+// quantiser would: row-major payload, neutral scales, precision per tile, map)
+struct mpc_fp32_panel {
+    uint8_t* payload;
+    int64_t row_stride;
+    uint8_t* scales;
+    uint8_t* prec;            // per tile
+    uint8_t* map_col;         // or nullptr: map_rep entries per tile, at most map_len
+    int map_rep;
+    int64_t map_len;
+};
 int mpc_launch_trsm_stats(hipStream_t st, float* A21, int64_t lda, int64_t s, int nb,
                           const float* dinv_j, const float* Ljj, float* rowss, float* tracker,
                           int tile_rows, mpc_small* sm, uint32_t* tile_amax, uint32_t* tile_maxrs,
                           int64_t row0 = 0, int64_t row1 = -1, const float* diag0 = nullptr,
-                          int slot = 0);
+                          int slot = 0,
+                          const mpc_fp32_panel* out = nullptr);
 int mpc_launch_quantize_ex(hipStream_t st, const float* P, int64_t m, int k, int64_t ld,
                            int tile_rows, const uint8_t* prec_in, const uint32_t* tile_amax,
                            const uint32_t* tile_maxrs, mpc_small* sm, int update_prec,
@@ -302,8 +314,9 @@ int mpc_launch_axpby(hipStream_t st, int64_t n, int nrhs, double a, const double
                      int64_t ldx, double b, double* Y, int64_t ldy);
 int mpc_launch_copy2d(hipStream_t st, int64_t n, int nrhs, const double* X, int64_t ldx,
                       double* Y, int64_t ldy);
-int mpc_launch_copy_f32(hipStream_t st, int64_t rows, int64_t cols, const float* A,
-                        int64_t lda, float* B, int64_t ldb);
+// B = A on and below the diagonal (rows x cols, cols <= rows)
+int mpc_launch_copy_lower(hipStream_t st, int64_t rows, int64_t cols, const float* A, int64_t lda,
+                          float* B, int64_t ldb);
 // k_matgen.hip
 int mpc_launch_hh_matrix(hipStream_t st, int64_t n, const double* lam, const double* W,
                          const double* P, const double* g, float* A, int64_t lda);

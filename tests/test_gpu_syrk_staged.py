@@ -84,3 +84,21 @@ def test_factor_one_stream_tail(handle, n, nb, prec):
         outs.append(T)
     assert torch.equal(outs[1], outs[2])
     assert err[1] <= 1.1 * err[0], err
+
+
+@pytest.mark.parametrize("n,nb", [(130, 64), (517, 128), (1031, 256), (4101, 256)])
+def test_factor_restored_after_breakdown(handle, n, nb):
+    """E4M3 updates break down on a kernel matrix with eigenvalues down to
+    1e-5; the fallback restores A (its lower triangle, 16-byte pieces, ragged
+    ends) and ends with FP32 updates: the outcome is that of an FP32 run on A,
+    the same factor bit for bit or (4101 points: cond 1e8) the same failing
+    column, and the strict upper triangle is A's."""
+    print("[case]", n, nb, flush=True)
+    x = torch.linspace(0, 8, n, device="cuda")
+    A = torch.exp(-0.5 * (x[:, None] - x[None, :]) ** 2) + 1e-5 * torch.eye(n, device="cuda")
+    T1, T2 = A.clone(), A.clone()
+    rc1, fi, _, _ = S.factor(handle, T1, S.factor_opts(nb=nb, update_prec=L.PREC_E4M3, fallback=1))
+    rc2, _, _, _ = S.factor(handle, T2, S.factor_opts(nb=nb, update_prec=L.PREC_FP32, fallback=0))
+    assert fi.retries == 1 and rc1 == rc2
+    assert rc1 or torch.equal(T1, T2)
+    assert torch.equal(torch.tril(T1, -1), torch.tril(A, -1))      # (the tensor is the transpose)
