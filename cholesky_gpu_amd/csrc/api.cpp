@@ -669,13 +669,18 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     // 8192 columns of n = 16384 that way cost an FP32 solve 21.3 -> 21.7 ms,
     // E4M3/FP32 14.01 -> 14.28.
     constexpr int64_t kOneStream = 4096;
-    // FP32-only updates of at least kWide columns take the 128-row kernel (too
-    // few workgroups for the chip below: n = 4000 factor 1774 us without it,
-    // 1754, 1717, 1696, 1694 and 1713 from 1024, 1536, 2048, 2560 and 3072)
+    // Updates of at least kWide columns whose operands are all of one class take
+    // that class's 128-row kernel (too few workgroups for the chip below: n = 4000
+    // FP32 factor 1774 us without it, 1754, 1717, 1696, 1694 and 1713 from 1024,
+    // 1536, 2048, 2560 and 3072; n = 4096 BF16 1337, 1277, 1270, 1263 and 1284
+    // without it and from 1536, 2048, 2560 and 3072).  With several classes it
+    // would be a launch each (E4M3/FP32 1168, and 1221 to 1186).
     constexpr int64_t kWide = 2304;
+    const bool one_launch = __builtin_popcount(cmask) == 1 &&
+                            (cmask != (1u << MPC_PREC_E4M3) || __builtin_popcount(fmask) == 1);
     auto one_stream = [&](int64_t j0, hipStream_t ps) -> int {
         for (int64_t j = j0; j + 1 < nt; ++j) {
-            const int wide = n - (j + 1) * nb >= kWide && cmask == (1u << MPC_PREC_FP32);
+            const int wide = one_launch && n - (j + 1) * nb >= kWide;
             int r;
             if ((r = AG > 1 ? agg(j, 1, j + 1, 0, -1, ps, wide ? 2 : 1)
                             : update(j, 0, -1, ps, !wide)))
