@@ -50,6 +50,27 @@ int mpc_ws_reserve(mpc_workspace& w, size_t bytes) {
     return 0;
 }
 
+// Grow-only page-locked staging memory of a handle.  What lies in it belongs to
+// one entry point call, which synchronises before it reads or returns.
+static int host_reserve(mpc_handle* h, size_t bytes) {
+    if (h->host && bytes <= h->host_bytes) return 0;
+    if (h->host) {
+        (void)hipHostFree(h->host);
+        h->host = nullptr;
+        h->host_bytes = 0;
+    }
+    const size_t b = (bytes + 4095) & ~(size_t)4095;
+    const hipError_t e = hipHostMalloc(&h->host, b, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        h->host = nullptr;
+        mpc_set_error("host allocation of %zu bytes failed: %s", b, hipGetErrorString(e));
+        return MPC_ERR_NOMEM;
+    }
+    h->host_bytes = b;
+    return 0;
+}
+
 // Arrival counters for kernels whose last workgroup finishes a split
 // reduction.  Every such launch leaves its counters at zero, so they are
 // cleared only when the buffer is (re)allocated, which happens outside any
@@ -192,6 +213,7 @@ extern "C" int mpc_handle_destroy(mpc_handle* h) {
                              &h->pcg, &h->scratch, &h->winv, &h->gp64, &h->gp32, &h->gpvec,
                              &h->tlist, &h->tick})
         ws_free(*w);
+    if (h->host) (void)hipHostFree(h->host);
     if (h->pcg_exec) (void)hipGraphExecDestroy(h->pcg_exec);
     if (h->ev_col) (void)hipEventDestroy(h->ev_col);
     if (h->ev_panel) (void)hipEventDestroy(h->ev_panel);
@@ -519,6 +541,11 @@ void mpc_syrk_masks(int update_prec, const int* ladder, int n_ladder, unsigned* 
 static int agg_panels_of(const mpc_factor_opts* o) {
     return (o->profile != 0 || tile_rows_for(o->nb) != o->nb) ? 1 : o->agg_panels;
 }
+
+// where a factor's results lie in the handle's staging memory: the leading
+// scalars of mpc_small, then the precision map
+constexpr size_t kHostMap = 256;
+static_assert(offsetof(mpc_small, tile_amax) <= kHostMap, "staging");
 
 // first_src (optional, aggregated schedule only): dA holds only the first
 // agg_panels block columns (the caller copied them); the rest of its lower
@@ -892,9 +919,11 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         h->winv_pending = true;
     }
     MPC_HIP(hipEventRecord(e1, st));
-    mpc_small hs;
-    MPC_HIP(hipMemcpyAsync(&hs, sm, offsetof(mpc_small, tile_amax), hipMemcpyDeviceToHost, st));
+    if ((rc = host_reserve(h, kHostMap + (size_t)nt * nt))) return rc;
+    MPC_HIP(hipMemcpyAsync(h->host, sm, offsetof(mpc_small, tile_amax), hipMemcpyDeviceToHost, st));
+    MPC_HIP(hipMemcpyAsync((uint8_t*)h->host + kHostMap, map, (size_t)nt * nt, hipMemcpyDeviceToHost, st));
     MPC_HIP(hipStreamSynchronize(st));
+    const mpc_small& hs = *(const mpc_small*)h->host;      // (up to tile_amax)
     float ms_total = 0;
     (void)hipEventElapsedTime(&ms_total, e0, e1);
     fi->ms_total += ms_total;
@@ -1023,12 +1052,7 @@ static int factor_impl(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     fi.eps_prime_used = eps;
     const double nd = (double)n;
     fi.flops_total = nd * nd * nd / 3.0 + nd * nd / 2.0 + nd / 6.0;
-    if (rc >= 0) {
-        std::vector<uint8_t> hm((size_t)nt * nt);
-        MPC_HIP(hipMemcpyAsync(hm.data(), map, hm.size(), hipMemcpyDeviceToHost, h->stream));
-        MPC_HIP(hipStreamSynchronize(h->stream));
-        flops_from_map(hm.data(), n, nb, &fi);
-    }
+    if (rc >= 0) flops_from_map((const uint8_t*)h->host + kHostMap, n, nb, &fi);
     if (info) *info = fi;
     // the dinv blocks now describe this factor, and so do the big-block
     // inverses when they were built along with it
@@ -1208,12 +1232,18 @@ static int pcg_impl(mpc_handle* h, const pcg_operator& op, int64_t lda, const fl
     std::vector<double> relres(nrhs, 0.0), alphas, betas;
     // the scalars rz, rz_new, pq, rr, bb are contiguous (nrhs each): one copy
     // (each copy is a separate transfer with its own latency)
-    std::vector<double> hsc(5 * (size_t)nrhs);
-    MPC_HIP(hipMemcpyAsync(hsc.data(), b.rz, sizeof(double) * 5 * nrhs, hipMemcpyDeviceToHost, st));
+    // staging: the scalars (hsc), relres (hrel), then the flags (hflags)
+    if ((rc = host_reserve(h, sizeof(double) * std::max<size_t>(6 * (size_t)nrhs, 2 * (size_t)hmax) +
+                                  sizeof(int) * 3 * (size_t)nrhs)))
+        return rc;
+    double* hsc = (double*)h->host;
+    double* hrel = hsc + 5 * (size_t)nrhs;
+    int* hflags = (int*)(hsc + std::max<size_t>(6 * (size_t)nrhs, 2 * (size_t)hmax));
+    MPC_HIP(hipMemcpyAsync(hsc, b.rz, sizeof(double) * 5 * nrhs, hipMemcpyDeviceToHost, st));
     MPC_HIP(hipStreamSynchronize(st));
-    std::copy(hsc.begin(), hsc.begin() + nrhs, hrz.begin());
-    std::copy(hsc.begin() + 3 * nrhs, hsc.begin() + 4 * nrhs, hrr.begin());
-    std::copy(hsc.begin() + 4 * nrhs, hsc.begin() + 5 * nrhs, hb.begin());
+    std::copy(hsc, hsc + nrhs, hrz.begin());
+    std::copy(hsc + 3 * nrhs, hsc + 4 * nrhs, hrr.begin());
+    std::copy(hsc + 4 * nrhs, hsc + 5 * nrhs, hb.begin());
     std::vector<double> nb2(nrhs);
     int nactive = 0;
     for (int j = 0; j < nrhs; ++j) {
@@ -1224,13 +1254,13 @@ static int pcg_impl(mpc_handle* h, const pcg_operator& op, int64_t lda, const fl
         if (res <= o->tol) act[j] = 0; else ++nactive;
     }
     // the flags active, cand, iters are contiguous on the device: one copy
-    // each way (hflags is the host staging area of all three)
-    std::vector<int> hflags(3 * (size_t)nrhs);
+    // each way (hflags is the host staging area of all three; the host writes it
+    // only after a synchronisation)
     auto flags_to_device = [&](int count) -> int {
-        std::copy(act.begin(), act.end(), hflags.begin());
-        std::copy(cand.begin(), cand.end(), hflags.begin() + nrhs);
-        std::copy(iters.begin(), iters.end(), hflags.begin() + 2 * nrhs);
-        MPC_HIP(hipMemcpyAsync(b.active, hflags.data(), sizeof(int) * count * nrhs,
+        std::copy(act.begin(), act.end(), hflags);
+        std::copy(cand.begin(), cand.end(), hflags + nrhs);
+        std::copy(iters.begin(), iters.end(), hflags + 2 * nrhs);
+        MPC_HIP(hipMemcpyAsync(b.active, hflags, sizeof(int) * count * nrhs,
                                hipMemcpyHostToDevice, st));
         return 0;
     };
@@ -1308,13 +1338,14 @@ static int pcg_impl(mpc_handle* h, const pcg_operator& op, int64_t lda, const fl
         for (int q = 0; q < nbody; ++q)
             if ((rc = run_body())) return rc;
         done += nbody;
-        MPC_HIP(hipMemcpyAsync(hflags.data(), b.active, sizeof(int) * 3 * nrhs,
+        MPC_HIP(hipMemcpyAsync(hflags, b.active, sizeof(int) * 3 * nrhs,
                                hipMemcpyDeviceToHost, st));
-        MPC_HIP(hipMemcpyAsync(relres.data(), d_relres, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
+        MPC_HIP(hipMemcpyAsync(hrel, d_relres, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
         MPC_HIP(hipStreamSynchronize(st));
-        std::copy(hflags.begin(), hflags.begin() + nrhs, act.begin());
-        std::copy(hflags.begin() + nrhs, hflags.begin() + 2 * nrhs, cand.begin());
-        std::copy(hflags.begin() + 2 * nrhs, hflags.begin() + 3 * nrhs, iters.begin());
+        std::copy(hflags, hflags + nrhs, act.begin());
+        std::copy(hflags + nrhs, hflags + 2 * nrhs, cand.begin());
+        std::copy(hflags + 2 * nrhs, hflags + 3 * nrhs, iters.begin());
+        std::copy(hrel, hrel + nrhs, relres.begin());
         bool any_cand = false;
         for (int j = 0; j < nrhs; ++j) any_cand |= cand[j] != 0;
         if (any_cand) {
@@ -1324,8 +1355,9 @@ static int pcg_impl(mpc_handle* h, const pcg_operator& op, int64_t lda, const fl
                 if ((rc = mpc_launch_copy2d(st, n, nrhs, dB, ldb, b.W, n))) return rc;
                 if ((rc = mpc_launch_axpby(st, n, nrhs, -1.0, b.Q, n, 1.0, b.W, n))) return rc;
                 if ((rc = mpc_launch_dot(st, n, nrhs, b.W, n, b.W, n, b.rr, b.part))) return rc;
-                MPC_HIP(hipMemcpyAsync(hrr.data(), b.rr, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
+                MPC_HIP(hipMemcpyAsync(hrel, b.rr, sizeof(double) * nrhs, hipMemcpyDeviceToHost, st));
                 MPC_HIP(hipStreamSynchronize(st));
+                std::copy(hrel, hrel + nrhs, hrr.begin());
             }
             for (int j = 0; j < nrhs; ++j) {
                 if (!cand[j]) continue;
@@ -1360,15 +1392,15 @@ static int pcg_impl(mpc_handle* h, const pcg_operator& op, int64_t lda, const fl
     if ((rc = mpc_launch_copy2d(st, n, nrhs, b.X, ldw, dX, ldx))) return rc;
     // the alpha and beta histories are contiguous (hmax each): one copy
     const int mh = iters[0] > 0 ? std::min(iters[0], hmax) : 0;
-    std::vector<double> hab((size_t)hmax + mh);
+    double* hab = hsc;
     if (mh > 0)
-        MPC_HIP(hipMemcpyAsync(hab.data(), d_ahist, sizeof(double) * (hmax + mh),
+        MPC_HIP(hipMemcpyAsync(hab, d_ahist, sizeof(double) * (hmax + mh),
                                hipMemcpyDeviceToHost, st));
     MPC_HIP(hipEventRecord(e1, st));
     MPC_HIP(hipStreamSynchronize(st));
     if (mh > 0) {
-        alphas.assign(hab.begin(), hab.begin() + mh);
-        betas.assign(hab.begin() + hmax, hab.begin() + hmax + mh);
+        alphas.assign(hab, hab + mh);
+        betas.assign(hab + hmax, hab + hmax + mh);
     }
     h->last_alpha = alphas;
     h->last_beta = betas;
@@ -1610,7 +1642,10 @@ extern "C" int mpc_block_pcg(mpc_handle* h, const float* dA, int64_t lda, const 
     if ((rc = ext_x0(h, dL, ldl, n, nb, s, dB, ldb, dX, ldx, o->x0_mode, b))) return rc;
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, st, e.flag, 1, 0);
     MPC_LAUNCH_CHECK();
-    int k = 0, restarts = 0, hflag = 0;
+    if ((rc = host_reserve(h, sizeof(int)))) return rc;
+    int& hflag = *(int*)h->host;
+    hflag = 0;
+    int k = 0, restarts = 0;
     bool restart = true, conv = false;
     // R = B - A X, Z = M^-1 R, P = Z, G = Z^T R
     auto start = [&]() -> int {

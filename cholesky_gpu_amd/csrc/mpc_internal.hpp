@@ -125,6 +125,11 @@ struct mpc_handle {
     mpc_workspace gp32;       // GP: FP32 copy of A (factor source)
     mpc_workspace gpvec;      // GP: right-hand sides, solutions, U, V, partials
     mpc_workspace tick;       // arrival counters of split reductions (zero between launches)
+    // page-locked host memory that results are copied to: a copy to pageable
+    // memory blocks the host by itself (15..20 us), so that two of them before a
+    // synchronisation cost two round trips
+    void*        host = nullptr;
+    size_t       host_bytes = 0;
     // provenance of the dinv blocks: the factor they belong to
     const float* dinv_owner = nullptr;
     int64_t      dinv_n = 0;
