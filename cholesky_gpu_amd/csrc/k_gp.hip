@@ -24,29 +24,6 @@ namespace {
 constexpr int GT = 64;        // tile edge
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-// sum over the 64 lanes, in every lane: rotations within 16 lanes, then the
-// four sixteens in order
-template <int CTRL>
-__device__ __forceinline__ double rotate16(double v) {
-    const uint64_t u = __double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-__device__ __forceinline__ double lane_value(double v, int l) {
-    const uint64_t u = __double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-__device__ __forceinline__ double sum64(double v) {
-    v += rotate16<0x128>(v);
-    v += rotate16<0x124>(v);
-    v += rotate16<0x122>(v);
-    v += rotate16<0x121>(v);
-    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-
 // One 64 x 64 tile of the lower triangle per workgroup, a 32 x 32 quarter per
 // wave.  m comes from the FP64 matrix cores (v_mfma_f64_16x16x4, operands
 // straight from L2: lane (q, k) of a product holds row q, solve column k, and
@@ -161,7 +138,7 @@ __global__ __launch_bounds__(256, 2) void gp_grad_tile_kernel(
             }
     const int nout = (n_ls == 1 ? 1 : d) + 2;
     auto out = [&](int c, double v) {
-        v = sum64(v);
+        v = mpc_sum64(v);
         if (lane == 0) red[wave][c] = v;
     };
     if (n_ls == 1) {

@@ -253,49 +253,78 @@ __global__ __launch_bounds__(256) void symv_reduce_kernel(int64_t n, int E, int 
 }
 
 // ---------------------------------------------------------------- dots and updates
+// Sum of a workgroup's NW waves, in thread 0
+template <int NW>
+__device__ __forceinline__ double wg_sum(double v) {
+    __shared__ double red[NW];
+    v = mpc_sum64(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += red[w];
+    }
+    return s;
+}
+
+// sum of a[r] b[r] over r = r0 + thread, + nthr, ..: E of them, clamped loads all
+// in flight (rows from n on weigh nothing)
+template <int E>
+__device__ __forceinline__ double dot_rows(int64_t r0, int nthr, int64_t n, const double* __restrict__ a,
+                                           const double* __restrict__ b) {
+    double x[E], y[E], s = 0.0;
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int64_t r = r0 + (int64_t)q * nthr + threadIdx.x, rc = r < n ? r : n - 1;
+        x[q] = a[rc];
+        y[q] = b[rc];
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q) s = r0 + (int64_t)q * nthr + threadIdx.x < n ? fma(x[q], y[q], s) : s;
+    return s;
+}
+
+// Dots of column j = blockIdx.x of a and b (blockIdx.y = 1: b2), a workgroup for
+// each.  Up to kDotOne rows the second launch for a split sum takes longer than
+// the split saves (n = 500 / 2048 / 8192 / 16384: 3.9 / 3.9 / 4.6 / 6.9 us, split
+// 5.2 / 6.0 / 8.1 / 10.0).
+constexpr int64_t kDotOne = 16384;
+__global__ __launch_bounds__(1024) void dot_kernel(int64_t n, const double* __restrict__ a, int64_t lda_,
+                                                  const double* __restrict__ b0, int64_t ldb0,
+                                                  const double* __restrict__ b2, int64_t ldb2,
+                                                  double* __restrict__ out0, double* __restrict__ out2) {
+    const int j = blockIdx.x;
+    const double* __restrict__ b = blockIdx.y ? b2 + j * ldb2 : b0 + j * ldb0;
+    double s = 0.0;
+    for (int64_t r0 = 0; r0 < n; r0 += 8 * 1024) s += dot_rows<8>(r0, 1024, n, a + j * lda_, b);
+    s = wg_sum<16>(s);
+    if (threadIdx.x == 0) (blockIdx.y ? out2 : out0)[j] = s;
+}
+
 // blockIdx.z selects the second operand: 0 -> b, 1 -> b2 (two dots with the
 // same first operand in one launch); partials of z at part + z nrhs nparts
 __global__ __launch_bounds__(RB) void dot_partial_kernel(int64_t n, const double* __restrict__ a,
                                                         int64_t lda_, const double* __restrict__ b0,
                                                         int64_t ldb0, const double* __restrict__ b2,
                                                         int64_t ldb2, double* __restrict__ part) {
-    __shared__ double red[RB];
     const int j = blockIdx.y;
-    const double* __restrict__ b = blockIdx.z ? b2 : b0;
-    const int64_t ldb = blockIdx.z ? ldb2 : ldb0;
-    const int64_t r0 = (int64_t)blockIdx.x * RB * 8;
-    double s = 0.0;
-    for (int q = 0; q < 8; ++q) {
-        int64_t r = r0 + q * RB + threadIdx.x;
-        if (r < n) s = fma(a[j * lda_ + r], b[j * ldb + r], s);
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = RB / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
+    const double* __restrict__ b = blockIdx.z ? b2 + j * ldb2 : b0 + j * ldb0;
+    const double s = wg_sum<RB / 64>(dot_rows<8>((int64_t)blockIdx.x * RB * 8, RB, n, a + j * lda_, b));
     if (threadIdx.x == 0)
-        part[((int64_t)blockIdx.z * gridDim.y + j) * gridDim.x + blockIdx.x] = red[0];
+        part[((int64_t)blockIdx.z * gridDim.y + j) * gridDim.x + blockIdx.x] = s;
 }
 
 // blockIdx.y selects the dot: 0 -> out, 1 -> out2
 __global__ __launch_bounds__(RB) void dot_final_kernel(int nparts, const double* __restrict__ part,
                                                       double* __restrict__ out0,
                                                       double* __restrict__ out2) {
-    __shared__ double red[RB];
     const int j = blockIdx.x;
-    double* __restrict__ out = blockIdx.y ? out2 : out0;
-    part += (int64_t)blockIdx.y * gridDim.x * nparts;
+    part += ((int64_t)blockIdx.y * gridDim.x + j) * nparts;
     double s = 0.0;
-    for (int q = threadIdx.x; q < nparts; q += RB) s += part[(int64_t)j * nparts + q];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = RB / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[j] = red[0];
+    for (int q = threadIdx.x; q < nparts; q += RB) s += part[q];
+    s = wg_sum<RB / 64>(s);
+    if (threadIdx.x == 0) (blockIdx.y ? out2 : out0)[j] = s;
 }
 
 __global__ __launch_bounds__(RB) void update_xr_kernel(int64_t n, double* __restrict__ X,
@@ -491,12 +520,6 @@ __global__ __launch_bounds__(256, 2) void gram_kernel(int64_t n, int s, int64_t 
 // and gives Xo = 0, so the updates that use Xo leave their blocks unchanged.
 // (One thread for the factor: 45 us at s = 16.)
 constexpr double kSpdRelPivot = 1e-13;
-__device__ __forceinline__ double lane_double(double v, int l) {
-    const uint64_t u = __double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
 __global__ __launch_bounds__(64) void spd_solve_kernel(int s, const double* __restrict__ Gm,
                                                       const double* __restrict__ H,
                                                       double* __restrict__ Xo,
@@ -514,7 +537,7 @@ __global__ __launch_bounds__(64) void spd_solve_kernel(int s, const double* __re
 #pragma unroll
     for (int j = 0; j < BS; ++j) {
         if (j < s && !bad) {                     // (uniform)
-            const double d = lane_double(c[j], j), g = Gm[j + j * s];
+            const double d = mpc_lane_value(c[j], j), g = Gm[j + j * s];
             if (!(d > kSpdRelPivot * g) || !(d < INFINITY)) {
                 bad = true;
             } else {
@@ -522,7 +545,7 @@ __global__ __launch_bounds__(64) void spd_solve_kernel(int s, const double* __re
                 c[j] = tid == j ? l : c[j] / l;  // lanes above j hold nothing of use
 #pragma unroll
                 for (int k = j + 1; k < BS; ++k)
-                    if (k < s) c[k] = fma(-c[j], lane_double(c[j], k), c[k]);
+                    if (k < s) c[k] = fma(-c[j], mpc_lane_value(c[j], k), c[k]);
             }
         }
         if (tid < BS) C[j][tid] = c[j];
@@ -663,29 +686,35 @@ int mpc_launch_symv64(hipStream_t st, const double* A, int64_t lda, int64_t n, i
     return launch_symv_t<double>(st, A, lda, n, nrhs, X, ldx, Y, ldy, part);
 }
 
-int mpc_launch_dot(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
-                   const double* b, int64_t ldb, double* out, double* part) {
+// ndot dots of a with b and (2) c, to out_b and out_c
+static int launch_dots(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
+                       const double* b, int64_t ldb, double* out_b, const double* c, int64_t ldc,
+                       double* out_c, unsigned ndot, double* part) {
+    if (n <= kDotOne) {
+        hipLaunchKernelGGL(dot_kernel, dim3((unsigned)nrhs, ndot), dim3(1024), 0, st, n, a, lda_, b, ldb, c,
+                           ldc, out_b, out_c);
+        MPC_LAUNCH_CHECK();
+        return 0;
+    }
     const unsigned nparts = (unsigned)((n + RB * 8 - 1) / (RB * 8));
-    hipLaunchKernelGGL(dot_partial_kernel, dim3(nparts, (unsigned)nrhs, 1), dim3(RB), 0, st, n, a,
-                       lda_, b, ldb, b, ldb, part);
+    hipLaunchKernelGGL(dot_partial_kernel, dim3(nparts, (unsigned)nrhs, ndot), dim3(RB), 0, st, n, a,
+                       lda_, b, ldb, c, ldc, part);
     MPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(dot_final_kernel, dim3((unsigned)nrhs, 1), dim3(RB), 0, st, (int)nparts, part,
-                       out, out);
+    hipLaunchKernelGGL(dot_final_kernel, dim3((unsigned)nrhs, ndot), dim3(RB), 0, st, (int)nparts, part,
+                       out_b, out_c);
     MPC_LAUNCH_CHECK();
     return 0;
+}
+
+int mpc_launch_dot(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
+                   const double* b, int64_t ldb, double* out, double* part) {
+    return launch_dots(st, n, nrhs, a, lda_, b, ldb, out, b, ldb, out, 1, part);
 }
 
 int mpc_launch_dot2(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
                     const double* b, int64_t ldb, double* out_b, const double* c, int64_t ldc,
                     double* out_c, double* part) {
-    const unsigned nparts = (unsigned)((n + RB * 8 - 1) / (RB * 8));
-    hipLaunchKernelGGL(dot_partial_kernel, dim3(nparts, (unsigned)nrhs, 2), dim3(RB), 0, st, n, a,
-                       lda_, b, ldb, c, ldc, part);
-    MPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(dot_final_kernel, dim3((unsigned)nrhs, 2), dim3(RB), 0, st, (int)nparts, part,
-                       out_b, out_c);
-    MPC_LAUNCH_CHECK();
-    return 0;
+    return launch_dots(st, n, nrhs, a, lda_, b, ldb, out_b, c, ldc, out_c, 2, part);
 }
 
 int mpc_launch_pcg_update_xr(hipStream_t st, int64_t n, int nrhs, double* X, int64_t ldx,

@@ -393,29 +393,6 @@ __global__ __launch_bounds__(256) void bwd_gemv_partial_kernel(
     }
 }
 
-// Sum over the 64 lanes, in every lane: rotations within 16 lanes, then the
-// four sixteens in order
-template <int CTRL>
-__device__ __forceinline__ double rotate16(double v) {
-    const uint64_t u = __double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-__device__ __forceinline__ double lane_value(double v, int l) {
-    const uint64_t u = __double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-__device__ __forceinline__ double sum64(double v) {
-    v += rotate16<0x128>(v);
-    v += rotate16<0x124>(v);
-    v += rotate16<0x122>(v);
-    v += rotate16<0x121>(v);
-    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-
 typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));     // 16-byte load, any column start
 typedef double d2 __attribute__((ext_vector_type(2)));
 
@@ -500,7 +477,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dot_kernel(const float* __restrict
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const double sum = sum64(acc[j]);
+        const double sum = mpc_sum64(acc[j]);
         if (lane == 0 && j < nj && c < bI) v[(int64_t)j * bI + c] = V[(int64_t)j * ldv + c] - sum;
     }
 }
@@ -581,7 +558,7 @@ __global__ __launch_bounds__(256, 2) void tri_dot_kernel(const float* __restrict
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const double sum = sum64(acc[j]);
+        const double sum = mpc_sum64(acc[j]);
         if (lane == 0 && j < nj && r < bI) out[(int64_t)j * ldo + r] = sum;
     }
 }

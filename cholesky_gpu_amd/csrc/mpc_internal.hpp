@@ -30,6 +30,29 @@ static __device__ __forceinline__ bool mpc_last_arrival(int* t, int total) {
     return last;
 }
 
+// Sum over a wave's 64 lanes, in every lane: rotations within 16 lanes (no LDS),
+// then the four sixteens in order
+template <int CTRL>
+static __device__ __forceinline__ double mpc_rotate16(double v) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+static __device__ __forceinline__ double mpc_lane_value(double v, int l) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+static __device__ __forceinline__ double mpc_sum64(double v) {
+    v += mpc_rotate16<0x128>(v);
+    v += mpc_rotate16<0x124>(v);
+    v += mpc_rotate16<0x122>(v);
+    v += mpc_rotate16<0x121>(v);
+    return (mpc_lane_value(v, 0) + mpc_lane_value(v, 16)) + (mpc_lane_value(v, 32) + mpc_lane_value(v, 48));
+}
+
 // ---------------------------------------------------------------- errors
 void mpc_set_error(const char* fmt, ...);
 

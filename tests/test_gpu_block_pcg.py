@@ -27,3 +27,19 @@ def test_three_eigenvalues(handle, n, s):
     want = B / lam.to(torch.float64)[None, :]
     err = (X - want).norm(dim=1) / want.norm(dim=1)
     assert float(err.max()) <= 4e-12, float(err.max())
+
+
+@pytest.mark.parametrize("n", [1, 1023, 8193, 16384, 16385])
+@pytest.mark.parametrize("s", [1, 3])
+def test_dots_where_they_split(handle, n, s):
+    """Independent PCGs on the same kind of matrix at the sizes where a dot
+    takes a second batch of rows and a second launch: same bounds as above."""
+    print("[case]", n, s, flush=True)
+    lam = torch.tensor([1.0, 2.0, 4.0]).repeat(n // 3 + 1)[:n].cuda()
+    B = torch.from_numpy(np.random.default_rng(n + s).standard_normal((s, n))).cuda()
+    X, pi, rc = S.pcg(handle, torch.diag(lam).contiguous(), torch.eye(n, device="cuda"), B, nb=64,
+                      opts=S.pcg_opts(tol=1e-12, maxit=50, x0_mode=1))
+    assert rc == 0 and 0 < pi.iters <= 4, (rc, pi.iters)
+    want = B / lam.to(torch.float64)[None, :]
+    err = (X - want).norm(dim=1) / want.norm(dim=1)
+    assert float(err.max()) <= 4e-12, float(err.max())
