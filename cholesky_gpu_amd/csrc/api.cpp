@@ -676,14 +676,29 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     const int64_t nI = (n + Bo - 1) / Bo;
     float* WT = W ? W + (size_t)nI * Bo * Bo : nullptr;
     // after the panel of step s (on stream ps): build the inverse of the big
-    // block that step s completes, on wstream
+    // block that step s completes, on wstream.  The last block's is waited for:
+    // what its first half and three quarters allow is built when they are
+    // factored (one event on the chain each; at 2048 rows the build ends 131 us
+    // after the last panel, at once 195)
+    int64_t tail_rows = 0;                       // rows of the last block built so far
     auto build_w = [&](int64_t s, hipStream_t ps) -> int {
-        if (!W || !((((s + 1) * nb) % Bo) == 0 || s == nt - 1)) return 0;
-        const int64_t I = (s * nb) / Bo;
+        if (!W) return 0;
+        const int64_t I = (s * nb) / Bo, rows = std::min<int64_t>((s + 1) * nb, n) - I * Bo;
+        const bool end = (((s + 1) * nb) % Bo) == 0 || s == nt - 1;
+        if (I < nI - 1 && !end) return 0;
+        if (I == nI - 1 && !end) {
+            int64_t half = 128;                  // half of the power of two that covers the block
+            while (2 * half < n - I * Bo) half *= 2;
+            if (half < 256 || rows % 128 || (rows != half && rows != half + half / 2)) return 0;
+        }
         MPC_HIP(hipEventRecord(h->ev_wready, ps));
         MPC_HIP(hipStreamWaitEvent(h->wstream, h->ev_wready, 0));
-        if (I == nI - 1) MPC_HIP(hipEventRecord(h->ev_wpre, h->wstream));
-        return mpc_build_block_inverses_range(h->wstream, dA, lda, n, Bo, dinv, W, WT, I, I + 1);
+        if (I < nI - 1)
+            return mpc_build_block_inverses_range(h->wstream, dA, lda, n, Bo, dinv, W, WT, I, I + 1);
+        if (tail_rows == 0) MPC_HIP(hipEventRecord(h->ev_wpre, h->wstream));
+        const int64_t from = tail_rows;
+        tail_rows = rows;
+        return mpc_build_block_inverse_stage(h->wstream, dA, lda, n, Bo, dinv, W, WT, I, from, rows);
     };
 
     // The last kOneStream columns go on one stream: panel, then its whole

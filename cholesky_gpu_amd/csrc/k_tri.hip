@@ -575,43 +575,100 @@ int launch_gemm(hipStream_t st, const gemm_batch& g, int nbatch, bool f64) {
 
 }  // namespace
 
-// Build Winv_I = L_II^{-1} for every big block (Bo x Bo, column-major, ld Bo,
-// block I at W + I*Bo*Bo) and WT_I = Winv_I^T from L and its 32x32 diagonal
-// inverses.  Full big blocks are batched per level; a ragged last big block is
-// handled by its own launches with clipped sizes.
-static int double_level(hipStream_t st, const float* L, int64_t ldl, int Bo, float* W, float* WT,
-                        int h, int64_t I0, int nblk, int q0, int nq, int hc, bool f64) {
+// Winv_I = L_II^{-1} for a big block (Bo x Bo, column-major, ld Bo, block I at
+// W + I*Bo*Bo) and WT_I = Winv_I^T come from L and its 32x32 diagonal inverses,
+// 128 x 128 blocks first, then by doubling: for the pairs q0 .. q0 + nq - 1 of
+// blocks of h rows (the second of them with hc <= h rows) of nblk big blocks
+//   T = B A^-1 (kept in the upper part at (p, p + h)), X21 = -C^-1 T at (p + h, p).
+static int double_first(hipStream_t st, const float* L, int64_t ldl, int Bo, float* W, int h, int64_t I0,
+                        int nblk, int q0, int nq, int hc, bool f64) {
     const int64_t base = I0 * Bo;
     const int64_t p = 2 * (int64_t)h * q0;
     float* Wi = W + I0 * (int64_t)Bo * Bo;
-    const int64_t bs = (int64_t)Bo * Bo;                 // stride between big blocks in W
-    gemm_batch g1;                                       // T = B * Ainv -> upper part (p, p+h)
-    g1.A = L + (base + p + h) + (base + p) * ldl;  g1.lda = ldl;
-    g1.B = Wi + p + p * (int64_t)Bo;              g1.ldb = Bo;
-    g1.C = Wi + p + (p + h) * (int64_t)Bo;        g1.ldc = Bo;
-    g1.CT = nullptr;
-    g1.sA = 2 * (int64_t)h * (1 + ldl);
-    g1.sB = g1.sC = 2 * (int64_t)h * (1 + Bo);
-    g1.tA = (int64_t)Bo * (1 + ldl);
-    g1.tB = g1.tC = bs;
-    g1.nq = nq;
-    g1.m = hc; g1.n = h; g1.k = h; g1.alpha = 1.f; g1.a_lower = 0; g1.b_lower = 1;
-    int rc = launch_gemm(st, g1, nq * nblk, f64);
+    gemm_batch g;
+    g.A = L + (base + p + h) + (base + p) * ldl;  g.lda = ldl;
+    g.B = Wi + p + p * (int64_t)Bo;              g.ldb = Bo;
+    g.C = Wi + p + (p + h) * (int64_t)Bo;        g.ldc = Bo;
+    g.CT = nullptr;
+    g.sA = 2 * (int64_t)h * (1 + ldl);
+    g.sB = g.sC = 2 * (int64_t)h * (1 + Bo);
+    g.tA = (int64_t)Bo * (1 + ldl);
+    g.tB = g.tC = (int64_t)Bo * Bo;
+    g.nq = nq;
+    g.m = hc; g.n = h; g.k = h; g.alpha = 1.f; g.a_lower = 0; g.b_lower = 1;
+    return launch_gemm(st, g, nq * nblk, f64);
+}
+static int double_second(hipStream_t st, int Bo, float* W, float* WT, int h, int64_t I0, int nblk, int q0,
+                         int nq, int hc, bool f64) {
+    const int64_t p = 2 * (int64_t)h * q0, bs = (int64_t)Bo * Bo;
+    float* Wi = W + I0 * bs;
+    gemm_batch g;
+    g.A = Wi + (p + h) + (p + h) * (int64_t)Bo;  g.lda = Bo;
+    g.B = Wi + p + (p + h) * (int64_t)Bo;        g.ldb = Bo;
+    g.C = Wi + (p + h) + p * (int64_t)Bo;        g.ldc = Bo;
+    g.CT = WT + I0 * bs + p + (p + h) * (int64_t)Bo;
+    g.sA = g.sB = g.sC = 2 * (int64_t)h * (1 + Bo);
+    g.tA = g.tB = g.tC = bs;
+    g.nq = nq;
+    g.m = hc; g.n = h; g.k = hc; g.alpha = -1.f; g.a_lower = 1; g.b_lower = 0;
+    return launch_gemm(st, g, nq * nblk, f64);
+}
+
+static int leaves(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo, const float* dinv,
+                  float* W, float* WT, int64_t b0, int64_t b1) {
+    if (b1 > b0)
+        hipLaunchKernelGGL(winv_leaf_kernel, dim3((unsigned)(b1 - b0)), dim3(256), 0, st, L, ldl, dinv, n,
+                           Bo, W, WT, b0);
+    MPC_LAUNCH_CHECK();
+    return 0;
+}
+
+int mpc_build_block_inverse_stage(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
+                                  const float* dinv, float* W, float* WT, int64_t I, int64_t from,
+                                  int64_t to) {
+    const int64_t rows = std::min<int64_t>(Bo, n - I * Bo);
+    if (Bo % LF || Bo < LF || from % LF || from < 0 || to > rows || (to < rows && to % LF)) {
+        mpc_set_error("block inverse: rows %lld to %lld of %lld, block %d", (long long)from, (long long)to,
+                      (long long)rows, Bo);
+        return MPC_ERR_ARG;
+    }
+    const bool f64 = n <= 8192;
+    int rc = leaves(st, L, ldl, n, Bo, dinv, W, WT, I * (Bo / LF) + from / LF, I * (Bo / LF) + cdiv(to, LF));
     if (rc) return rc;
-    gemm_batch g2;                                       // X21 = -Cinv * T -> (p+h, p)
-    g2.A = Wi + (p + h) + (p + h) * (int64_t)Bo;  g2.lda = Bo;
-    g2.B = Wi + p + (p + h) * (int64_t)Bo;        g2.ldb = Bo;
-    g2.C = Wi + (p + h) + p * (int64_t)Bo;        g2.ldc = Bo;
-    g2.CT = WT + I0 * bs + p + (p + h) * (int64_t)Bo;
-    g2.sA = g2.sB = g2.sC = 2 * (int64_t)h * (1 + Bo);
-    g2.tA = g2.tB = g2.tC = bs;
-    g2.nq = nq;
-    g2.m = hc; g2.n = h; g2.k = hc; g2.alpha = -1.f; g2.a_lower = 1; g2.b_lower = 0;
-    return launch_gemm(st, g2, nq * nblk, f64);
+    for (int h = LF; h < Bo; h *= 2) {
+        // pairs whose first (second) half ends in (from, to]: q with
+        // from < 2 h q + h <= to, and from < min(2 h q + 2 h, rows) <= to
+        int f0 = -1, f1 = 0, s0 = -1, s1 = 0;
+        for (int q = 0; 2 * (int64_t)h * q + h < rows; ++q) {
+            const int64_t a = 2 * (int64_t)h * q + h, c = std::min<int64_t>(a + h, rows);
+            if (a > from && a <= to) { if (f0 < 0) f0 = q; f1 = q + 1; }
+            if (c > from && c <= to) { if (s0 < 0) s0 = q; s1 = q + 1; }
+        }
+        // (the last pair of the block on its own where its second half is short)
+        auto each = [&](int q0, int q1, auto&& run) -> int {
+            if (q0 < 0) return 0;
+            const int64_t lastc = rows - (2 * (int64_t)h * (q1 - 1) + h);
+            const int full = lastc >= h ? q1 : q1 - 1;
+            int r = 0;
+            if (full > q0) r = run(q0, full - q0, h);
+            if (!r && full < q1) r = run(full, 1, (int)lastc);
+            return r;
+        };
+        if ((rc = each(f0, f1, [&](int q, int nq, int hc) {
+                 return double_first(st, L, ldl, Bo, W, h, I, 1, q, nq, hc, f64);
+             })))
+            return rc;
+        if ((rc = each(s0, s1, [&](int q, int nq, int hc) {
+                 return double_second(st, Bo, W, WT, h, I, 1, q, nq, hc, f64);
+             })))
+            return rc;
+    }
+    return 0;
 }
 
 // Big blocks [I0, I1) only (each depends on L_II and the 32x32 inverses of
 // its diagonal alone, so blocks can be built as soon as they are factored).
+// Full big blocks are batched per level.
 int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
                                    const float* dinv, float* W, float* WT, int64_t I0,
                                    int64_t I1) {
@@ -619,36 +676,20 @@ int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, 
         mpc_set_error("block inverse: Bo must be a multiple of %d", LF);
         return MPC_ERR_ARG;
     }
-    const int64_t nI = (n + Bo - 1) / Bo;
-    const int64_t nfull = n / Bo;                 // big blocks with Bo rows
-    if (I1 > nI) I1 = nI;
-    if (I0 >= I1) return 0;
-    const int64_t b0 = I0 * (Bo / LF), b1 = std::min<int64_t>(cdiv(n, LF), I1 * (Bo / LF));
-    hipLaunchKernelGGL(winv_leaf_kernel, dim3((unsigned)(b1 - b0)), dim3(256), 0, st, L, ldl, dinv, n,
-                       Bo, W, WT, b0);
-    MPC_LAUNCH_CHECK();
-    const int64_t f1 = std::min(I1, nfull);      // full blocks in the range: [I0, f1)
+    const int64_t nI = (n + Bo - 1) / Bo, f1 = std::min(I1, n / Bo);     // full blocks: [I0, f1)
     const bool f64 = n <= 8192;
     int rc;
-    for (int h = LF; h < Bo; h *= 2) {
-        const int pairs = Bo / (2 * h);
-        if (f1 > I0 && (rc = double_level(st, L, ldl, Bo, W, WT, h, I0, (int)(f1 - I0), 0, pairs, h, f64)))
-            return rc;
-        if (nI > nfull && nfull >= I0 && nfull < I1) {   // ragged last big block
-            const int64_t I = nfull, rows = n - I * Bo;
-            int npair = 0;
-            for (int q = 0; q < pairs; ++q)
-                if (2 * h * q + h < rows) npair = q + 1;
-            if (npair == 0) continue;
-            const int full = (2 * h * (npair - 1) + 2 * h <= rows) ? npair : npair - 1;
-            if (full > 0 && (rc = double_level(st, L, ldl, Bo, W, WT, h, I, 1, 0, full, h, f64)))
+    if (f1 > I0) {
+        if ((rc = leaves(st, L, ldl, n, Bo, dinv, W, WT, I0 * (Bo / LF), f1 * (Bo / LF)))) return rc;
+        for (int h = LF; h < Bo; h *= 2) {
+            const int pairs = Bo / (2 * h);
+            if ((rc = double_first(st, L, ldl, Bo, W, h, I0, (int)(f1 - I0), 0, pairs, h, f64)) ||
+                (rc = double_second(st, Bo, W, WT, h, I0, (int)(f1 - I0), 0, pairs, h, f64)))
                 return rc;
-            if (npair > full) {
-                const int hc = (int)(rows - 2 * (int64_t)h * full - h);
-                if ((rc = double_level(st, L, ldl, Bo, W, WT, h, I, 1, full, 1, hc, f64))) return rc;
-            }
         }
     }
+    if (nI > n / Bo && n / Bo >= I0 && n / Bo < I1)                      // ragged last big block
+        return mpc_build_block_inverse_stage(st, L, ldl, n, Bo, dinv, W, WT, n / Bo, 0, n % Bo);
     return 0;
 }
 

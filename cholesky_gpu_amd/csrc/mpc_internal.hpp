@@ -379,6 +379,12 @@ int mpc_launch_block_axpy(hipStream_t st, int64_t n, int s, const double* M, int
                           const double* Cm, double a, const double* Z, int64_t ldz, double* Y,
                           int64_t ldy);
 // k_tri.hip
+// what rows [from, to) of big block I add to its inverse once columns up to `to`
+// of the block are factored (from: where the last call ended; both multiples of
+// 128, or `to` the block's end)
+int mpc_build_block_inverse_stage(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
+                                  const float* dinv, float* W, float* WT, int64_t I, int64_t from,
+                                  int64_t to);
 int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
                                    const float* dinv, float* W, float* WT, int64_t I0, int64_t I1);
 int mpc_build_block_inverses(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,

@@ -65,3 +65,22 @@ def test_apply_precond_edges(handle, n, nrhs):
     past 1024 (the backward products' step), pieces of 256 that are not full,
     last row blocks of 1 to 63 rows.  Tolerance as above."""
     test_apply_precond_blocks(handle, n, nrhs)
+
+
+@pytest.mark.parametrize("n,nb", [(300, 64), (500, 64), (512, 128), (513, 256), (777, 128), (1100, 128),
+                                  (2047, 256), (2048, 128), (2500, 256), (3001, 256), (3600, 128)])
+def test_inverses_built_in_stages(handle, n, nb):
+    """The last big block's inverse built in stages during the factor (half,
+    three quarters, the end; whole and ragged blocks) is the one built at once
+    from a finished factor: the solutions agree bit for bit."""
+    say("staged inverses", n, nb)
+    A, _ = S.matgen_householder(handle, n, cond=1e3, lam_max=1e3, seed=n)
+    B = torch.from_numpy(np.random.default_rng(n).standard_normal((2, n))).cuda()
+    fo = S.factor_opts(nb=nb, update_prec=L.PREC_FP32, fallback=0)
+    po = S.pcg_opts(tol=1e-10, maxit=100)
+    X1, _, pi1, rc1 = S.precond_cg(handle, A, B, fo, po)
+    Lf = A.clone()
+    rc, _, _, _ = S.factor(handle, Lf, fo)
+    X2, pi2, rc2 = S.pcg(handle, A, Lf, B, nb=nb, opts=po)
+    assert rc == 0 and rc1 == 0 and rc2 == 0 and pi1.iters == pi2.iters
+    assert torch.equal(X1, X2)
