@@ -569,11 +569,17 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         mpc_set_error("factor: a deferred copy needs the aggregated schedule");
         return MPC_ERR_ARG;
     }
-    // groups whose far updates go together: two, unless every update is FP32
-    // (bound by the matrix cores, not by C's traffic; n = 16384: 22.1 ms a solve
-    // with one, 22.7 with two, where E4M3/FP32 switching takes 15.08 and 14.66 and
-    // the 60000-point MXFP8 solve 446 and 367) or the panel ring has no room
-    const int PG = AG == 2 && o->update_prec != MPC_PREC_FP32 ? 2 : 1;
+    // groups whose far updates go together (AG = 2 only: the panel ring has room
+    // for eight): two, which halves C's traffic (n = 16384 E4M3/FP32 switching 15.08
+    // ms a solve with one and 14.66 with two, 60000 points MXFP8 446 and 367).  FP32
+    // updates are bound by the matrix cores; there the chain gains, which waits for a
+    // far update's first strip only, once the update outlasts two groups' panels:
+    // FP32 factors with one and two at nb = 256: n = 5000 1.93 and 2.04 ms, 8192 4.08
+    // and 4.13, 12000 8.76 and 8.68, 16384 18.0 and 17.6, 32768 114.0 and 109.8; nb = 128:
+    // 8192 4.57 and 4.77, 12000 9.72 and 9.81, 16384 20.0 and 19.2.  Backward errors
+    // there 4.2e-7 and 3.9e-7 (nb = 256), 3.8e-7 and 3.1e-7 (128).
+    constexpr int64_t kPairFp32 = 12288;
+    const int PG = AG == 2 && (o->update_prec != MPC_PREC_FP32 || n >= kPairFp32) ? 2 : 1;
     const int nslot = 2 * PG * AG;
     if ((rc = mpc_ws_reserve(h->panel, (size_t)nslot * (n + 128) * nb * 4))) return rc;
     if ((rc = mpc_ws_reserve(h->scales, (size_t)nslot * (n + 128) * (nb / 32)))) return rc;
