@@ -570,16 +570,20 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         return MPC_ERR_ARG;
     }
     // groups whose far updates go together (AG = 2 only: the panel ring has room
-    // for eight): two, which halves C's traffic (n = 16384 E4M3/FP32 switching 15.08
-    // ms a solve with one and 14.66 with two, 60000 points MXFP8 446 and 367).  FP32
-    // updates are bound by the matrix cores; there the chain gains, which waits for a
-    // far update's first strip only, once the update outlasts two groups' panels:
-    // FP32 factors with one and two at nb = 256: n = 5000 1.93 and 2.04 ms, 8192 4.08
-    // and 4.13, 12000 8.76 and 8.68, 16384 18.0 and 17.6, 32768 114.0 and 109.8; nb = 128:
-    // 8192 4.57 and 4.77, 12000 9.72 and 9.81, 16384 20.0 and 19.2.  Backward errors
-    // there 4.2e-7 and 3.9e-7 (nb = 256), 3.8e-7 and 3.1e-7 (128).
-    constexpr int64_t kPairFp32 = 12288;
-    const int PG = AG == 2 && (o->update_prec != MPC_PREC_FP32 || n >= kPairFp32) ? 2 : 1;
+    // for eight): two, which halves C's traffic, once the update outlasts the
+    // chain of two groups; before that the later start of half of it costs more.
+    // Factors with one and two (ms): nb = 256 E4M3/FP32 switching n = 5000 1.81 and
+    // 1.92, 8192 3.17 and 3.28, 9001 4.30 and 4.17, 16384 9.08 and 8.46; BF16 6000 2.07
+    // and 2.12, 12000 5.37 and 5.17.  nb = 128 (more traffic for the same columns)
+    // 6000 2.54 and 2.54, 8192 3.82 and 3.88 (BF16 3.61 and 3.49), 12000 6.81 and 6.43.
+    // FP32 updates are bound by the matrix cores; there the chain gains, which
+    // waits for a far update's first strip only: nb = 256 8192 4.08 and 4.13, 12000
+    // 8.76 and 8.68, 16384 18.0 and 17.6, 32768 114.0 and 109.8; nb = 128 8192 4.57 and
+    // 4.77, 12000 9.72 and 9.81, 16384 20.0 and 19.2, with backward errors at 16384 of
+    // 4.2e-7 and 3.9e-7 (nb = 256), 3.8e-7 and 3.1e-7 (128).
+    constexpr int64_t kPair = 8448, kPairFp32 = 12288;
+    const bool pairs = o->update_prec == MPC_PREC_FP32 ? n >= kPairFp32 : nb < 256 || n >= kPair;
+    const int PG = AG == 2 && pairs ? 2 : 1;
     const int nslot = 2 * PG * AG;
     if ((rc = mpc_ws_reserve(h->panel, (size_t)nslot * (n + 128) * nb * 4))) return rc;
     if ((rc = mpc_ws_reserve(h->scales, (size_t)nslot * (n + 128) * (nb / 32)))) return rc;

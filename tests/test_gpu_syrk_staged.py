@@ -125,3 +125,27 @@ def test_factor_group_pairs_fp32(handle, n, nb):
     print("backward errors", err, flush=True)
     assert err[2] <= 1.1 * err[1]
     assert torch.equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("n,nb", [(8447, 256), (8448, 256), (8750, 256), (4225, 128), (5000, 128)])
+@pytest.mark.parametrize("prec", [L.PREC_BF16, L.PREC_MXE4M3])
+def test_factor_group_pairs_large(handle, n, nb, prec):
+    """The sizes from which two groups' panels go into one far update, before
+    the one-stream tail: the backward error of the factor is that of the
+    per-panel updates (agg_panels = 1) up to 10 %, and two runs agree bit for
+    bit."""
+    print("[case]", n, nb, L.PREC_NAMES[prec], flush=True)
+    A, _ = S.matgen_householder(handle, n, cond=20.0, lam_max=20.0, seed=n)
+    err, outs = {}, []
+    for agg in (1, 2, 2):
+        T = A.clone()
+        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=prec, ladder=(prec,),
+                                                        fallback=0, agg_panels=agg))
+        assert rc == 0
+        L64 = torch.triu(T).to(torch.float64).T.contiguous()
+        err[agg] = float((L64 @ L64.T.contiguous() - A.to(torch.float64)).norm()
+                         / A.to(torch.float64).norm())
+        outs.append(T)
+    print("backward errors", err, flush=True)
+    assert err[2] <= 1.1 * err[1]
+    assert torch.equal(outs[1], outs[2])
