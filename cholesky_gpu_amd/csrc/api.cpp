@@ -576,13 +576,19 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     // 1.92, 8192 3.17 and 3.28, 9001 4.30 and 4.17, 16384 9.08 and 8.46; BF16 6000 2.07
     // and 2.12, 12000 5.37 and 5.17.  nb = 128 (more traffic for the same columns)
     // 6000 2.54 and 2.54, 8192 3.82 and 3.88 (BF16 3.61 and 3.49), 12000 6.81 and 6.43.
-    // FP32 updates are bound by the matrix cores; there the chain gains, which
-    // waits for a far update's first strip only: nb = 256 8192 4.08 and 4.13, 12000
-    // 8.76 and 8.68, 16384 18.0 and 17.6, 32768 114.0 and 109.8; nb = 128 8192 4.57 and
-    // 4.77, 12000 9.72 and 9.81, 16384 20.0 and 19.2, with backward errors at 16384 of
-    // 4.2e-7 and 3.9e-7 (nb = 256), 3.8e-7 and 3.1e-7 (128).
-    constexpr int64_t kPair = 8448, kPairFp32 = 12288;
-    const bool pairs = o->update_prec == MPC_PREC_FP32 ? n >= kPairFp32 : nb < 256 || n >= kPair;
+    // Not where (nearly) every update is FP32: those are bound by the matrix cores
+    // (n = 16384 18.0 and 17.6 ms, 8192 4.08 and 4.13), and the longer FP32 sums
+    // cost precision: FP32 factor, cond 1e6, nb = 256, kappa - 1 of the preconditioned
+    // matrix 6e-3 with one, 1.0e-2 with two, 5e-2 with four; E4M3/FP32 at eps' = 0.001
+    // (a third of the work FP32) 1.9e-2, 2.2e-2 and 3.0e-2, at 0.005 4.9e-2 with each
+    // (the Schur-diagonal rule leaves most tiles FP32 whatever eps').
+    constexpr int64_t kPair = 8448;
+    constexpr double kMostlyFp32 = 1.0 / 256;    // eps' below which a switching factor counts
+    bool fp32_sums = o->update_prec == MPC_PREC_FP32;
+    for (int l = 0; l < o->n_ladder && o->update_prec == MPC_PREC_SWITCH; ++l)
+        fp32_sums |= o->ladder[l] == MPC_PREC_FP32 &&
+                     (eps < kMostlyFp32 || o->rule == MPC_RULE_SCHUR);
+    const bool pairs = !fp32_sums && (nb < 256 || n >= kPair);
     const int PG = AG == 2 && pairs ? 2 : 1;
     const int nslot = 2 * PG * AG;
     if ((rc = mpc_ws_reserve(h->panel, (size_t)nslot * (n + 128) * nb * 4))) return rc;

@@ -104,29 +104,6 @@ def test_factor_restored_after_breakdown(handle, n, nb):
     assert torch.equal(torch.tril(T1, -1), torch.tril(A, -1))      # (the tensor is the transpose)
 
 
-@pytest.mark.parametrize("n,nb", [(12287, 256), (12288, 256), (12588, 256), (12417, 128)])
-def test_factor_group_pairs_fp32(handle, n, nb):
-    """FP32 updates on both sides of the size from which two groups' panels
-    go into one far update: the backward error of the factor is that of the
-    per-panel updates (agg_panels = 1) up to 10 %, and two runs agree bit for
-    bit."""
-    print("[case]", n, nb, flush=True)
-    A, _ = S.matgen_householder(handle, n, cond=1e4, lam_max=1e4, seed=n)
-    err, outs = {}, []
-    for agg in (1, 2, 2):
-        T = A.clone()
-        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=L.PREC_FP32,
-                                                        ladder=(L.PREC_FP32,), agg_panels=agg))
-        assert rc == 0
-        L64 = torch.triu(T).to(torch.float64).T.contiguous()
-        err[agg] = float((L64 @ L64.T.contiguous() - A.to(torch.float64)).norm()
-                         / A.to(torch.float64).norm())
-        outs.append(T)
-    print("backward errors", err, flush=True)
-    assert err[2] <= 1.1 * err[1]
-    assert torch.equal(outs[1], outs[2])
-
-
 @pytest.mark.parametrize("n,nb", [(8447, 256), (8448, 256), (8750, 256), (4225, 128), (5000, 128)])
 @pytest.mark.parametrize("prec", [L.PREC_BF16, L.PREC_MXE4M3])
 def test_factor_group_pairs_large(handle, n, nb, prec):
