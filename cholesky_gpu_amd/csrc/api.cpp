@@ -569,30 +569,40 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         mpc_set_error("factor: a deferred copy needs the aggregated schedule");
         return MPC_ERR_ARG;
     }
-    // groups whose far updates go together (AG = 2 only: the panel ring has room
-    // for eight): two, which halves C's traffic, once the update outlasts the
-    // chain of two groups; before that the later start of half of it costs more.
-    // Factors with one and two (ms): nb = 256 E4M3/FP32 switching n = 5000 1.81 and
-    // 1.92, 8192 3.17 and 3.28, 9001 4.30 and 4.17, 16384 9.08 and 8.46; BF16 6000 2.07
-    // and 2.12, 12000 5.37 and 5.17.  nb = 128 (more traffic for the same columns)
-    // 6000 2.54 and 2.54, 8192 3.82 and 3.88 (BF16 3.61 and 3.49), 12000 6.81 and 6.43.
+    // groups whose far updates go together (AG = 2 only: an update takes at most
+    // eight panels): two or four, which halves or quarters C's traffic, once the
+    // update outlasts the chain of as many groups; before that the later start of
+    // a part of it costs more.  Factors with one and two (ms): nb = 256 E4M3/FP32
+    // switching n = 5000 1.81 and 1.92, 8192 3.17 and 3.28, 9001 4.30 and 4.17, 16384
+    // 9.08 and 8.46; BF16 6000 2.07 and 2.12, 12000 5.37 and 5.17.  nb = 128 (more
+    // traffic for the same columns) 6000 2.54 and 2.54, 8192 3.82 and 3.88 (BF16
+    // 3.61 and 3.49), 12000 6.81 and 6.43.  With two and four: 12000 nb = 256 5.39 and
+    // 5.47, 128 6.36 and 6.37; 16384 nb = 256 8.43 and 8.45 (MXFP8 6.32 and 6.00, BF16 8.93
+    // and 8.66), 128 9.87 and 9.70; 24576 17.0 and 16.4; 32768 30.6 and 28.9; 60000
+    // 124.5 and 110.6 (MXFP8 105.2 and 88.0).  A ring that does not fit in memory
+    // takes fewer groups.
     // Not where (nearly) every update is FP32: those are bound by the matrix cores
     // (n = 16384 18.0 and 17.6 ms, 8192 4.08 and 4.13), and the longer FP32 sums
     // cost precision: FP32 factor, cond 1e6, nb = 256, kappa - 1 of the preconditioned
     // matrix 6e-3 with one, 1.0e-2 with two, 5e-2 with four; E4M3/FP32 at eps' = 0.001
     // (a third of the work FP32) 1.9e-2, 2.2e-2 and 3.0e-2, at 0.005 4.9e-2 with each
     // (the Schur-diagonal rule leaves most tiles FP32 whatever eps').
-    constexpr int64_t kPair = 8448;
+    constexpr int64_t kPair = 8448, kQuad = 15360;
     constexpr double kMostlyFp32 = 1.0 / 256;    // eps' below which a switching factor counts
     bool fp32_sums = o->update_prec == MPC_PREC_FP32;
     for (int l = 0; l < o->n_ladder && o->update_prec == MPC_PREC_SWITCH; ++l)
         fp32_sums |= o->ladder[l] == MPC_PREC_FP32 &&
                      (eps < kMostlyFp32 || o->rule == MPC_RULE_SCHUR);
-    const bool pairs = !fp32_sums && (nb < 256 || n >= kPair);
-    const int PG = AG == 2 && pairs ? 2 : 1;
+    int PG = 1;
+    if (AG == 2 && !fp32_sums) PG = n >= kQuad ? 4 : nb < 256 || n >= kPair ? 2 : 1;
+    auto ring = [&](int groups) -> int {
+        const size_t slots = (size_t)2 * groups * AG;
+        const int r = mpc_ws_reserve(h->panel, slots * (n + 128) * nb * 4);
+        return r ? r : mpc_ws_reserve(h->scales, slots * (n + 128) * (nb / 32));
+    };
+    while ((rc = ring(PG)) != 0 && PG > 1) PG /= 2;
+    if (rc) return rc;
     const int nslot = 2 * PG * AG;
-    if ((rc = mpc_ws_reserve(h->panel, (size_t)nslot * (n + 128) * nb * 4))) return rc;
-    if ((rc = mpc_ws_reserve(h->scales, (size_t)nslot * (n + 128) * (nb / 32)))) return rc;
     if ((rc = mpc_ws_reserve(h->dinv, (size_t)(nt * nb / 32 + 8) * 1024 * sizeof(float)))) return rc;
     // row sums of squares, then the original diagonal (switching rule SCHUR)
     if ((rc = mpc_ws_reserve(h->rowstat, 2 * (size_t)(n + 128) * sizeof(float)))) return rc;
@@ -769,12 +779,12 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // the group (K = AG nb): block column E (the next group's first) on
         // pstream, the rest of the next group on st, everything beyond that
         // on fstream, where it overlaps the next groups' panels.
-        // With PG = 2 the columns beyond the next two groups take two groups'
-        // panels at once (K = 2 AG nb), which halves the traffic of C that
-        // bounds those updates: after an even group fstream updates only the
-        // strip of the group after next; after an odd one the next group but
-        // one first (the chain waits for it at the end of the next group),
-        // then the rest, each with both groups.
+        // With PG > 1 the columns beyond the next two groups take PG groups'
+        // panels at once (K = PG AG nb), which divides the traffic of C that
+        // bounds those updates: after each group fstream updates the strip of
+        // the group after next (the chain waits for it at the end of the next
+        // group) with the panels of all groups not yet applied to it, and after
+        // every PG-th group the rest with the same panels.
         // The next panel is enqueued before the updates on st and fstream: the
         // chain does not wait for the host to issue those, and POTRF's one
         // workgroup gets a CU before their thousands.
@@ -830,16 +840,15 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, gt, st, 2))) return rc;
                 MPC_HIP(hipEventRecord(h->ev_bulk, st));
                 bulk_seen = false;
+                const int64_t q = g % PG, pp = p0 - q * AG;    // the groups not applied yet
+                const int pn = (int)q * AG + np;
                 if (PG == 1) {
                     if ((rc = agg(p0, np, E, gt, -1, fs, 2))) return rc;
                     MPC_HIP(hipEventRecord(h->ev_far, fs));
-                } else if (g % 2 == 0) {
-                    if ((rc = agg(p0, np, E, gt, 2 * gt, fs, 2))) return rc;
-                    MPC_HIP(hipEventRecord(h->ev_far, fs));
                 } else {
-                    if ((rc = agg(p0 - AG, 2 * AG, E, gt, 2 * gt, fs, 2))) return rc;
+                    if ((rc = agg(pp, pn, E, gt, 2 * gt, fs, 2))) return rc;
                     MPC_HIP(hipEventRecord(h->ev_far, fs));
-                    if ((rc = agg(p0 - AG, 2 * AG, E, 2 * gt, -1, fs, 2))) return rc;
+                    if (q == PG - 1 && (rc = agg(pp, pn, E, 2 * gt, -1, fs, 2))) return rc;
                 }
                 far_pending = true;
             }

@@ -188,7 +188,7 @@ int mpc_noalloc_init_device(int device);
 struct mpc_small {
     int      info;            // 1-based failing column, 0 = ok
     int      nan_flag;        // NaN/Inf seen in a panel
-    uint32_t mu_bits;         // min pivot^2 so far (bits of a positive float; atomicMin)
+    uint32_t mu_bits;         // min pivot^2 so far (bits of a positive float; POTRF alone writes it)
     // mu_bits as the POTRF of a step left it, by step parity: the tile
     // decisions of that step's panel read this copy, which stays fixed while
     // the next step's POTRF lowers mu_bits
@@ -206,10 +206,10 @@ struct mpc_small {
     uint32_t tile_maxrs[2][1024];  // max row sum of squares
     // decided precision per panel tile, one slot per panel buffer (a panel
     // stays live until the aggregated update of its group has read it)
-    uint8_t  tile_prec[2 * 4][1024];
+    uint8_t  tile_prec[16][1024];
 };
-constexpr int MPC_AGG_MAX = 4;                    // panels per aggregated update
-constexpr int MPC_PANEL_SLOTS = 2 * MPC_AGG_MAX;  // panel buffers in the ring
+constexpr int MPC_AGG_MAX = 4;                    // panels per group (agg_panels)
+constexpr int MPC_PANEL_SLOTS = 16;               // panel buffers in the ring: twice an update's
 static_assert(sizeof(((mpc_small*)nullptr)->tile_prec) / 1024 == MPC_PANEL_SLOTS, "slots");
 
 // ---------------------------------------------------------------- kernels (launchers)
@@ -259,6 +259,7 @@ constexpr int MPC_SYRK_TILE = 128;   // output tile edge of the SYRK kernels
 // rows0 - q * nb (each panel starts nb rows below the previous one).
 // Scalars only: a kernel argument of pointer arrays costs scalar registers.
 constexpr int MPC_SYRK_MAXP = 8;
+static_assert(MPC_PANEL_SLOTS >= 2 * MPC_SYRK_MAXP && MPC_SYRK_MAXP >= MPC_AGG_MAX, "panel ring");
 struct mpc_syrk_panels {
     const uint8_t* payload;
     const uint8_t* scales;
@@ -389,7 +390,7 @@ int mpc_build_block_inverses_range(hipStream_t st, const float* L, int64_t ldl, 
                                    const float* dinv, float* W, float* WT, int64_t I0, int64_t I1);
 int mpc_build_block_inverses(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
                              const float* dinv, float* W, float* WT);
-// part: mpc_block_prec_partial_doubles(Bo, nrhs) doubles of scratch
+// part: mpc_block_prec_partial_doubles(n, Bo, nrhs) doubles of scratch
 // z = L^-T L^-1 r (R in, Y work, Z out; ld each)
 int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n, int Bo,
                          const float* Winv, const float* WinvT, const double* R, double* Y,
@@ -397,7 +398,7 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
                          hipEvent_t late_ev = nullptr, int64_t I_late = -1);
 int64_t mpc_block_prec_partial_doubles(int64_t n, int Bo, int nrhs);
 // Big-block edge of the sweeps: the whole matrix up to 2048 rows (rounded up to
-// a power of two), else 2048.  A stage costs six dependent launches per
+// a power of two), else 2048.  A stage costs five dependent launches per
 // application; a larger block costs its inverse, which for the last one is not
 // hidden by the factor.  Solves (us, Bo = 1024 / 2048 / 4096): n = 2048 2244 /
 // 2149 / -, 4096 3335 / 3172 / 3555, 8192 6397 / 6111 / 6802, 12000 11041 / 10060

@@ -126,3 +126,44 @@ def test_factor_group_pairs_large(handle, n, nb, prec):
     print("backward errors", err, flush=True)
     assert err[2] <= 1.1 * err[1]
     assert torch.equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("n,nb", [(15359, 256), (15360, 256), (16001, 256), (15487, 128)])
+@pytest.mark.parametrize("prec", [L.PREC_BF16, L.PREC_SWITCH])
+def test_factor_group_quads(handle, n, nb, prec):
+    """The size from which four groups' panels go into one far update: the
+    backward error of the factor, on random vectors, is that of the per-panel
+    updates (agg_panels = 1) up to 10 %, two runs agree bit for bit, and the
+    solve that factors a partly copied matrix equals factor and solve."""
+    print("[case]", n, nb, prec, flush=True)
+    A, _ = S.matgen_householder(handle, n, cond=20.0, lam_max=20.0, seed=n)
+    V = torch.randn(n, 8, dtype=torch.float64, generator=torch.Generator().manual_seed(n)).cuda()
+    ladder = (L.PREC_E4M3, L.PREC_FP32) if prec == L.PREC_SWITCH else (prec,)
+
+    def product(M):                  # M V by row blocks, in FP64
+        return torch.cat([M[r:r + 2048].to(torch.float64) @ V for r in range(0, n, 2048)])
+
+    ref = product(A)
+    err, outs = {}, []
+    for agg in (1, 2, 2):
+        T = A.clone()
+        fo = S.factor_opts(nb=nb, update_prec=prec, ladder=ladder, eps_prime=0.125, fallback=0,
+                           agg_panels=agg)
+        rc, _, _, _ = S.factor(handle, T, fo)
+        assert rc == 0
+        Lt = torch.triu(T)
+        w = product(Lt)
+        y = sum(Lt[r:r + 2048].to(torch.float64).T.contiguous() @ w[r:r + 2048]
+                for r in range(0, n, 2048))
+        err[agg] = float((y - ref).norm() / ref.norm())
+        outs.append(T)
+    print("backward errors", err, flush=True)
+    assert err[2] <= 1.1 * err[1]
+    assert torch.equal(outs[1], outs[2])
+    B = V[:, :1].T.contiguous()
+    po = S.pcg_opts(tol=1e-10)
+    # (first the solve with the handle's last factor, whose 32x32 inverses it
+    # still has; for another factor it computes them again, in other bits)
+    X2 = S.pcg(handle, A, outs[2], B, nb=nb, opts=po)[0]
+    X1 = S.precond_cg(handle, A, B, fo, po)[0]
+    assert torch.equal(X1, X2)
