@@ -3,7 +3,7 @@
 //
 //  trsm_stats: L21 = A21 * L_jj^{-T} (the RIGHT/LOWER/TRANS form of
 //    fp8_chol.cuh:73-85; switching_chol.cuh:98-110 calls a LEFT form that is
-//    out of bounds).  One wave owns a 32-row slab and substitutes over the
+//    out of bounds).  A workgroup owns a 32-row slab and substitutes over the
 //    32-column blocks of the panel with the inverses of L_jj's 32x32 diagonal
 //    sub-blocks (MFMA 32x32x2 f32).  The epilogue computes each row's sum of
 //    squares, subtracts it from the Schur-diagonal tracker (update_diag,
@@ -33,9 +33,9 @@ __device__ __forceinline__ int sigma(int s, int h) { return 8 * (s >> 2) + 4 * h
 // MFMAs of 64 cycles a step) bounds the launch: nothing else may sit on it.  The
 // inverse is read at the start, the L operands of step b + 1 during step b,
 // statistics and stores follow the barrier, and the chain's wave has priority
-// over the wave that shares its SIMD.  A wave per block (two blocks each on four
-// waves, operands read where they are used: nb = 256 30 us for 2000 to 10000
-// rows, nb = 128 11.3).
+// over the wave that shares its SIMD.  Four waves (two blocks each at nb = 256,
+// operands read where they are used) took, alone, 22.2 us for 2000 rows and 29.6
+// for 10000 at nb = 256, and 11.3 at nb = 128; this takes 16.1, 24.0 and 8.4.
 // MFMA roles (32x32x2 f32, k index sig(t, h) on both operands): A = L or
 // Dinv rows (lane m = lane % 32), B = X or acc columns (lane n = row of the
 // slab); accumulator register i of lane (n, h) holds column sig(i, h), row n,

@@ -6,8 +6,9 @@
 // for all right-hand sides; vectors are FP64.
 //
 // A row-by-row substitution over n = 16384 rows is a dependency chain; the
-// sweep is instead blocked with big diagonal blocks of Bo rows (Bo = 1024 or
-// 2048) whose inverses Winv_I = L_II^{-1} are formed once per factor:
+// sweep is instead blocked with big diagonal blocks of Bo rows (mpc_block_bo:
+// the power of two from n up, at most 2048) whose inverses Winv_I = L_II^{-1}
+// are formed once per factor:
 //   forward   for I:   y_I = Winv_I w_I ;  w_{>I} -= L_{>I,I} y_I
 //   backward  for I:   x_I = Winv_I^T w_I; w_{<I} -= L_{I,<I}^T x_I
 // so a sweep is 2 * n / Bo bandwidth-bound kernels with no serial work
