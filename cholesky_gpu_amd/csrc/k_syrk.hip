@@ -1105,9 +1105,10 @@ __device__ __forceinline__ void syrk_f8_tile(float* __restrict__ C, int64_t m, i
 }
 
 // ---------------------------------------------------------------- 16-bit classes
-// The pairs of the BF16 class (BF16 or FP8 tiles, at least one BF16; CLS BF16)
-// and of two FP16 tiles (CLS FP16), in the K order of mm_16 (bit for bit the
-// same sums), staged like the bf16 planes above with one plane a side.
+// The pairs of the BF16 class (at least one BF16 tile, the other BF16, FP8 or, in
+// mpc_syrk only, FP16, whose values lose their last three bits; CLS BF16) and of
+// two FP16 tiles (CLS FP16), in the K order of mm_16 (bit for bit the same sums),
+// staged like the bf16 planes above with one plane a side.
 constexpr int S16B = 8 * 1024;                // bytes of a buffer
 
 template <int CLS>
@@ -1174,7 +1175,7 @@ __device__ __forceinline__ void syrk_16_tile(float* __restrict__ C, int64_t m, i
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
             sf[side] = pf[side];
-            if (CLS == MPC_PREC_FP16 || pf[side] == MPC_PREC_BF16) {
+            if (CLS == MPC_PREC_FP16 || pf[side] == MPC_PREC_BF16 || pf[side] == MPC_PREC_FP16) {
 #pragma unroll
                 for (int u = 2 * side; u < 2 * side + 2; ++u) {
                     const u32x2 v = *reinterpret_cast<const u32x2*>(pay + row[u] * row_stride + 2 * kk);
@@ -1204,7 +1205,13 @@ __device__ __forceinline__ void syrk_16_tile(float* __restrict__ C, int64_t m, i
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             u32x2 w = {st[u][0], st[u][1]};
-            if (CLS != MPC_PREC_FP16 && sf[u >> 1] != MPC_PREC_BF16) {
+            if (CLS != MPC_PREC_FP16 && sf[u >> 1] == MPC_PREC_FP16) {
+                float f[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    f[e] = (float)__builtin_bit_cast(_Float16, (unsigned short)(st[u][e >> 1] >> (16 * (e & 1))));
+                w = u32x2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
+            } else if (CLS != MPC_PREC_FP16 && sf[u >> 1] != MPC_PREC_BF16) {
                 const float s = mpc_dev_exp2i((int)st[u][1] - 127);
                 v2f a, b;
                 if (mpc_dev_is_e4m3(sf[u >> 1])) {

@@ -167,3 +167,28 @@ def test_factor_group_quads(handle, n, nb, prec):
     X2 = S.pcg(handle, A, outs[2], B, nb=nb, opts=po)[0]
     X1 = S.precond_cg(handle, A, B, fo, po)[0]
     assert torch.equal(X1, X2)
+
+
+@pytest.mark.parametrize("m,k", [(129, 64), (257, 192), (640, 256)])
+def test_staged_bf16_with_fp16(handle, oracle, m, k):
+    """BF16 and FP16 tiles alternating: a pair of one of each is computed in
+    BF16, the FP16 values cut to their leading 8 bits, a pair of two FP16 tiles
+    from the values themselves: every element within k u32 of the FP64 result on
+    these operands, relative to |C| + |Q| |Q|^T."""
+    print("[case]", m, k, flush=True)
+    rng = np.random.default_rng(m + k)
+    P = rng.standard_normal((m, k)).astype(np.float32)
+    Cm = rng.standard_normal((m, m)).astype(np.float32)
+    precs = [L.PREC_FP16 if t % 2 else L.PREC_BF16 for t in range((m + 127) // 128)]
+    pay, sc, pt = S.quantize_panel(handle, torch.from_numpy(P.T.copy()).cuda(), precs, 128)
+    Q = np.ascontiguousarray(oracle.quantize_panel(P, precs, 128)[2], dtype=np.float32)
+    cut = (Q.view(np.uint32) & np.uint32(0xffff0000)).view(np.float32).astype(np.float64)
+    Q = Q.astype(np.float64)
+    Cd = torch.from_numpy(Cm.T.copy()).cuda()
+    S.syrk(handle, Cd, pay, sc, k, 128, pt)
+    got = Cd.cpu().numpy().T
+    half = np.repeat([p == L.PREC_FP16 for p in precs], 128)[:m]
+    ref = Cm - np.where(half[:, None] & half[None, :], Q @ Q.T, cut @ cut.T)
+    err = np.abs(got - ref) / (np.abs(Cm) + np.abs(Q) @ np.abs(Q).T)
+    assert err[np.tril(np.ones((m, m), bool))].max() <= k * 2.0 ** -24
+    assert np.array_equal(np.triu(got, 1), np.triu(Cm, 1))
