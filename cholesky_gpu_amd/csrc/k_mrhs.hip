@@ -9,13 +9,18 @@
 //     one column, 16 bytes, so 16 lanes read a 256-byte column segment, and
 //     its element i is the operand of the product whose n stands for row
 //     4n + i: no transpose and no LDS.
+//     Symmetric A (mode 3) is read from its upper triangle only, as the kernels
+//     for fewer right-hand sides do: left of the diagonal the product's columns
+//     are rows there, so a lane takes rows 4k .. 4k+3 of columns 4q .. 4q+3
+//     (FP32: through LDS) and names the 16 values the other way round.
 //   mm_t (columns are the outputs): lane (q, k) loads rows 4k .. 4k+3 of
 //     column q; element i is the operand with k <-> row 4k + i.
 // The right-hand sides are read as operands straight from L2.  Per 8 KB of an
 // FP32 matrix a wave issues 32 products of 64 cycles, 9.8 TB/s over 1024 SIMDs:
-// above what HBM delivers.  With 16 right-hand sides (A X, FP32 A) n = 8192
-// takes 55 us (4.9 TB/s), where two passes of 8 over half the symmetric matrix
-// with FP64 FMAs from LDS took 244.
+// above what HBM delivers.  With 16 right-hand sides (A X, symmetric FP32 A)
+// n = 8192 takes 62 us, each element read twice (4.3 TB/s; 57 where both
+// triangles are read directly), where two passes of 8 that read the elements
+// once, with FP64 FMAs from LDS, took 244.
 #include "mpc_internal.hpp"
 #include <algorithm>
 
@@ -48,14 +53,14 @@ __device__ __forceinline__ void split_range(int mode, int64_t r0, int64_t rows, 
 //
 // A last row block that is not full (m >= 64) moves up to end at row m and
 // stores only its own rows: with predicated 4-byte loads its workgroups ran
-// several times as long as the others (16 right-hand sides: n = 12000 185 us,
-// now 112; n = 8684 108, now 72).
+// several times as long as the others (16 right-hand sides, mode 0: n = 12000
+// 185 us, moved up 112; n = 8684 108 and 72).
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int64_t lda, int64_t m,
                                                   int64_t kc, int64_t cw, const double* __restrict__ X,
                                                   int64_t ldx, int nj, double* __restrict__ part) {
     typedef T vec4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-    __shared__ double red[4][MPC_MM_NJ][MR];
+    __shared__ __align__(16) double red[4][MPC_MM_NJ][MR];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane & 15, k = lane >> 4;
     const int64_t rb = (int64_t)blockIdx.x * MR, cs = (int64_t)blockIdx.y * cw;
@@ -73,8 +78,21 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
     auto load = [&](int64_t c0) {
         const int64_t c = c0 + MU * k;            // this lane's columns
         if (rfull && c0 + MG <= kc) {
+            if (MODE == 3 && c0 < r0 + MR - 1) {      // not above the diagonal as a whole
+                vec4 t[4];
 #pragma unroll
-            for (int s = 0; s < MU; ++s) v[s] = *reinterpret_cast<const vec4*>(A + r + (c + s) * lda);
+                for (int i = 0; i < 4; ++i) t[i] = *reinterpret_cast<const vec4*>(A + c + (r + i) * lda);
+                const bool mirror = c0 + MG <= r0 + 1;    // below it
+#pragma unroll
+                for (int s = 0; s < MU; ++s) {
+                    if (!mirror) v[s] = *reinterpret_cast<const vec4*>(A + r + (c + s) * lda);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[s][i] = mirror || c + s < r + i ? t[i][s] : v[s][i];
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < MU; ++s) v[s] = *reinterpret_cast<const vec4*>(A + r + (c + s) * lda);
+            }
 #pragma unroll
             for (int s = 0; s < MU; s += 2) {
                 const d2 y = *reinterpret_cast<const d2*>(Xj + c + s);
@@ -87,7 +105,9 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
                 const int64_t cc = c + s < kc ? c + s : kc - 1;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const T y = A[(r + i < m ? r + i : m - 1) + cc * lda];
+                    const int64_t rc = r + i < m ? r + i : m - 1;
+                    const bool up = MODE != 3 || rc <= cc;
+                    const T y = A[(up ? rc : cc) + (up ? cc : rc) * lda];
                     v[s][i] = (r + i < m && c + s < kc) ? y : T(0);
                 }
                 const double y = Xj[cc];
@@ -114,8 +134,61 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = tot[i] = v4d{};
     int64_t c0 = cb + MG * wave;
+    int g = 1;
+    if constexpr (MODE == 3 && sizeof(T) == 4) {
+        // Left of the diagonal a wave's 16 columns of the product are 64-byte
+        // pieces of 64 columns of A.  Loaded as such they cost a third more than
+        // 256-byte ones (n = 16384, both triangles read directly 200 us, this way
+        // 266; FP64, 128 bytes: no difference).  So the workgroup loads 64 x 64
+        // elements at a time in 256-byte pieces, wave w columns 16 w + .., and the
+        // waves read theirs from LDS (224 us): column x's 4-row piece y lies at
+        // 16-byte slot y ^ (x / 4), which is free of conflicts both ways.
+        typedef T lds4 __attribute__((ext_vector_type(4)));
+        lds4* const buf = reinterpret_cast<lds4*>(&red[0][0][0]);
+        const int64_t steps = rfull && r0 + 1 > cb ? ((ce < r0 + 1 ? ce : r0 + 1) - cb) / (4 * MG) : 0;
+        const T* src = A + cb + 4 * q + (r0 + 16 * wave + k) * lda;
+        lds4 st[4], w[4];
+        double y[MU];
+        auto fetch = [&](int64_t t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                st[i] = *reinterpret_cast<const vec4*>(src + 4 * MG * t + (int64_t)(4 * i) * lda);
+#pragma unroll
+            for (int s = 0; s < MU; s += 2) {
+                const d2 z = *reinterpret_cast<const d2*>(Xj + c0 + 4 * MG * t + MU * k + s);
+                x[s] = z[0];
+                x[s + 1] = z[1];
+            }
+        };
+        if (steps > 0) fetch(0);
+        for (int64_t t = 0; t < steps; ++t) {
+            lds4* const b = buf + 1024 * (t & 1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[16 * (16 * wave + 4 * i + k) + (q ^ (4 * wave + i))] = st[i];
+#pragma unroll
+            for (int s = 0; s < MU; ++s) y[s] = x[s];
+            mpc_lds_barrier();                   // (the other buffer is read to the end)
+            if (t + 1 < steps) fetch(t + 1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = b[16 * (4 * q + i) + ((4 * wave + k) ^ q)];
+#pragma unroll
+            for (int s = 0; s < MU; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[s], (double)w[i][s], acc[i], 0, 0, 0);
+            if (g++ % MFL == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    tot[i] += acc[i];
+                    acc[i] = v4d{};
+                }
+            }
+        }
+        c0 += 4 * MG * steps;
+        __syncthreads();                         // red is written below
+    }
     if (c0 < ce) load(c0);
-    for (int g = 1; c0 < ce; c0 += 4 * MG, ++g) {
+    for (; c0 < ce; c0 += 4 * MG, ++g) {
         vec4 w[MU];
         double y[MU];
 #pragma unroll
@@ -284,6 +357,7 @@ int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc, 
     const dim3 g((unsigned)cdiv(m, MR), (unsigned)cdiv(kc, cw)), b(256);
     if (mode == 1) hipLaunchKernelGGL((mm_n_kernel<T, 1>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     else if (mode == 2) hipLaunchKernelGGL((mm_n_kernel<T, 2>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
+    else if (mode == 3) hipLaunchKernelGGL((mm_n_kernel<T, 3>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     else hipLaunchKernelGGL((mm_n_kernel<T, 0>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     MPC_LAUNCH_CHECK();
     return 0;

@@ -32,10 +32,10 @@ constexpr int RB = 256;          // rows per workgroup
 // symv_reduce adds P[K][0..nst) in order (deterministic).  The partials take
 // nst^2 E NJ doubles, NJ <= 4 right-hand sides per pass (at n = 16384, S = 4,
 // one right-hand side: 1/64 of the bytes read from A).  More than four
-// right-hand sides go through the matrix cores in passes of 16 over the whole
-// matrix (k_mrhs.hip): twice the bytes, but the FMAs here read x from LDS per
+// right-hand sides go through the matrix cores in passes of 16 that read every
+// element of the triangle twice (k_mrhs.hip): the FMAs here read x from LDS per
 // element and right-hand side and so cost more than the bytes (n = 8192: 48 us
-// for 4, where 16 take 62 there; n = 6000: 34 and 53).
+// for 4, where 16 take 62 there; n = 6000: 34 and 42).
 constexpr int SY_T = 64;
 constexpr int SY_JMAX = 4;
 // 16-byte loads of columns that are aligned to their elements only (an odd
@@ -617,7 +617,7 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + RB - 1) / RB); }
 }  // namespace
 
 // right-hand sides of the next pass: at most SY_JMAX (padded to 1, 2 or 4) with
-// the symmetric kernel, at most MPC_MM_NJ as a product with the whole matrix
+// the kernel above, at most MPC_MM_NJ on the matrix cores
 static int symv_pass_rhs(int nrhs) {
     return nrhs > SY_JMAX ? std::min(nrhs, MPC_MM_NJ) : nrhs <= 1 ? 1 : nrhs <= 2 ? 2 : SY_JMAX;
 }
@@ -626,10 +626,9 @@ static int symv_pass_rhs(int nrhs) {
 // 25), large ones the fewer partial sums (n = 6000: 25.6 / 25.1 / 27.7, 12000:
 // 72 / 55 / 62, 16384: 145 / 132 / 121, 36864: 671 / 580 / 540).
 static int symv_tiles(int64_t n) { return n >= 14336 ? 4 : n >= 4608 ? 2 : 1; }
-// Workgroups of the product with the whole matrix: 768 run at once (16 columns:
-// n = 3000 15.0 / 17.4 / 18.0 / 20.2 us with 512 / 1024 / 1536 / 2048, 8192 53 /
-// 56 / 57 / 61, 8684 79 / 73 / 72 / 74, 12000 138 / 116 / 112 / 120, 16384 192 /
-// 191 / 196 / 201)
+// Workgroups of the product on the matrix cores (16 columns: n = 3000 16.5 /
+// 19.7 / 21.4 / 23.5 us with 512 / 1024 / 1536 / 2048, 8192 61 / 62 / 67 / 66, 8684
+// 85 / 78 / 78 / 80, 12000 164 / 134 / 128 / 136, 16384 222 / 223 / 230 / 225)
 static int64_t symv_splits(int64_t n) { return mpc_mm_splits(n, n, n <= 4096 ? 512 : 1024); }
 
 int64_t mpc_symv_partial_doubles(int64_t n, int nrhs) {
@@ -660,7 +659,7 @@ static int launch_symv_t(hipStream_t st, const T* A, int64_t lda, int64_t n, int
         const int NJ = symv_pass_rhs(nrhs - j0), nj = std::min(nrhs - j0, NJ);
         if (NJ > SY_JMAX) {
             const int64_t S = symv_splits(n);
-            int rc = mpc_launch_mm_n(st, A, lda, n, n, 0, X + j0 * ldx, ldx, nj, part, S);
+            int rc = mpc_launch_mm_n(st, A, lda, n, n, 3, X + j0 * ldx, ldx, nj, part, S);
             if (!rc) rc = mpc_launch_mm_sum(st, n, nj, n, S, 0, MPC_MM_GROUP_N, part, nullptr, 0, 1.0, Y + j0 * ldy, ldy);
             if (rc) return rc;
         } else {

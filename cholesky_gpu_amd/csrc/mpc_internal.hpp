@@ -303,7 +303,8 @@ constexpr int MPC_MM_GROUP_N = 16, MPC_MM_GROUP_T = 64;      // chunk granularit
 int64_t mpc_mm_splits(int64_t rows, int64_t kc, int64_t wgs);   // chunks of mm_n
 int64_t mpc_mm_splits_t(int64_t cols, int64_t kc);              // chunks of mm_t
 // part[(s nj + j) m + r] = sum over chunk s of A[r][c] X[j][c]; mode 1: c <= r,
-// 2: c >= r (square A; the rest is not read as data)
+// 2: c >= r (square A; the rest is not read as data), 3: A symmetric, its upper
+// triangle read
 int mpc_launch_mm_n(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t kc, int mode,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S);
 int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int64_t kc, int mode,

@@ -84,3 +84,24 @@ def test_inverses_built_in_stages(handle, n, nb):
     X2, pi2, rc2 = S.pcg(handle, A, Lf, B, nb=nb, opts=po)
     assert rc == 0 and rc1 == 0 and rc2 == 0 and pi1.iters == pi2.iters
     assert torch.equal(X1, X2)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 130, 777, 4609])
+@pytest.mark.parametrize("nrhs", [4, 5, 16, 21])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_product_reads_upper_triangle(handle, n, nrhs, dtype):
+    """The operator's product takes A from its upper triangle (column-major) for
+    any number of right-hand sides: with NaN below the diagonal the residual is,
+    bit for bit, that of the full matrix."""
+    say("upper triangle", n, nrhs, dtype)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.randn(n, n, generator=g, device="cuda", dtype=torch.float32).to(dtype)
+    A = torch.tril(A) + torch.tril(A, -1).T.contiguous()
+    half = torch.tril(A) + torch.triu(torch.full_like(A, float("nan")), 1)   # tensor = transpose
+    X = torch.randn(nrhs, n, generator=g, device="cuda", dtype=torch.float64)
+    B = torch.randn(nrhs, n, generator=g, device="cuda", dtype=torch.float64)
+    eye = torch.eye(n, device="cuda", dtype=torch.float32)
+    f = S.pcg if dtype is torch.float32 else S.pcg64
+    res = [f(handle, M.contiguous(), eye, B, nb=64, X=X.clone(),
+             opts=S.pcg_opts(x0_mode=2, maxit=0))[1].relres for M in (A, half)]
+    assert res[0] == res[1], res
