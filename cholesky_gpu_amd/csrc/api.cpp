@@ -727,32 +727,37 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         return mpc_build_block_inverse_stage(h->wstream, dA, lda, n, Bo, dinv, W, WT, I, from, rows);
     };
 
-    // The last kOneStream columns go on one stream: panel, then its whole
-    // trailing update, with no event in between.  There the update is no
-    // longer than the waits that overlapping it would take (5..10 us for each
-    // event on the chain, and as much of host time).  Measured as whole
-    // factors, overlapped and on one stream: n = 4096, nb = 128 FP32 2181 and
-    // 1670 us, E4M3/FP32 1750 and 1393, nb = 256 FP32 1784 and 1590; n = 768,
-    // nb = 64 570 and 405.  Beyond it the update is the longer part: the last
-    // 8192 columns of n = 16384 that way cost an FP32 solve 21.3 -> 21.7 ms,
-    // E4M3/FP32 14.01 -> 14.28.
+    // The last kOneStream columns go on one stream: panel, then its trailing
+    // update (in groups as below: C is rounded as often as in the overlapped
+    // schedule), with no event in between.  There the update is no longer than the
+    // waits that overlapping it would take (5..10 us for each event on the chain,
+    // and as much of host time).  Measured as whole factors, overlapped and on one
+    // stream: n = 4096, nb = 128 FP32 2014 and 1436 us, E4M3/FP32 2068 and 1388, nb =
+    // 256 FP32 1565 and 1376, BF16 1306 and 1226; n = 768, nb = 64 538 and 320.
+    // Beyond it the update is the longer part: the last 8192 columns of n = 16384
+    // that way cost an FP32 factor 17.91 -> 18.11 ms, E4M3/FP32 8.57 -> 8.75.
     constexpr int64_t kOneStream = 4096;
-    // Updates of at least kWide columns whose operands are all of one class take
-    // that class's 128-row kernel (too few workgroups for the chip below: n = 4000
-    // FP32 factor 1774 us without it, 1754, 1717, 1696, 1694 and 1713 from 1024,
-    // 1536, 2048, 2560 and 3072; n = 4096 BF16 1337, 1277, 1270, 1263 and 1284
-    // without it and from 1536, 2048, 2560 and 3072).  With several classes it
-    // would be a launch each (E4M3/FP32 1168, and 1221 to 1186).
+    // Group updates of at least kWide columns whose operands are all of one class
+    // take that class's 128-row kernel (too few workgroups for the chip below: n =
+    // 4000, nb = 128 FP32 factor 1479 us without it, 1469, 1444, 1427, 1426, 1435 and
+    // 1460 from 1024, 1536, 2048, 2304, 2560 and 3072; n = 4096 BF16 1292 without it,
+    // 1247, 1240, 1236, 1238 and 1254 from 1536, 2048, 2304, 2560 and 3072).  With
+    // several classes it would be a launch each.
     constexpr int64_t kWide = 2304;
     const bool one_launch = __builtin_popcount(cmask) == 1 &&
                             (cmask != (1u << MPC_PREC_E4M3) || __builtin_popcount(fmask) == 1);
     auto one_stream = [&](int64_t j0, hipStream_t ps) -> int {
         for (int64_t j = j0; j + 1 < nt; ++j) {
+            const int64_t g = j / AG, E = std::min<int64_t>((g + 1) * AG, nt);
             const int wide = one_launch && n - (j + 1) * nb >= kWide;
             int r;
-            if ((r = AG > 1 ? agg(j, 1, j + 1, 0, -1, ps, wide ? 2 : 1)
-                            : update(j, 0, -1, ps, !wide)))
-                return r;
+            if (AG == 1)
+                r = update(j, 0, -1, ps, !wide);
+            else if (j + 1 < E)          // the columns of the group
+                r = update(j, 0, E < nt ? (E - (j + 1)) * nb / 64 : -1, ps, 1);
+            else                         // the rest, all panels of the group at once
+                r = agg(g * AG, AG, E, 0, -1, ps, wide ? 2 : 1);
+            if (r) return r;
             if ((r = panel(j + 1, ps))) return r;
             if ((r = build_w(j + 1, ps))) return r;
         }

@@ -192,3 +192,32 @@ def test_staged_bf16_with_fp16(handle, oracle, m, k):
     err = np.abs(got - ref) / (np.abs(Cm) + np.abs(Q) @ np.abs(Q).T)
     assert err[np.tril(np.ones((m, m), bool))].max() <= k * 2.0 ** -24
     assert np.array_equal(np.triu(got, 1), np.triu(Cm, 1))
+
+
+@pytest.mark.parametrize("n,nb", [(640, 128), (1111, 128), (1500, 256), (4096, 256), (4864, 128), (6000, 256)])
+@pytest.mark.parametrize("agg", [1, 2, 3, 4])
+def test_factor_group_sums(handle, n, nb, agg):
+    """The products of a group's panels are added before C takes them, in whole
+    factors of any size and in the last columns of larger ones.  I in front, then
+    rows of constant b: a panel adds nb b^2, less than half the spacing of the
+    floats below 1, to every entry of C.  Entries of C that are 1 stay 1 when
+    panels are subtracted one by one and become fl(1 - agg nb b^2), one or two
+    spacings less, in groups; divided by a pivot of 4 they come out halved.  All
+    of it is exact in FP32."""
+    print("[case]", n, nb, agg, flush=True)
+    b = 0.875 * 2.0 ** -16 if nb == 128 else 1.25 * 2.0 ** -17
+    last = max(k for k in range(1, 200) if k * agg * nb + nb // 2 < n)    # the last group with rows below
+    for group in {1, last}:
+        e, p = group * agg * nb, (group - 1) * agg * nb
+        T = torch.eye(n, device="cuda")
+        T[p:e, e:] = b                           # the tensor is the transpose
+        T[torch.arange(e, n), torch.arange(e, n)] = 4.0
+        rows = sorted({e + 1, (e + n) // 2, n - 1} - {e})
+        T[e, rows] = 1.0
+        T = torch.triu(T) + torch.triu(T, 1).T.contiguous()
+        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=L.PREC_FP32, fallback=0,
+                                                        agg_panels=agg))
+        assert rc == 0
+        want = 0.5 * float(np.float32(1.0 - agg * nb * b * b))
+        got = T[e, rows].cpu().numpy()
+        assert (got == want).all(), (group, rows, got - 0.5, want - 0.5)
