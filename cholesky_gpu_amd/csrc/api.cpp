@@ -560,6 +560,9 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     hipStream_t st = h->stream;
     int rc;
     if ((rc = wait_winv(h, st))) return rc;       // it reads dinv and the factor
+    const int ladder[4] = {o->ladder[0], o->ladder[1], o->ladder[2], o->ladder[3]};
+    unsigned cmask = 0, fmask = 0;
+    mpc_syrk_masks(o->update_prec, ladder, o->n_ladder, &cmask, &fmask);
     // panels live in a ring: 2 buffers, or 2 * PG * agg_panels when the updates
     // beyond a group of agg_panels block columns are aggregated (the PG groups
     // being aggregated and the groups being factored meanwhile)
@@ -573,28 +576,27 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     // eight panels): two or four, which halves or quarters C's traffic, once the
     // update outlasts the chain of as many groups; before that the later start of
     // a part of it costs more.  Factors with one and two (ms): nb = 256 E4M3/FP32
-    // switching n = 5000 1.81 and 1.92, 8192 3.17 and 3.28, 9001 4.30 and 4.17, 16384
-    // 9.08 and 8.46; BF16 6000 2.07 and 2.12, 12000 5.37 and 5.17.  nb = 128 (more
-    // traffic for the same columns) 6000 2.54 and 2.54, 8192 3.82 and 3.88 (BF16
-    // 3.61 and 3.49), 12000 6.81 and 6.43.  With two and four: 12000 nb = 256 5.39 and
-    // 5.47, 128 6.36 and 6.37; 16384 nb = 256 8.43 and 8.45 (MXFP8 6.32 and 6.00, BF16 8.93
-    // and 8.66), 128 9.87 and 9.70; 24576 17.0 and 16.4; 32768 30.6 and 28.9; 60000
-    // 124.5 and 110.6 (MXFP8 105.2 and 88.0).  A ring that does not fit in memory
-    // takes fewer groups.
-    // Not where (nearly) every update is FP32: those are bound by the matrix cores
-    // (n = 16384 18.0 and 17.6 ms, 8192 4.08 and 4.13), and the longer FP32 sums
-    // cost precision: FP32 factor, cond 1e6, nb = 256, kappa - 1 of the preconditioned
-    // matrix 6e-3 with one, 1.0e-2 with two, 5e-2 with four; E4M3/FP32 at eps' = 0.001
-    // (a third of the work FP32) 1.9e-2, 2.2e-2 and 3.0e-2, at 0.005 4.9e-2 with each
-    // (the Schur-diagonal rule leaves most tiles FP32 whatever eps').
+    // switching n = 5000 1.84 and 1.96, 8192 3.22 and 3.34, 12000 5.48 and 5.40, 16384
+    // 9.10 and 8.49; BF16 6000 2.07 and 2.12, 12000 5.37 and 5.17.  nb = 128 (more
+    // traffic for the same columns) 6000 2.53 and 2.53, 8192 3.84 and 3.90 (BF16
+    // 3.61 and 3.49), 12000 6.81 and 6.48.  With two and four: 12000 nb = 256 5.40 and
+    // 5.53, 128 6.48 and 6.52; 16384 nb = 256 8.49 and 8.62 (MXFP8 6.30 and 6.00, BF16 9.14
+    // and 8.96), 128 10.04 and 9.89; 24576 17.2 and 16.7; 32768 31.0 and 29.1.  A ring
+    // that does not fit in memory takes fewer groups.
+    // The products of two FP32 tiles are added per group all the same (P.sum
+    // below), so no factor's FP32 sums get longer: with K = 2048 kappa - 1 of the
+    // preconditioned matrix (FP32 factor, cond 1e6, n = 16384) was 5e-2 instead of
+    // 6.5e-3.  For these tiles, then, C's traffic stays, and where (nearly) every
+    // update is FP32 the grouping only delays a part of them: FP32 factor n = 16384
+    // 18.1, 18.5 and 19.1 ms with one, two and four; E4M3/FP32 at eps' = 1e-5 17.5, 18.3
+    // and 19.0 (the Schur-diagonal rule leaves most tiles FP32 whatever eps').
     constexpr int64_t kPair = 8448, kQuad = 15360;
     constexpr double kMostlyFp32 = 1.0 / 256;    // eps' below which a switching factor counts
-    bool fp32_sums = o->update_prec == MPC_PREC_FP32;
-    for (int l = 0; l < o->n_ladder && o->update_prec == MPC_PREC_SWITCH; ++l)
-        fp32_sums |= o->ladder[l] == MPC_PREC_FP32 &&
-                     (eps < kMostlyFp32 || o->rule == MPC_RULE_SCHUR);
+    const bool mostly_fp32 = cmask == (1u << MPC_PREC_FP32) ||
+                             (o->update_prec == MPC_PREC_SWITCH && (cmask >> MPC_PREC_FP32 & 1u) &&
+                              (eps < kMostlyFp32 || o->rule == MPC_RULE_SCHUR));
     int PG = 1;
-    if (AG == 2 && !fp32_sums) PG = n >= kQuad ? 4 : nb < 256 || n >= kPair ? 2 : 1;
+    if (AG == 2 && !mostly_fp32) PG = n >= kQuad ? 4 : nb < 256 || n >= kPair ? 2 : 1;
     auto ring = [&](int groups) -> int {
         const size_t slots = (size_t)2 * groups * AG;
         const int r = mpc_ws_reserve(h->panel, slots * (n + 128) * nb * 4);
@@ -620,9 +622,6 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     float* rowss = (float*)h->rowstat.ptr;
     float* diag0 = rowss + (n + 128);
     const int rule = o->rule;
-    const int ladder[4] = {o->ladder[0], o->ladder[1], o->ladder[2], o->ladder[3]};
-    unsigned cmask = 0, fmask = 0;
-    mpc_syrk_masks(o->update_prec, ladder, o->n_ladder, &cmask, &fmask);
 
     hipLaunchKernelGGL(init_small_kernel, dim3(1), dim3(256), 0, st, sm);
     int64_t ninit = std::max<int64_t>(n, nt * nt);
@@ -692,6 +691,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         P.p0 = (int)(p0 % nslot);
         P.np = np;
         P.nb = nb;
+        P.sum = AG;
         // (panel 0 is in the first update of every column beyond its group)
         P.csrc = (first_src && p0 == 0) ? first_src + e + e * lda : nullptr;
         return mpc_launch_syrk_panels(us, dA + e + e * lda, n - e, lda, nb, P, (int64_t)nb * 4, tr,

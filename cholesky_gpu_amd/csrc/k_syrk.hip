@@ -199,9 +199,9 @@ struct c_frag {
 // addressing every load would keep its own 64-bit VGPR address alive until
 // the matching store.
 template <int QA>
-__device__ __forceinline__ void load_c(const tile_ctx& t, c_frag<QA>& c) {
+__device__ __forceinline__ void load_c(const tile_ctx& t, c_frag<QA>& c, int lane = threadIdx.x & 63) {
     constexpr int QE = 32 * QA;
-    const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
+    const int h = lane >> 5, n = lane & 31;
     const __amdgpu_buffer_rsrc_t rsl = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(t.Cs) + t.rowbase + t.colbase * t.ldc, 0, 0x7fffffff, 0x00020000);
     const int ld4 = (int)t.ldc * 4;
@@ -239,8 +239,8 @@ __device__ __forceinline__ void load_c(const tile_ctx& t, c_frag<QA>& c) {
 
 template <int QA>
 __device__ __forceinline__ void store_c(const tile_ctx& t, const c_frag<QA>& c,
-                                        const v16f acc[QA][QA]) {
-    const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
+                                        const v16f acc[QA][QA], int lane = threadIdx.x & 63) {
+    const int h = lane >> 5, n = lane & 31;
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(t.C + t.rowbase + t.colbase * t.ldc, 0, 0x7fffffff,
                                           0x00020000);
@@ -644,10 +644,16 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
 // K = 256: 832 us = 80 TFLOP/s of the 157 peak).  In LDS a block of 32 rows is in operand
 // order, two groups of 16-byte elements (k 8h .. +3 and 8h + 4 .. +7 of lane
 // half h), so a wave's operand is one 1 KB read.
+// C takes the products of P.sum panels at a time, at most: the rounding errors of
+// an FP32 sum grow with its length and are all the error there is here, while in
+// the other kernels the operands' rounding is larger by orders of magnitude.
+// (GROUPED: more than one sum; the loop costs 20 registers, n = 32768 FP32 factor
+// 113.0 -> 114.8 ms.)
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int FSK = 16;                       // K of a chunk
 constexpr int FSB = 8 * 2 * 1024;             // bytes of a buffer: 8 blocks of 2 groups
 
+template <bool GROUPED>
 __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                               const mpc_syrk_panels& P, int64_t row_stride,
                                               int tile_rows, const syrk_shape& G, int64_t pid,
@@ -660,16 +666,16 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
     if (L.mode == 1) note_pair(L, P, tile_rows, trow, tcol, pid, rank);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
 
-    unsigned use = 0;                        // the panels of this launch
+    unsigned todo = 0;                       // the panels of this launch
     int lo = 99;                             // first launch with work on the tile
     for (int q = 0; q < P.np; ++q) {
         const int slot = (P.p0 + q) % P.slots;
         const uint8_t* prec = P.prec + slot * 1024 + (P.rows0 - (int64_t)q * P.nb) / tile_rows;
         const int r = launch_rank(prec[trow], prec[tcol]);
         lo = r < lo ? r : lo;
-        if (r == rank) use |= 1u << q;
+        if (r == rank) todo |= 1u << q;
     }
-    if (!use) return;
+    if (!todo) return;
 
     tile_ctx t;
     t.C = C;
@@ -699,7 +705,8 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
             src[u] = reinterpret_cast<const float*>(pay + row * row_stride);
         }
     };
-    int q = __builtin_ctz(use), kc = 0;
+    unsigned use = 0;                        // of the sum in the making
+    int q = 0, kc = 0;
     bool more = true;
     auto load = [&]() {                      // the next chunk into st
 #pragma unroll
@@ -719,52 +726,67 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
 #pragma unroll
         for (int u = 0; u < 4; ++u) *reinterpret_cast<v4f*>(sd + buf * FSB + u * 4096) = st[u];
     };
-    v16f acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
     const char* const opa = lds + (2 * wc) * 2048 + lane * 16;
     const char* const opb = lds + (4 + 2 * wr) * 2048 + lane * 16;
-    panel(q);
-    load();
-    store(0);
-    bool staged = true;                      // a chunk is in the current buffer
-    bool held = more;                        // a chunk is in st
-    if (more) load();
-    for (int buf = 0; staged; buf ^= 1) {
-        mpc_lds_barrier();
-        if (live) {
-            v4f A[2][2], B[2][2];
+    unsigned group = (1u << (GROUPED ? P.sum : MPC_SYRK_MAXP)) - 1;
+    do {
+        use = todo & group;
+        group <<= P.sum;
+        if (GROUPED && !use) continue;
+        todo &= ~use;
+        v16f acc[2][2];
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    A[b][g] = *reinterpret_cast<const v4f*>(opa + buf * FSB + b * 2048 + g * 1024);
-                    B[b][g] = *reinterpret_cast<const v4f*>(opb + buf * FSB + b * 2048 + g * 1024);
-                }
+            for (int b = 0; b < 2; ++b) acc[a][b] = v16f{};
+        q = __builtin_ctz(use);
+        kc = 0;
+        more = true;
+        panel(q);
+        load();
+        store(0);
+        bool staged = true;                  // a chunk is in the current buffer
+        bool held = more;                    // a chunk is in st
+        if (more) load();
+        for (int buf = 0; staged; buf ^= 1) {
+            mpc_lds_barrier();
+            if (live) {
+                v4f A[2][2], B[2][2];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+                for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) {
-                        const float av = A[b][e >> 2][e & 3];
-                        const float bv = B[a][e >> 2][e & 3];
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[a][b], 0, 0, 0);
+                    for (int g = 0; g < 2; ++g) {
+                        A[b][g] = *reinterpret_cast<const v4f*>(opa + buf * FSB + b * 2048 + g * 1024);
+                        B[b][g] = *reinterpret_cast<const v4f*>(opb + buf * FSB + b * 2048 + g * 1024);
                     }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int a = 0; a < 2; ++a)
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) {
+                            const float av = A[b][e >> 2][e & 3];
+                            const float bv = B[a][e >> 2][e & 3];
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[a][b], 0, 0, 0);
+                        }
+            }
+            staged = held;
+            if (held) {
+                store(buf ^ 1);              // (last read before this chunk's barrier)
+                held = more;
+                if (more) load();
+            }
         }
-        staged = held;
-        if (held) {
-            store(buf ^ 1);                  // (last read before this chunk's barrier)
-            held = more;
-            if (more) load();
+        if (live) {
+            int l = lane;                    // (C's offsets and masks are worked out here: kept
+            if (GROUPED) asm volatile("" : "+v"(l));     // over the loop they take 50 registers)
+            c_frag<2> cv;
+            load_c<2>(t, cv, l);
+            store_c<2>(t, cv, acc, l);
         }
-    }
-    if (!live) return;
-    c_frag<2> cv;
-    load_c<2>(t, cv);
-    store_c<2>(t, cv, acc);
+        t.Cs = C;
+        if (GROUPED && todo) mpc_lds_barrier();          // the buffers are rewritten
+    } while (GROUPED && todo);
 }
 
 // ---------------------------------------------------------------- FP32 x FP8 / BF16
@@ -1273,7 +1295,8 @@ __device__ __forceinline__ void syrk_16_tile(float* __restrict__ C, int64_t m, i
 }
 
 // The staged kernels by launch rank: 0-3 FP8 element pairs, 4 BF16, 5 FP16,
-// 6 FP32 x FP32, 7 FP32 x FP8 / BF16.
+// 6 FP32 x FP32, 7 FP32 x FP8 / BF16; kF32Groups: 6 with several sums.
+constexpr int kF32Groups = 9;
 template <int RANK, bool LISTED>
 __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
                                                           int k, const mpc_syrk_panels P,
@@ -1281,7 +1304,7 @@ __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__
                                                           const mpc_small* __restrict__ sm, int64_t npair,
                                                           int64_t per_xcd, const syrk_shape G,
                                                           const syrk_lists L) {
-    constexpr int kBuf = RANK < 4 ? F8B : RANK < 6 ? S16B : RANK == 6 ? FSB : SPB;
+    constexpr int kBuf = RANK < 4 ? F8B : RANK < 6 ? S16B : RANK == 7 ? SPB : FSB;
     __shared__ __align__(16) char lds[2 * kBuf];
     if (sm && sm->info != 0) return;
     auto tile = [&](int64_t pid) {
@@ -1290,14 +1313,15 @@ __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__
         else if constexpr (RANK < 6)
             syrk_16_tile<RANK == 4 ? MPC_PREC_BF16 : MPC_PREC_FP16>(C, m, ldc, k, P, row_stride, tile_rows,
                                                                     G, pid, L, lds);
-        else if constexpr (RANK == 6)
-            syrk_f32_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        else if constexpr (RANK == 6 || RANK == kF32Groups)
+            syrk_f32_tile<RANK == kF32Groups>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
         else
             syrk_split_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
     };
     if constexpr (LISTED) {
-        const int count = L.base[RANK];
-        const int* list = L.base + kListHead + (int64_t)RANK * L.cap;
+        constexpr int rank = RANK == kF32Groups ? 6 : RANK;
+        const int count = L.base[rank];
+        const int* list = L.base + kListHead + (int64_t)rank * L.cap;
         for (int it = blockIdx.x; it < count; it += gridDim.x) {
             tile(list[it]);
             mpc_lds_barrier();               // the buffers are rewritten
@@ -1463,7 +1487,8 @@ int mpc_launch_syrk_panels(hipStream_t st, float* C, int64_t m, int64_t ldc, int
     if (e5) MPC_SYRK_LAUNCH(syrk_staged_kernel, 3);
     if (class_mask & (1u << MPC_PREC_BF16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 4);
     if (class_mask & (1u << MPC_PREC_FP16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 5);
-    if (f32) MPC_SYRK_LAUNCH(syrk_staged_kernel, 6);             // FP32 x FP32
+    if (f32 && P.sum > 0 && P.np > P.sum) MPC_SYRK_LAUNCH(syrk_staged_kernel, kF32Groups);
+    else if (f32) MPC_SYRK_LAUNCH(syrk_staged_kernel, 6);        // FP32 x FP32
     if (f32s) MPC_SYRK_LAUNCH(syrk_staged_kernel, 7);            // FP32 x FP8 / BF16 (split)
     if (f32h) MPC_SYRK_LAUNCH(syrk_kernel, 2, true);             // FP32 x FP16
     MPC_LAUNCH_CHECK();

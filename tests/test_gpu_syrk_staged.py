@@ -221,3 +221,32 @@ def test_factor_group_sums(handle, n, nb, agg):
         want = 0.5 * float(np.float32(1.0 - agg * nb * b * b))
         got = T[e, rows].cpu().numpy()
         assert (got == want).all(), (group, rows, got - 0.5, want - 0.5)
+
+
+@pytest.mark.parametrize("n,nb,ladder", [(15360, 256, (L.PREC_FP32,)), (8500, 256, (L.PREC_E4M3, L.PREC_FP32)),
+                                         (15400, 256, (L.PREC_E4M3, L.PREC_FP32)),
+                                         (15500, 128, (L.PREC_E4M3, L.PREC_FP32))])
+def test_factor_fp32_sums_per_group(handle, n, nb, ladder):
+    """A switching factor that keeps every tile FP32, with a ladder that has
+    nothing else or on a matrix whose rows grow by sqrt(2) per 128 (so that no
+    tile is small beside the first pivots: the first panel's next tile has row
+    sums of squares of about a tenth of them, E4M3 takes 1/16 at this eps'), is
+    the fixed FP32 factor bit for bit: updates with several groups' panels add
+    FP32 products group by group."""
+    print("[case]", n, nb, ladder, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    G = torch.randn(n, n // 32, generator=g, device="cuda")
+    d = torch.exp2(torch.arange(n, device="cuda").div(128, rounding_mode="floor") / 2 - 30)
+    A = G @ G.T / (n // 32) + torch.eye(n, device="cuda")
+    A = torch.tril(A) + torch.tril(A, -1).T
+    A = (A * d[:, None] * d[None, :]).contiguous()
+    outs = []
+    for prec, lad in ((L.PREC_FP32, (L.PREC_FP32,)), (L.PREC_SWITCH, ladder)):
+        T = A.clone()
+        rc, _, mp, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=prec, ladder=lad,
+                                                         eps_prime=1 / 256, fallback=0), want_map=True)
+        assert rc == 0
+        low = np.tril(np.ones(tuple(mp.shape), bool), -1)
+        assert (mp.cpu().numpy().T[low] == L.PREC_FP32).all()
+        outs.append(T)
+    assert torch.equal(outs[0], outs[1])
