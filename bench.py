@@ -141,12 +141,12 @@ def main():
         log("accuracy", acc)
 
     # ---- SYRK roofline at the first-step shape (m = n - nb, k = nb), E4M3 tiles,
-    # and at the aggregated shape the factor issues (k = agg_panels * nb)
+    # and at one group's depth (k = agg_panels * nb)
     sy = syrk_roofline(h, stream, n, nb, args.syrk_reps, C0=A)
     m, k, syrk_ms, syrk_gbs, syrk_tf = sy["m"], sy["k"], sy["ms"], sy["gbs"], sy["tflops"]
     agg = args.agg if args.agg is not None else fo8.agg_panels
     sya = syrk_roofline(h, stream, n, nb, args.syrk_reps, C0=A, k=agg * nb) if agg > 1 else None
-    # the same update at K = 2048 (a depth the factor does not issue): where the
+    # the same update at K = 2048, the depth of the far updates at this size: where the
     # arithmetic intensity reaches the FP8 ridge and the matrix cores take over
     syd = syrk_roofline(h, stream, n, nb, max(2, args.syrk_reps // 4), C0=A, k=2048)
     # the streaming rate this device attains: a 1 GiB elementwise copy on the same stream
@@ -207,7 +207,7 @@ def main():
         "pcg_gbs": pcg_gbs,
         "pcg_frac_hbm": {kk: round(v / HBM_PEAK_GBS, 4) for kk, v in pcg_gbs.items()},
         "accuracy": acc,
-        "roofline": {"kernel": "syrk_kernel<E4M3> (one trailing update, m=%d k=%d)" % (m, k),
+        "roofline": {"kernel": "syrk_staged_kernel, E4M3 (one panel's trailing update, m=%d k=%d)" % (m, k),
                      "bound": "hbm", "achieved": round(syrk_gbs, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(syrk_gbs / HBM_PEAK_GBS, 4),
                      "traffic": syrk_traffic(m, k),
@@ -216,7 +216,7 @@ def main():
                      "copy_gbs": round(cpy["gbs"], 1),
                      "frac_of_copy": round(syrk_gbs / cpy["gbs"], 4)},
         "roofline_aggregated": None if sya is None else {
-            "kernel": "syrk_kernel<E4M3> (the factor's aggregated update, m=%d k=%d)"
+            "kernel": "syrk_staged_kernel, E4M3 (one group's update, m=%d k=%d)"
                       % (sya["m"], sya["k"]),
             "bound": "hbm", "achieved": round(sya["gbs"], 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(sya["gbs"] / HBM_PEAK_GBS, 4),
@@ -224,7 +224,8 @@ def main():
             "tflops": round(sya["tflops"], 1),
             "mfma_frac_fp8": round(sya["tflops"] / FP8_PEAK_TFLOPS, 4)},
         "syrk_deep": {
-            "kernel": "syrk_kernel<E4M3> (m=%d k=%d, not issued by the factor)" % (syd["m"], syd["k"]),
+            "kernel": "syrk_staged_kernel, E4M3 (a far update of eight panels, m=%d k=%d)"
+                      % (syd["m"], syd["k"]),
             "avg_ms": round(syd["ms"], 4), "gbs": round(syd["gbs"], 1),
             "hbm_frac": round(syd["gbs"] / HBM_PEAK_GBS, 4), "tflops": round(syd["tflops"], 1),
             "mfma_frac_fp8": round(syd["tflops"] / FP8_PEAK_TFLOPS, 4)},

@@ -127,9 +127,9 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
                 for (int i = 0; i < 4; ++i) v[s][i] = c + s >= r + i ? v[s][i] : T(0);
         }
     };
-    // Sums of MFL groups (128 terms) are added up apart: one running sum over
-    // the chunk loses accuracy with its length, which a residual at cond 1e8
-    // shows (n = 65536: 8192 terms a wave).
+    // Sums of MFL groups (128 terms) are added up apart: one running sum over a
+    // wave's part of the chunk (2048 terms of the longest) loses accuracy with its
+    // length, which the residual of a solve at cond 1e8 shows (n = 65536).
     v4d acc[4], tot[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = tot[i] = v4d{};
@@ -230,7 +230,8 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 
 // part[(s nj + j) nc + c] = sum_{r in chunk s} A[r][c] X[j][r] for the 32
 // columns of blockIdx.x, chunk s = blockIdx.y of rw rows (a multiple of MTG).
-// Wave w takes the chunk's row groups w, w + 4, ..
+// Wave w takes the chunk's row groups w, w + 4, .., each sum in one piece: this
+// product is part of a preconditioner with FP32 entries, never of a residual.
 __global__ __launch_bounds__(256) void mm_t_kernel(const float* __restrict__ A, int64_t lda,
                                                   int64_t m, int64_t nc, int64_t rw,
                                                   const double* __restrict__ X, int64_t ldx, int nj,

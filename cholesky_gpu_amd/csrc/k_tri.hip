@@ -24,11 +24,14 @@
 namespace {
 
 // ---------------------------------------------------------------- block inverses
-// The products of the build are FP32 operands with FP64 sums
-// (v_mfma_f64_16x16x4), rounded to FP32 once when stored: the rounding errors
-// of FP32 sums grow with the block (z of a 2048-point RBF factor is then off
-// by 1.5e-7 with Bo = 256 and 7e-7 with Bo = 2048; with FP64 sums 7e-8 for
-// every Bo).  D = a b: lane (q, k) = (lane % 16, lane / 16) supplies a[q][k] and
+// The products of the build are FP32 operands, for up to 8192 rows (and in the
+// 128-row blocks of any) with FP64 sums (v_mfma_f64_16x16x4), rounded to FP32
+// once when stored: the rounding errors of FP32 sums grow with the block (z of a
+// 2048-point RBF factor is then off by 1.5e-7 with Bo = 256 and 7e-7 with Bo =
+// 2048; with FP64 sums 7e-8 for every Bo).  Larger matrices, whose blocks had
+// 2048 rows and FP32 sums all along, keep them (see gemm_kernel): z of an FP32
+// factor at cond 1e6 is off by 1.2e-7 at n = 8192, 1.7e-7 at 8200 and 1.9e-7 at
+// 16384.  D = a b: lane (q, k) = (lane % 16, lane / 16) supplies a[q][k] and
 // b[k][q]; its register e is D[4e + k][q].
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));

@@ -325,8 +325,9 @@ int mpc_launch_symv64(hipStream_t st, const double* A, int64_t lda, int64_t n, i
 int64_t mpc_symv_partial_doubles(int64_t n, int nrhs);
 int mpc_launch_dot(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
                    const double* b, int64_t ldb, double* out, double* part);
-// out_b = a . b and out_c = a . c per column in two launches (part: twice
-// the partials of one dot); each sum in the same order as mpc_launch_dot's
+// out_b = a . b and out_c = a . c per column in the launches of one dot (one up
+// to 16384 rows, two beyond; part: twice the partials of one dot); each sum in the
+// same order as mpc_launch_dot's
 int mpc_launch_dot2(hipStream_t st, int64_t n, int nrhs, const double* a, int64_t lda_,
                     const double* b, int64_t ldb, double* out_b, const double* c, int64_t ldc,
                     double* out_c, double* part);

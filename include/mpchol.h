@@ -127,9 +127,18 @@ typedef struct {
     int    fallback;        /* 1: on a non-positive pivot restore A, divide
                                eps_prime by 16 and retry (twice), then all-FP32 */
     int    profile;         /* 1: time the phases with events (adds syncs) */
-    int    agg_panels;      /* panels whose trailing updates beyond their group
-                               of block columns are applied together
-                               (K = agg_panels * nb): 1..4, default 2 */
+    int    agg_panels;      /* panels of a group, 1..4, default 2.  Block columns
+                               beyond the group take the products of its panels
+                               together, summed before they are subtracted (K =
+                               agg_panels * nb); those inside it, panel by
+                               panel.  With 2, large factors (nb = 256: n >=
+                               8448, four groups from 15360; nb = 128: n >
+                               4096, 15360) sum two or four groups so where that
+                               saves time (K <= 8 nb), products of two FP32
+                               tiles excepted.  1 at nb = 64 and with profile.
+                               Panel buffers: up to 16 * (n + 128) * nb * 4
+                               bytes with 2 (fewer groups if they do not fit),
+                               2 * agg_panels such slots otherwise */
     int    rule;            /* MPC_RULE_* below (default MPC_RULE_MINPIVOT) */
 } mpc_factor_opts;
 /* Switching rules.  Each picks, for a panel tile L_ij (i > j) of panel j, the
