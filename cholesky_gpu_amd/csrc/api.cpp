@@ -675,9 +675,10 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     };
     // aggregated update of panels p0 .. p0+np-1 on the trailing matrix from
     // block column E (rows and columns >= E nb), tile columns [t0, t1) of
-    // 64 * qa; qa = 1 one mixed-class launch, qa = 2 one launch per class
+    // 64 * qa; qa = 1 one mixed-class launch, qa = 2 one launch per class; sum:
+    // panels in one FP32 x FP32 chain of additions (qa = 1: always one)
     auto agg = [&](int64_t p0, int np, int64_t E, int64_t t0, int64_t t1, hipStream_t us,
-                   int qa) -> int {
+                   int qa, int sum) -> int {
         const int64_t e = E * nb;
         if (e >= n || np < 1) return 0;
         mpc_syrk_panels P{};
@@ -691,7 +692,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         P.p0 = (int)(p0 % nslot);
         P.np = np;
         P.nb = nb;
-        P.sum = AG;
+        P.sum = sum;
         // (panel 0 is in the first update of every column beyond its group)
         P.csrc = (first_src && p0 == 0) ? first_src + e + e * lda : nullptr;
         return mpc_launch_syrk_panels(us, dA + e + e * lda, n - e, lda, nb, P, (int64_t)nb * 4, tr,
@@ -732,16 +733,17 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
     // schedule), with no event in between.  There the update is no longer than the
     // waits that overlapping it would take (5..10 us for each event on the chain,
     // and as much of host time).  Measured as whole factors, overlapped and on one
-    // stream: n = 4096, nb = 128 FP32 2014 and 1436 us, E4M3/FP32 2068 and 1388, nb =
-    // 256 FP32 1565 and 1376, BF16 1306 and 1226; n = 768, nb = 64 538 and 320.
+    // stream: n = 4096, nb = 128 FP32 1996 and 1445 us, E4M3/FP32 2069 and 1407, nb =
+    // 256 FP32 1562 and 1391, BF16 1297 and 1227; n = 768, nb = 64 528 and 323.
     // Beyond it the update is the longer part: the last 8192 columns of n = 16384
     // that way cost an FP32 factor 17.91 -> 18.11 ms, E4M3/FP32 8.57 -> 8.75.
+    // Here the panels of a group are added up panel by panel (sum = 1).
     constexpr int64_t kOneStream = 4096;
     // Group updates of at least kWide columns whose operands are all of one class
     // take that class's 128-row kernel (too few workgroups for the chip below: n =
-    // 4000, nb = 128 FP32 factor 1479 us without it, 1469, 1444, 1427, 1426, 1435 and
-    // 1460 from 1024, 1536, 2048, 2304, 2560 and 3072; n = 4096 BF16 1292 without it,
-    // 1247, 1240, 1236, 1238 and 1254 from 1536, 2048, 2304, 2560 and 3072).  With
+    // 4000, nb = 128 FP32 factor 1472 us without it, 1452, 1445, 1425, 1430, 1430 and
+    // 1436 from 1024, 1536, 2048, 2304, 2560 and 3072; n = 4096 BF16 1284 without it,
+    // 1251, 1241, 1239, 1239 and 1237 from 1536, 2048, 2304, 2560 and 3072).  With
     // several classes it would be a launch each.
     constexpr int64_t kWide = 2304;
     const bool one_launch = __builtin_popcount(cmask) == 1 &&
@@ -756,7 +758,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
             else if (j + 1 < E)          // the columns of the group
                 r = update(j, 0, E < nt ? (E - (j + 1)) * nb / 64 : -1, ps, 1);
             else                         // the rest, all panels of the group at once
-                r = agg(g * AG, AG, E, 0, -1, ps, wide ? 2 : 1);
+                r = agg(g * AG, AG, E, 0, -1, ps, wide ? 2 : 1, 1);
             if (r) return r;
             if ((r = panel(j + 1, ps))) return r;
             if ((r = build_w(j + 1, ps))) return r;
@@ -789,7 +791,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         // bounds those updates: after each group fstream updates the strip of
         // the group after next (the chain waits for it at the end of the next
         // group) with the panels of all groups not yet applied to it, and after
-        // every PG-th group the rest with the same panels.
+        // every PG-th group, or the last one, the rest with the same panels.
         // The next panel is enqueued before the updates on st and fstream: the
         // chain does not wait for the host to issue those, and POTRF's one
         // workgroup gets a CU before their thousands.
@@ -812,7 +814,7 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
         const int64_t gt = (int64_t)AG * nb / MPC_SYRK_TILE;      // SYRK tiles of a group
         int64_t j = 0;
         for (; j + 1 < nt; ++j) {
-            if (j % (PG * AG) == 0 && n - j * nb <= kOneStream) break;
+            if (j % AG == 0 && n - j * nb <= kOneStream) break;
             const int64_t g = j / AG, E = std::min<int64_t>((g + 1) * AG, nt);
             const int64_t bs1 = std::min<int64_t>(nb, n - (j + 1) * nb);
             const int64_t split = (bs1 + MPC_SYRK_TILE - 1) / MPC_SYRK_TILE;
@@ -837,23 +839,24 @@ static int factor_once(mpc_handle* h, float* dA, int64_t n, int64_t lda, const m
                 const int64_t p0 = g * AG;
                 const int np = (int)(j - p0 + 1);
                 if (far_pending) MPC_HIP(hipStreamWaitEvent(ps, h->ev_far, 0));
-                if ((rc = agg(p0, np, E, 0, nb / 64, ps, 1))) return rc;
+                if ((rc = agg(p0, np, E, 0, nb / 64, ps, 1, 1))) return rc;
                 MPC_HIP(hipEventRecord(h->ev_panel, ps));
                 if ((rc = panel(j + 1, ps))) return rc;
                 MPC_HIP(hipStreamWaitEvent(st, h->ev_panel, 0));
                 MPC_HIP(hipStreamWaitEvent(fs, h->ev_panel, 0));
-                if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, gt, st, 2))) return rc;
+                if ((rc = agg(p0, np, E, nb / MPC_SYRK_TILE, gt, st, 2, AG))) return rc;
                 MPC_HIP(hipEventRecord(h->ev_bulk, st));
                 bulk_seen = false;
                 const int64_t q = g % PG, pp = p0 - q * AG;    // the groups not applied yet
                 const int pn = (int)q * AG + np;
                 if (PG == 1) {
-                    if ((rc = agg(p0, np, E, gt, -1, fs, 2))) return rc;
+                    if ((rc = agg(p0, np, E, gt, -1, fs, 2, AG))) return rc;
                     MPC_HIP(hipEventRecord(h->ev_far, fs));
                 } else {
-                    if ((rc = agg(pp, pn, E, gt, 2 * gt, fs, 2))) return rc;
+                    if ((rc = agg(pp, pn, E, gt, 2 * gt, fs, 2, AG))) return rc;
                     MPC_HIP(hipEventRecord(h->ev_far, fs));
-                    if (q == PG - 1 && (rc = agg(pp, pn, E, 2 * gt, -1, fs, 2))) return rc;
+                    const bool rest = q == PG - 1 || n - E * nb <= kOneStream;   // (the loop ends)
+                    if (rest && (rc = agg(pp, pn, E, 2 * gt, -1, fs, 2, AG))) return rc;
                 }
                 far_pending = true;
             }

@@ -507,7 +507,7 @@ template <int QA, bool F32H>
 __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                           const mpc_syrk_panels& P, int64_t row_stride,
                                           int tile_rows, const syrk_shape& G, int64_t pid,
-                                          const syrk_lists& L);
+                                          const syrk_lists& L, float* sums);
 
 // The products of the P.np panels are summed in the accumulators (K = np*k)
 // and subtracted from C once.  F32H: only the pairs of FP32 and FP16 tiles (a
@@ -524,27 +524,28 @@ __global__ __launch_bounds__(256, 2) void syrk_kernel(float* __restrict__ C, int
                                                    const mpc_small* __restrict__ sm, int64_t npair,
                                                    int64_t per_xcd, const syrk_shape G,
                                                    const syrk_lists L) {
+    __shared__ float sums[QA == 1 ? 16 * 256 : 1];
     if (sm && sm->info != 0) return;
     if constexpr (LISTED) {
         const int rank = launch_rank_of(MPC_PREC_FP32, 0, 0);
         const int count = L.base[rank];
         const int* list = L.base + kListHead + (int64_t)rank * L.cap;
         for (int it = blockIdx.x; it < count; it += gridDim.x)
-            syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L);
+            syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, list[it], L, sums);
         return;
     }
     // XCD-aware remap: hardware places block b on XCD b % 8
     const int64_t b = blockIdx.x;
     const int64_t pid = (b & 7) * per_xcd + (b >> 3);
     if (pid >= npair) return;
-    syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L);
+    syrk_tile<QA, F32H>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, sums);
 }
 
 template <int QA, bool F32H>
 __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                           const mpc_syrk_panels& P, int64_t row_stride,
                                           int tile_rows, const syrk_shape& G, int64_t pid,
-                                          const syrk_lists& L) {
+                                          const syrk_lists& L, float* sums) {
     constexpr int TILE = 64 * QA;
     int64_t ti, tj;
     tile_of<TILE>(G, pid, ti, tj);
@@ -607,8 +608,20 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
     constexpr bool kPrefetchC = QA == 1;
     c_frag<QA> cv;
     if constexpr (kPrefetchC) load_c<QA>(t, cv);
+    // Each panel's sum apart (see kSumPanels below); the sum of the panels so far
+    // waits in LDS, as three workgroups per CU have no 16 registers to spare.
     for (int q = 0; q < P.np; ++q) {
         if (!((use >> q) & 1u)) continue;
+        if constexpr (QA == 1) {
+            if (q > 0) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    float* s = sums + 256 * i + threadIdx.x;
+                    *s = q > 1 ? *s + acc[0][0][i] : acc[0][0][i];
+                }
+                acc[0][0] = v16f{};
+            }
+        }
         operand_src orow, ocol;
         operands(q, orow, ocol);
         if constexpr (F32H) {
@@ -630,6 +643,12 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
             }
         }
     }
+    if constexpr (QA == 1) {
+        if (P.np > 1) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[0][0][i] += sums[256 * i + threadIdx.x];
+        }
+    }
     if constexpr (!kPrefetchC) load_c<QA>(t, cv);
     store_c<QA>(t, cv, acc);
 }
@@ -644,16 +663,24 @@ __device__ __forceinline__ void syrk_tile(float* __restrict__ C, int64_t m, int6
 // K = 256: 832 us = 80 TFLOP/s of the 157 peak).  In LDS a block of 32 rows is in operand
 // order, two groups of 16-byte elements (k 8h .. +3 and 8h + 4 .. +7 of lane
 // half h), so a wave's operand is one 1 KB read.
-// C takes the products of P.sum panels at a time, at most: the rounding errors of
-// an FP32 sum grow with its length and are all the error there is here, while in
-// the other kernels the operands' rounding is larger by orders of magnitude.
-// (GROUPED: more than one sum; the loop costs 20 registers, n = 32768 FP32 factor
-// 113.0 -> 114.8 ms.)
+// The rounding errors of an FP32 sum grow with the length of its chain of
+// additions, systematically where the products vary slowly, and are all the error
+// there is here (in the other kernels the operands' rounding is larger by orders
+// of magnitude).  So a chain covers P.sum panels:
+//   kSumGroups: C takes each chain's result (20 more registers: n = 32768 FP32
+//     factor 113.0 -> 114.8 ms, so it has an instance of its own);
+//   kSumPanels (P.sum = 1): the panels' results are added in registers and C takes
+//     the sum once.  212 registers, two workgroups a CU, for updates of up to 4096
+//     rows, which have no more.  FP32 factor of a matrix with cond 1e6, n = 4000,
+//     nb = 128, groups of 2: ||L - exact|| 1.4e-5, 1.7e-5 with one chain and with C
+//     taking every panel's (n = 4096, nb = 256: 2.6e-5, 7.7e-5 and 2.9e-5), at 1425
+//     us, 1402 and 1395.
 typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int FSK = 16;                       // K of a chunk
 constexpr int FSB = 8 * 2 * 1024;             // bytes of a buffer: 8 blocks of 2 groups
+constexpr int kSumAll = 0, kSumGroups = 1, kSumPanels = 2;
 
-template <bool GROUPED>
+template <int SUMS>
 __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, int64_t ldc, int k,
                                               const mpc_syrk_panels& P, int64_t row_stride,
                                               int tile_rows, const syrk_shape& G, int64_t pid,
@@ -728,11 +755,19 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
     };
     const char* const opa = lds + (2 * wc) * 2048 + lane * 16;
     const char* const opb = lds + (4 + 2 * wr) * 2048 + lane * 16;
-    unsigned group = (1u << (GROUPED ? P.sum : MPC_SYRK_MAXP)) - 1;
+    constexpr bool kGroups = SUMS == kSumGroups;
+    v16f tot[2][2];                          // kSumPanels: the panels before the current one
+    if constexpr (SUMS == kSumPanels) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) tot[a][b] = v16f{};
+    }
+    unsigned group = (1u << (kGroups ? P.sum : MPC_SYRK_MAXP)) - 1;
     do {
         use = todo & group;
         group <<= P.sum;
-        if (GROUPED && !use) continue;
+        if (kGroups && !use) continue;
         todo &= ~use;
         v16f acc[2][2];
 #pragma unroll
@@ -748,6 +783,7 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
         bool staged = true;                  // a chunk is in the current buffer
         bool held = more;                    // a chunk is in st
         if (more) load();
+        int left = k;                        // of the panel being multiplied
         for (int buf = 0; staged; buf ^= 1) {
             mpc_lds_barrier();
             if (live) {
@@ -771,6 +807,19 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
                         }
             }
             staged = held;
+            if constexpr (SUMS == kSumPanels) {
+                left -= FSK;
+                if (left == 0 && held) {
+                    left = k;
+#pragma unroll
+                    for (int a = 0; a < 2; ++a)
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) {
+                            tot[a][b] += acc[a][b];
+                            acc[a][b] = v16f{};
+                        }
+                }
+            }
             if (held) {
                 store(buf ^ 1);              // (last read before this chunk's barrier)
                 held = more;
@@ -778,15 +827,21 @@ __device__ __forceinline__ void syrk_f32_tile(float* __restrict__ C, int64_t m, 
             }
         }
         if (live) {
+            if constexpr (SUMS == kSumPanels) {
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) acc[a][b] += tot[a][b];
+            }
             int l = lane;                    // (C's offsets and masks are worked out here: kept
-            if (GROUPED) asm volatile("" : "+v"(l));     // over the loop they take 50 registers)
+            if (kGroups) asm volatile("" : "+v"(l));     // over the loop they take 50 registers)
             c_frag<2> cv;
             load_c<2>(t, cv, l);
             store_c<2>(t, cv, acc, l);
         }
         t.Cs = C;
-        if (GROUPED && todo) mpc_lds_barrier();          // the buffers are rewritten
-    } while (GROUPED && todo);
+        if (kGroups && todo) mpc_lds_barrier();          // the buffers are rewritten
+    } while (kGroups && todo);
 }
 
 // ---------------------------------------------------------------- FP32 x FP8 / BF16
@@ -1295,8 +1350,8 @@ __device__ __forceinline__ void syrk_16_tile(float* __restrict__ C, int64_t m, i
 }
 
 // The staged kernels by launch rank: 0-3 FP8 element pairs, 4 BF16, 5 FP16,
-// 6 FP32 x FP32, 7 FP32 x FP8 / BF16; kF32Groups: 6 with several sums.
-constexpr int kF32Groups = 9;
+// 6 FP32 x FP32, 7 FP32 x FP8 / BF16; kF32Groups, kF32Panels: 6 with other sums.
+constexpr int kF32Groups = 9, kF32Panels = 10;
 template <int RANK, bool LISTED>
 __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__ C, int64_t m, int64_t ldc,
                                                           int k, const mpc_syrk_panels P,
@@ -1313,13 +1368,14 @@ __global__ __launch_bounds__(256, 2) void syrk_staged_kernel(float* __restrict__
         else if constexpr (RANK < 6)
             syrk_16_tile<RANK == 4 ? MPC_PREC_BF16 : MPC_PREC_FP16>(C, m, ldc, k, P, row_stride, tile_rows,
                                                                     G, pid, L, lds);
-        else if constexpr (RANK == 6 || RANK == kF32Groups)
-            syrk_f32_tile<RANK == kF32Groups>(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
+        else if constexpr (RANK == 6 || RANK == kF32Groups || RANK == kF32Panels)
+            syrk_f32_tile<RANK == 6 ? kSumAll : RANK == kF32Groups ? kSumGroups : kSumPanels>(
+                C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
         else
             syrk_split_tile(C, m, ldc, k, P, row_stride, tile_rows, G, pid, L, lds);
     };
     if constexpr (LISTED) {
-        constexpr int rank = RANK == kF32Groups ? 6 : RANK;
+        constexpr int rank = RANK > 7 ? 6 : RANK;
         const int count = L.base[rank];
         const int* list = L.base + kListHead + (int64_t)rank * L.cap;
         for (int it = blockIdx.x; it < count; it += gridDim.x) {
@@ -1487,7 +1543,8 @@ int mpc_launch_syrk_panels(hipStream_t st, float* C, int64_t m, int64_t ldc, int
     if (e5) MPC_SYRK_LAUNCH(syrk_staged_kernel, 3);
     if (class_mask & (1u << MPC_PREC_BF16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 4);
     if (class_mask & (1u << MPC_PREC_FP16)) MPC_SYRK_LAUNCH(syrk_staged_kernel, 5);
-    if (f32 && P.sum > 0 && P.np > P.sum) MPC_SYRK_LAUNCH(syrk_staged_kernel, kF32Groups);
+    if (f32 && P.sum == 1 && P.np > 1) MPC_SYRK_LAUNCH(syrk_staged_kernel, kF32Panels);
+    else if (f32 && P.sum > 0 && P.np > P.sum) MPC_SYRK_LAUNCH(syrk_staged_kernel, kF32Groups);
     else if (f32) MPC_SYRK_LAUNCH(syrk_staged_kernel, 6);        // FP32 x FP32
     if (f32s) MPC_SYRK_LAUNCH(syrk_staged_kernel, 7);            // FP32 x FP8 / BF16 (split)
     if (f32h) MPC_SYRK_LAUNCH(syrk_kernel, 2, true);             // FP32 x FP16

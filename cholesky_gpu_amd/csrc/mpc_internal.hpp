@@ -267,7 +267,7 @@ struct mpc_syrk_panels {
     int64_t pstride, sstride;    // bytes between slots (prec: 1024 per slot)
     int64_t rows0;
     int slots, p0, np, nb;
-    int sum;                     // panels per FP32 x FP32 sum (0: np)
+    int sum;                     // panels per chain of FP32 x FP32 additions (0: np)
     // optional: C's values are read from csrc (same leading dimension) by
     // the first launch of the class sequence that touches a tile, and written
     // to C; later launches read C.  nullptr: C in place.

@@ -250,3 +250,34 @@ def test_factor_fp32_sums_per_group(handle, n, nb, ladder):
         assert (mp.cpu().numpy().T[low] == L.PREC_FP32).all()
         outs.append(T)
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n,nb", [(1111, 128), (1500, 256), (4000, 128), (4096, 256), (6000, 256)])
+@pytest.mark.parametrize("agg", [2, 3, 4])
+def test_factor_panel_sums(handle, n, nb, agg):
+    """Each panel's products are added apart from the other panels of the group:
+    where the group's first panel gives 1 and every product of the others is
+    2^-25, a quarter of the spacing of the floats there, one chain would stay at
+    1; apart they give 1 + (agg - 1) nb 2^-25 exactly.  The pivot beside it is 4
+    exactly when its sum is right, and halves the entries."""
+    print("[case]", n, nb, agg, flush=True)
+    last = max(k for k in range(1, 200) if k * agg * nb + nb // 2 < n)    # the last group with rows below
+    for group in {1, last}:
+        e, p = group * agg * nb, (group - 1) * agg * nb
+        T = torch.eye(n, device="cuda")
+        T[torch.arange(e, n), torch.arange(e, n)] = 8.0
+        rows = sorted({e + 1, (e + n) // 2, n - 1} - {e})
+        small = (agg - 1) * nb * 2.0 ** -25
+        T[p, e] = 1.0                            # (the tensor is the transpose)
+        T[p, rows] = 1.0
+        T[p + nb:e, e] = 2.0 ** -13
+        T[p + nb:e, rows] = 2.0 ** -12
+        T[e, e] = 5.0 + 0.5 * small
+        T[e, rows] = 2.0
+        T = torch.triu(T) + torch.triu(T, 1).T.contiguous()
+        rc, _, _, _ = S.factor(handle, T, S.factor_opts(nb=nb, update_prec=L.PREC_FP32, fallback=0,
+                                                        agg_panels=agg))
+        assert rc == 0
+        assert float(T[e, e]) == 2.0
+        got = T[e, rows].cpu().numpy()
+        assert (got == 0.5 * (1.0 - small)).all(), (group, rows, got - 0.5, -0.5 * small)
