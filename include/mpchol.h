@@ -199,7 +199,8 @@ typedef struct {
     double ms_total;
 } mpc_pcg_info;
 void mpc_pcg_opts_default(mpc_pcg_opts* o);
-/* Solves A X = B for nrhs columns.  A: FP32 n x n (full storage, only read);
+/* Solves A X = B for nrhs columns.  A: FP32 n x n (full storage, only read;
+   products with it take the upper triangle, i <= j);
    L: FP32 lower factor from mpc_factor with block size nb; B, X: FP64 n x nrhs.
    Returns 0 if all columns converged, MPC_ERR_NOT_CONVERGED otherwise. */
 int mpc_pcg(mpc_handle* h, const float* dA, int64_t lda, const float* dL, int64_t ldl,
