@@ -1,4 +1,4 @@
-// k_mrhs.hip -- products of a matrix with a block of up to 16 right-hand sides
+// k_mrhs.hip -- products of a matrix with blocks of up to 16 right-hand sides
 // (FP64 vectors, FP32 or FP64 matrix), on the FP64 matrix cores
 // (v_mfma_f64_16x16x4: exact FP32-to-FP64 operands, FP64 sums).
 //
@@ -49,7 +49,7 @@ __device__ __forceinline__ void split_range(int mode, int64_t r0, int64_t rows, 
 // part[(s nj + j) m + r] = sum_{c in chunk s} A[r][c] X[j][c] for the 64 rows of
 // blockIdx.x, chunk s = blockIdx.y of cw columns (a multiple of MG).  Wave w
 // takes the chunk's column groups w, w + 4, ..; the four waves' sums are added
-// in wave order through LDS.
+// in wave order through LDS.  blockIdx.z: 16 of the right-hand sides.
 //
 // A last row block that is not full (m >= 64) moves up to end at row m and
 // stores only its own rows: with predicated 4-byte loads its workgroups ran
@@ -70,7 +70,8 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
     int64_t cb = cs;
     if (MODE == 2 && cb < r0) cb = r0 & ~(int64_t)(MG - 1);
     if (cb >= ce) return;                        // (the sum skips this chunk)
-    const double* __restrict__ Xj = X + (int64_t)(q < nj ? q : nj - 1) * ldx;
+    const int j0 = blockIdx.z * MPC_MM_NJ;
+    const double* __restrict__ Xj = X + (int64_t)(j0 + q < nj ? j0 + q : nj - 1) * ldx;
     const int64_t r = r0 + 4 * q;
     const bool rfull = r0 + MR <= m;
     vec4 v[MU];
@@ -221,8 +222,8 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int j = wave + 4 * u;
-            if (j < nj)
-                part[((int64_t)blockIdx.y * nj + j) * m + r0 + lane] =
+            if (j0 + j < nj)
+                part[((int64_t)blockIdx.y * nj + j0 + j) * m + r0 + lane] =
                     ((red[0][j][lane] + red[1][j][lane]) + red[2][j][lane]) + red[3][j][lane];
         }
     }
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(256) void mm_n_kernel(const T* __restrict__ A, int6
 
 // part[(s nj + j) nc + c] = sum_{r in chunk s} A[r][c] X[j][r] for the 32
 // columns of blockIdx.x, chunk s = blockIdx.y of rw rows (a multiple of MTG).
-// Wave w takes the chunk's row groups w, w + 4, .., each sum in one piece: this
+// Wave w takes the chunk's row groups w, w + 4, .. (blockIdx.z as above), each sum in one piece: this
 // product is part of a preconditioner with FP32 entries, never of a residual.
 __global__ __launch_bounds__(256) void mm_t_kernel(const float* __restrict__ A, int64_t lda,
                                                   int64_t m, int64_t nc, int64_t rw,
@@ -242,7 +243,8 @@ __global__ __launch_bounds__(256) void mm_t_kernel(const float* __restrict__ A, 
     const int q = lane & 15, k = lane >> 4;
     const int64_t c0 = (int64_t)blockIdx.x * MTC, rs = (int64_t)blockIdx.y * rw;
     const int64_t re = rs + rw < m ? rs + rw : m;
-    const double* __restrict__ Xj = X + (int64_t)(q < nj ? q : nj - 1) * ldx;
+    const int j0 = blockIdx.z * MPC_MM_NJ;
+    const double* __restrict__ Xj = X + (int64_t)(j0 + q < nj ? j0 + q : nj - 1) * ldx;
     const float* __restrict__ col[2];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
@@ -315,8 +317,8 @@ __global__ __launch_bounds__(256) void mm_t_kernel(const float* __restrict__ A, 
     if (c0 + c < nc) {
 #pragma unroll
         for (int j = tid >> 5; j < MPC_MM_NJ; j += 8)
-            if (j < nj)
-                part[((int64_t)blockIdx.y * nj + j) * nc + c0 + c] =
+            if (j0 + j < nj)
+                part[((int64_t)blockIdx.y * nj + j0 + j) * nc + c0 + c] =
                     ((red[0][j][c] + red[1][j][c]) + red[2][j][c]) + red[3][j][c];
     }
 }
@@ -350,12 +352,12 @@ inline int64_t chunk(int64_t kc, int64_t S, int64_t unit) { return cdiv(cdiv(kc,
 template <typename T>
 int launch_mm_n(hipStream_t st, const T* A, int64_t lda, int64_t m, int64_t kc, int mode,
                 const double* X, int64_t ldx, int nj, double* part, int64_t S) {
-    if (nj < 1 || nj > MPC_MM_NJ || S < 1) {
+    if (nj < 1 || S < 1) {
         mpc_set_error("mm_n: %d right-hand sides, %lld chunks", nj, (long long)S);
         return MPC_ERR_ARG;
     }
     const int64_t cw = chunk(kc, S, MG);
-    const dim3 g((unsigned)cdiv(m, MR), (unsigned)cdiv(kc, cw)), b(256);
+    const dim3 g((unsigned)cdiv(m, MR), (unsigned)cdiv(kc, cw), (unsigned)cdiv(nj, MPC_MM_NJ)), b(256);
     if (mode == 1) hipLaunchKernelGGL((mm_n_kernel<T, 1>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     else if (mode == 2) hipLaunchKernelGGL((mm_n_kernel<T, 2>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
     else if (mode == 3) hipLaunchKernelGGL((mm_n_kernel<T, 3>), g, b, 0, st, A, lda, m, kc, cw, X, ldx, nj, part);
@@ -393,13 +395,14 @@ int mpc_launch_mm_n(hipStream_t st, const double* A, int64_t lda, int64_t m, int
 
 int mpc_launch_mm_t(hipStream_t st, const float* A, int64_t lda, int64_t m, int64_t nc,
                     const double* X, int64_t ldx, int nj, double* part, int64_t S) {
-    if (nj < 1 || nj > MPC_MM_NJ || S < 1) {
+    if (nj < 1 || S < 1) {
         mpc_set_error("mm_t: %d right-hand sides, %lld chunks", nj, (long long)S);
         return MPC_ERR_ARG;
     }
     const int64_t rw = chunk(m, S, MTG);
-    hipLaunchKernelGGL(mm_t_kernel, dim3((unsigned)cdiv(nc, MTC), (unsigned)cdiv(m, rw)), dim3(256), 0,
-                       st, A, lda, m, nc, rw, X, ldx, nj, part);
+    hipLaunchKernelGGL(mm_t_kernel,
+                       dim3((unsigned)cdiv(nc, MTC), (unsigned)cdiv(m, rw), (unsigned)cdiv(nj, MPC_MM_NJ)), dim3(256), 0, st,
+                       A, lda, m, nc, rw, X, ldx, nj, part);
     MPC_LAUNCH_CHECK();
     return 0;
 }

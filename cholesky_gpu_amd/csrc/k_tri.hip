@@ -519,6 +519,7 @@ __global__ __launch_bounds__(256) void gemv_sum_kernel(const double* __restrict_
 // 256-row piece outside the triangle replaced by its neighbour) times v from
 // LDS.  bI = 2048, one right-hand side 5.3 us, four 7.0 (two outputs a wave 6.0
 // and 7.6; 64 x 64 tiles over rows of M and a launch to add them up 10 and 15).
+// blockIdx.y: NJ of the right-hand sides.
 template <bool UPPER, int NJ>
 __global__ __launch_bounds__(256, 2) void tri_dot_kernel(const float* __restrict__ Mt, int ld, int bI,
                                                         const double* __restrict__ V, int64_t ldv,
@@ -531,6 +532,9 @@ __global__ __launch_bounds__(256, 2) void tri_dot_kernel(const float* __restrict
     const int klo = UPPER ? kd : 0, khi = UPPER ? (bI - 1) >> 8 : kd;
     v4f m[NK];
     const float* col = Mt + (int64_t)(r < bI ? r : bI - 1) * ld;
+    V += (int64_t)blockIdx.y * NJ * ldv;
+    out += (int64_t)blockIdx.y * NJ * ldo;
+    nj -= blockIdx.y * NJ;
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
         const int c = 256 * (k < klo ? klo : k > khi ? khi : k) + 4 * lane;
@@ -704,7 +708,7 @@ int mpc_build_block_inverses(hipStream_t st, const float* L, int64_t ldl, int64_
 
 static int tri_dot(hipStream_t st, const float* Mt, int Bo, int bI, bool upper, const double* V,
                    int64_t ldv, int nj, double* out, int64_t ldo) {
-    const dim3 g(cdiv(bI, 4)), b(256);
+    const dim3 g(cdiv(bI, 4), cdiv(nj, NR)), b(256);
 #define MPC_TRI_DOT(U, J) \
     hipLaunchKernelGGL((tri_dot_kernel<U, J>), g, b, 0, st, Mt, Bo, bI, V, ldv, nj, out, ldo)
     if (upper) {
@@ -740,9 +744,18 @@ static int bwd_gemv(hipStream_t st, const float* L, int64_t ldl, int64_t p0, int
     return 0;
 }
 
-// right-hand sides of the next pass over the factor: at most NR in the GEMV
-// kernels above, else at most MPC_MM_NJ on the matrix cores
-static int sweep_pass(int nrhs) { return nrhs > NR ? std::min(nrhs, MPC_MM_NJ) : nrhs; }
+// Right-hand sides of the next pass over the factor: at most NR in the GEMV
+// kernels above, on the matrix cores as many as kPass keeps the partial sums
+// small for (40 MB at most).  A pass for every MPC_MM_NJ of them repeats a stage's
+// launches and leaves the chip idle between them (applications with 33 columns, us,
+// in passes of 16 and in one: n = 128 65 and 37, 2049 163 and 99, 6200 426 and 303,
+// 16000 1313 and 1059).
+constexpr int kPass = 64;
+// Up to kDotRows rows (one block, no product beside it) the triangles of any number
+// of right-hand sides go by column dots, two launches instead of four: n = 65, 16
+// columns, 30 us and 40; 200, 64 columns 34 and 39; 300 39 and 40; 1000 68 and 52.
+constexpr int64_t kDotRows = 256;
+static int sweep_pass(int nrhs) { return std::min(nrhs, kPass); }
 
 // Chunks of the products with a big block's rows: two workgroups a CU (2048
 // rows, 16 right-hand sides: the triangle 7.2 us, 9.7 with three or four; 2048 /
@@ -762,7 +775,7 @@ static int64_t mm_chunks(int Bo, int64_t kc) {
 int64_t mpc_block_prec_partial_doubles(int64_t n, int Bo, int nrhs) {
     const int64_t gemv = (1 + (n + FW_CW - 1) / FW_CW) * Bo * std::min(nrhs, NR);
     if (nrhs <= NR) return gemv;
-    return std::max(gemv, (mm_chunks(Bo, n) + mm_chunks(Bo, Bo) + 1) * Bo * std::min(nrhs, MPC_MM_NJ));
+    return std::max(gemv, (mm_chunks(Bo, n) + mm_chunks(Bo, Bo) + 1) * Bo * sweep_pass(nrhs));
 }
 
 // One stage on the matrix cores: v = R_I - (sum of the S chunks of the off-
@@ -792,7 +805,7 @@ int mpc_apply_block_prec(hipStream_t st, const float* L, int64_t ldl, int64_t n,
     int rc;
     for (int j0 = 0, nj; j0 < nrhs; j0 += nj, R += nj * ld, Y += nj * ld, Z += nj * ld) {
         nj = sweep_pass(nrhs - j0);
-        const bool mm = nj > NR;
+        const bool mm = nj > NR && n > kDotRows;
         double* v = part + (mm ? mm_chunks(Bo, Bo) * Bo * nj : 0);
         double* gpart = v + (int64_t)Bo * nj;
         for (int64_t I = 0; I < nI; ++I) {

@@ -297,8 +297,9 @@ int mpc_launch_syrk_classes(hipStream_t st, float* C, int64_t m, int64_t ldc, in
 // compute classes / FP8 element formats that a factor configuration can produce
 void mpc_syrk_masks(int update_prec, const int* ladder, int n_ladder, unsigned* class_mask,
                     unsigned* fp8_mask);
-// k_mrhs.hip: products with up to MPC_MM_NJ right-hand sides X (nj columns,
-// ld ldx), as partial sums over S column (row) chunks, and their sum
+// k_mrhs.hip: products with right-hand sides X (nj columns, ld ldx; the matrix is
+// read once for every MPC_MM_NJ of them), as partial sums over S column (row)
+// chunks, and their sum
 constexpr int MPC_MM_NJ = 16;
 constexpr int MPC_MM_GROUP_N = 16, MPC_MM_GROUP_T = 64;      // chunk granularity of mm_n, mm_t
 int64_t mpc_mm_splits(int64_t rows, int64_t kc, int64_t wgs);   // chunks of mm_n

@@ -105,3 +105,11 @@ def test_product_reads_upper_triangle(handle, n, nrhs, dtype):
     res = [f(handle, M.contiguous(), eye, B, nb=64, X=X.clone(),
              opts=S.pcg_opts(x0_mode=2, maxit=0))[1].relres for M in (A, half)]
     assert res[0] == res[1], res
+
+
+@pytest.mark.parametrize("n", [63, 256, 257, 2100, 4500])
+@pytest.mark.parametrize("nrhs", [6, 33, 64, 65, 70])
+def test_apply_precond_many(handle, n, nrhs):
+    """More right-hand sides than one product takes and than one pass takes, by
+    column dots (up to 256 rows) and on the matrix cores.  Tolerance as above."""
+    test_apply_precond_blocks(handle, n, nrhs)
